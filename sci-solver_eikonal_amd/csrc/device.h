@@ -84,6 +84,15 @@ struct DeviceState {
   size_t lds_bytes = 0;         // a visit with its records staged (when rec_lds)
   size_t lds_bytes_direct = 0;  // a visit reading its records from memory
   int32_t queue_cap = 0;
+  // the visits that keep a block's element data in registers (k_visit_resident): items or
+  // elements per thread (0: the blocks do not fit), threads, LDS strides and bytes, and for
+  // triangles the items (resident.h, TriItems)
+  int32_t res_n = 0, res_bt = 0;
+  int32_t max_local = 0, max_elem = 0;
+  size_t res_lds = 0;
+  int2* item_range = nullptr;
+  uint32_t* item_id = nullptr;
+  float4* item_len = nullptr;
   bool has_result = false;
   // split element records of the multi-solve visits that read them from memory (ensure_split)
   void* esel = nullptr;

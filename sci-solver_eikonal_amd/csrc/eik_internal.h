@@ -72,6 +72,10 @@ struct Layout {
   std::vector<uint64_t> vmask;
   int32_t max_dep = 0;
   int32_t max_local = 0, max_own = 0, max_elem = 0;
+  // per block: its (element, corner) pairs that a visit may update (owned corners, and of a
+  // virtual face only the obtuse one)
+  std::vector<int32_t> items;
+  int32_t max_items = 0;
   int64_t total_elems = 0;
   bool valid = false;
 };

@@ -210,6 +210,7 @@ int build_layout(Mesh& m) {
   });
   L.blocks.resize(nb);
   if (m.dim == 3) L.tets.resize(total); else L.tris.resize(total);
+  L.items.assign(nb, 0);
   L.rec_elem.resize(total);
   for (int64_t q = 0; q < total; ++q)
     L.rec_elem[q] = (int32_t)(elist[q] < m.ne ? elist[q] : m.vorigin[elist[q] - m.ne]);
@@ -247,6 +248,7 @@ int build_layout(Mesh& m) {
         bad[b] = 1;
         break;
       }
+      for (int j = 0; j < (e < m.ne ? k : 1); ++j) L.items[b] += lv[j] < d.nown;
       const float* Le = &eL[(size_t)e * nl];
       const float* He = &eH[(size_t)e * k];
       if (m.dim == 3) {
@@ -289,6 +291,7 @@ int build_layout(Mesh& m) {
       L.max_local = std::max(L.max_local, d.nown + d.nhalo);
       L.max_own = std::max(L.max_own, d.nown);
       L.max_elem = std::max(L.max_elem, d.nelem);
+      L.max_items = std::max(L.max_items, L.items[b]);
     }
   }
 

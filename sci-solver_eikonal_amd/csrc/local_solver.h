@@ -156,21 +156,34 @@ __device__ __noinline__ float face_cost_fp64(float a1, float a2, float L1, float
   return v < double(EIK_INF) ? (float)v : EIK_INF;
 }
 
+// What a corner solve does with its ill-conditioned pieces: kMixed evaluates them in fp64 (calls);
+// kReport leaves them out and sets *ill, for callers that solve such a corner again with kMixed
+// out of line, so that the common path holds no call (whose register convention costs the calling
+// kernel a third of its resident waves).
+enum IllPieces { kMixed, kReport };
+
 // fp32 face with the fp64 fallback; inputs already scaled (trace of the 2x2 Gram = 1 is not
 // needed for the face: the 2x2 adjugate entries are products of two lengths).
-__device__ __forceinline__ float face_cost_mixed(float a1, float a2, float L1, float L2, float L12) {
+template <IllPieces MODE = kMixed>
+__device__ __forceinline__ float face_cost_mixed(float a1, float a2, float L1, float L2, float L12,
+                                                 bool* ill = nullptr) {
   const float g12 = 0.5f * (L1 + L2 - L12);
   const float det = fma_(L1, L2, -g12 * g12);
-  if (det < kCondFp64 * L1 * L2) return face_cost_fp64(a1, a2, L1, L2, L12);
+  if constexpr (MODE == kReport) {
+    *ill = *ill || det < kCondFp64 * L1 * L2;
+  } else {
+    if (det < kCondFp64 * L1 * L2) return face_cost_fp64(a1, a2, L1, L2, L12);
+  }
   return face_cost<float>(a1, a2, L1, L2, L12);
 }
 
 // Target D of a tet from corners 1..3.  L1..L3 = |X_i - D|^2, L12, L13, L23 = |X_i - X_j|^2.
 // Unknown corners (t >= large) are left out, as the reference's candidates through them are
 // never the minimum.  Returns +inf when no corner is known.
+template <IllPieces MODE = kMixed>
 __device__ __forceinline__ float tet_corner_solve(float t1, float t2, float t3, float L1, float L2,
                                                   float L3, float L12, float L13, float L23,
-                                                  float large) {
+                                                  float large, bool* ill_out = nullptr) {
   const bool k1 = t1 < large, k2 = t2 < large, k3 = t3 < large;
   const float t0 = __builtin_fminf(t1, __builtin_fminf(t2, t3));
   // unit-trace scaling
@@ -183,13 +196,17 @@ __device__ __forceinline__ float tet_corner_solve(float t1, float t2, float t3, 
   if (k1 && k2 && k3) {
     bool ill;
     float v = interior_cost<float>(b1, b2, b3, n1, n2, n3, n12, n13, n23, kCondFp64, &ill);
-    if (ill) v = interior_cost_fp64(b1, b2, b3, n1, n2, n3, n12, n13, n23);
+    if constexpr (MODE == kReport) {
+      if (ill) *ill_out = true;
+    } else {
+      if (ill) v = interior_cost_fp64(b1, b2, b3, n1, n2, n3, n12, n13, n23);
+    }
     if (v < EIK_INF) return t0 + v * sq;  // a causal interior point is the minimum
   }
   float best = EIK_INF;
-  if (k1 && k2) best = __builtin_fminf(best, face_cost_mixed(b1, b2, n1, n2, n12));
-  if (k1 && k3) best = __builtin_fminf(best, face_cost_mixed(b1, b3, n1, n3, n13));
-  if (k2 && k3) best = __builtin_fminf(best, face_cost_mixed(b2, b3, n2, n3, n23));
+  if (k1 && k2) best = __builtin_fminf(best, face_cost_mixed<MODE>(b1, b2, n1, n2, n12, ill_out));
+  if (k1 && k3) best = __builtin_fminf(best, face_cost_mixed<MODE>(b1, b3, n1, n3, n13, ill_out));
+  if (k2 && k3) best = __builtin_fminf(best, face_cost_mixed<MODE>(b2, b3, n2, n3, n23, ill_out));
   if (k1) best = __builtin_fminf(best, b1 + sqrt_(n1));
   if (k2) best = __builtin_fminf(best, b2 + sqrt_(n2));
   if (k3) best = __builtin_fminf(best, b3 + sqrt_(n3));
@@ -197,8 +214,9 @@ __device__ __forceinline__ float tet_corner_solve(float t1, float t2, float t3, 
 }
 
 // Target Z of a triangle from X1, X2.  L1 = |X1 - Z|^2, L2 = |X2 - Z|^2, L12 = |X1 - X2|^2.
+template <IllPieces MODE = kMixed>
 __device__ __forceinline__ float tri_corner_solve(float t1, float t2, float L1, float L2, float L12,
-                                                  float large) {
+                                                  float large, bool* ill = nullptr) {
   const bool k1 = t1 < large, k2 = t2 < large;
   const float t0 = k1 && k2 ? __builtin_fminf(t1, t2) : (k1 ? t1 : t2);
   const float tr = L1 + L2;
@@ -208,7 +226,7 @@ __device__ __forceinline__ float tri_corner_solve(float t1, float t2, float L1, 
   const float b1 = (t1 - t0) * isq, b2 = (t2 - t0) * isq;
   float best = EIK_INF;
   if (k1 && k2) {
-    best = face_cost_mixed(b1, b2, n1, n2, n12);
+    best = face_cost_mixed<MODE>(b1, b2, n1, n2, n12, ill);
     if (best < EIK_INF) return t0 + best * sq;
   }
   if (k1) best = __builtin_fminf(best, b1 + sqrt_(n1));
@@ -220,9 +238,10 @@ __device__ __forceinline__ float tri_corner_solve(float t1, float t2, float L1, 
 // {01,02,03,12,13,23}.  The other corners are taken in increasing order; the inputs are
 // permuted with selects on scalar values so that every lane runs the same solver code whatever
 // its corner (no divergent switch, no runtime-indexed arrays, which would live in scratch).
+template <IllPieces MODE = kMixed>
 __device__ __forceinline__ float tet_rotation(int c, float t0, float t1, float t2, float t3,
                                               float L0, float L1, float L2, float L3, float L4,
-                                              float L5, float large) {
+                                              float L5, float large, bool* ill = nullptr) {
   const bool c0 = c == 0, c1 = c == 1, c2 = c == 2, le1 = c <= 1, le2 = c <= 2;
   float a1 = c0 ? t1 : t0;
   float a2 = le1 ? t2 : t1;
@@ -233,7 +252,18 @@ __device__ __forceinline__ float tet_rotation(int c, float t0, float t1, float t
   float E12 = c0 ? L3 : (c1 ? L1 : L0);
   float E13 = c0 ? L4 : (le2 ? L2 : L1);
   float E23 = le1 ? L5 : (c2 ? L4 : L3);
-  return tet_corner_solve(a1, a2, a3, D1, D2, D3, E12, E13, E23, large);
+  return tet_corner_solve<MODE>(a1, a2, a3, D1, D2, D3, E12, E13, E23, large, ill);
+}
+
+// The same solves with their ill-conditioned pieces in fp64, out of line (see kReport).
+__device__ __noinline__ float tet_rotation_wide(int c, float t0, float t1, float t2, float t3,
+                                                float L0, float L1, float L2, float L3, float L4,
+                                                float L5, float large) {
+  return tet_rotation(c, t0, t1, t2, t3, L0, L1, L2, L3, L4, L5, large);
+}
+__device__ __noinline__ float tri_corner_solve_wide(float t1, float t2, float L1, float L2,
+                                                    float L12, float large) {
+  return tri_corner_solve(t1, t2, L1, L2, L12, large);
 }
 
 // Corner c (0..2) of a triangle with times t0..t2 and squared edge lengths L0..L2 = {01,12,20}.

@@ -1,0 +1,255 @@
+// resident.h -- block visits that keep a block's element data in registers (device code).
+//
+// A persistent workgroup visits the same block several times in a row (a re-run is five of six
+// visits of the 64^3 cube), and a visit of a 64-vertex block is a chain of short phases, each a
+// few LDS round trips long, not a volume of work.  So what a sweep reads is placed for the
+// shortest chain:
+//   * triangles: one (target, two others) item per updatable corner, rotated once when the block
+//     is loaded, N items per thread in registers with the times they were last solved with.  A
+//     sweep is three LDS reads per item, the test, the solve in place and an LDS minimum: one
+//     barrier, no work-item queue, no records in LDS.
+//   * tets: N elements per thread in registers for the selection (corner slots, heights, the
+//     corner times last seen), four LDS reads per element; the selected (element, corner) pairs
+//     go through the LDS queue, since a sweep solves one in fifteen of them, and only what the
+//     solve reads (corner slots, lengths: 32 bytes) is staged in LDS.
+// Freshness is per item: it is solved again only if one of the *other* corners fell since its last
+// evaluation by this visit's workgroup (across visits: since the `seen` times).
+#pragma once
+
+#include "fim_kernels.h"
+
+namespace eik {
+
+// Items of the triangle blocks: block b's items are [start, start + count) of the arrays.
+// id: slots of the two other corners and the target, 10 bits each (a | b << 10 | target << 20);
+// len: {|a - target|^2, |b - target|^2, |a - b|^2, height of the target}.
+struct TriItems {
+  const int2* range;
+  const uint32_t* id;
+  const float4* len;
+};
+constexpr int kItemSlotBits = 10;
+constexpr int kItemSlots = 1 << kItemSlotBits;  // local vertices of a block with items
+
+// A time that has fallen since `last`, by more than eps relative (eps = 0: at all).
+__device__ __forceinline__ bool fell(float last, float now, float eps) {
+  return last - now > eps * now;
+}
+
+template <int N>
+struct TriRegs {
+  uint32_t id[N];
+  float la[N], lb[N], lab[N], h[N];
+  float pa[N], pb[N];  // times of the two other corners at the last evaluation
+};
+
+template <int N, int BT>
+__device__ __forceinline__ void tri_load(TriRegs<N>& r, const TriItems& t, int2 range) {
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int i = u * BT + (int)threadIdx.x;
+    const bool in = i < range.y;
+    r.id[u] = in ? t.id[range.x + i] : 0u;
+    const float4 l = in ? t.len[range.x + i] : make_float4(1.f, 1.f, 1.f, EIK_INF);
+    r.la[u] = l.x;
+    r.lb[u] = l.y;
+    r.lab[u] = l.z;
+    r.h[u] = l.w;
+  }
+}
+
+__device__ __forceinline__ int slot_a(uint32_t id) { return id & (kItemSlots - 1); }
+__device__ __forceinline__ int slot_b(uint32_t id) { return (id >> kItemSlotBits) & (kItemSlots - 1); }
+__device__ __forceinline__ int slot_t(uint32_t id) { return id >> (2 * kItemSlotBits); }
+
+template <int N>
+__device__ __forceinline__ void tri_seen(TriRegs<N>& r, const float* sP) {
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    r.pa[u] = sP[slot_a(r.id[u])];
+    r.pb[u] = sP[slot_b(r.id[u])];
+  }
+}
+
+// One sweep over the thread's items.  Returns whether it lowered a time.
+template <int N>
+__device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large, float eps,
+                                          unsigned& solves) {
+  float ta[N], tb[N], tk[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    ta[u] = sT[slot_a(r.id[u])];
+    tb[u] = sT[slot_b(r.id[u])];
+    tk[u] = sT[slot_t(r.id[u])];
+  }
+  bool changed = false;
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    if (!(fell(r.pa[u], ta[u], eps) || fell(r.pb[u], tb[u], eps))) continue;
+    r.pa[u] = ta[u];
+    r.pb[u] = tb[u];
+    // nothing below the smaller time plus the height; unknown times are `large`, and no time
+    // is above that
+    if (!(tk[u] > __builtin_fminf(ta[u], tb[u]) + r.h[u])) continue;
+    ++solves;
+    bool bad = false;
+    float cand = tri_corner_solve<kReport>(ta[u], tb[u], r.la[u], r.lb[u], r.lab[u], large, &bad);
+    if (bad) cand = tri_corner_solve_wide(ta[u], tb[u], r.la[u], r.lb[u], r.lab[u], large);
+    cand = __builtin_fmaxf(cand, 0.f);
+    if (cand < tk[u]) {
+      atomicMin(reinterpret_cast<unsigned*>(&sT[slot_t(r.id[u])]), __float_as_uint(cand));
+      changed |= fell(tk[u], cand, eps);
+    }
+  }
+  return changed;
+}
+
+template <int N>
+struct TetRegs {
+  uint32_t v01[N], v23[N];     // corner slots, 16 bits each
+  float h0[N], h1[N], h2[N], h3[N];  // heights; +inf: the corner is not owned
+  float p0[N], p1[N], p2[N], p3[N];  // corner times at the last selection
+};
+
+// Loads the thread's records: slots and heights to registers, slots and lengths to LDS.
+template <int N, int BT>
+__device__ __forceinline__ void tet_load(TetRegs<N>& r, const void* recs, const BlockDesc& d,
+                                         uint4* sA, uint4* sB) {
+  const uint4* p = reinterpret_cast<const uint4*>(recs) + 3 * (int64_t)d.estart;
+  uint4 q0[N], q1[N], q2[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int e = u * BT + (int)threadIdx.x;
+    const int k = 3 * (e < d.nelem ? e : 0);
+    q0[u] = p[k];
+    q1[u] = p[k + 1];
+    q2[u] = p[k + 2];
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int e = u * BT + (int)threadIdx.x;
+    const bool in = e < d.nelem;
+    if (in) {
+      sA[e] = q0[u];
+      sB[e] = q1[u];
+    }
+    const unsigned n = in ? (unsigned)d.nown : 0u;
+    r.v01[u] = q0[u].x;
+    r.v23[u] = q0[u].y;
+    r.h0[u] = (q0[u].x & 0xffffu) < n ? __uint_as_float(q2[u].x) : EIK_INF;
+    r.h1[u] = (q0[u].x >> 16) < n ? __uint_as_float(q2[u].y) : EIK_INF;
+    r.h2[u] = (q0[u].y & 0xffffu) < n ? __uint_as_float(q2[u].z) : EIK_INF;
+    r.h3[u] = (q0[u].y >> 16) < n ? __uint_as_float(q2[u].w) : EIK_INF;
+  }
+}
+
+template <int N>
+__device__ __forceinline__ void tet_seen(TetRegs<N>& r, const float* sP) {
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    r.p0[u] = sP[r.v01[u] & 0xffffu];
+    r.p1[u] = sP[r.v01[u] >> 16];
+    r.p2[u] = sP[r.v23[u] & 0xffffu];
+    r.p3[u] = sP[r.v23[u] >> 16];
+  }
+}
+
+// Inclusive sum over the lanes of a wave, in six DPP steps.
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return x;
+}
+
+// Bitwise or over the lanes of a wave (valid in lane 63).
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+  int x = (int)v;
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return (uint32_t)x;
+}
+
+// Appends the (element, corner) pairs of the thread's elements that can improve to the queue.
+template <int N, int BT>
+__device__ __forceinline__ void tet_select(TetRegs<N>& r, const float* sT, float eps, uint16_t* sQ,
+                                           int* qn) {
+  float t0[N], t1[N], t2[N], t3[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    t0[u] = sT[r.v01[u] & 0xffffu];
+    t1[u] = sT[r.v01[u] >> 16];
+    t2[u] = sT[r.v23[u] & 0xffffu];
+    t3[u] = sT[r.v23[u] >> 16];
+  }
+  unsigned sel = 0;
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const bool f0 = fell(r.p0[u], t0[u], eps), f1 = fell(r.p1[u], t1[u], eps);
+    const bool f2 = fell(r.p2[u], t2[u], eps), f3 = fell(r.p3[u], t3[u], eps);
+    if (!(f0 || f1 || f2 || f3)) continue;
+    r.p0[u] = t0[u];
+    r.p1[u] = t1[u];
+    r.p2[u] = t2[u];
+    r.p3[u] = t3[u];
+    const float m01 = __builtin_fminf(t0[u], t1[u]), m23 = __builtin_fminf(t2[u], t3[u]);
+    const float mn0 = __builtin_fminf(t1[u], m23), mn1 = __builtin_fminf(t0[u], m23);
+    const float mn2 = __builtin_fminf(m01, t3[u]), mn3 = __builtin_fminf(m01, t2[u]);
+    unsigned s = (t0[u] > mn0 + r.h0[u] ? 1u : 0u) | (t1[u] > mn1 + r.h1[u] ? 2u : 0u) |
+                 (t2[u] > mn2 + r.h2[u] ? 4u : 0u) | (t3[u] > mn3 + r.h3[u] ? 8u : 0u);
+    // one corner alone changed: it has no new solve itself
+    const unsigned f = (f0 ? 1u : 0u) | (f1 ? 2u : 0u) | (f2 ? 4u : 0u) | (f3 ? 8u : 0u);
+    if ((f & (f - 1u)) == 0u) s &= ~f;
+    sel |= s << (4 * u);
+  }
+  if (__ballot(sel != 0u) == 0ull) return;
+  const int n = __popc(sel);
+  const int end = wave_scan(n);
+  int base = 0;
+  if (__lane_id() == 63) base = atomicAdd(qn, end);
+  base = __builtin_amdgcn_readlane(base, 63);
+  for (int q = base + end - n; sel; ++q, sel &= sel - 1u) {
+    const int k = __ffs(sel) - 1;
+    sQ[q] = (uint16_t)((((k >> 2) * BT + (int)threadIdx.x) << 2) | (k & 3));
+  }
+}
+
+// Solves the queued pairs.  Returns whether the thread lowered a time.
+template <int BT>
+__device__ __forceinline__ bool tet_solve(const uint4* sA, const uint4* sB, const uint16_t* sQ, int nq,
+                                          float* sT, float large, float eps, unsigned& solves) {
+  bool changed = false;
+  for (int q = threadIdx.x; q < nq; q += BT) {
+    const int item = (int)sQ[q];
+    const int k = item & 3;
+    const uint4 a = sA[item >> 2], b = sB[item >> 2];
+    const int v0 = a.x & 0xffffu, v1 = a.x >> 16, v2 = a.y & 0xffffu, v3 = a.y >> 16;
+    const float t0 = sT[v0], t1 = sT[v1], t2 = sT[v2], t3 = sT[v3];
+    const float tk = k == 0 ? t0 : k == 1 ? t1 : k == 2 ? t2 : t3;
+    const int vk = k == 0 ? v0 : k == 1 ? v1 : k == 2 ? v2 : v3;
+    ++solves;
+    bool ill = false;
+    float cand = tet_rotation<kReport>(k, t0, t1, t2, t3, __uint_as_float(a.z), __uint_as_float(a.w),
+                                       __uint_as_float(b.x), __uint_as_float(b.y),
+                                       __uint_as_float(b.z), __uint_as_float(b.w), large, &ill);
+    if (ill)
+      cand = tet_rotation_wide(k, t0, t1, t2, t3, __uint_as_float(a.z), __uint_as_float(a.w),
+                               __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z),
+                               __uint_as_float(b.w), large);
+    cand = __builtin_fmaxf(cand, 0.f);
+    if (cand < tk) {
+      atomicMin(reinterpret_cast<unsigned*>(&sT[vk]), __float_as_uint(cand));
+      changed |= fell(tk, cand, eps);
+    }
+  }
+  return changed;
+}
+
+}  // namespace eik

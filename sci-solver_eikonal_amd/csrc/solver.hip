@@ -7,9 +7,11 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "device.h"
+#include "resident.h"
 
 namespace eik {
 
@@ -19,7 +21,8 @@ static int dev_free(DeviceState* d) {
   void* ptrs[] = {d->esel, d->elen, d->rec_elem, d->vmask, d->vh_start, d->vh_pos, d->seen, d->blocks, d->elems,  d->halo,  d->iperm,   d->sup_start, d->sup,
                   d->dep_start, d->dep, d->owner, d->T,      d->out,      d->chg,
                   d->self,   d->list[0], d->list[1], d->count, d->counters, d->sync_acc, d->seeds,
-                  d->seedvals, d->queue, d->qflag, d->bstate, d->qctl};
+                  d->seedvals, d->queue, d->qflag, d->bstate, d->qctl,
+                  d->item_range, d->item_id, d->item_len};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (d->h_seed) (void)hipHostFree(d->h_seed);
@@ -416,6 +419,289 @@ __global__ __launch_bounds__(kBlockThreads) void k_visit_async(AsyncArgs a) {
     atomicAdd(&a.counters[threadIdx.x], sAcc[threadIdx.x]);
 }
 
+struct ResidentArgs {
+  AsyncArgs a;
+  TriItems items;      // triangles
+  int32_t max_local;   // LDS strides: local vertices and elements of the largest block
+  int32_t max_elem;
+};
+
+// The persistent kernel over blocks whose element data fits the workgroup's registers
+// (resident.h): N items or elements per thread.  Same queue, claims and visit policy as
+// k_visit_async; a workgroup that visits a block again keeps its registers and LDS, and only the
+// halo times are read again.
+// What bounds it: a chain of short phases per visit (a sweep of two to seven hundred dependent
+// instructions per wave and the device round trips that hand its result on), on fronts too small
+// to fill the chip.  Whole solves against the staged records and LDS queue of k_visit_async: level-5
+// icosphere (10,242 vertices) 0.349 -> 0.197 ms, level-7 anisotropic icosphere 1.191 -> 0.734,
+// 32^2 square 0.247 -> 0.176, 16^3 cube 0.350 -> 0.276, 33^3 tensor cube 0.463 -> 0.326, 64^3 cube
+// 1.222 -> 0.968 ms.  Held to 128 VGPRs so that four workgroups fit a CU.
+template <int DIM, int N, int BT>
+__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_resident(ResidentArgs ra) {
+  const AsyncArgs& a = ra.a;
+  extern __shared__ uint4 lds4[];
+  __shared__ int sFlag[3];      // a sweep's "a time fell", in a ring over the sweeps
+  __shared__ int sQn[2];        // work-item counters of alternate sweeps (tets)
+  __shared__ unsigned sMark[2]; // dependents whose halo holds a vertex lowered since the last push
+  __shared__ int sBlock;
+  __shared__ int sAgain;
+  __shared__ int sNext;  // block taken while the previous visit queued its dependents, or -2
+  __shared__ unsigned sPend;  // pending count returned by this workgroup's last push
+  __shared__ unsigned long long sAcc[kNumCounters];
+  const int tid = threadIdx.x;
+  uint4* sA = lds4;
+  uint4* sB = sA + (DIM == 3 ? ra.max_elem : 0);
+  float* sT = reinterpret_cast<float*>(sB + (DIM == 3 ? ra.max_elem : 0));
+  float* sP = sT + ra.max_local;
+  int* sHidx = reinterpret_cast<int*>(sP + ra.max_local);
+  uint16_t* sQ = reinterpret_cast<uint16_t*>(sHidx + ra.max_local);
+  const float large = a.v.large, eps = a.v.eps;
+  if (tid < kNumCounters) sAcc[tid] = 0;
+  if (tid < 3) sFlag[tid] = 0;
+  if (tid < 2) sQn[tid] = 0;
+  if (tid < 2) sMark[tid] = 0;
+  if (tid == 0) {
+    sNext = -2;
+    sPend = 0;
+  }
+  int ring = 0;  // sweeps run so far, modulo 3
+  int qc = 0;
+  uint64_t solves = 0;
+  for (;;) {
+    if (tid == 0) {
+      int nb = sNext;
+      if (nb == -2) {
+        const unsigned long long w0 = wall_clock64();
+        nb = q_take(a);
+        sAcc[6] += wall_clock64() - w0;
+        if (nb == kAbandoned) sAcc[kCntAbandoned] += 1;
+      }
+      sBlock = nb;
+      sNext = -2;
+    }
+    __syncthreads();
+    const int b = __builtin_amdgcn_readfirstlane(sBlock);
+    if (b < 0) break;
+    unsigned long long t0 = wall_clock64();
+    // the block's state: one owned vertex per thread, its items or elements in registers
+    const BlockDesc d = a.v.blocks[b];
+    float* seen = a.v.seen + d.vstart + d.hstart;
+    float own = 0.f;      // the owned vertex's time as last published
+    float own_last = 0.f; // ... at the start of the last sweep
+    uint64_t vm = 0;
+    int32_t dep = 0;
+    const int32_t s0 = a.dep_start[b];
+    const int ndep = a.dep_start[b + 1] - s0;
+    std::conditional_t<DIM == 2, TriRegs<N>, TetRegs<N>> r;
+    if (tid < d.nown) {
+      own = load_T<true>(a.v.T + d.vstart + tid);
+      sP[tid] = seen[tid];
+      vm = a.v.vmask[d.vstart + tid];
+      sT[tid] = own;
+    }
+    for (int i = tid; i < d.nhalo; i += BT) {
+      const int32_t h = a.v.halo[d.hstart + i];
+      sHidx[i] = h;
+      sP[d.nown + i] = seen[d.nown + i];
+      sT[d.nown + i] = load_T<true>(a.v.T + h);
+    }
+    if (tid < ndep) dep = a.dep[s0 + tid];
+    if constexpr (DIM == 2)
+      tri_load<N, BT>(r, ra.items, ra.items.range[b]);
+    else
+      tet_load<N, BT>(r, a.v.elems, d, sA, sB);
+    __syncthreads();
+    if constexpr (DIM == 2) tri_seen<N>(r, sP);
+    else tet_seen<N>(r, sP);
+    unsigned long long t1 = wall_clock64();
+    bool rerun = false;
+    for (;;) {
+      // latency-bound regime (see kLatencyPending); sPend is written after the barrier that
+      // follows this read
+      const bool latency = sPend < kLatencyPending * gridDim.x;
+      const int inner = latency ? latency_sweeps<DIM>(a.v.max_inner) : a.v.max_inner;
+      unsigned nsolve = 0;
+      uint64_t marks = 0;  // dependents holding this thread's vertex, if it fell
+      int sweep = 0;
+      bool conv = false;
+      while (sweep < inner) {
+        bool ch = false;
+        int nq = 1;
+        if constexpr (DIM == 2) {
+          ch = tri_sweep<N>(r, sT, large, eps, nsolve);
+        } else {
+          tet_select<N, BT>(r, sT, eps, sQ, &sQn[qc]);
+          __syncthreads();
+          nq = sQn[qc];
+          if (tid == 0) sQn[qc ^ 1] = 0;
+          qc ^= 1;
+          if (nq) ch = tet_solve<BT>(sA, sB, sQ, nq, sT, large, eps, nsolve);
+        }
+        if (ch) sFlag[ring] = 1;
+        // (no pair selected: no time fell, and no thread waits for another's solve)
+        if (nq) __syncthreads();
+        const int any = nq ? sFlag[ring] : 0;
+        ring = ring == 2 ? 0 : ring + 1;
+        if (tid == 0) sFlag[ring == 2 ? 0 : ring + 1] = 0;
+        ++sweep;
+        // publish the owned times that fell
+        own_last = own;
+        if (tid < d.nown) {
+          const float v = sT[tid];
+          if (v < own) {
+            own = v;
+            (void)__hip_atomic_fetch_min(reinterpret_cast<unsigned*>(a.v.T + d.vstart + tid),
+                                         __float_as_uint(v), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+            marks |= vm;
+          }
+        }
+        if (!any) {
+          conv = true;
+          break;
+        }
+      }
+      solves += nsolve;
+      const unsigned long long t2 = wall_clock64();
+      // reduced over the wave first: the compiler turns an LDS or with a uniform address into a
+      // scalar loop over the lanes (a third of a triangle sweep)
+      if (__ballot(marks != 0ull)) {
+        const uint32_t lo = wave_or((uint32_t)marks), hi = wave_or((uint32_t)(marks >> 32));
+        if (__lane_id() == 63) {
+          if (lo) atomicOr(&sMark[0], lo);
+          if (hi) atomicOr(&sMark[1], hi);
+        }
+      }
+      // the published times have reached the device's coherence point (vmcnt covers atomics
+      // without a result) before the dependents are queued
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_s_waitcnt(0);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __syncthreads();
+      const unsigned long long tq = wall_clock64();
+      // visits beyond the bound queue nothing more (runaway guard)
+      const bool cap_ok = (int64_t)sAcc[0] < a.max_visits;
+      bool want = false;
+      if (tid < 64) {
+        const uint64_t mask = (uint64_t)sMark[0] | ((uint64_t)sMark[1] << 32);
+        want = cap_ok && tid < ndep && ((mask >> tid) & 1ull) != 0ull;
+        if (want) want = atomicExch(&a.qflag[dep], 1u) == 0u;
+        if (tid == 0)
+          sAgain = (latency && !conv && cap_ok) || (release_or_rerun(a, b) && cap_ok);
+      }
+      __syncthreads();
+      const bool again = sAgain != 0;
+      if (tid < 64) {
+        if (tid < 2) sMark[tid] = 0;
+        // an unconverged block that is left goes back to the queue
+        bool self = tid == 0 && !again && !conv && cap_ok;
+        if (self) self = atomicExch(&a.qflag[b], 1u) == 0u;
+        const uint64_t bal = __ballot(want);
+        const unsigned nself = __ballot(self) ? 1u : 0u;
+        const unsigned n = (unsigned)__popcll(bal) + nself;
+        const unsigned dec = again ? 0u : 1u;
+        if (n + dec > 0u) {
+          uint32_t base = 0;
+          if (tid == 0) {
+            // tail += n, pending += n - dec, in one 64-bit add (pending >= 1 while this visit
+            // counts, so the low word cannot borrow)
+            const unsigned long long inc = ((unsigned long long)n << 32) + n - dec;
+            const unsigned long long old = __hip_atomic_fetch_add(
+                &a.ctl->tp, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            base = (uint32_t)(old >> 32);
+            sPend = (unsigned)(old & 0xffffffffull);
+            if (n == 0u && (old & 0xffffffffull) == 1ull) q_finish(a);
+            if (self)
+              __hip_atomic_store(q_slot(a, base + n - 1u), b + 1, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+          }
+          base = __shfl(base, 0, 64);
+          if (want)
+            __hip_atomic_store(q_slot(a, base + (uint32_t)__popcll(bal & lane_mask_lt())), dep + 1,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (tid == 0) {
+          VisitResult vr;
+          vr.sweeps = sweep;
+          vr.t_load = t1 - t0;
+          vr.t_sweep = t2 - t1;
+          vr.t_wb = tq - t2;
+          tally_visit(sAcc, d, vr, 0, a.elem_bytes, tq - t0, rerun, rerun);
+          sAcc[10] += wall_clock64() - tq;
+        }
+      } else if (again) {
+        // the other waves read the halo times of the next visit
+        for (int i = tid - 64; i < d.nhalo; i += BT - 64)
+          sT[d.nown + i] = load_T<true>(a.v.T + sHidx[i]);
+      } else if (tid == 64) {
+        // the next block is taken while wave 0 queues the dependents: this visit is over, so the
+        // workgroup holds no work that the wait for a ticket could depend on
+        const unsigned long long w0 = wall_clock64();
+        const int32_t nx = q_take(a);
+        sNext = nx;
+        sAcc[6] += wall_clock64() - w0;
+        if (nx == kAbandoned) sAcc[kCntAbandoned] += 1;
+      }
+      if (!again) {
+        // what this visit evaluated the block's elements with: every time, but for the owned
+        // vertices that fell in the last sweep of a visit cut off by the sweep cap.  A later
+        // visit that misses these (they are plain stores) evaluates more than it has to.
+        if (tid < d.nown) seen[tid] = conv ? own : own_last;
+        for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = sT[d.nown + i];
+      }
+      __syncthreads();
+      if (!again) break;
+      rerun = true;
+      t0 = t1 = wall_clock64();
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) solves += __shfl_down(solves, off, 64);
+  if (__lane_id() == 0 && solves) atomicAdd(&sAcc[3], (unsigned long long)solves);
+  __syncthreads();
+  if (tid < kNumCounters && sAcc[tid]) atomicAdd(&a.counters[tid], sAcc[tid]);
+}
+
+// The items of every triangle block (TriItems) from its records: one workgroup per block, items in
+// record order.  mask: the record's updatable corners; corners not owned have no item.
+__global__ __launch_bounds__(256) void k_tri_items(const BlockDesc* blocks, const uint4* recs,
+                                                   const int2* range, uint32_t* id, float4* len) {
+  __shared__ int sWave[4];
+  const BlockDesc d = blocks[blockIdx.x];
+  int at = range[blockIdx.x].x;
+  for (int e0 = 0; e0 < d.nelem; e0 += 256) {
+    const int e = e0 + (int)threadIdx.x;
+    const Elem x = load_elem<2>(recs, d.estart + (e < d.nelem ? e : 0));
+    unsigned m = e < d.nelem ? x.mask & 7u : 0u;
+    if (x.v0 >= d.nown) m &= ~1u;
+    if (x.v1 >= d.nown) m &= ~2u;
+    if (x.v2 >= d.nown) m &= ~4u;
+    const int n = __popc(m), end = wave_scan(n);
+    if (__lane_id() == 63) sWave[threadIdx.x >> 6] = end;
+    __syncthreads();
+    int q = at + end - n, total = 0;
+    for (int w = 0; w < 4; ++w) {
+      if (w < (int)(threadIdx.x >> 6)) q += sWave[w];
+      total += sWave[w];
+    }
+    // the corner order and lengths of tri_rotation
+    if (m & 1u) {
+      id[q] = x.v1 | (x.v2 << kItemSlotBits) | ((uint32_t)x.v0 << (2 * kItemSlotBits));
+      len[q++] = make_float4(x.L0, x.L2, x.L1, x.H0);
+    }
+    if (m & 2u) {
+      id[q] = x.v0 | (x.v2 << kItemSlotBits) | ((uint32_t)x.v1 << (2 * kItemSlotBits));
+      len[q++] = make_float4(x.L0, x.L1, x.L2, x.H1);
+    }
+    if (m & 4u) {
+      id[q] = x.v0 | (x.v1 << kItemSlotBits) | ((uint32_t)x.v2 << (2 * kItemSlotBits));
+      len[q++] = make_float4(x.L2, x.L1, x.L0, x.H2);
+    }
+    at += total;
+    __syncthreads();
+  }
+}
+
 // T_out[caller id] = T[new id]
 __global__ void k_gather(const float* T, const int32_t* iperm, int64_t nv, float* out) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -455,6 +741,8 @@ size_t visit_lds_bytes(const Layout& L, int dim, int32_t queue_cap, size_t rec_b
          sizeof(uint16_t) * (((size_t)queue_cap + 1) & ~(size_t)1) +
          sizeof(int32_t) * std::max<size_t>(L.max_dep, 2);
 }
+
+static int setup_resident(Mesh& m, size_t max_lds);
 
 int upload_layout(Mesh& m) {
   int rc = ensure_stream(m);
@@ -547,7 +835,61 @@ int upload_layout(Mesh& m) {
   HIP_TRY(hipMalloc((void**)&d->counters, sizeof(unsigned long long) * kNumCounters));
   HIP_TRY(hipMalloc((void**)&d->sync_acc, sizeof(unsigned long long) * kSyncSlots * kSyncSlotWords));
   HIP_TRY(hipStreamSynchronize(s));
+  rc = setup_resident(m, (size_t)max_lds);
+  if (rc) return rc;
   m.device_dirty = false;
+  return EIK_OK;
+}
+
+// The shape of the register-resident visits for this layout, and the triangle items.  A block
+// qualifies when one thread can hold each owned vertex and N x BT items (triangles) or elements
+// (tets) cover it; N and BT grow with the largest block.
+static int setup_resident(Mesh& m, size_t max_lds) {
+  DeviceState* d = m.dev;
+  const Layout& L = m.layout;
+  d->max_local = L.max_local;
+  d->max_elem = L.max_elem;
+  d->res_n = 0;
+  if (L.vmask.empty()) return EIK_OK;
+  const int32_t need = m.dim == 3 ? L.max_elem : L.max_items;
+  if (m.dim == 2 && need <= 2 * 256) d->res_n = 2, d->res_bt = 256;
+  else if (need <= 4 * 256) d->res_n = 4, d->res_bt = 256;
+  else if (need <= 4 * 512) d->res_n = 4, d->res_bt = 512;
+  if (d->res_n == 0 || L.max_own > d->res_bt || (m.dim == 2 && L.max_local > kItemSlots)) {
+    d->res_n = 0;
+    return EIK_OK;
+  }
+  d->res_lds = sizeof(float) * 3 * (size_t)L.max_local;
+  if (m.dim == 3)
+    d->res_lds += 2 * sizeof(uint4) * (size_t)L.max_elem + sizeof(uint16_t) * (size_t)L.max_items;
+  if (d->res_lds > max_lds) {
+    d->res_n = 0;
+    return EIK_OK;
+  }
+  if (d->res_lds > 65536)
+    HIP_TRY(hipFuncSetAttribute(
+        d->res_bt == 256 ? (const void*)k_visit_resident<3, 4, 256>
+                         : (const void*)k_visit_resident<3, 4, 512>,
+        hipFuncAttributeMaxDynamicSharedMemorySize, (int)d->res_lds));
+  if (m.dim == 3) return EIK_OK;
+  std::vector<int2> range(L.nblocks);
+  int64_t n = 0;
+  for (int32_t b = 0; b < L.nblocks; ++b) {
+    range[b] = make_int2((int)n, L.items[b]);
+    n += L.items[b];
+  }
+  if (n >= INT32_MAX) {
+    d->res_n = 0;
+    return EIK_OK;
+  }
+  int rc = upload(&d->item_range, range, d->stream);
+  if (rc) return rc;
+  HIP_TRY(hipMalloc((void**)&d->item_id, sizeof(uint32_t) * std::max<int64_t>(n, 1)));
+  HIP_TRY(hipMalloc((void**)&d->item_len, sizeof(float4) * std::max<int64_t>(n, 1)));
+  hipLaunchKernelGGL(k_tri_items, dim3(L.nblocks), dim3(256), 0, d->stream, d->blocks,
+                     (const uint4*)d->elems, d->item_range, d->item_id, d->item_len);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(d->stream));  // the host copy of the ranges has been read
   return EIK_OK;
 }
 
@@ -652,6 +994,39 @@ static int solve_sync(Mesh& m, const eik_solve_opts_t& o, eik_solve_stats_t& st)
   return EIK_OK;
 }
 
+// The visit kernel of the persistent single solve.
+struct VisitKernel {
+  const void* fn;
+  int threads;
+  size_t lds;
+  bool resident;
+};
+
+// Register-resident visits where the blocks fit them, unless the records are to be read from
+// memory; else the general kernel, its records staged in LDS where they fit.
+static VisitKernel visit_kernel(const DeviceState* d, int32_t stage_records) {
+  VisitKernel k;
+  if (d->res_n && stage_records != EIK_STAGE_MEMORY) {
+    k.resident = true;
+    k.threads = d->res_bt;
+    k.lds = d->res_lds;
+    if (d->dim == 3)
+      k.fn = d->res_bt == 256 ? (const void*)k_visit_resident<3, 4, 256>
+                              : (const void*)k_visit_resident<3, 4, 512>;
+    else
+      k.fn = d->res_n == 2      ? (const void*)k_visit_resident<2, 2, 256>
+             : d->res_bt == 256 ? (const void*)k_visit_resident<2, 4, 256>
+                                : (const void*)k_visit_resident<2, 4, 512>;
+    return k;
+  }
+  const bool stage = d->rec_lds && stage_records != EIK_STAGE_MEMORY;
+  k.resident = false;
+  k.threads = kBlockThreads;
+  k.lds = stage ? d->lds_bytes : d->lds_bytes_direct;
+  k.fn = d->dim == 3 ? (const void*)k_visit_async<3> : (const void*)k_visit_async<2>;
+  return k;
+}
+
 // Workgroups of the single-solve persistent kernel.  A workgroup for every queued block mostly
 // visits blocks whose suppliers are still changing, which only makes more visits, while too few
 // workgroups leave the fronts' blocks waiting; the grid is sized to the fronts.  Triangle
@@ -664,15 +1039,12 @@ static int solve_sync(Mesh& m, const eik_solve_opts_t& o, eik_solve_stats_t& st)
 // blocks; five workgroups per front block measured best over cubes with one source: 32^3
 // 0.59 -> 0.47 ms, 16^3 and 24^3 about 10% faster, from 48^3 on (the 64^3 cube included) every
 // workgroup that fits (64^3: 1.17 ms at 768, 1.31 at 640, 1.59 at 512).  At least one per CU.
-static int persistent_grid(int dim, size_t lds, int requested, int64_t nblocks, int64_t nseeds,
-                           int* out) {
+static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t nblocks,
+                           int64_t nseeds, int* out) {
   int dev = 0, ncu = 0, per_cu = 0;
   HIP_TRY(hipGetDevice(&dev));
   HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  if (dim == 3)
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_visit_async<3>, kBlockThreads, lds));
-  else
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_visit_async<2>, kBlockThreads, lds));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, k.threads, k.lds));
   int resident = std::max(1, ncu * std::max(per_cu, 1));
   resident = std::min(resident, 64 * ncu);
   if (requested > 0) {
@@ -766,13 +1138,25 @@ static AsyncArgs async_args(const Mesh& m, const eik_solve_opts_t& o, const Asyn
   return a;
 }
 
+static int launch_visits(const DeviceState* d, const VisitKernel& k, const AsyncArgs& a, int grid,
+                         hipStream_t s) {
+  ResidentArgs ra;
+  ra.a = a;
+  ra.items = {d->item_range, d->item_id, d->item_len};
+  ra.max_local = d->max_local;
+  ra.max_elem = d->max_elem;
+  void* args[] = {k.resident ? (void*)&ra : (void*)&a};
+  HIP_TRY(hipLaunchKernel(k.fn, dim3(grid), dim3(k.threads), args, k.lds, s));
+  return EIK_OK;
+}
+
 static int solve_async(Mesh& m, const eik_solve_opts_t& o, int64_t nseeds, eik_solve_stats_t& st) {
   DeviceState* d = m.dev;
   hipStream_t s = d->stream;
   int rc0 = ensure_queue(d);
   if (rc0) return rc0;
   const bool stage = d->rec_lds && o.stage_records != EIK_STAGE_MEMORY;
-  const size_t lds = stage ? d->lds_bytes : d->lds_bytes_direct;
+  const VisitKernel vk = visit_kernel(d, o.stage_records);
   const AsyncBufs bufs = {d->T,     d->seen,   d->queue, d->qflag, d->bstate,
                           reinterpret_cast<QueueCtl*>(d->qctl), d->counters, (uint32_t)d->qcap};
   const AsyncArgs a = async_args(m, o, bufs, stage);
@@ -782,14 +1166,10 @@ static int solve_async(Mesh& m, const eik_solve_opts_t& o, int64_t nseeds, eik_s
                      d->iperm, d->owner, m.nv);
   HIP_TRY(hipGetLastError());
   int grid = 0;
-  int rc = persistent_grid(m.dim, lds, o.workgroups, d->nblocks, nseeds, &grid);
+  int rc = persistent_grid(m.dim, vk, o.workgroups, d->nblocks, nseeds, &grid);
   if (rc) return rc;
   HIP_TRY(hipEventRecord(d->evA, s));
-  if (m.dim == 3)
-    hipLaunchKernelGGL(k_visit_async<3>, dim3(grid), dim3(kBlockThreads), lds, s, a);
-  else
-    hipLaunchKernelGGL(k_visit_async<2>, dim3(grid), dim3(kBlockThreads), lds, s, a);
-  HIP_TRY(hipGetLastError());
+  if ((rc = launch_visits(d, vk, a, grid, s))) return rc;
   HIP_TRY(hipEventRecord(d->evB, s));
   HIP_TRY(hipStreamSynchronize(s));
   float vms = 0.f;
@@ -1096,7 +1476,7 @@ int eik_solve_noalloc(eik_mesh_t h, const int32_t* seeds_dev, int64_t nseeds, fl
   eik_solve_opts_t o;
   eik_solve_opts_default(&o);
   const bool stage = d->rec_lds != 0;
-  const size_t lds = stage ? d->lds_bytes : d->lds_bytes_direct;
+  const VisitKernel vk = visit_kernel(d, o.stage_records);
   const float large = m->dim == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
   // the array keeps the previous call's contents: everything the solve reads first is reset,
   // with a fill kernel (no memset nodes if the caller captures this into a graph)
@@ -1119,11 +1499,8 @@ int eik_solve_noalloc(eik_mesh_t h, const int32_t* seeds_dev, int64_t nseeds, fl
   hipLaunchKernelGGL(k_async_seed, seed_grid(nseeds), dim3(64), 0, s, a, seeds_dev, nseeds,
                      d->iperm, d->owner, m->nv);
   int grid = 0;
-  if ((rc = persistent_grid(m->dim, lds, 0, d->nblocks, nseeds, &grid))) return rc;
-  if (m->dim == 3)
-    hipLaunchKernelGGL(k_visit_async<3>, dim3(grid), dim3(kBlockThreads), lds, s, a);
-  else
-    hipLaunchKernelGGL(k_visit_async<2>, dim3(grid), dim3(kBlockThreads), lds, s, a);
+  if ((rc = persistent_grid(m->dim, vk, 0, d->nblocks, nseeds, &grid))) return rc;
+  if ((rc = launch_visits(d, vk, a, grid, s))) return rc;
   hipLaunchKernelGGL(k_gather, dim3(grid1d(m->nv, 256)), dim3(256), 0, s, b.T, d->iperm, m->nv,
                      T_out_dev);
   HIP_TRY(hipGetLastError());
