@@ -74,12 +74,10 @@ struct DeviceState {
   // (2 * seed_cap words) on the way in, the counters on the way out
   int32_t* h_seed = nullptr;
   unsigned long long* h_cnt = nullptr;
-  // async scheduler
-  int32_t* queue = nullptr;
-  uint32_t* qflag = nullptr;
-  uint32_t* bstate = nullptr;
-  void* qctl = nullptr;  // QueueCtl
-  int32_t qcap = 0;
+  float* h_out = nullptr;  // behind h_cnt: a small mesh's times (kSmallOut)
+  // persistent scheduler (block_sched.h): block words and control words
+  unsigned long long* words = nullptr;
+  unsigned char* sctl = nullptr;
   int32_t max_workgroups = 0;
   size_t lds_bytes = 0;         // a visit with its records staged (when rec_lds)
   size_t lds_bytes_direct = 0;  // a visit reading its records from memory

@@ -43,11 +43,20 @@ struct TriRegs {
   float pa[N], pb[N];  // times of the two other corners at the last evaluation
 };
 
+// The thread index, opaque: what is computed from it is computed where it is used, not hoisted out of
+// the loop over the blocks and spilled (a reload waits for every load issued before it).
+__device__ __forceinline__ int this_thread() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 template <int N, int BT>
 __device__ __forceinline__ void tri_load(TriRegs<N>& r, const TriItems& t, int2 range) {
+  const int tid = this_thread();
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    const int i = u * BT + (int)threadIdx.x;
+    const int i = u * BT + tid;
     const bool in = i < range.y;
     r.id[u] = in ? t.id[range.x + i] : 0u;
     const float4 l = in ? t.len[range.x + i] : make_float4(1.f, 1.f, 1.f, EIK_INF);
@@ -76,6 +85,12 @@ template <int N>
 __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large, float eps,
                                           unsigned& solves) {
   float ta[N], tb[N], tk[N];
+  // What a solve computes from the lengths alone stays in registers from sweep to sweep where there
+  // is room (N = 2); for more items it would be spilled, so it is computed again.
+  if constexpr (N > 2) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) asm volatile("" : "+v"(r.la[u]), "+v"(r.lb[u]), "+v"(r.lab[u]));
+  }
 #pragma unroll
   for (int u = 0; u < N; ++u) {
     ta[u] = sT[slot_a(r.id[u])];
@@ -94,7 +109,8 @@ __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large,
     ++solves;
     bool bad = false;
     float cand = tri_corner_solve<kReport>(ta[u], tb[u], r.la[u], r.lb[u], r.lab[u], large, &bad);
-    if (bad) cand = tri_corner_solve_wide(ta[u], tb[u], r.la[u], r.lb[u], r.lab[u], large);
+    if (__builtin_expect(bad, 0))
+      cand = tri_corner_solve_wide(ta[u], tb[u], r.la[u], r.lb[u], r.lab[u], large);
     cand = __builtin_fmaxf(cand, 0.f);
     if (cand < tk[u]) {
       atomicMin(reinterpret_cast<unsigned*>(&sT[slot_t(r.id[u])]), __float_as_uint(cand));
@@ -111,35 +127,45 @@ struct TetRegs {
   float p0[N], p1[N], p2[N], p3[N];  // corner times at the last selection
 };
 
+// Copies 16 bytes per lane from memory straight to LDS (lane i of the wave to base + 16 i), so that
+// no register holds them on the way.
+__device__ __forceinline__ void copy_to_lds(const uint4* from, uint4* wave_base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                   (__attribute__((address_space(3))) void*)wave_base, 16, 0, 0);
+}
+
 // Loads the thread's records: slots and heights to registers, slots and lengths to LDS.
 template <int N, int BT>
 __device__ __forceinline__ void tet_load(TetRegs<N>& r, const void* recs, const BlockDesc& d,
                                          uint4* sA, uint4* sB) {
   const uint4* p = reinterpret_cast<const uint4*>(recs) + 3 * (int64_t)d.estart;
-  uint4 q0[N], q1[N], q2[N];
+  const int tid = this_thread();
+  const int wave = __builtin_amdgcn_readfirstlane(tid & ~63);
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    const int e = u * BT + (int)threadIdx.x;
-    const int k = 3 * (e < d.nelem ? e : 0);
-    q0[u] = p[k];
-    q1[u] = p[k + 1];
-    q2[u] = p[k + 2];
+    const int e = u * BT + tid;
+    const bool in = e < d.nelem;
+    const uint4* q = p + 3 * (in ? e : 0);
+    if (in) {
+      copy_to_lds(q, sA + u * BT + wave);
+      copy_to_lds(q + 1, sB + u * BT + wave);
+    }
+    const uint2 v = *reinterpret_cast<const uint2*>(q);
+    const uint4 h = q[2];
+    r.v01[u] = v.x;
+    r.v23[u] = v.y;
+    r.h0[u] = __uint_as_float(h.x);
+    r.h1[u] = __uint_as_float(h.y);
+    r.h2[u] = __uint_as_float(h.z);
+    r.h3[u] = __uint_as_float(h.w);
   }
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    const int e = u * BT + (int)threadIdx.x;
-    const bool in = e < d.nelem;
-    if (in) {
-      sA[e] = q0[u];
-      sB[e] = q1[u];
-    }
-    const unsigned n = in ? (unsigned)d.nown : 0u;
-    r.v01[u] = q0[u].x;
-    r.v23[u] = q0[u].y;
-    r.h0[u] = (q0[u].x & 0xffffu) < n ? __uint_as_float(q2[u].x) : EIK_INF;
-    r.h1[u] = (q0[u].x >> 16) < n ? __uint_as_float(q2[u].y) : EIK_INF;
-    r.h2[u] = (q0[u].y & 0xffffu) < n ? __uint_as_float(q2[u].z) : EIK_INF;
-    r.h3[u] = (q0[u].y >> 16) < n ? __uint_as_float(q2[u].w) : EIK_INF;
+    const unsigned n = u * BT + tid < d.nelem ? (unsigned)d.nown : 0u;
+    r.h0[u] = (r.v01[u] & 0xffffu) < n ? r.h0[u] : EIK_INF;
+    r.h1[u] = (r.v01[u] >> 16) < n ? r.h1[u] : EIK_INF;
+    r.h2[u] = (r.v23[u] & 0xffffu) < n ? r.h2[u] : EIK_INF;
+    r.h3[u] = (r.v23[u] >> 16) < n ? r.h3[u] : EIK_INF;
   }
 }
 
@@ -221,34 +247,78 @@ __device__ __forceinline__ void tet_select(TetRegs<N>& r, const float* sT, float
   }
 }
 
-// Solves the queued pairs.  Returns whether the thread lowered a time.
-template <int BT>
-__device__ __forceinline__ bool tet_solve(const uint4* sA, const uint4* sB, const uint16_t* sQ, int nq,
-                                          float* sT, float large, float eps, unsigned& solves) {
+struct TetItem {
+  float t0, t1, t2, t3;
+  uint4 a, b;  // slots and lengths
+  int k;
+};
+
+__device__ __forceinline__ TetItem tet_item(const uint4* sA, const uint4* sB, int item,
+                                            const float* sT) {
+  TetItem x;
+  x.k = item & 3;
+  x.a = sA[item >> 2];
+  x.b = sB[item >> 2];
+  x.t0 = sT[x.a.x & 0xffffu];
+  x.t1 = sT[x.a.x >> 16];
+  x.t2 = sT[x.a.y & 0xffffu];
+  x.t3 = sT[x.a.y >> 16];
+  return x;
+}
+
+// Lowers the target of an item to a candidate; returns whether it fell.
+__device__ __forceinline__ bool tet_lower(const TetItem& x, float cand, float* sT, float eps) {
+  const float tk = x.k == 0 ? x.t0 : x.k == 1 ? x.t1 : x.k == 2 ? x.t2 : x.t3;
+  const uint32_t pair = x.k < 2 ? x.a.x : x.a.y;
+  const int vk = (x.k & 1) ? pair >> 16 : pair & 0xffffu;
+  cand = __builtin_fmaxf(cand, 0.f);
+  if (!(cand < tk)) return false;
+  atomicMin(reinterpret_cast<unsigned*>(&sT[vk]), __float_as_uint(cand));
+  return fell(tk, cand, eps);
+}
+
+// The queued pairs of ill-conditioned tets, again, in fp64.  What the thread holds of its elements
+// goes to memory meanwhile: kept in registers across the calls, the compiler spills most of it on
+// every load of a block, whether the block has such tets or not.
+template <int N, int BT>
+__device__ __forceinline__ bool tet_solve_ill(TetRegs<N>& r, const uint4* sA, const uint4* sB,
+                                              const uint16_t* sQ, int nq, float* sT, float large,
+                                              float eps) {
+  TetRegs<N> keep = r;
+  asm volatile("" : : "v"(&keep) : "memory");  // in memory, not in registers
   bool changed = false;
   for (int q = threadIdx.x; q < nq; q += BT) {
-    const int item = (int)sQ[q];
-    const int k = item & 3;
-    const uint4 a = sA[item >> 2], b = sB[item >> 2];
-    const int v0 = a.x & 0xffffu, v1 = a.x >> 16, v2 = a.y & 0xffffu, v3 = a.y >> 16;
-    const float t0 = sT[v0], t1 = sT[v1], t2 = sT[v2], t3 = sT[v3];
-    const float tk = k == 0 ? t0 : k == 1 ? t1 : k == 2 ? t2 : t3;
-    const int vk = k == 0 ? v0 : k == 1 ? v1 : k == 2 ? v2 : v3;
-    ++solves;
-    bool ill = false;
-    float cand = tet_rotation<kReport>(k, t0, t1, t2, t3, __uint_as_float(a.z), __uint_as_float(a.w),
-                                       __uint_as_float(b.x), __uint_as_float(b.y),
-                                       __uint_as_float(b.z), __uint_as_float(b.w), large, &ill);
-    if (ill)
-      cand = tet_rotation_wide(k, t0, t1, t2, t3, __uint_as_float(a.z), __uint_as_float(a.w),
-                               __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z),
-                               __uint_as_float(b.w), large);
-    cand = __builtin_fmaxf(cand, 0.f);
-    if (cand < tk) {
-      atomicMin(reinterpret_cast<unsigned*>(&sT[vk]), __float_as_uint(cand));
-      changed |= fell(tk, cand, eps);
-    }
+    const TetItem x = tet_item(sA, sB, sQ[q], sT);
+    const float cand = tet_rotation_wide(
+        x.k, x.t0, x.t1, x.t2, x.t3, __uint_as_float(x.a.z), __uint_as_float(x.a.w),
+        __uint_as_float(x.b.x), __uint_as_float(x.b.y), __uint_as_float(x.b.z),
+        __uint_as_float(x.b.w), large);
+    changed |= tet_lower(x, cand, sT, eps);
   }
+  asm volatile("" : : "v"(&keep) : "memory");
+  r = keep;
+  return changed;
+}
+
+// Solves the queued pairs.  Returns whether the thread lowered a time.
+template <int N, int BT>
+__device__ __forceinline__ bool tet_solve(TetRegs<N>& r, const uint4* sA, const uint4* sB,
+                                          const uint16_t* sQ, int nq, float* sT, float large,
+                                          float eps, unsigned& solves) {
+  bool changed = false, ill = false;
+  for (int q = threadIdx.x; q < nq; q += BT) {
+    const TetItem x = tet_item(sA, sB, sQ[q], sT);
+    ++solves;
+    bool bad = false;
+    const float cand = tet_rotation<kReport>(
+        x.k, x.t0, x.t1, x.t2, x.t3, __uint_as_float(x.a.z), __uint_as_float(x.a.w),
+        __uint_as_float(x.b.x), __uint_as_float(x.b.y), __uint_as_float(x.b.z),
+        __uint_as_float(x.b.w), large, &bad);
+    ill |= bad;
+    if (!bad) changed |= tet_lower(x, cand, sT, eps);
+  }
+  if (__builtin_expect(__ballot(ill) != 0ull, 0))
+    changed |= tet_solve_ill<N, BT>(r, sA, sB, sQ, nq, sT, large, eps);
   return changed;
 }
 

@@ -12,8 +12,13 @@
 
 #include "device.h"
 #include "resident.h"
+#include "block_sched.h"
 
 namespace eik {
+
+// Results of up to this many vertices are copied out through pinned memory in the solve's one wait;
+// larger ones straight to the caller's memory after it.
+constexpr int64_t kSmallOut = 65536;
 
 static int dev_free(DeviceState* d) {
   if (!d) return EIK_OK;
@@ -21,7 +26,7 @@ static int dev_free(DeviceState* d) {
   void* ptrs[] = {d->esel, d->elen, d->rec_elem, d->vmask, d->vh_start, d->vh_pos, d->seen, d->blocks, d->elems,  d->halo,  d->iperm,   d->sup_start, d->sup,
                   d->dep_start, d->dep, d->owner, d->T,      d->out,      d->chg,
                   d->self,   d->list[0], d->list[1], d->count, d->counters, d->sync_acc, d->seeds,
-                  d->seedvals, d->queue, d->qflag, d->bstate, d->qctl,
+                  d->seedvals, d->words, d->sctl,
                   d->item_range, d->item_id, d->item_len};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -74,6 +79,8 @@ struct FillSegs {
   int64_t n[kMax];
   int32_t v[kMax];
   int count;
+  unsigned long long* words = nullptr;  // block words, set to clean (block_sched.h)
+  int64_t nwords = 0;
   void add(void* ptr, int64_t words, int32_t value) {
     p[count] = reinterpret_cast<int32_t*>(ptr);
     n[count] = words;
@@ -90,6 +97,16 @@ __global__ void k_fill_segs(FillSegs f) {
     const int32_t v = f.v[k];
     for (int64_t i = i0; i < f.n[k]; i += stride) p[i] = v;
   }
+  for (int64_t i = i0; i < f.nwords; i += stride) f.words[i] = kClean;
+}
+
+static unsigned fill_grid(const FillSegs& f) {
+  int64_t most = 0;
+  for (int k = 0; k < f.count; ++k) most = std::max(most, f.n[k]);
+  return (unsigned)std::min<int64_t>(grid1d(most, 256), 2048);
+}
+static void launch_fill(const FillSegs& f, hipStream_t s) {
+  hipLaunchKernelGGL(k_fill_segs, dim3(fill_grid(f)), dim3(256), 0, s, f);
 }
 
 // seeds: caller ids -> new ids; T = value; the owner block of each seed is marked changed
@@ -231,311 +248,164 @@ __global__ __launch_bounds__(kBlockThreads) void k_visit_sync(SyncArgs a) {
   block_counters(a.acc, d, r.sweeps, solves, a.elem_bytes, wall_clock64() - t0, r, &sRed);
 }
 
-struct AsyncArgs {
-  VisitArgs v;
-  size_t rec_lds_bytes;
-  int32_t* queue;     // qcap slots of kSlotStride ints: 0 = empty, else block + 1 or kDoneMark
-  uint32_t* qflag;    // per block: 1 while queued
-  uint32_t* bstate;   // per block: entries taken since its current visit began (0 = idle)
-  QueueCtl* ctl;
-  uint32_t qmask;     // qcap - 1
-  int32_t bmask;      // entries carry the block index only
-  const int32_t* dep_start;
-  const int32_t* dep;
-  unsigned long long* counters;
-  int32_t elem_bytes;  // algorithmic bytes per element (visit_algo_bytes)
-  int32_t nblocks;
-  int64_t max_visits;  // runaway guard: visits of one workgroup after which it queues nothing
-  unsigned long long wait_limit;  // wall-clock ticks a queue wait may last (q_take)
-};
-
-// initial queue: the owner block of every seed and that block's dependents, one workgroup per
-// seed (grid-stride beyond the grid) and one lane per block to queue (lane 0 the owner), so the
-// pushes' device-scope round trips overlap instead of following each other
-__global__ void k_async_seed(AsyncArgs a, const int32_t* seeds, int64_t n, const int32_t* iperm,
-                             const int32_t* owner, int64_t nv) {
-  for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
-    if (seeds[i] < 0 || seeds[i] >= nv) continue;
-    const int32_t b = owner[iperm[seeds[i]]];
-    const int32_t s0 = a.dep_start[b], nd = a.dep_start[b + 1] - s0;
-    for (int j = threadIdx.x; j <= nd; j += blockDim.x) q_push(a, j == 0 ? b : a.dep[s0 + j - 1]);
-  }
-}
-
 static dim3 seed_grid(int64_t nseeds) {
   return dim3((unsigned)std::min<int64_t>(nseeds, 1 << 16));
 }
 
-template <int DIM>
-__global__ __launch_bounds__(kBlockThreads) void k_visit_async(AsyncArgs a) {
-  extern __shared__ uint4 lds4[];
-  __shared__ int sFlag[4];
-  __shared__ int sQn[2];  // work-item counters of alternate chunks
-  __shared__ int sBlock;
-  __shared__ unsigned long long sRed;
-  __shared__ unsigned long long sAcc[kNumCounters];
-  __shared__ int sAgain;
-  __shared__ int sNext;  // block taken while the previous visit queued its dependents, or -2
-  __shared__ unsigned sPend;  // pending count returned by this workgroup's last push
-  if (threadIdx.x < kNumCounters) sAcc[threadIdx.x] = 0;
-  if (threadIdx.x == 0) {
-    sNext = -2;
-    sPend = 0;
-  }
-  for (;;) {
-    if (threadIdx.x == 0) {
-      int nb = sNext;
-      if (nb == -2) {
-        const unsigned long long w0 = wall_clock64();
-        nb = q_take(a);
-        sAcc[6] += wall_clock64() - w0;
-        if (nb == kAbandoned) sAcc[kCntAbandoned] += 1;
-      }
-      sBlock = nb;
-      sNext = -2;
-    }
-    __syncthreads();
-    const int b = sBlock;
-    if (b < 0) break;
-    bool rerun = false;      // the previous visit of this workgroup was of block b
-    bool preloaded = false;  // ... and its times for this visit are in LDS already (rerun_load)
-    do {
-      if (threadIdx.x == 0) sRed = 0;
-      const unsigned long long t0 = wall_clock64();
-      const BlockDesc d = a.v.blocks[b];
-      VisitLds l = carve_lds<DIM>(lds4, a.rec_lds_bytes, a.v.queue_cap, d);
-      uint64_t solves = 0;
-      // latency-bound regime (see kLatencyPending); sPend is only written after the barrier
-      // that follows this read
-      const bool latency = sPend < kLatencyPending * gridDim.x;
-      const int inner = latency ? latency_sweeps<DIM>(a.v.max_inner) : 0;
-      VisitResult r = visit_block<DIM, true>(a.v, b, l.rec, l.T, l.old, l.chg, l.hidx, l.vm, l.q, l.mark,
-                                             sFlag, sQn, &solves, rerun, inner, preloaded);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) solves += __shfl_down(solves, off, 64);
-      // sRed is read by thread 0 after the next barrier
-      if (__lane_id() == 0) atomicAdd(&sRed, (unsigned long long)solves);
-      const unsigned long long tq = wall_clock64();
-      // visits beyond the bound queue nothing more (runaway guard; converging solves stay far
-      // below it)
-      const bool cap_ok = (int64_t)sAcc[0] < a.max_visits;
-      // items: the dependents whose halo holds a lowered boundary vertex, then the block itself
-      // when it hit the sweep cap.  The first 64 dependents are flagged (qflag) while thread 0
-      // releases the block: whether the block runs again decides if this visit's pending count
-      // is dropped in the same atomic that queues the items, and whether the next block is
-      // taken now.  In the latency-bound regime an unconverged block is not released: this
-      // workgroup runs it again.
-      const int32_t s0 = a.dep_start[b];
-      const int ndep = r.bnd_changed && cap_ok ? a.dep_start[b + 1] - s0 : 0;
-      bool want0 = false;
-      int32_t c0 = b;
-      if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        if (lane < ndep) {
-          const uint64_t mask = a.v.vmask ? ((uint64_t)(uint32_t)l.mark[0] |
-                                             ((uint64_t)(uint32_t)l.mark[1] << 32))
-                                          : 0ull;
-          want0 = a.v.vmask ? ((mask >> lane) & 1ull) != 0ull : l.mark[lane] != 0;
-          c0 = a.dep[s0 + lane];
-          if (want0) want0 = atomicExch(&a.qflag[c0], 1u) == 0u;
-        }
-        if (lane == 0)
-          sAgain = (latency && !r.converged && cap_ok) || (release_or_rerun(a, b) && cap_ok);
-      }
-      __syncthreads();
-      const int again = sAgain;
-      if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        const uint64_t mask = a.v.vmask ? ((uint64_t)(uint32_t)l.mark[0] |
-                                           ((uint64_t)(uint32_t)l.mark[1] << 32))
-                                        : 0ull;
-        const int nitems = ndep + 1;
-        for (int j0 = 0; j0 < nitems; j0 += 64) {
-          const int j = j0 + lane;
-          bool want = false;
-          int32_t c = b;
-          if (j0 == 0 && j < ndep) {
-            want = want0;
-            c = c0;
-          } else {
-            if (j < ndep) {
-              want = a.v.vmask ? ((mask >> j) & 1ull) != 0ull : l.mark[j] != 0;
-              c = a.dep[s0 + j];
-            } else if (j == ndep) {
-              want = !r.converged && !again && cap_ok;  // a re-run continues the block anyway
-            }
-            if (want) want = atomicExch(&a.qflag[c], 1u) == 0u;
-          }
-          const uint64_t bal = __ballot(want);
-          const unsigned n = (unsigned)__popcll(bal);
-          const unsigned dec = (j0 + 64 >= nitems && !again) ? 1u : 0u;
-          if (n == 0u && dec == 0u) continue;
-          uint32_t base = 0;
-          if (lane == 0) {
-            // tail += n, pending += n - dec, in one 64-bit add (pending >= 1 while this visit
-            // counts, so the low word cannot borrow)
-            const unsigned long long inc = ((unsigned long long)n << 32) + n - dec;
-            const unsigned long long old = __hip_atomic_fetch_add(
-                &a.ctl->tp, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            base = (uint32_t)(old >> 32);
-            sPend = (unsigned)(old & 0xffffffffull);
-            if (n == 0u && (old & 0xffffffffull) == 1ull) q_finish(a);
-          }
-          base = __shfl(base, 0, 64);
-          if (want)
-            __hip_atomic_store(q_slot(a, base + (uint32_t)__popcll(bal & lane_mask_lt())), c + 1,
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (lane == 0) {
-          tally_visit(sAcc, d, r, sRed, a.elem_bytes, tq - t0, rerun, rerun && a.v.rec_lds);
-          sAcc[10] += wall_clock64() - tq;
-        }
-        if (again) {
-          // the re-run starts with clear dependent marks (they have all been read above)
-          if (a.v.vmask) {
-            if (lane < 2) l.mark[lane] = 0;
-          } else if (a.v.vh_start) {
-            for (int i = lane; i < a.dep_start[b + 1] - s0; i += 64) l.mark[i] = 0;
-          }
-        }
-      } else if (again) {
-        // the other waves prepare the re-run while wave 0 queues the dependents
-        rerun_load<true, kBlockThreads>(a.v, d, r.sweeps, l.T, l.old, l.chg, l.hidx, sFlag, 64);
-      } else if (threadIdx.x == 64) {
-        // the next block is taken while wave 0 queues the dependents: this visit is over (no
-        // re-run), so the workgroup holds no work that the wait for a ticket could depend on
-        const unsigned long long w0 = wall_clock64();
-        const int32_t nx = q_take(a);
-        sNext = nx;
-        sAcc[6] += wall_clock64() - w0;
-        if (nx == kAbandoned) sAcc[kCntAbandoned] += 1;
-      }
-      __syncthreads();
-      rerun = true;
-      preloaded = again;
-    } while (sAgain);
-  }
-  if (threadIdx.x < kNumCounters && sAcc[threadIdx.x])
-    atomicAdd(&a.counters[threadIdx.x], sAcc[threadIdx.x]);
-}
-
-struct ResidentArgs {
-  AsyncArgs a;
+struct SolveArgs {
+  VisitArgs v;
+  Sched s;
   TriItems items;      // triangles
+  const int32_t* dep_start;
+  const int32_t* dep;
+  const int32_t* iperm;
+  float* out;          // the times in caller order, written when the solve has ended (or null)
+  int64_t nv;
+  unsigned long long* counters;
+  int64_t max_visits;  // runaway guard: visits of one workgroup after which it marks nothing
+  int32_t elem_bytes;  // algorithmic bytes per element (visit_algo_bytes)
   int32_t max_local;   // LDS strides: local vertices and elements of the largest block
   int32_t max_elem;
+  size_t rec_lds_bytes;  // k_visit_general: staged records
 };
 
+// After the end of the solve (block == kNoWork: every visit has ended and every published time has
+// landed), the launch's workgroups write the times in caller order.
+__device__ __forceinline__ void write_out(const SolveArgs& a, int block) {
+  if (!a.out || block != kNoWork) return;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.nv; i += stride)
+    a.out[i] = load_T<true>(a.v.T + a.iperm[i]);
+}
+
+// Blocks seen waiting when a tet block is claimed from which on its visit runs up to max_inner sweeps:
+// while work waits, a block is loaded for more than one sweep (96^3 cube with 16 sources, 1 sweep
+// always / 1 / 8 / 16 waiting blocks: 1.66 / 1.52 / 1.52 / 1.57 ms); while workgroups wait for work,
+// one sweep, whose times reach the dependents sooner.
+constexpr int kCrowd = 8;
+
+// One whole wave: the next block, with the time spent looking in the workgroup's tally.
+__device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned long long* acc) {
+  const unsigned long long w0 = wall_clock64();
+  const int32_t b = sched_find(s, f);
+  if (__lane_id() == 0) {
+    acc[6] += wall_clock64() - w0;
+    if (b == kGaveUp) acc[kCntAbandoned] += 1;
+  }
+  return b;
+}
+
 // The persistent kernel over blocks whose element data fits the workgroup's registers
-// (resident.h): N items or elements per thread.  Same queue, claims and visit policy as
-// k_visit_async; a workgroup that visits a block again keeps its registers and LDS, and only the
-// halo times are read again.
-// What bounds it: a chain of short phases per visit (a sweep of two to seven hundred dependent
-// instructions per wave and the device round trips that hand its result on), on fronts too small
-// to fill the chip.  Whole solves against the staged records and LDS queue of k_visit_async: level-5
-// icosphere (10,242 vertices) 0.349 -> 0.197 ms, level-7 anisotropic icosphere 1.191 -> 0.734,
-// 32^2 square 0.247 -> 0.176, 16^3 cube 0.350 -> 0.276, 33^3 tensor cube 0.463 -> 0.326, 64^3 cube
-// 1.222 -> 0.968 ms.  Held to 128 VGPRs so that four workgroups fit a CU.
+// (resident.h): N items or elements per thread.  Blocks are found and handed on as block_sched.h
+// says; a workgroup that visits a block again, at once or when it is dirty again and nothing smaller
+// waits, keeps its registers and LDS, and only times are read again.  A visit of a tet block is one
+// sweep while few blocks wait (kCrowd); a block that has not converged is visited again at once
+// unless a block of the same owner waits with a smaller time.
+// What bounds it: the chain of a visit (64^3 cube: 3.0 us a sweep, 0.4 us until its times have landed,
+// 0.8 us of marks and release, 2 us to load a block into the registers and LDS every third visit), and
+// on large tet meshes the loads too (96^3: 86,000 of 40 KB in 1.5 ms).  Held to 128 VGPRs, so that four
+// workgroups fit a CU: with 45 of them spilled the 96^3 solve took 2.1 ms, without 1.7.
+// Visit kernels, against the staged records of visit_block and one queue ring: 64^3 cube 1.045 ->
+// 0.664 ms, 96^3 with 16 sources 3.67 -> 1.53, 33^3 tensor 0.448 -> 0.295, 16^3 0.285 -> 0.172; level-8
+// icosphere 3.29 -> 1.70, level-7 anisotropic 1.02 -> 0.55, level 5 0.328 -> 0.169, 32^2 square 0.158 ->
+// 0.081.
 template <int DIM, int N, int BT>
-__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_resident(ResidentArgs ra) {
-  const AsyncArgs& a = ra.a;
+__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_resident(SolveArgs a) {
   extern __shared__ uint4 lds4[];
   __shared__ int sFlag[3];      // a sweep's "a time fell", in a ring over the sweeps
   __shared__ int sQn[2];        // work-item counters of alternate sweeps (tets)
-  __shared__ unsigned sMark[2]; // dependents whose halo holds a vertex lowered since the last push
+  __shared__ unsigned sMark[2]; // dependents whose halo holds a vertex lowered in this visit
   __shared__ int sBlock;
-  __shared__ int sAgain;
-  __shared__ int sNext;  // block taken while the previous visit queued its dependents, or -2
-  __shared__ unsigned sPend;  // pending count returned by this workgroup's last push
+  __shared__ unsigned sWaiting; // smallest key of the owner's waiting blocks when last looked
+  __shared__ unsigned sKey;     // smallest time the visit lowered
+  __shared__ int sCrowd;        // dirty blocks seen waiting when this one was claimed
   __shared__ unsigned long long sAcc[kNumCounters];
   const int tid = threadIdx.x;
   uint4* sA = lds4;
-  uint4* sB = sA + (DIM == 3 ? ra.max_elem : 0);
-  float* sT = reinterpret_cast<float*>(sB + (DIM == 3 ? ra.max_elem : 0));
-  float* sP = sT + ra.max_local;
-  int* sHidx = reinterpret_cast<int*>(sP + ra.max_local);
-  uint16_t* sQ = reinterpret_cast<uint16_t*>(sHidx + ra.max_local);
+  uint4* sB = sA + (DIM == 3 ? a.max_elem : 0);
+  float* sT = reinterpret_cast<float*>(sB + (DIM == 3 ? a.max_elem : 0));
+  float* sP = sT + a.max_local;
+  int* sHidx = reinterpret_cast<int*>(sP + a.max_local);
+  uint16_t* sQ = reinterpret_cast<uint16_t*>(sHidx + a.max_local);
   const float large = a.v.large, eps = a.v.eps;
   if (tid < kNumCounters) sAcc[tid] = 0;
   if (tid < 3) sFlag[tid] = 0;
   if (tid < 2) sQn[tid] = 0;
   if (tid < 2) sMark[tid] = 0;
-  if (tid == 0) {
-    sNext = -2;
-    sPend = 0;
-  }
+  if (tid == 0) sKey = kClean;
+  Finder f;
+  if (tid < 64) sched_enter(a.s, f);
   int ring = 0;  // sweeps run so far, modulo 3
   int qc = 0;
-  uint64_t solves = 0;
-  for (;;) {
+  uint32_t solves = 0;
+  if (tid < 64) {
+    const int32_t nb = find_next(a.s, f, sAcc);
     if (tid == 0) {
-      int nb = sNext;
-      if (nb == -2) {
-        const unsigned long long w0 = wall_clock64();
-        nb = q_take(a);
-        sAcc[6] += wall_clock64() - w0;
-        if (nb == kAbandoned) sAcc[kCntAbandoned] += 1;
-      }
       sBlock = nb;
-      sNext = -2;
+      sCrowd = f.others;
     }
-    __syncthreads();
-    const int b = __builtin_amdgcn_readfirstlane(sBlock);
-    if (b < 0) break;
+  }
+  __syncthreads();
+  int b = __builtin_amdgcn_readfirstlane(sBlock);
+  while (b >= 0) {
     unsigned long long t0 = wall_clock64();
-    // the block's state: one owned vertex per thread, its items or elements in registers
+    const int cur = b;
+    // the resident block: one owned vertex per thread, its items or elements in registers
     const BlockDesc d = a.v.blocks[b];
+    const uint32_t slot = sched_slot(a.s, b);
     float* seen = a.v.seen + d.vstart + d.hstart;
-    float own = 0.f;      // the owned vertex's time as last published
-    float own_last = 0.f; // ... at the start of the last sweep
-    uint64_t vm = 0;
-    int32_t dep = 0;
     const int32_t s0 = a.dep_start[b];
     const int ndep = a.dep_start[b + 1] - s0;
+    float own = 0.f;  // the owned vertex's time as last published
+    uint64_t vm = 0;
+    uint32_t dep_slot = 0;
     std::conditional_t<DIM == 2, TriRegs<N>, TetRegs<N>> r;
-    if (tid < d.nown) {
-      own = load_T<true>(a.v.T + d.vstart + tid);
-      sP[tid] = seen[tid];
-      vm = a.v.vmask[d.vstart + tid];
-      sT[tid] = own;
+    const int t = this_thread();
+    if (t < d.nown) {
+      own = load_T<true>(a.v.T + d.vstart + t);
+      sP[t] = seen[t];
+      vm = a.v.vmask[d.vstart + t];
+      sT[t] = own;
     }
-    for (int i = tid; i < d.nhalo; i += BT) {
+    for (int i = t; i < d.nhalo; i += BT) {
       const int32_t h = a.v.halo[d.hstart + i];
       sHidx[i] = h;
       sP[d.nown + i] = seen[d.nown + i];
       sT[d.nown + i] = load_T<true>(a.v.T + h);
     }
-    if (tid < ndep) dep = a.dep[s0 + tid];
+    if (t < ndep) dep_slot = sched_slot(a.s, a.dep[s0 + t]);
     if constexpr (DIM == 2)
-      tri_load<N, BT>(r, ra.items, ra.items.range[b]);
+      tri_load<N, BT>(r, a.items, a.items.range[b]);
     else
       tet_load<N, BT>(r, a.v.elems, d, sA, sB);
+    wait_memory();  // the copies to LDS too
     __syncthreads();
     if constexpr (DIM == 2) tri_seen<N>(r, sP);
     else tet_seen<N>(r, sP);
     unsigned long long t1 = wall_clock64();
     bool rerun = false;
+    unsigned waiting = kClean;  // smallest key of the owner's other blocks when last looked
+    // visits of this block: the next one at once, or when the block is dirty again and nothing
+    // smaller waits
     for (;;) {
-      // latency-bound regime (see kLatencyPending); sPend is written after the barrier that
-      // follows this read
-      const bool latency = sPend < kLatencyPending * gridDim.x;
-      const int inner = latency ? latency_sweeps<DIM>(a.v.max_inner) : a.v.max_inner;
-      unsigned nsolve = 0;
+      const int inner = DIM == 2 || sCrowd >= kCrowd ? a.v.max_inner : 1;
       uint64_t marks = 0;  // dependents holding this thread's vertex, if it fell
+      uint32_t key = kClean;
+      float own_last = own;
       int sweep = 0;
       bool conv = false;
       while (sweep < inner) {
         bool ch = false;
         int nq = 1;
         if constexpr (DIM == 2) {
-          ch = tri_sweep<N>(r, sT, large, eps, nsolve);
+          ch = tri_sweep<N>(r, sT, large, eps, solves);
         } else {
           tet_select<N, BT>(r, sT, eps, sQ, &sQn[qc]);
           __syncthreads();
           nq = sQn[qc];
           if (tid == 0) sQn[qc ^ 1] = 0;
           qc ^= 1;
-          if (nq) ch = tet_solve<BT>(sA, sB, sQ, nq, sT, large, eps, nsolve);
+          if (nq) ch = tet_solve<N, BT>(r, sA, sB, sQ, nq, sT, large, eps, solves);
         }
         if (ch) sFlag[ring] = 1;
         // (no pair selected: no time fell, and no thread waits for another's solve)
@@ -554,6 +424,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                                          __float_as_uint(v), __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
             marks |= vm;
+            key = __float_as_uint(v);
           }
         }
         if (!any) {
@@ -561,65 +432,35 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
           break;
         }
       }
-      solves += nsolve;
       const unsigned long long t2 = wall_clock64();
+      // visits beyond the bound mark nothing more (runaway guard)
+      const bool cap_ok = (int64_t)sAcc[0] < a.max_visits;
+      const bool more = !conv && cap_ok;
+      // marks made from here on are seen by the halo loads of the next visit or after it
+      if (more && tid == 0) sched_again(a.s, slot);
       // reduced over the wave first: the compiler turns an LDS or with a uniform address into a
       // scalar loop over the lanes (a third of a triangle sweep)
-      if (__ballot(marks != 0ull)) {
+      if (__ballot(key != kClean)) {
         const uint32_t lo = wave_or((uint32_t)marks), hi = wave_or((uint32_t)(marks >> 32));
+        key = wave_umin(key);
         if (__lane_id() == 63) {
+          atomicMin(&sKey, key);
           if (lo) atomicOr(&sMark[0], lo);
           if (hi) atomicOr(&sMark[1], hi);
         }
       }
-      // the published times have reached the device's coherence point (vmcnt covers atomics
-      // without a result) before the dependents are queued
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      __builtin_amdgcn_s_waitcnt(0);
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      // the published times have reached the device's coherence point before the dependents are
+      // marked
+      wait_memory();
       __syncthreads();
       const unsigned long long tq = wall_clock64();
-      // visits beyond the bound queue nothing more (runaway guard)
-      const bool cap_ok = (int64_t)sAcc[0] < a.max_visits;
-      bool want = false;
+      const uint32_t vkey = sKey;
+      // visited again at once, unless another of the owner's blocks waits with a smaller time
+      const bool again = more && !(waiting < vkey);
       if (tid < 64) {
         const uint64_t mask = (uint64_t)sMark[0] | ((uint64_t)sMark[1] << 32);
-        want = cap_ok && tid < ndep && ((mask >> tid) & 1ull) != 0ull;
-        if (want) want = atomicExch(&a.qflag[dep], 1u) == 0u;
-        if (tid == 0)
-          sAgain = (latency && !conv && cap_ok) || (release_or_rerun(a, b) && cap_ok);
-      }
-      __syncthreads();
-      const bool again = sAgain != 0;
-      if (tid < 64) {
+        if (cap_ok && tid < ndep && ((mask >> tid) & 1ull)) sched_mark(a.s, dep_slot, vkey);
         if (tid < 2) sMark[tid] = 0;
-        // an unconverged block that is left goes back to the queue
-        bool self = tid == 0 && !again && !conv && cap_ok;
-        if (self) self = atomicExch(&a.qflag[b], 1u) == 0u;
-        const uint64_t bal = __ballot(want);
-        const unsigned nself = __ballot(self) ? 1u : 0u;
-        const unsigned n = (unsigned)__popcll(bal) + nself;
-        const unsigned dec = again ? 0u : 1u;
-        if (n + dec > 0u) {
-          uint32_t base = 0;
-          if (tid == 0) {
-            // tail += n, pending += n - dec, in one 64-bit add (pending >= 1 while this visit
-            // counts, so the low word cannot borrow)
-            const unsigned long long inc = ((unsigned long long)n << 32) + n - dec;
-            const unsigned long long old = __hip_atomic_fetch_add(
-                &a.ctl->tp, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            base = (uint32_t)(old >> 32);
-            sPend = (unsigned)(old & 0xffffffffull);
-            if (n == 0u && (old & 0xffffffffull) == 1ull) q_finish(a);
-            if (self)
-              __hip_atomic_store(q_slot(a, base + n - 1u), b + 1, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-          }
-          base = __shfl(base, 0, 64);
-          if (want)
-            __hip_atomic_store(q_slot(a, base + (uint32_t)__popcll(bal & lane_mask_lt())), dep + 1,
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
         if (tid == 0) {
           VisitResult vr;
           vr.sweeps = sweep;
@@ -627,20 +468,26 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
           vr.t_sweep = t2 - t1;
           vr.t_wb = tq - t2;
           tally_visit(sAcc, d, vr, 0, a.elem_bytes, tq - t0, rerun, rerun);
-          sAcc[10] += wall_clock64() - tq;
+        }
+        if (again) {
+          const uint32_t w = sched_waiting(a.s);
+          if (tid == 0) sWaiting = w;
+          if (tid == 0) sAcc[10] += wall_clock64() - tq;
+        } else {
+          wait_memory();  // the marks have landed before this block can count as clean
+          if (tid == 0) sched_leave(a.s, slot, more ? vkey : kClean);
+          if (tid == 0) sAcc[10] += wall_clock64() - tq;
+          const int32_t nb = find_next(a.s, f, sAcc);
+          if (tid == 0) {
+            sBlock = nb;
+            sCrowd = f.others;
+            sWaiting = kClean;
+          }
         }
       } else if (again) {
-        // the other waves read the halo times of the next visit
+        // the halo times of the next visit (by the waves that mark nothing)
         for (int i = tid - 64; i < d.nhalo; i += BT - 64)
           sT[d.nown + i] = load_T<true>(a.v.T + sHidx[i]);
-      } else if (tid == 64) {
-        // the next block is taken while wave 0 queues the dependents: this visit is over, so the
-        // workgroup holds no work that the wait for a ticket could depend on
-        const unsigned long long w0 = wall_clock64();
-        const int32_t nx = q_take(a);
-        sNext = nx;
-        sAcc[6] += wall_clock64() - w0;
-        if (nx == kAbandoned) sAcc[kCntAbandoned] += 1;
       }
       if (!again) {
         // what this visit evaluated the block's elements with: every time, but for the owned
@@ -650,15 +497,143 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = sT[d.nown + i];
       }
       __syncthreads();
-      if (!again) break;
-      rerun = true;
+      waiting = sWaiting;
+      if (tid == 0) sKey = kClean;
       t0 = t1 = wall_clock64();
+      rerun = again;
+      if (again) continue;
+      b = __builtin_amdgcn_readfirstlane(sBlock);
+      if (b != cur) break;
+      // the same block, still resident: only times may have fallen (the owned ones if another
+      // workgroup visited the block meanwhile)
+      if (tid < d.nown) {
+        own = load_T<true>(a.v.T + d.vstart + tid);
+        sT[tid] = own;
+      }
+      for (int i = tid; i < d.nhalo; i += BT) sT[d.nown + i] = load_T<true>(a.v.T + sHidx[i]);
+      __syncthreads();
+      t1 = wall_clock64();
     }
   }
+  write_out(a, sBlock);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) solves += __shfl_down(solves, off, 64);
   if (__lane_id() == 0 && solves) atomicAdd(&sAcc[3], (unsigned long long)solves);
   __syncthreads();
+  if (tid < kNumCounters && sAcc[tid]) atomicAdd(&a.counters[tid], sAcc[tid]);
+}
+
+// Seeds of a solve of the scheduler above: the sources' times, and the owner block of each source
+// and that block's dependents marked (one workgroup per source, one lane per block to mark).
+__global__ void k_sched_seed(Sched s, const int32_t* seeds, const float* vals, int64_t n,
+                             const int32_t* iperm, const int32_t* owner, const int32_t* dep_start,
+                             const int32_t* dep, float* T, int64_t nv) {
+  for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
+    if (seeds[i] < 0 || seeds[i] >= nv) continue;
+    const int32_t v = iperm[seeds[i]];
+    const int32_t b = owner[v];
+    if (threadIdx.x == 0)
+      atomicMin(reinterpret_cast<unsigned*>(&T[v]), __float_as_uint(vals ? vals[i] : 0.f));
+    const int32_t s0 = dep_start[b], nd = dep_start[b + 1] - s0;
+    for (int j = threadIdx.x; j <= nd; j += blockDim.x)
+      sched_mark(s, sched_slot(s, j == 0 ? b : dep[s0 + j - 1]), __float_as_uint(vals ? vals[i] : 0.f));
+  }
+}
+
+// The persistent kernel over blocks of any size: the records staged in LDS or read from memory,
+// the selected pairs through the LDS queue (visit_block).  Scheduling as in k_visit_resident.
+template <int DIM>
+__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_visit_general(SolveArgs a) {
+  extern __shared__ uint4 lds4[];
+  __shared__ int sFlag[4];
+  __shared__ int sQn[2];  // work-item counters of alternate chunks
+  __shared__ int sBlock;
+  __shared__ unsigned sKey;  // smallest time the visit lowered
+  __shared__ int sCrowd;     // dirty blocks seen waiting when this one was claimed
+  __shared__ unsigned long long sRed;
+  __shared__ unsigned long long sAcc[kNumCounters];
+  const int tid = threadIdx.x;
+  if (tid < kNumCounters) sAcc[tid] = 0;
+  Finder f;
+  if (tid < 64) sched_enter(a.s, f);
+  for (;;) {
+    if (tid < 64) {
+      const int32_t nb = find_next(a.s, f, sAcc);
+      if (tid == 0) {
+        sBlock = nb;
+        sCrowd = f.others;
+      }
+    }
+    __syncthreads();
+    const int b = __builtin_amdgcn_readfirstlane(sBlock);
+    if (b < 0) break;
+    const BlockDesc d = a.v.blocks[b];
+    const VisitLds l = carve_lds<DIM>(lds4, a.rec_lds_bytes, a.v.queue_cap, d);
+    const uint32_t slot = sched_slot(a.s, b);
+    const int32_t s0 = a.dep_start[b];
+    const int ndep = a.dep_start[b + 1] - s0;
+    bool rerun = false;  // the previous visit of this workgroup was of block b, and this one's
+                         // times are in LDS already (rerun_load)
+    // few blocks wait: one sweep of a tet block per visit (see kCrowd; larger here, where a load costs
+    // less beside the sweeps)
+    const int inner = DIM == 3 && sCrowd < 3 * kCrowd ? 1 : 0;
+    for (;;) {
+      if (tid == 0) {
+        sRed = 0;
+        sKey = kClean;
+      }
+      const unsigned long long t0 = wall_clock64();
+      uint64_t solves = 0;
+      const VisitResult r =
+          visit_block<DIM, true>(a.v, b, l.rec, l.T, l.old, l.chg, l.hidx, l.vm, l.q, l.mark, sFlag,
+                                 sQn, &solves, rerun, inner, rerun);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) solves += __shfl_down(solves, off, 64);
+      if (__lane_id() == 0) atomicAdd(&sRed, (unsigned long long)solves);
+      uint32_t key = kClean;
+      for (int i = tid; i < d.nown; i += kBlockThreads)
+        if (l.T[i] < l.old[i]) key = min(key, __float_as_uint(l.T[i]));
+      key = wave_umin(key);
+      if (__lane_id() == 0 && key != kClean) atomicMin(&sKey, key);
+      // visits beyond the bound mark nothing more (runaway guard)
+      const bool again = !r.converged && (int64_t)sAcc[0] < a.max_visits;
+      // (marks made meanwhile stay: clearing them here would cost every visit a round trip, and the
+      // block a further visit at the end where there were any)
+      __syncthreads();
+      const unsigned long long tq = wall_clock64();
+      if (tid < 64) {
+        // the visit's times have reached the device's coherence point (visit_block)
+        const uint64_t mask = a.v.vmask ? ((uint64_t)(uint32_t)l.mark[0] |
+                                           ((uint64_t)(uint32_t)l.mark[1] << 32))
+                                        : 0ull;
+        if (r.bnd_changed && (int64_t)sAcc[0] < a.max_visits)
+          for (int j = tid; j < ndep; j += 64)
+            if (a.v.vmask ? ((mask >> j) & 1ull) != 0ull : l.mark[j] != 0)
+              sched_mark(a.s, sched_slot(a.s, a.dep[s0 + j]), sKey);
+        if (again) {
+          // the next visit starts with clear marks (they have all been read above)
+          if (a.v.vmask) {
+            if (tid < 2) l.mark[tid] = 0;
+          } else {
+            for (int j = tid; j < ndep; j += 64) l.mark[j] = 0;
+          }
+        } else {
+          wait_memory();  // the marks have landed before this block can count as clean
+          if (tid == 0) sched_leave(a.s, slot, kClean);
+        }
+        if (tid == 0) {
+          tally_visit(sAcc, d, r, sRed, a.elem_bytes, tq - t0, rerun, rerun && a.v.rec_lds);
+          sAcc[10] += wall_clock64() - tq;
+        }
+      } else if (again) {
+        rerun_load<true, kBlockThreads>(a.v, d, r.sweeps, l.T, l.old, l.chg, l.hidx, sFlag, 64);
+      }
+      __syncthreads();
+      if (!again) break;
+      rerun = true;
+    }
+  }
+  write_out(a, sBlock);
   if (tid < kNumCounters && sAcc[tid]) atomicAdd(&a.counters[tid], sAcc[tid]);
 }
 
@@ -797,7 +772,7 @@ int upload_layout(Mesh& m) {
   if (lds > 65536) {
     // dynamic LDS beyond 64 KB (MI355X has 160 KB per CU) is opted into per kernel
     const void* ks[] = {(const void*)k_visit_sync<3>, (const void*)k_visit_sync<2>,
-                        (const void*)k_visit_async<3>, (const void*)k_visit_async<2>};
+                        (const void*)k_visit_general<3>, (const void*)k_visit_general<2>};
     for (const void* k : ks)
       HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   }
@@ -841,6 +816,17 @@ int upload_layout(Mesh& m) {
   return EIK_OK;
 }
 
+static const void* resident_kernel(int dim, int n, int bt) {
+  if (dim == 3)
+    return bt == 256   ? (const void*)k_visit_resident<3, 4, 256>
+           : bt == 512 ? (const void*)k_visit_resident<3, 4, 512>
+                       : (const void*)k_visit_resident<3, 4, 1024>;
+  return n == 2      ? (const void*)k_visit_resident<2, 2, 256>
+         : bt == 256 ? (const void*)k_visit_resident<2, 4, 256>
+         : bt == 512 ? (const void*)k_visit_resident<2, 4, 512>
+                     : (const void*)k_visit_resident<2, 4, 1024>;
+}
+
 // The shape of the register-resident visits for this layout, and the triangle items.  A block
 // qualifies when one thread can hold each owned vertex and N x BT items (triangles) or elements
 // (tets) cover it; N and BT grow with the largest block.
@@ -855,6 +841,7 @@ static int setup_resident(Mesh& m, size_t max_lds) {
   if (m.dim == 2 && need <= 2 * 256) d->res_n = 2, d->res_bt = 256;
   else if (need <= 4 * 256) d->res_n = 4, d->res_bt = 256;
   else if (need <= 4 * 512) d->res_n = 4, d->res_bt = 512;
+  else if (need <= 4 * 1024) d->res_n = 4, d->res_bt = 1024;
   if (d->res_n == 0 || L.max_own > d->res_bt || (m.dim == 2 && L.max_local > kItemSlots)) {
     d->res_n = 0;
     return EIK_OK;
@@ -867,10 +854,8 @@ static int setup_resident(Mesh& m, size_t max_lds) {
     return EIK_OK;
   }
   if (d->res_lds > 65536)
-    HIP_TRY(hipFuncSetAttribute(
-        d->res_bt == 256 ? (const void*)k_visit_resident<3, 4, 256>
-                         : (const void*)k_visit_resident<3, 4, 512>,
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)d->res_lds));
+    HIP_TRY(hipFuncSetAttribute(resident_kernel(m.dim, d->res_n, d->res_bt),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)d->res_lds));
   if (m.dim == 3) return EIK_OK;
   std::vector<int2> range(L.nblocks);
   int64_t n = 0;
@@ -999,48 +984,32 @@ struct VisitKernel {
   const void* fn;
   int threads;
   size_t lds;
-  bool resident;
+  bool stage;  // k_visit_general: records staged in LDS
 };
 
 // Register-resident visits where the blocks fit them, unless the records are to be read from
 // memory; else the general kernel, its records staged in LDS where they fit.
 static VisitKernel visit_kernel(const DeviceState* d, int32_t stage_records) {
   VisitKernel k;
+  k.stage = d->rec_lds && stage_records != EIK_STAGE_MEMORY;
   if (d->res_n && stage_records != EIK_STAGE_MEMORY) {
-    k.resident = true;
     k.threads = d->res_bt;
     k.lds = d->res_lds;
-    if (d->dim == 3)
-      k.fn = d->res_bt == 256 ? (const void*)k_visit_resident<3, 4, 256>
-                              : (const void*)k_visit_resident<3, 4, 512>;
-    else
-      k.fn = d->res_n == 2      ? (const void*)k_visit_resident<2, 2, 256>
-             : d->res_bt == 256 ? (const void*)k_visit_resident<2, 4, 256>
-                                : (const void*)k_visit_resident<2, 4, 512>;
+    k.fn = resident_kernel(d->dim, d->res_n, d->res_bt);
     return k;
   }
-  const bool stage = d->rec_lds && stage_records != EIK_STAGE_MEMORY;
-  k.resident = false;
   k.threads = kBlockThreads;
-  k.lds = stage ? d->lds_bytes : d->lds_bytes_direct;
-  k.fn = d->dim == 3 ? (const void*)k_visit_async<3> : (const void*)k_visit_async<2>;
+  k.lds = k.stage ? d->lds_bytes : d->lds_bytes_direct;
+  k.fn = d->dim == 3 ? (const void*)k_visit_general<3> : (const void*)k_visit_general<2>;
   return k;
 }
 
-// Workgroups of the single-solve persistent kernel.  A workgroup for every queued block mostly
-// visits blocks whose suppliers are still changing, which only makes more visits, while too few
-// workgroups leave the fronts' blocks waiting; the grid is sized to the fronts.  Triangle
-// meshes: the fronts are curves, about sqrt(blocks x sources) blocks, and triangle visits
-// publish lowered times during their sweeps; three workgroups per front block, with three
-// sweeps per visit, against every workgroup that fits with four: level-7 anisotropic icosphere
-// with 4 sources 1.47 -> 1.23 ms (13.1M -> 5.3M local solves), 16 and 64 sources 5% faster,
-// isotropic with 1 source 1.96 -> 1.72 ms, 257^2 square 1.27 -> 1.14 ms, 32^2 square 0.24 ->
-// 0.21 ms, level-8 icosphere equal.  Tet meshes: surfaces, about blocks^(2/3) x sources^(1/3)
-// blocks; five workgroups per front block measured best over cubes with one source: 32^3
-// 0.59 -> 0.47 ms, 16^3 and 24^3 about 10% faster, from 48^3 on (the 64^3 cube included) every
-// workgroup that fits (64^3: 1.17 ms at 768, 1.31 at 640, 1.59 at 512).  At least one per CU.
-static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t nblocks,
-                           int64_t nseeds, int* out) {
+// Workgroups of the single-solve persistent kernel: one per block while they all fit, so that every
+// block stays resident with its owner, else all that fit (64^3 cube, 4,292 blocks: 1.61 ms at 256,
+// 0.99 at 512, 0.72 at 1,024; 96^3, 14,261 blocks: 5.12, 2.90, 1.82).  Triangle meshes stop at three
+// per CU (level-7 anisotropic icosphere, 2,560 blocks: 0.76 ms at 256, 0.57 at 512, 0.55 at 768, 0.60
+// at 1,024; level 8, 10,240 blocks: 2.65, 1.88, 1.70, 1.69).
+static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t nblocks, int* out) {
   int dev = 0, ncu = 0, per_cu = 0;
   HIP_TRY(hipGetDevice(&dev));
   HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1051,9 +1020,8 @@ static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t
     *out = std::min(requested, resident);
     return EIK_OK;
   }
-  const double nb = (double)std::max<int64_t>(nblocks, 1), ns = (double)std::max<int64_t>(nseeds, 1);
-  const double front = dim == 2 ? 3.0 * std::sqrt(nb * ns) : 5.0 * std::cbrt(nb * nb * ns);
-  *out = (int)std::min<double>(resident, std::max<double>(ncu, front));
+  const int most = dim == 2 ? std::min(resident, 3 * ncu) : resident;
+  *out = (int)std::min<int64_t>(most, std::max<int64_t>(nblocks, 1));
   return EIK_OK;
 }
 
@@ -1065,22 +1033,28 @@ static int32_t async_inner_sweeps(int dim, int32_t requested) {
   return requested > 0 ? requested : (dim == 2 ? 3 : default_inner_sweeps(dim, 0));
 }
 
-// The work queue of the single-solve persistent scheduler, allocated on first use.  Ring
-// capacity: every block queued at once plus a waiting ticket per resident workgroup (at most 64
-// per CU), twice over.
-static int ensure_queue(DeviceState* d) {
-  if (d->queue) return EIK_OK;
+// After a launch whose workgroups gave up waiting: EIK_OK if the solve still reached its end (the
+// result is complete), else EIK_ERR_TIMEOUT.  Synchronises stream s.
+static int check_end(const unsigned char* sctl, hipStream_t s, unsigned long long abandoned) {
+  uint32_t done = 0;
+  HIP_TRY(hipMemcpyAsync(&done, sctl + kSchedCtlBytes / 2, sizeof(done), hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
+  if (done) return EIK_OK;
+  return fail(EIK_ERR_TIMEOUT, std::to_string(abandoned) +
+                                   " queue waits outlasted wait_limit_us and the solve did not "
+                                   "finish (incomplete result)");
+}
+
+// The block words of the persistent scheduler, allocated on first use: one per block and, since
+// every owner has as many, up to one more per workgroup (at most 64 per CU).
+static int ensure_words(DeviceState* d) {
+  if (d->words) return EIK_OK;
   int dev = 0, ncu = 0;
   HIP_TRY(hipGetDevice(&dev));
   HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   d->max_workgroups = 64 * std::max(ncu, 1);
-  uint32_t qcap = 1;
-  while (qcap < 2u * ((uint32_t)d->nblocks + (uint32_t)d->max_workgroups) + 2u) qcap <<= 1;
-  d->qcap = (int32_t)qcap;
-  HIP_TRY(hipMalloc((void**)&d->queue, sizeof(int32_t) * kSlotStride * qcap));
-  HIP_TRY(hipMalloc((void**)&d->qflag, sizeof(uint32_t) * d->nblocks));
-  HIP_TRY(hipMalloc((void**)&d->bstate, sizeof(uint32_t) * d->nblocks));
-  HIP_TRY(hipMalloc((void**)&d->qctl, sizeof(QueueCtl)));
+  HIP_TRY(hipMalloc((void**)&d->words, sizeof(unsigned long long) * sched_max_words(d->nblocks, d->max_workgroups)));
+  HIP_TRY(hipMalloc((void**)&d->sctl, kSchedCtlBytes));
   return EIK_OK;
 }
 
@@ -1089,18 +1063,23 @@ static int ensure_queue(DeviceState* d) {
 struct AsyncBufs {
   float* T;
   float* seen;
-  int32_t* queue;
-  uint32_t* qflag;
-  uint32_t* bstate;
-  QueueCtl* ctl;
+  unsigned long long* words;
+  unsigned char* sctl;
   unsigned long long* counters;
-  uint32_t qcap;
 };
 
-static AsyncArgs async_args(const Mesh& m, const eik_solve_opts_t& o, const AsyncBufs& b,
-                            bool stage) {
+// Enqueues a persistent solve on stream s: the resets, the seeds, and the visits, which write the
+// times in caller order to `out` (device memory, or null) when they are done.  A fill kernel
+// rather than memsets, so that a caller may capture this into a graph.
+static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBufs& b,
+                         const int32_t* seeds, const float* seedvals, int64_t nseeds, float* out,
+                         hipStream_t s, hipEvent_t before, hipEvent_t after) {
   const DeviceState* d = m.dev;
-  AsyncArgs a;
+  const VisitKernel k = visit_kernel(d, o.stage_records);
+  int grid = 0;
+  int rc = persistent_grid(m.dim, k, o.workgroups, d->nblocks, &grid);
+  if (rc) return rc;
+  SolveArgs a;
   a.v.blocks = d->blocks;
   a.v.elems = d->elems;
   a.v.halo = d->halo;
@@ -1110,73 +1089,50 @@ static AsyncArgs async_args(const Mesh& m, const eik_solve_opts_t& o, const Asyn
   a.v.max_inner = async_inner_sweeps(m.dim, o.max_inner);
   a.v.queue_cap = d->queue_cap;
   a.v.seen = b.seen;
-  a.v.rec_lds = stage ? 1 : 0;
+  a.v.rec_lds = k.stage ? 1 : 0;
   a.v.vh_start = d->vh_start;
   a.v.vh_pos = d->vh_pos;
   a.v.vmask = d->vmask;
   a.v.rmult = nullptr;
   a.v.lens = nullptr;
   a.v.dep_start = d->dep_start;
-  a.rec_lds_bytes = stage ? d->rec_lds_bytes : 0;
-  a.queue = b.queue;
-  a.qflag = b.qflag;
-  a.bstate = b.bstate;
-  a.ctl = b.ctl;
-  a.qmask = b.qcap - 1u;
-  a.bmask = 0x7fffffff;
+  a.s.word = b.words;
+  a.s.ctl = reinterpret_cast<unsigned long long*>(b.sctl);
+  a.s.done = reinterpret_cast<uint32_t*>(b.sctl + kSchedCtlBytes / 2);
+  sched_shape(a.s, d->nblocks, grid);
+  a.s.wait_limit = wait_limit_ticks(d->device, o.wait_limit_us);
+  a.items = {d->item_range, d->item_id, d->item_len};
   a.dep_start = d->dep_start;
   a.dep = d->dep;
+  a.iperm = d->iperm;
+  a.out = out;
+  a.nv = m.nv;
   a.counters = b.counters;
-  a.elem_bytes = m.dim == 3 ? kAlgoElemBytes<3> : kAlgoElemBytes<2>;
-  a.nblocks = d->nblocks;
-  // runaway guard: a workgroup that has made this many visits queues no more work (its visits
+  // runaway guard: a workgroup that has made this many visits marks no more blocks (its visits
   // still finish), so a solve ends even if it never converged; the bound is max_iterations
   // outer iterations' worth of visits of every block (1000 without a cap), far above what a
   // converging solve needs
   a.max_visits = (int64_t)(o.max_iterations > 0 ? o.max_iterations : 1000) * d->nblocks;
-  a.wait_limit = wait_limit_ticks(d->device, o.wait_limit_us);
-  return a;
-}
-
-static int launch_visits(const DeviceState* d, const VisitKernel& k, const AsyncArgs& a, int grid,
-                         hipStream_t s) {
-  ResidentArgs ra;
-  ra.a = a;
-  ra.items = {d->item_range, d->item_id, d->item_len};
-  ra.max_local = d->max_local;
-  ra.max_elem = d->max_elem;
-  void* args[] = {k.resident ? (void*)&ra : (void*)&a};
-  HIP_TRY(hipLaunchKernel(k.fn, dim3(grid), dim3(k.threads), args, k.lds, s));
-  return EIK_OK;
-}
-
-static int solve_async(Mesh& m, const eik_solve_opts_t& o, int64_t nseeds, eik_solve_stats_t& st) {
-  DeviceState* d = m.dev;
-  hipStream_t s = d->stream;
-  int rc0 = ensure_queue(d);
-  if (rc0) return rc0;
-  const bool stage = d->rec_lds && o.stage_records != EIK_STAGE_MEMORY;
-  const VisitKernel vk = visit_kernel(d, o.stage_records);
-  const AsyncBufs bufs = {d->T,     d->seen,   d->queue, d->qflag, d->bstate,
-                          reinterpret_cast<QueueCtl*>(d->qctl), d->counters, (uint32_t)d->qcap};
-  const AsyncArgs a = async_args(m, o, bufs, stage);
-  // the queue, its flags, block states and control words were reset with the solve's other
-  // arrays (eik_solve)
-  hipLaunchKernelGGL(k_async_seed, seed_grid(nseeds), dim3(64), 0, s, a, d->seeds, nseeds,
-                     d->iperm, d->owner, m.nv);
+  a.elem_bytes = m.dim == 3 ? kAlgoElemBytes<3> : kAlgoElemBytes<2>;
+  a.max_local = d->max_local;
+  a.max_elem = d->max_elem;
+  a.rec_lds_bytes = k.stage ? d->rec_lds_bytes : 0;
+  FillSegs f;
+  f.count = 0;
+  f.add(b.T, m.nv, (int32_t)__builtin_bit_cast(uint32_t, a.v.large));
+  f.add(b.seen, d->nseen, (int32_t)__builtin_bit_cast(uint32_t, EIK_INF));
+  f.add(b.counters, 2 * kNumCounters, 0);
+  f.words = b.words;
+  f.nwords = (int64_t)a.s.owners * a.s.stride;
+  f.add(b.sctl, kSchedCtlBytes / 4, 0);
+  launch_fill(f, s);
+  hipLaunchKernelGGL(k_sched_seed, seed_grid(nseeds), dim3(64), 0, s, a.s, seeds, seedvals, nseeds,
+                     d->iperm, d->owner, d->dep_start, d->dep, b.T, m.nv);
   HIP_TRY(hipGetLastError());
-  int grid = 0;
-  int rc = persistent_grid(m.dim, vk, o.workgroups, d->nblocks, nseeds, &grid);
-  if (rc) return rc;
-  HIP_TRY(hipEventRecord(d->evA, s));
-  if ((rc = launch_visits(d, vk, a, grid, s))) return rc;
-  HIP_TRY(hipEventRecord(d->evB, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  float vms = 0.f;
-  HIP_TRY(hipEventElapsedTime(&vms, d->evA, d->evB));
-  st.visit_ms = vms;
-  st.visit_launches = 1;
-  st.outer_iterations = 1;
+  if (before) HIP_TRY(hipEventRecord(before, s));
+  void* args[] = {(void*)&a};
+  HIP_TRY(hipLaunchKernel(k.fn, dim3(grid), dim3(k.threads), args, k.lds, s));
+  if (after) HIP_TRY(hipEventRecord(after, s));
   return EIK_OK;
 }
 
@@ -1256,7 +1212,11 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     HIP_TRY(hipHostMalloc((void**)&d->h_seed, sizeof(int32_t) * 2 * nseeds));
     d->seed_cap = nseeds;
   }
-  if (!d->h_cnt) HIP_TRY(hipHostMalloc((void**)&d->h_cnt, sizeof(unsigned long long) * kNumCounters));
+  if (!d->h_cnt) {
+    HIP_TRY(hipHostMalloc((void**)&d->h_cnt, sizeof(unsigned long long) * kNumCounters +
+                                                 sizeof(float) * std::min(m->nv, kSmallOut)));
+    d->h_out = reinterpret_cast<float*>(d->h_cnt + kNumCounters);
+  }
   d->hist_len = 0;
   int32_t* h_vals = d->h_seed + d->seed_cap;
   std::memcpy(d->h_seed, seeds, sizeof(int32_t) * nseeds);
@@ -1265,8 +1225,16 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
   HIP_TRY(hipMemcpyAsync(d->seeds, d->h_seed, sizeof(int32_t) * nseeds, hipMemcpyHostToDevice, s));
   if (seed_vals)
     HIP_TRY(hipMemcpyAsync(d->seedvals, h_vals, sizeof(float) * nseeds, hipMemcpyHostToDevice, s));
-  if (o.scheduler == EIK_SCHED_ASYNC && (rc = ensure_queue(d))) return rc;
-  {
+  eik_solve_stats_t st;
+  std::memset(&st, 0, sizeof(st));
+  const bool async = o.scheduler == EIK_SCHED_ASYNC;
+  if (async) {
+    if ((rc = ensure_words(d))) return rc;
+    const AsyncBufs bufs = {d->T, d->seen, d->words, d->sctl, d->counters};
+    rc = enqueue_async(*m, o, bufs, d->seeds, seed_vals ? d->seedvals : nullptr, nseeds,
+                       T_out ? d->out : nullptr, s, d->evA, d->evB);
+    if (rc) return rc;
+  } else {
     FillSegs f;
     f.count = 0;
     f.add(d->T, m->nv, (int32_t)__builtin_bit_cast(uint32_t, large));
@@ -1275,32 +1243,33 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     f.add(d->self, d->nblocks, -1);
     f.add(d->counters, 2 * kNumCounters, 0);
     f.add(d->count, 4, 0);
-    if (o.scheduler != EIK_SCHED_ASYNC)
-      f.add(d->sync_acc, 2 * kSyncSlots * kSyncSlotWords, 0);
-    if (o.scheduler == EIK_SCHED_ASYNC) {
-      f.add(d->queue, (int64_t)d->qcap * kSlotStride, 0);
-      f.add(d->qflag, d->nblocks, 0);
-      f.add(d->bstate, d->nblocks, 0);
-      f.add(d->qctl, (int64_t)(sizeof(QueueCtl) / 4), 0);
-    }
-    int64_t most = 0;
-    for (int k = 0; k < f.count; ++k) most = std::max(most, f.n[k]);
-    hipLaunchKernelGGL(k_fill_segs, dim3((unsigned)std::min<int64_t>(grid1d(most, 256), 2048)),
-                       dim3(256), 0, s, f);
+    f.add(d->sync_acc, 2 * kSyncSlots * kSyncSlotWords, 0);
+    launch_fill(f, s);
+    hipLaunchKernelGGL(k_seed, dim3(grid1d(nseeds, 256)), dim3(256), 0, s, d->seeds,
+                       seed_vals ? d->seedvals : nullptr, nseeds, d->iperm, d->owner, d->T, d->chg,
+                       d->self, m->nv);
+    HIP_TRY(hipGetLastError());
+    if ((rc = solve_sync(*m, o, st))) return rc;
+    if (T_out)
+      hipLaunchKernelGGL(k_gather, dim3(grid1d(m->nv, 256)), dim3(256), 0, s, d->T, d->iperm, m->nv,
+                         d->out);
   }
-  hipLaunchKernelGGL(k_seed, dim3(grid1d(nseeds, 256)), dim3(256), 0, s, d->seeds,
-                     seed_vals ? d->seedvals : nullptr, nseeds, d->iperm, d->owner, d->T, d->chg,
-                     d->self, m->nv);
-  HIP_TRY(hipGetLastError());
-  eik_solve_stats_t st;
-  std::memset(&st, 0, sizeof(st));
-  rc = o.scheduler == EIK_SCHED_ASYNC ? solve_async(*m, o, nseeds, st) : solve_sync(*m, o, st);
-  if (rc) return rc;
   HIP_TRY(hipEventRecord(d->ev1, s));
   HIP_TRY(hipMemcpyAsync(d->h_cnt, d->counters, sizeof(unsigned long long) * kNumCounters,
                          hipMemcpyDeviceToHost, s));
+  // a small result comes back in the same wait, through pinned memory
+  const bool small = T_out && m->nv <= kSmallOut;
+  if (small)
+    HIP_TRY(hipMemcpyAsync(d->h_out, d->out, sizeof(float) * m->nv, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
   const unsigned long long* cnt = d->h_cnt;
+  if (async) {
+    float vms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&vms, d->evA, d->evB));
+    st.visit_ms = vms;
+    st.visit_launches = 1;
+    st.outer_iterations = 1;
+  }
   auto t1 = std::chrono::steady_clock::now();
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, d->ev0, d->ev1));
@@ -1329,13 +1298,13 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
   st.history_len = d->hist_len;
   if (st.abandoned_waits > 0) {
     if (stats) *stats = st;
-    rc = check_queue_end(reinterpret_cast<const QueueCtl*>(d->qctl), s, cnt[kCntAbandoned]);
+    rc = check_end(d->sctl, s, cnt[kCntAbandoned]);
     if (rc) return rc;
   }
   d->has_result = true;
-  if (T_out) {
-    hipLaunchKernelGGL(k_gather, dim3(grid1d(m->nv, 256)), dim3(256), 0, s, d->T, d->iperm, m->nv,
-                       d->out);
+  if (small) {
+    std::memcpy(T_out, d->h_out, sizeof(float) * m->nv);
+  } else if (T_out) {
     HIP_TRY(hipMemcpyAsync(T_out, d->out, sizeof(float) * m->nv, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
   }
@@ -1446,14 +1415,10 @@ int eik_solve_noalloc(eik_mesh_t h, const int32_t* seeds_dev, int64_t nseeds, fl
     return fail(EIK_ERR_STATE, "the current device is not the one the mesh was uploaded to");
   int ncu = 0;
   HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  uint32_t qcap = 1;
-  while (qcap < 2u * ((uint32_t)d->nblocks + 64u * (uint32_t)std::max(ncu, 1)) + 2u) qcap <<= 1;
-  // [control block][counters][queued flags][block states][ring][T][seen], 256-byte aligned
-  const size_t o_cnt = align256(sizeof(QueueCtl));
-  const size_t o_flag = o_cnt + align256(sizeof(unsigned long long) * kNumCounters);
-  const size_t o_state = o_flag + align256(sizeof(uint32_t) * (size_t)d->nblocks);
-  const size_t o_ring = o_state + align256(sizeof(uint32_t) * (size_t)d->nblocks);
-  const size_t o_T = o_ring + align256(sizeof(int32_t) * kSlotStride * (size_t)qcap);
+  // [control words][counters][block words][T][seen], 256-byte aligned
+  const size_t o_cnt = align256(kSchedCtlBytes);
+  const size_t o_word = o_cnt + align256(sizeof(unsigned long long) * kNumCounters);
+  const size_t o_T = o_word + align256(sizeof(unsigned long long) * sched_max_words((size_t)d->nblocks, 64 * (size_t)std::max(ncu, 1)));
   const size_t o_seen = o_T + align256(sizeof(float) * (size_t)m->nv);
   const size_t need = o_seen + align256(sizeof(float) * (size_t)d->nseen);
   if (need > kScratchBytes)
@@ -1463,48 +1428,14 @@ int eik_solve_noalloc(eik_mesh_t h, const int32_t* seeds_dev, int64_t nseeds, fl
   unsigned char* base = nullptr;
   int rc = scratch_address(dev, &base);
   if (rc) return rc;
-  AsyncBufs b;
-  b.ctl = reinterpret_cast<QueueCtl*>(base);
-  b.counters = reinterpret_cast<unsigned long long*>(base + o_cnt);
-  b.qflag = reinterpret_cast<uint32_t*>(base + o_flag);
-  b.bstate = reinterpret_cast<uint32_t*>(base + o_state);
-  b.queue = reinterpret_cast<int32_t*>(base + o_ring);
-  b.T = reinterpret_cast<float*>(base + o_T);
-  b.seen = reinterpret_cast<float*>(base + o_seen);
-  b.qcap = qcap;
-  hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : d->stream;
+  // the array keeps the previous call's contents: everything the solve reads first is reset
+  const AsyncBufs b = {reinterpret_cast<float*>(base + o_T), reinterpret_cast<float*>(base + o_seen),
+                       reinterpret_cast<unsigned long long*>(base + o_word), base,
+                       reinterpret_cast<unsigned long long*>(base + o_cnt)};
   eik_solve_opts_t o;
   eik_solve_opts_default(&o);
-  const bool stage = d->rec_lds != 0;
-  const VisitKernel vk = visit_kernel(d, o.stage_records);
-  const float large = m->dim == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
-  // the array keeps the previous call's contents: everything the solve reads first is reset,
-  // with a fill kernel (no memset nodes if the caller captures this into a graph)
-  FillSegs f;
-  f.count = 0;
-  f.add(b.T, m->nv, (int32_t)__builtin_bit_cast(uint32_t, large));
-  f.add(b.seen, d->nseen, (int32_t)__builtin_bit_cast(uint32_t, EIK_INF));
-  f.add(b.counters, 2 * kNumCounters, 0);
-  f.add(b.queue, (int64_t)qcap * kSlotStride, 0);
-  f.add(b.qflag, d->nblocks, 0);
-  f.add(b.bstate, d->nblocks, 0);
-  f.add(b.ctl, (int64_t)(sizeof(QueueCtl) / 4), 0);
-  int64_t most = 0;
-  for (int k = 0; k < f.count; ++k) most = std::max(most, f.n[k]);
-  hipLaunchKernelGGL(k_fill_segs, dim3((unsigned)std::min<int64_t>(grid1d(most, 256), 2048)),
-                     dim3(256), 0, s, f);
-  hipLaunchKernelGGL(k_seed, dim3(grid1d(nseeds, 256)), dim3(256), 0, s, seeds_dev, nullptr,
-                     nseeds, d->iperm, d->owner, b.T, nullptr, nullptr, m->nv);
-  const AsyncArgs a = async_args(*m, o, b, stage);
-  hipLaunchKernelGGL(k_async_seed, seed_grid(nseeds), dim3(64), 0, s, a, seeds_dev, nseeds,
-                     d->iperm, d->owner, m->nv);
-  int grid = 0;
-  if ((rc = persistent_grid(m->dim, vk, 0, d->nblocks, nseeds, &grid))) return rc;
-  if ((rc = launch_visits(d, vk, a, grid, s))) return rc;
-  hipLaunchKernelGGL(k_gather, dim3(grid1d(m->nv, 256)), dim3(256), 0, s, b.T, d->iperm, m->nv,
-                     T_out_dev);
-  HIP_TRY(hipGetLastError());
-  return EIK_OK;
+  return enqueue_async(*m, o, b, seeds_dev, nullptr, nseeds, T_out_dev,
+                       stream ? reinterpret_cast<hipStream_t>(stream) : d->stream, nullptr, nullptr);
 }
 
 }  // extern "C"
