@@ -125,23 +125,25 @@ __device__ __forceinline__ bool sched_all_clean(const Sched& s) {
   return true;
 }
 
-// Claims a slot for a visit.  The workgroup is counted busy in the same round trip.
-__device__ __forceinline__ bool sched_claim(const Sched& s, Finder& f, uint32_t slot) {
-  uint32_t held = 0;
+// Claims a slot seen unlocked with this key, for a visit: nothing is taken if the word has changed.  (An
+// exchange would take a mark that came in under another workgroup's visit and put it back: for that
+// moment, before the count of the one that took it has landed, every word could look clean.)  The
+// workgroup is counted busy in the same round trip.
+__device__ __forceinline__ bool sched_claim(const Sched& s, Finder& f, uint32_t slot, uint32_t key) {
+  uint32_t got = 0;
   if (__lane_id() == 0) {
     if (!f.busy)
       (void)__hip_atomic_fetch_add(s.ctl, (1ull << 32) + 1ull, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long old = __hip_atomic_exchange(
-        &s.word[slot], (1ull << 32) | kClean, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // under visit already: the mark taken here is put back (the holder unlocks its half alone)
-    held = (uint32_t)(old >> 32);
-    if (held && (uint32_t)old != kClean) sched_mark(s, slot, (uint32_t)old);
+    unsigned long long seen = key;
+    got = __hip_atomic_compare_exchange_strong(&s.word[slot], &seen, (1ull << 32) | kClean,
+                                               __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
   }
   f.busy = true;
   // the count has landed before the visit marks anything
   wait_memory();
-  return __builtin_amdgcn_readfirstlane(held) == 0u;
+  return __builtin_amdgcn_readfirstlane(got) != 0u;
 }
 
 // The next block for this workgroup, claimed; kNoWork at the end of the solve; kGaveUp when the
@@ -186,10 +188,10 @@ __device__ __forceinline__ int32_t sched_find(const Sched& s, Finder& f) {
       const int l = __ffsll((unsigned long long)__ballot(key == best)) - 1;
       f.others = __popcll(__ballot(key != kClean)) - 1;
       const uint32_t slot = (uint32_t)__builtin_amdgcn_readlane((int)at, l);
-      if (sched_claim(s, f, slot)) return sched_block(s, slot);
+      if (sched_claim(s, f, slot, best)) return sched_block(s, slot);
       continue;
     }
-    if (__builtin_amdgcn_readfirstlane(dn)) return kNoWork;
+    if (!f.busy && __builtin_amdgcn_readfirstlane(dn)) return kNoWork;
     if (f.busy) {
       // no more work: every mark of this workgroup's visits has landed
       wait_memory();
