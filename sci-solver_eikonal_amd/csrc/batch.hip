@@ -15,36 +15,35 @@
 
 namespace eik {
 
-// Per solve (blockIdx.y): T = LARGENUM, seen = +inf.
-__global__ void k_multi_init(const SolveDesc* solves) {
+// Per solve (blockIdx.y): T = LARGENUM, seen = +inf, and its blocks' entries of the kind's table.
+__global__ void k_multi_init(const SolveDesc* solves, int32_t* bsolve3, int32_t* bsolve2) {
   const SolveDesc& s = solves[blockIdx.y];
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < s.nseen; i += stride) {
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (int64_t i = i0; i < s.nseen; i += stride) {
     if (i < s.nv) s.T[i] = s.large;
     s.seen[i] = EIK_INF;
   }
+  int32_t* bsolve = s.dim == 3 ? bsolve3 : bsolve2;
+  for (int64_t i = i0; i < s.nblocks; i += stride) bsolve[s.kbase + i] = (int32_t)blockIdx.y;
 }
 
-// Seeds: (solve, caller vertex, value) triples; the owner block of each seed and its dependents
-// are queued, one workgroup per seed and one lane per block to queue (lane 0 the owner), so the
-// pushes' device-scope round trips overlap.  *n is read from device memory so a captured graph
-// serves any seed count.  The arguments of a kind without solves in the launch are all zero, so
-// the descriptors come from `solves`, and a seed's own kind (present by construction) gives the
-// queue.
-__global__ void k_multi_seed(const SolveDesc* solves, MultiArgs a3, MultiArgs a2,
-                             const int32_t* seed_solve, const int32_t* seed_vert,
-                             const float* seed_val, const int32_t* n) {
-  for (int64_t i = blockIdx.x; i < *n; i += gridDim.x) {
-    const int32_t si = seed_solve[i];
-    const SolveDesc& s = solves[si];
-    const MultiArgs& a = s.dim == 3 ? a3 : a2;
-    const int32_t v = s.iperm[seed_vert[i]];
-    if (threadIdx.x == 0) atomicMin(reinterpret_cast<unsigned*>(&s.T[v]), __float_as_uint(seed_val[i]));
+// Seeds: (solve, caller vertex, value) triples (three arrays of cap, then their number, read from
+// device memory so that a captured graph serves any seed count); the owner block of each seed and its
+// dependents are marked, one workgroup per seed and one lane per block to mark.
+__global__ void k_multi_seed(const SolveDesc* solves, Sched s3, Sched s2, const int32_t* seeds,
+                             int64_t cap) {
+  const int32_t n = seeds[3 * cap];
+  for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const SolveDesc& s = solves[seeds[i]];
+    const Sched& q = s.dim == 3 ? s3 : s2;
+    const int32_t v = s.iperm[seeds[cap + i]];
+    const uint32_t t = (uint32_t)seeds[2 * cap + i];
+    if (threadIdx.x == 0) atomicMin(reinterpret_cast<unsigned*>(&s.T[v]), t);
     const int32_t b = s.owner[v];
-    const int32_t tag = si << a.bbits;
     const int32_t s0 = s.dep_start[b], nd = s.dep_start[b + 1] - s0;
     for (int j = threadIdx.x; j <= nd; j += blockDim.x)
-      q_push(a, tag | (s.bbase + (j == 0 ? b : s.dep[s0 + j - 1])));
+      sched_mark(q, sched_slot(q, s.kbase + (j == 0 ? b : s.dep[s0 + j - 1])), t);
   }
 }
 
@@ -73,18 +72,15 @@ __global__ void k_check_factors(const float* f, int64_t n, int32_t* bad) {
   if (b) bad[0] = 1;
 }
 
-__global__ void k_fill_u64(unsigned long long* p, int64_t n) {
+__global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0ull;
+  if (i < n) p[i] = v;
 }
 
-// One launch per element kind: a launch's solves are all tets or all triangles (the two kinds
-// keep separate queues), so the kernel is compiled per kind and keeps the register budget of
-// the single-solve kernel.  Two shapes: BT = kBlockThreads with the element records staged in
-// LDS (the per-solve factors are applied while staging), and BT = kDirectThreads reading the
-// records from memory at every use, whose small LDS footprint lets twice as many workgroups
-// per CU hide each other's latencies (launches without factors: many independent solves keep
-// them all busy).
+// A launch's visits of blocks of any size, one kernel per element kind, in two shapes: BT =
+// kBlockThreads with the element records staged in LDS (the per-solve factors are applied while
+// staging), and BT = kDirectThreads reading the split records from memory at every use, whose small
+// LDS footprint lets twice as many workgroups per CU hide each other's latencies.
 constexpr int kDirectThreads = 128;
 
 // WPE: waves per SIMD the register allocation is sized for (4: at most 128 VGPRs, 3: at most
@@ -93,50 +89,43 @@ constexpr int kDirectThreads = 128;
 template <int DIM, int BT, int WPE>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_visit_multi(
     MultiArgs a, const SolveDesc* __restrict__ solves) {
-  // the shape reading records from memory uses the split records (selection part and lengths)
   constexpr bool kSplit = BT == kDirectThreads;
   extern __shared__ uint4 lds4[];
   __shared__ int sFlag[4];
   __shared__ int sQn[2];  // work-item counters of alternate chunks
-  __shared__ int sEntry;
+  __shared__ int sBlock;
+  __shared__ unsigned sKey;  // smallest time the visit lowered
   __shared__ unsigned long long sRed;
   __shared__ unsigned long long sAcc[kNumCounters];
-  __shared__ int sAgain;
-  __shared__ int sNext;  // entry taken while the previous visit queued its dependents, or -2
-  if (threadIdx.x < kNumCounters) sAcc[threadIdx.x] = 0;
-  if (threadIdx.x == 0) sNext = -2;
-  // No seed of this kind was queued (the seed kernel ran before this launch): nothing will ever
-  // bring `pending` to zero, so the launch ends at once.  Every workgroup checks on entry rather
-  // than one chosen workgroup: with several launches in flight, a given workgroup of this kernel
-  // may not become resident until other kernels' workgroups leave, and those may be waiting on
-  // their own launch in the same way.  pending is zero only before any seed or after the end,
-  // and a repeated q_finish only marks slots no workgroup waits on (it is skipped once the end
-  // is marked).
-  if (threadIdx.x == 0 &&
-      (__hip_atomic_load(&a.ctl->tp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffffffffull) == 0ull &&
-      (__hip_atomic_load(&a.ctl->head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kDoneBit) == 0u)
-    q_finish(a);
+  const Sched& s = a.loop.s;
+  const int tid = threadIdx.x;
+  if (tid < kNumCounters) sAcc[tid] = 0;
+  // the second wave looks for work, while the first hands on what the last visit did
+  const bool finder = tid >= 64 && tid < 128;
+  Finder f;
+  if (finder) sched_enter(s, f, blockIdx.x);
+  if (tid == 0) sBlock = kNothing;
+  wait_memory();
+  __syncthreads();
   for (;;) {
-    if (threadIdx.x == 0) {
-      int ne = sNext;
-      if (ne == -2) {
-        const unsigned long long w0 = wall_clock64();
-        ne = q_take(a);
-        sAcc[6] += wall_clock64() - w0;
-        if (ne == kAbandoned) sAcc[kCntAbandoned] += 1;
+    if (sBlock == kNothing) {
+      __syncthreads();
+      if (finder) {
+        const int32_t nb = find_next(s, f, sAcc);
+        if (tid == 64) sBlock = nb;
       }
-      sEntry = ne;
-      sNext = -2;
+      __syncthreads();
     }
-    __syncthreads();
+    if (tid == 0) {
+      sRed = 0;
+      sKey = kClean;
+    }
     // uniform across the workgroup: kept in scalar registers, the descriptor read with scalar
     // loads
-    const int entry = __builtin_amdgcn_readfirstlane(sEntry);
-    if (entry < 0) break;
-    const int si = entry >> a.bbits;
-    const SolveDesc& sD = solves[si];
-    const int g = entry & a.bmask;
-    const int b = g - sD.bbase;
+    const int g = __builtin_amdgcn_readfirstlane(sBlock);
+    if (g < 0) break;
+    const SolveDesc& sD = solves[a.bsolve[g]];
+    const int b = g - sD.kbase;
     VisitArgs v;
     v.blocks = sD.blocks;
     v.elems = kSplit ? sD.esel : sD.elems;
@@ -144,8 +133,8 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     v.T = sD.T;
     v.seen = sD.seen;
     v.large = sD.large;
-    v.eps = a.eps;
-    v.max_inner = a.max_inner;
+    v.eps = a.loop.eps;
+    v.max_inner = a.loop.max_inner;
     v.queue_cap = a.queue_cap;
     v.rec_lds = BT == kBlockThreads;
     v.vh_start = nullptr;
@@ -154,96 +143,99 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     v.vmask = sD.vmask;
     v.rmult = sD.rmult;
     v.lens = sD.elen;
-    bool rerun = false;  // the previous visit of this workgroup was of this block
-    do {
-      if (threadIdx.x == 0) sRed = 0;
-      const unsigned long long t0 = wall_clock64();
-      const BlockDesc d = v.blocks[b];
-      VisitLds l = carve_lds<DIM>(lds4, a.rec_lds_bytes, a.queue_cap, d);
-      uint64_t solves = 0;
-      VisitResult r = visit_block<DIM, true, BT, kSplit>(v, b, l.rec, l.T, l.old, l.chg, l.hidx, l.vm, l.q,
-                                                 l.mark, sFlag, sQn, &solves, rerun);
+    const unsigned long long t0 = wall_clock64();
+    const BlockDesc d = v.blocks[b];
+    const VisitLds l = carve_lds<DIM>(lds4, a.rec_lds_bytes, a.queue_cap, d);
+    uint64_t solves_done = 0;
+    const VisitResult r = visit_block<DIM, true, BT, kSplit>(v, b, l.rec, l.T, l.old, l.chg, l.hidx,
+                                                             l.vm, l.q, l.mark, sFlag, sQn,
+                                                             &solves_done);
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) solves += __shfl_down(solves, off, 64);
-      // sRed is read by thread 0 after the next barrier
-      if (__lane_id() == 0) atomicAdd(&sRed, (unsigned long long)solves);
-      const unsigned long long tq = wall_clock64();
-      const bool cap_ok = (int64_t)sAcc[0] < a.max_visits;
-      // the first 64 dependents are flagged while thread 0 releases the block (see
-      // k_visit_async)
-      const int32_t s0 = v.dep_start[b];
-      const int ndep = r.bnd_changed && cap_ok ? v.dep_start[b + 1] - s0 : 0;
+    for (int off = 32; off > 0; off >>= 1) solves_done += __shfl_down(solves_done, off, 64);
+    if (__lane_id() == 0) atomicAdd(&sRed, (unsigned long long)solves_done);
+    uint32_t key = kClean;
+    for (int i = tid; i < d.nown; i += BT)
+      if (l.T[i] < l.old[i]) key = min(key, __float_as_uint(l.T[i]));
+    key = wave_umin(key);
+    if (__lane_id() == 0 && key != kClean) atomicMin(&sKey, key);
+    __syncthreads();
+    const unsigned long long tq = wall_clock64();
+    if (tid < 64) {
+      // the visit's times have reached the device's coherence point (visit_block)
+      const bool open = (int64_t)sAcc[0] < a.loop.max_visits;
       const uint64_t mask = v.vmask ? ((uint64_t)(uint32_t)l.mark[0] |
                                        ((uint64_t)(uint32_t)l.mark[1] << 32))
                                     : ~0ull;
-      bool want0 = false;
-      int32_t c0 = g;
-      if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        if (lane < ndep) {
-          want0 = !v.vmask || ((mask >> lane) & 1ull) != 0ull;
-          c0 = sD.bbase + sD.dep[s0 + lane];
-          if (want0) want0 = atomicExch(&a.qflag[c0], 1u) == 0u;
-        }
-        if (lane == 0) sAgain = release_or_rerun(a, g) && cap_ok;
+      const int32_t s0 = v.dep_start[b];
+      const int ndep = r.bnd_changed && open ? v.dep_start[b + 1] - s0 : 0;
+      const uint32_t k = sKey;
+      for (int j = tid; j < ndep; j += 64)
+        if (!v.vmask || ((mask >> (j & 63)) & 1ull))
+          sched_mark(s, sched_slot(s, sD.kbase + sD.dep[s0 + j]), k);
+      wait_memory();  // the marks have landed before this block can count as clean
+      if (tid == 0) {
+        // an unconverged block waits with the smallest time it lowered
+        sched_leave(s, sched_slot(s, g), !r.converged && open ? k : kClean);
+        tally_visit(sAcc, d, r, sRed, kAlgoElemBytes<DIM>, tq - t0, false, false);
+        sAcc[10] += wall_clock64() - tq;
       }
-      __syncthreads();
-      const int again = sAgain;
-      if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        const int32_t tag = si << a.bbits;
-        const int nitems = ndep + 1;
-        for (int j0 = 0; j0 < nitems; j0 += 64) {
-          const int j = j0 + lane;
-          bool want = false;
-          int32_t c = g;
-          if (j0 == 0 && j < ndep) {
-            want = want0;
-            c = c0;
-          } else {
-            if (j < ndep) {
-              want = !v.vmask || ((mask >> (j & 63)) & 1ull) != 0ull;
-              c = sD.bbase + sD.dep[s0 + j];
-            } else if (j == ndep) {
-              want = !r.converged && !again && cap_ok;
-            }
-            if (want) want = atomicExch(&a.qflag[c], 1u) == 0u;
-          }
-          const uint64_t bal = __ballot(want);
-          const unsigned n = (unsigned)__popcll(bal);
-          const unsigned dec = (j0 + 64 >= nitems && !again) ? 1u : 0u;
-          if (n == 0u && dec == 0u) continue;
-          uint32_t base = 0;
-          if (lane == 0) {
-            const unsigned long long inc = ((unsigned long long)n << 32) + n - dec;
-            const unsigned long long old = __hip_atomic_fetch_add(
-                &a.ctl->tp, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            base = (uint32_t)(old >> 32);
-            if (n == 0u && (old & 0xffffffffull) == 1ull) q_finish(a);
-          }
-          base = __shfl(base, 0, 64);
-          if (want)
-            __hip_atomic_store(q_slot(a, base + (uint32_t)__popcll(bal & lane_mask_lt())),
-                               (tag | c) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (lane == 0) {
-          tally_visit(sAcc, d, r, sRed, kAlgoElemBytes<DIM>, tq - t0, rerun, rerun && v.rec_lds);
-          sAcc[10] += wall_clock64() - tq;
-        }
-      } else if (threadIdx.x == 64 && !again) {
-        // next entry taken while wave 0 queues the dependents (no re-run: nothing held)
-        const unsigned long long w0 = wall_clock64();
-        const int32_t nx = q_take(a);
-        sNext = nx;
-        sAcc[6] += wall_clock64() - w0;
-        if (nx == kAbandoned) sAcc[kCntAbandoned] += 1;
-      }
-      __syncthreads();
-      rerun = true;
-    } while (sAgain);
+    } else if (finder) {
+      const int32_t nb = find_next(s, f, sAcc, true);
+      if (tid == 64) sBlock = nb;
+    }
+    // The wait is written out: hipcc 7.2 leaves it away before a barrier that heads this loop, and a
+    // wave that passes the barrier then reads the block of the visit before.
+    wait_memory();
+    __syncthreads();
   }
-  if (threadIdx.x < kNumCounters && sAcc[threadIdx.x])
-    atomicAdd(&a.counters[threadIdx.x], sAcc[threadIdx.x]);
+  if (tid < kNumCounters && sAcc[tid]) atomicAdd(&a.counters[tid], sAcc[tid]);
+}
+
+struct MultiBlocks {
+  const SolveDesc* solves;
+  const int32_t* bsolve;
+  __device__ __forceinline__ BlockData operator()(int32_t g) const {
+    const SolveDesc& s = solves[bsolve[g]];
+    return {s.blocks, s.elems, s.halo,  s.T,     s.seen,      s.vmask,
+            s.dep_start, s.dep, s.rmult, s.items, g - s.kbase, s.kbase};
+  }
+};
+
+// A launch's visits of register-resident blocks (visit_loop.h).  KINDS: 1 tets, 2 triangles, 3 both: half
+// the workgroups begin with each kind and go on to the other when it has ended, so that a launch of
+// both takes about as long as the longer one instead of the sum, without two persistent kernels
+// waiting for each other's slots.
+template <int KINDS, int BT>
+__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_multi_resident(
+    MultiArgs a3, MultiArgs a2) {
+  extern __shared__ uint4 lds4[];
+  __shared__ LoopShared sh;
+  if (threadIdx.x < kNumCounters) sh.acc[threadIdx.x] = 0;
+  for (int pass = 0; pass < (KINDS == 3 ? 2 : 1); ++pass) {
+    const bool tets = KINDS == 1 || (KINDS == 3 && ((blockIdx.x ^ (unsigned)pass) & 1u) == 0u);
+    // both: even workgroups own tet blocks, odd ones triangle blocks (a lone workgroup both)
+    const uint32_t me = KINDS != 3 ? blockIdx.x
+                        : pass == 0 ? blockIdx.x >> 1 : gridDim.x == 1 ? 0u : 0xffffffffu;
+    if constexpr ((KINDS & 1) != 0) {
+      if (tets) resident_loop<3, kTetN<BT>, BT>(a3.loop, MultiBlocks{a3.solves, a3.bsolve}, me, lds4, sh);
+    }
+    if constexpr ((KINDS & 2) != 0) {
+      if (!tets) resident_loop<2, 4, BT>(a2.loop, MultiBlocks{a2.solves, a2.bsolve}, me, lds4, sh);
+    }
+  }
+  unsigned long long* counters = KINDS == 2 ? a2.counters : a3.counters;
+  if (threadIdx.x < kNumCounters && sh.acc[threadIdx.x])
+    atomicAdd(&counters[threadIdx.x], sh.acc[threadIdx.x]);
+}
+
+template <int KINDS>
+static const void* multi_resident(int bt) {
+  return bt == 256   ? (const void*)k_visit_multi_resident<KINDS, 256>
+         : bt == 512 ? (const void*)k_visit_multi_resident<KINDS, 512>
+                     : (const void*)k_visit_multi_resident<KINDS, 1024>;
+}
+static const void* multi_resident(int kinds, int bt) {
+  return kinds == 1 ? multi_resident<1>(bt) : kinds == 2 ? multi_resident<2>(bt) : multi_resident<3>(bt);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -333,10 +325,23 @@ static void launch_visits(const Group& g, size_t lds, hipStream_t s, const Multi
     hipLaunchKernelGGL((k_visit_multi<DIM, BT, 4>), dim3(g.grid), dim3(BT), lds, s, a, sd);
 }
 
+// Blocks per resident workgroup from which on a launch of tet blocks reads its records from memory.
+constexpr int kBusyBlocks = 24;
+
+// Resident workgroups of a register-resident launch.
+static int resident_grid(const void* fn, int bt, size_t lds, int requested, int* out) {
+  int dev = 0, ncu = 0, per = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, bt, lds));
+  const int resident = std::min(std::max(1, ncu * std::max(per, 1)), 64 * ncu);
+  *out = requested > 0 ? std::min(requested, resident) : resident;
+  return EIK_OK;
+}
+
 void launch_free(Launch& L) {
-  void* ptrs[] = {L.grp[0].queue, L.grp[0].qctl, L.grp[1].queue, L.grp[1].qctl, L.dsolves,
-                  L.qflag,        L.bstate,      L.counters,     L.out,         L.d_sseed,
-                  L.d_vseed,      L.d_nseed,     L.d_fseed};
+  void* ptrs[] = {L.grp[0].words, L.grp[0].sctl, L.grp[0].bsolve, L.grp[1].words, L.grp[1].sctl,
+                  L.grp[1].bsolve, L.dsolves, L.counters, L.out, L.d_seed};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (L.hsolves) (void)hipHostFree(L.hsolves);
@@ -368,6 +373,7 @@ int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
     g.dim = gi == 0 ? 3 : 2;
     int32_t max_local = 0, max_own = 0, max_dep = 2, qcap_l = 256;
     size_t rec_bytes = 0;
+    bool resident = true;  // every block of the kind fits register-resident visits
     for (Mesh* m : kinds) {
       if (m->dim != g.dim) continue;
       g.present = true;
@@ -379,7 +385,13 @@ int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
       max_dep = std::max(max_dep, Ly.max_dep);
       qcap_l = std::max(qcap_l, std::min(8192, K * Ly.max_elem));
       rec_bytes = std::max(rec_bytes, ((size_t)Ly.max_elem * rb + 15) & ~(size_t)15);
+      g.max_local = std::max(g.max_local, Ly.max_local);
+      g.max_elem = std::max(g.max_elem, Ly.max_elem);
+      g.max_items = std::max(g.max_items, Ly.max_items);
+      resident = resident && m->dev->res_n != 0;
+      g.res_bt = std::max(g.res_bt, (int)m->dev->res_bt);
     }
+    if (!resident) g.res_bt = 0;
     if (!g.present) continue;
     Layout probe;
     probe.max_local = max_local;
@@ -410,13 +422,31 @@ int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
     }
     g.rec_lds_bytes = rec_bytes;
     g.queue_cap = qcap_l;
-    // ring capacity: every block queued at once plus a waiting ticket per resident workgroup
-    // (at most 64 per CU), twice over
-    uint32_t qcap = 1;
-    while (qcap < 2u * ((uint32_t)cap_blocks + 64u * (uint32_t)std::max(ncu, 1)) + 2u) qcap <<= 1;
-    g.qcap = qcap;
-    HIP_TRY(hipMalloc((void**)&g.queue, sizeof(int32_t) * kSlotStride * qcap));
-    HIP_TRY(hipMalloc((void**)&g.qctl, sizeof(QueueCtl)));
+    if (g.res_bt) {
+      g.lds[2] = loop_lds_bytes(g.dim, g.max_local, g.max_elem, g.max_items);
+      if (g.lds[2] > (size_t)max_lds) g.res_bt = 0;
+    }
+    // at most 64 workgroups per CU own words
+    HIP_TRY(hipMalloc((void**)&g.words, sizeof(unsigned long long) *
+                                            sched_max_words(cap_blocks, 64 * (size_t)std::max(ncu, 1))));
+    HIP_TRY(hipMalloc((void**)&g.sctl, kSchedCtlBytes));
+    HIP_TRY(hipMalloc((void**)&g.bsolve, sizeof(int32_t) * std::max<int64_t>(cap_blocks, 1)));
+  }
+  // the register-resident kernels that may run, for their LDS (a merged launch takes the larger
+  // workgroup and LDS of the two kinds)
+  for (int kinds = 1; kinds <= 3; ++kinds) {
+    int bt = 0;
+    size_t lds = 0;
+    bool all = true;
+    for (int gi = 0; gi < 2; ++gi) {
+      if (!((kinds >> gi) & 1)) continue;
+      all = all && L.grp[gi].res_bt > 0;
+      bt = std::max(bt, L.grp[gi].res_bt);
+      lds = std::max(lds, L.grp[gi].lds[2]);
+    }
+    if (all && lds > 65536)
+      HIP_TRY(hipFuncSetAttribute(multi_resident(kinds, bt),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   }
   L.cap_solves = cap_solves;
   L.cap_blocks = cap_blocks;
@@ -427,14 +457,9 @@ int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
   HIP_TRY(hipEventCreate(&L.ev1));
   HIP_TRY(hipMalloc((void**)&L.dsolves, sizeof(SolveDesc) * cap_solves));
   HIP_TRY(hipHostMalloc((void**)&L.hsolves, sizeof(SolveDesc) * cap_solves));
-  HIP_TRY(hipMalloc((void**)&L.qflag, sizeof(uint32_t) * cap_blocks));
-  HIP_TRY(hipMalloc((void**)&L.bstate, sizeof(uint32_t) * cap_blocks));
   HIP_TRY(hipMalloc((void**)&L.counters, sizeof(unsigned long long) * kNumCounters));
   HIP_TRY(hipMalloc((void**)&L.out, sizeof(float) * cap_nv));
-  HIP_TRY(hipMalloc((void**)&L.d_sseed, sizeof(int32_t) * L.cap_seeds));
-  HIP_TRY(hipMalloc((void**)&L.d_vseed, sizeof(int32_t) * L.cap_seeds));
-  HIP_TRY(hipMalloc((void**)&L.d_fseed, sizeof(float) * L.cap_seeds));
-  HIP_TRY(hipMalloc((void**)&L.d_nseed, sizeof(int32_t)));
+  HIP_TRY(hipMalloc((void**)&L.d_seed, sizeof(int32_t) * (3 * L.cap_seeds + 1)));
   HIP_TRY(hipHostMalloc((void**)&L.h_seed, sizeof(int32_t) * (3 * L.cap_seeds + 1)));
   HIP_TRY(hipHostMalloc((void**)&L.h_out, sizeof(float) * cap_nv));
   HIP_TRY(hipHostMalloc((void**)&L.h_cnt, sizeof(unsigned long long) * kNumCounters));
@@ -463,54 +488,88 @@ void solve_desc(SolveDesc& s, Mesh* m, float* T, float* seen, const float* rmult
   s.T = T;
   s.seen = seen;
   s.nv = m->nv;
+  s.items = {d->item_range, d->item_id, d->item_len, d->item_rec};
   s.nseen = d->nseen;
   s.nblocks = d->nblocks;
   s.dim = m->dim;
   s.large = m->dim == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
 }
 
+// Numbers the blocks of each element kind over the launch's solves; n[0], n[1]: their numbers.
+static void launch_bases(SolveDesc* sd, int32_t nsolves, int64_t n[2]) {
+  n[0] = n[1] = 0;
+  for (int32_t i = 0; i < nsolves; ++i) {
+    int64_t& k = n[sd[i].dim == 3 ? 0 : 1];
+    sd[i].kbase = (int32_t)k;
+    k += sd[i].nblocks;
+  }
+}
+
 int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solve_opts_t& o,
                 MultiArgs a[2]) {
-  // queue entries: solve index above the launch-wide block index, both in 31 bits
-  int32_t bbits = 1;
-  while ((1ll << bbits) <= total_blocks) ++bbits;
-  if (bbits > 30 || ((int64_t)nsolves << bbits) >= (1ll << 31) - 1)
-    return fail(EIK_ERR_CAPACITY, "too many blocks and solves in one launch");
+  if (total_blocks >= (1ll << 30)) return fail(EIK_ERR_CAPACITY, "too many blocks in one launch");
+  // the blocks of each kind, numbered together
+  int64_t kblocks[2];
+  launch_bases(L.hsolves, nsolves, kblocks);
   for (int gi = 0; gi < 2; ++gi) {
     Group& g = L.grp[gi];
     std::memset(&a[gi], 0, sizeof(MultiArgs));
     if (!g.present) continue;
-    // many independent solves keep every workgroup busy: records read from memory, smaller
-    // workgroups, unless staging is asked for
-    g.shape = o.stage_records == EIK_STAGE_LDS ? 0 : 1;
-    if (g.shape == 0 && g.lds[0] == 0)
+    if (o.stage_records == EIK_STAGE_LDS && g.lds[0] == 0)
       return fail(EIK_ERR_CAPACITY, "the element records of a block do not fit the LDS for "
                                     "staging; use fewer vertices per block or read the records "
                                     "from memory (EIK_STAGE_AUTO)");
+    g.shape = o.stage_records == EIK_STAGE_LDS ? 0 : 1;
+    if (o.stage_records != EIK_STAGE_AUTO || g.res_bt == 0) continue;
+    // Register-resident visits, whose chain is short, unless there are so many tet blocks that every
+    // workgroup stays busy from its first visit to its last: then the records are read from memory at
+    // every use by smaller workgroups, of which more fit a CU.  Cubes of 16..48 vertices a side, resident /
+    // direct, ms: 14 blocks per resident workgroup 2.41 / 3.83 (192 vertices per block), 21 3.34 / 3.44
+    // (128) and 3.06 / 3.17 (64), 28 4.39 / 3.64 (192), 48 8.6 / 5.6 (192).  Triangle blocks are as
+    // small resident: level-7 spheres 1.5 / 10.8.
+    int per = 0, rc = resident_grid(multi_resident(1 << gi, g.res_bt), g.res_bt, g.lds[2], 0, &per);
+    if (rc) return rc;
+    g.shape = gi == 0 && kblocks[0] > (int64_t)kBusyBlocks * per ? 1 : 2;
+  }
+  L.merged = L.grp[0].present && L.grp[1].present && L.grp[0].shape == 2 && L.grp[1].shape == 2;
+  for (int gi = 0; gi < 2; ++gi) {
+    Group& g = L.grp[gi];
+    if (!g.present) continue;
     int rc;
-    if (g.shape == 0)
+    if (g.shape == 2) {
+      const Group& h = L.merged ? L.grp[1 - gi] : g;
+      const int bt = std::max(g.res_bt, h.res_bt);
+      rc = resident_grid(multi_resident(L.merged ? 3 : 1 << gi, bt), bt, std::max(g.lds[2], h.lds[2]),
+                         o.workgroups, &g.grid);
+      // no more than one workgroup per block
+      const int64_t most = L.merged ? 2 * std::max(kblocks[0], kblocks[1]) : kblocks[gi];
+      g.grid = (int)std::min<int64_t>(g.grid, std::max<int64_t>(most, 1));
+    } else if (g.shape == 0) {
       rc = gi == 0 ? group_grid<3, kBlockThreads>(g.lds[0], o.workgroups, &g.grid, &g.wpe)
                    : group_grid<2, kBlockThreads>(g.lds[0], o.workgroups, &g.grid, &g.wpe);
-    else
+    } else {
       rc = gi == 0 ? group_grid<3, kDirectThreads>(g.lds[1], o.workgroups, &g.grid, &g.wpe)
                    : group_grid<2, kDirectThreads>(g.lds[1], o.workgroups, &g.grid, &g.wpe);
+    }
     if (rc) return rc;
     MultiArgs& x = a[gi];
     x.solves = L.dsolves;
-    x.queue = g.queue;
-    x.qflag = L.qflag;
-    x.bstate = L.bstate;
-    x.ctl = g.qctl;
-    x.qmask = g.qcap - 1u;
-    x.bbits = bbits;
-    x.bmask = (int32_t)((1u << bbits) - 1u);
+    x.loop.s.word = g.words;
+    x.loop.s.ctl = reinterpret_cast<unsigned long long*>(g.sctl);
+    x.loop.s.done = reinterpret_cast<uint32_t*>(g.sctl + kSchedCtlBytes / 2);
+    // a merged launch's even workgroups own the tet blocks, its odd ones the triangle blocks
+    sched_shape(x.loop.s, std::max<int64_t>(kblocks[gi], 1),
+                L.merged ? std::max(1, (g.grid + 1 - gi) / 2) : g.grid);
+    x.loop.s.wait_limit = wait_limit_ticks(L.device, o.wait_limit_us);
+    x.loop.eps = o.eps;
+    x.loop.max_inner = default_inner_sweeps(g.dim, o.max_inner);
+    x.loop.max_visits = (int64_t)(o.max_iterations > 0 ? o.max_iterations : 1000) * std::max<int64_t>(total_blocks, 1);
+    x.loop.max_local = g.max_local;
+    x.loop.max_elem = g.max_elem;
+    x.bsolve = g.bsolve;
     x.counters = L.counters;
-    x.eps = o.eps;
-    x.max_inner = default_inner_sweeps(g.dim, o.max_inner);
     x.queue_cap = g.queue_cap;
     x.rec_lds_bytes = g.shape == 0 ? g.rec_lds_bytes : 0;
-    x.max_visits = (int64_t)(o.max_iterations > 0 ? o.max_iterations : 1000) * std::max<int64_t>(total_blocks, 1);
-    x.wait_limit = wait_limit_ticks(L.device, o.wait_limit_us);
   }
   return EIK_OK;
 }
@@ -520,7 +579,7 @@ int launch_check_end(const Launch& L) {
   if (n == 0) return EIK_OK;
   for (int gi = 0; gi < 2; ++gi)
     if (L.grp[gi].present) {
-      int rc = check_queue_end(L.grp[gi].qctl, L.stream, n);
+      int rc = check_end(L.grp[gi].sctl, L.stream, n);
       if (rc) return rc;
     }
   return EIK_OK;
@@ -539,29 +598,21 @@ int launch_issue(Launch& L, int32_t nsolves, int64_t total_blocks, int64_t total
   const int64_t cap = L.cap_seeds;
   if (upload_desc)
     HIP_TRY(hipMemcpyAsync(L.dsolves, L.hsolves, sizeof(SolveDesc) * nsolves, hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(L.d_sseed, L.h_seed, sizeof(int32_t) * cap, hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(L.d_vseed, L.h_seed + cap, sizeof(int32_t) * cap, hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(L.d_fseed, L.h_seed + 2 * cap, sizeof(float) * cap, hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(L.d_nseed, L.h_seed + 3 * cap, sizeof(int32_t), hipMemcpyHostToDevice, s));
+  HIP_TRY(hipMemcpyAsync(L.d_seed, L.h_seed, sizeof(int32_t) * (3 * cap + 1), hipMemcpyHostToDevice, s));
+  FillSegs f;
+  f.add(L.counters, 2 * kNumCounters, 0);
   for (int gi = 0; gi < 2; ++gi) {
-    const Group& g = L.grp[gi];
-    if (!g.present) continue;
-    const int64_t qwords = (int64_t)g.qcap * kSlotStride;
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid1d(qwords, 256)), dim3(256), 0, s, g.queue, qwords, 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, s, reinterpret_cast<int32_t*>(g.qctl),
-                       (int64_t)(sizeof(QueueCtl) / 4), 0);
+    if (!L.grp[gi].present) continue;
+    f.add(L.grp[gi].sctl, kSchedCtlBytes / 4, 0);
+    f.words[gi] = a[gi].loop.s.word;
+    f.nwords[gi] = (int64_t)a[gi].loop.s.owners * a[gi].loop.s.stride;
   }
-  if (total_blocks > 0) {
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid1d(total_blocks, 256)), dim3(256), 0, s,
-                       reinterpret_cast<int32_t*>(L.qflag), total_blocks, 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid1d(total_blocks, 256)), dim3(256), 0, s,
-                       reinterpret_cast<int32_t*>(L.bstate), total_blocks, 0);
-  }
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, L.counters, (int64_t)kNumCounters);
-  hipLaunchKernelGGL(k_multi_init, dim3(64, nsolves), dim3(256), 0, s, L.dsolves);
+  launch_fill(f, s);
+  hipLaunchKernelGGL(k_multi_init, dim3(64, nsolves), dim3(256), 0, s, L.dsolves, L.grp[0].bsolve,
+                     L.grp[1].bsolve);
   hipLaunchKernelGGL(k_multi_seed, dim3((unsigned)std::min<int64_t>(cap, 1 << 16)), dim3(64), 0, s,
-                     (const SolveDesc*)L.dsolves, a[0], a[1], L.d_sseed, L.d_vseed, L.d_fseed,
-                     L.d_nseed);
+                     (const SolveDesc*)L.dsolves, a[0].loop.s, a[1].loop.s, (const int32_t*)L.d_seed,
+                     cap);
   const SolveDesc* sd = L.dsolves;
   const Group& g3 = L.grp[0];
   const Group& g2 = L.grp[1];
@@ -569,6 +620,17 @@ int launch_issue(Launch& L, int32_t nsolves, int64_t total_blocks, int64_t total
   if (g3.present && g3.shape == 1) launch_visits<3, kDirectThreads>(g3, g3.lds[1], s, a[0], sd);
   if (g2.present && g2.shape == 0) launch_visits<2, kBlockThreads>(g2, g2.lds[0], s, a[1], sd);
   if (g2.present && g2.shape == 1) launch_visits<2, kDirectThreads>(g2, g2.lds[1], s, a[1], sd);
+  void* args[] = {(void*)&a[0], (void*)&a[1]};
+  if (L.merged) {
+    const int bt = std::max(g3.res_bt, g2.res_bt);
+    HIP_TRY(hipLaunchKernel(multi_resident(3, bt), dim3(g3.grid), dim3(bt), args,
+                            std::max(g3.lds[2], g2.lds[2]), s));
+  } else {
+    for (int gi = 0; gi < 2; ++gi)
+      if (L.grp[gi].present && L.grp[gi].shape == 2)
+        HIP_TRY(hipLaunchKernel(multi_resident(1 << gi, L.grp[gi].res_bt), dim3(L.grp[gi].grid),
+                                dim3(L.grp[gi].res_bt), args, L.grp[gi].lds[2], s));
+  }
   HIP_TRY(hipMemcpyAsync(L.h_cnt, L.counters, sizeof(unsigned long long) * kNumCounters,
                          hipMemcpyDeviceToHost, s));
   HIP_TRY(hipGetLastError());
@@ -675,6 +737,8 @@ static int batch_alloc(Batch* b, int64_t seed_cap) {
     off += m->nv;
     bbase += s.nblocks;
   }
+  int64_t n[2];
+  launch_bases(b->L.hsolves, (int32_t)b->meshes.size(), n);
   HIP_TRY(hipMemcpy(b->L.dsolves, b->L.hsolves, sizeof(SolveDesc) * b->meshes.size(),
                     hipMemcpyHostToDevice));
   return EIK_OK;

@@ -35,6 +35,8 @@ struct Sched {
   uint32_t owners;           // G: workgroups of the launch
   uint32_t per_owner;        // words per owner
   uint32_t stride;           // slots from one owner's words to the next's
+  uint32_t windows;          // of 64 slots
+  uint32_t step;             // windows from one look to the next: a walk over all of them
   int32_t nblocks;
   unsigned long long wait_limit;  // wall-clock ticks a workgroup may find no work
 };
@@ -45,6 +47,8 @@ inline void sched_shape(Sched& s, int64_t nblocks, int64_t owners) {
   s.owners = (uint32_t)owners;
   s.per_owner = (uint32_t)((nblocks + owners - 1) / owners);
   s.stride = s.per_owner == 1 ? 16 : s.per_owner;
+  s.windows = (s.owners * s.stride + 63) / 64;
+  s.step = s.windows % 37 ? 37 % s.windows : 1;
   s.nblocks = (int32_t)nblocks;
 }
 inline size_t sched_max_words(size_t nblocks, size_t max_owners) {
@@ -87,12 +91,14 @@ __device__ __forceinline__ void wait_memory() {
 // What one wave of a workgroup keeps between its searches.
 struct Finder {
   bool busy = false;  // counted in ctl
+  uint32_t me;        // the workgroup's owner index; s.owners or more: it owns no blocks
   uint32_t probe;     // next slot to look at among all
   int others = 0;     // dirty blocks seen beside the one claimed
+  uint32_t idle = 0;  // looks so far (one block per owner)
   uint64_t waits = 0; // those of the last look that were dirty (one block per owner)
 };
 
-constexpr int32_t kNoWork = -1, kGaveUp = -3;
+constexpr int32_t kNoWork = -1, kNothing = -2, kGaveUp = -3;
 
 // Smallest value over the lanes of a wave (uniform).
 __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
@@ -146,61 +152,64 @@ __device__ __forceinline__ bool sched_claim(const Sched& s, Finder& f, uint32_t 
   return __builtin_amdgcn_readfirstlane(got) != 0u;
 }
 
-// The next block for this workgroup, claimed; kNoWork at the end of the solve; kGaveUp when the
-// wait outlasted s.wait_limit.  Called by one whole wave.
-__device__ __forceinline__ int32_t sched_find(const Sched& s, Finder& f) {
+// One look: a block for this workgroup, claimed; kNoWork at the end of the solve; kNothing if there is
+// none now.  Called by one whole wave.
+__device__ __forceinline__ int32_t sched_look(const Sched& s, Finder& f) {
   const uint32_t lane = __lane_id();
-  const uint32_t own = blockIdx.x * s.stride;
+  const uint32_t own = f.me * s.stride;
   const uint32_t total = s.owners * s.stride;
+  const uint32_t dn = __hip_atomic_load(s.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint32_t key = kClean, at = 0;
+  for (uint32_t base = lane; base < s.per_owner && f.me < s.owners; base += 64) {
+    const unsigned long long v = load_word(&s.word[own + base]);
+    if ((v >> 32) == 0ull && (uint32_t)v < key) key = (uint32_t)v, at = own + base;
+  }
+  // With several blocks per owner, a window of all words too: the smallest key of the two looks
+  // is near the smallest of the launch, and an idle workgroup finds what a busy owner leaves.
+  // With one block per owner its owner visits it, resident; now and then a window is looked at
+  // for blocks that stay dirty because their owner is not running (yet).
+  if (s.per_owner > 1 || (++f.idle & 63u) == 0u) {
+    const uint32_t i = f.probe + lane;
+    const unsigned long long v = i < total ? load_word(&s.word[i]) : (unsigned long long)kClean;
+    bool take = (v >> 32) == 0ull;
+    bool next = true;
+    if (s.per_owner == 1) {
+      const uint64_t waits = __ballot(v < (unsigned long long)kClean);
+      take = take && ((f.waits >> lane) & 1ull);
+      next = (f.waits & waits) == 0ull && f.waits != 0ull;
+      f.waits = f.waits ? 0ull : waits;
+      next = next || f.waits == 0ull;
+    }
+    if (take && (uint32_t)v < key) key = (uint32_t)v, at = i;
+    if (next) {
+      f.probe += 64 * s.step;
+      while (f.probe >= 64 * s.windows) f.probe -= 64 * s.windows;
+    }
+  }
+  const uint32_t best = wave_umin(key);
+  // (done is not set while a workgroup is busy; one that is never leaves without lowering ctl)
+  if (best == kClean) return !f.busy && __builtin_amdgcn_readfirstlane(dn) ? kNoWork : kNothing;
+  const int l = __ffsll((unsigned long long)__ballot(key == best)) - 1;
+  f.others = __popcll(__ballot(key != kClean)) - 1;
+  const uint32_t slot = (uint32_t)__builtin_amdgcn_readlane((int)at, l);
+  return sched_claim(s, f, slot, best) ? sched_block(s, slot) : kNothing;
+}
+
+// The next block for this workgroup, claimed; kNoWork at the end of the solve; kGaveUp when the
+// wait outlasted s.wait_limit.  Called by one whole wave, when every mark and release of the
+// workgroup's visits has landed.
+__device__ __forceinline__ int32_t sched_find(const Sched& s, Finder& f) {
   unsigned long long since = 0;
-  uint32_t idle = 0;
   for (;;) {
-    const uint32_t dn = __hip_atomic_load(s.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t key = kClean, at = 0;
-    for (uint32_t base = lane; base < s.per_owner; base += 64) {
-      const unsigned long long v = load_word(&s.word[own + base]);
-      if ((v >> 32) == 0ull && (uint32_t)v < key) key = (uint32_t)v, at = own + base;
-    }
-    // With several blocks per owner, a window of all words too: the smallest key of the two looks
-    // is near the smallest of the launch, and an idle workgroup finds what a busy owner leaves.
-    // With one block per owner its owner visits it, resident; now and then a window is looked at
-    // for blocks that stay dirty because their owner is not running (yet).
-    if (s.per_owner > 1 || (++idle & 63u) == 0u) {
-      const uint32_t i = f.probe + lane;
-      const unsigned long long v = i < total ? load_word(&s.word[i]) : (unsigned long long)kClean;
-      bool take = (v >> 32) == 0ull;
-      bool next = true;
-      if (s.per_owner == 1) {
-        const uint64_t waits = __ballot(v < (unsigned long long)kClean);
-        take = take && ((f.waits >> lane) & 1ull);
-        next = (f.waits & waits) == 0ull && f.waits != 0ull;
-        f.waits = f.waits ? 0ull : waits;
-        next = next || f.waits == 0ull;
-      }
-      if (take && (uint32_t)v < key) key = (uint32_t)v, at = i;
-      if (next) {
-        f.probe += 64 * 37;
-        if (f.probe >= total) f.probe = (f.probe % total) & ~63u;
-      }
-    }
-    const uint32_t best = wave_umin(key);
-    if (best != kClean) {
-      const int l = __ffsll((unsigned long long)__ballot(key == best)) - 1;
-      f.others = __popcll(__ballot(key != kClean)) - 1;
-      const uint32_t slot = (uint32_t)__builtin_amdgcn_readlane((int)at, l);
-      if (sched_claim(s, f, slot, best)) return sched_block(s, slot);
-      continue;
-    }
-    if (!f.busy && __builtin_amdgcn_readfirstlane(dn)) return kNoWork;
+    const int32_t b = sched_look(s, f);
+    if (b != kNothing) return b;
     if (f.busy) {
-      // no more work: every mark of this workgroup's visits has landed
-      wait_memory();
       unsigned long long old = 0;
-      if (lane == 0)
+      if (__lane_id() == 0)
         old = __hip_atomic_fetch_add(s.ctl, ~0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       f.busy = false;
       const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)old);
-      if (lo == 1u && sched_all_clean(s) && lane == 0 &&
+      if (lo == 1u && sched_all_clean(s) && __lane_id() == 0 &&
           __hip_atomic_load(s.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == old - 1ull)
         __hip_atomic_store(s.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       since = wall_clock64();
@@ -213,10 +222,11 @@ __device__ __forceinline__ int32_t sched_find(const Sched& s, Finder& f) {
 }
 
 // One workgroup starts busy, so that a solve without work (no valid source) ends too.  Called by
-// one whole wave before its first search.
-__device__ __forceinline__ void sched_enter(const Sched& s, Finder& f) {
-  f.probe = 64 * (blockIdx.x % 61) % (s.owners * s.stride) & ~63u;
-  if (blockIdx.x != 0) return;
+// one whole wave before its first search.  me: the workgroup's owner index.
+__device__ __forceinline__ void sched_enter(const Sched& s, Finder& f, uint32_t me) {
+  f.me = me;
+  f.probe = 64 * (f.me % 61 % s.windows);
+  if (f.me != 0) return;
   if (__lane_id() == 0)
     (void)__hip_atomic_fetch_add(s.ctl, (1ull << 32) + 1ull, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
@@ -224,10 +234,10 @@ __device__ __forceinline__ void sched_enter(const Sched& s, Finder& f) {
 }
 
 // The smallest key of this owner's blocks that no workgroup visits (one whole wave).
-__device__ __forceinline__ uint32_t sched_waiting(const Sched& s) {
+__device__ __forceinline__ uint32_t sched_waiting(const Sched& s, uint32_t me) {
   uint32_t key = kClean;
-  for (uint32_t i = __lane_id(); i < s.per_owner; i += 64) {
-    const unsigned long long v = load_word(&s.word[blockIdx.x * s.stride + i]);
+  for (uint32_t i = __lane_id(); i < s.per_owner && me < s.owners; i += 64) {
+    const unsigned long long v = load_word(&s.word[me * s.stride + i]);
     if ((v >> 32) == 0ull && (uint32_t)v < key) key = (uint32_t)v;
   }
   return wave_umin(key);
@@ -239,13 +249,15 @@ __device__ __forceinline__ void sched_again(const Sched& s, uint32_t slot) {
   __hip_atomic_store(key_of(s, slot), kClean, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Gives a claimed block back after its marks have landed; key: kClean, or what it waits with.
+// Gives a claimed block back after its marks have landed; key: kClean, or what it waits with.  Returns
+// when the release has landed, so that the end of the solve can be found.
 __device__ __forceinline__ void sched_leave(const Sched& s, uint32_t slot, uint32_t key) {
   if (key != kClean) {
     sched_mark(s, slot, key);
     wait_memory();
   }
   __hip_atomic_store(lock_of(s, slot), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  wait_memory();
 }
 
 }  // namespace eik

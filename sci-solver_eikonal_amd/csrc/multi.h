@@ -4,10 +4,9 @@
 //
 // Every solve of a launch has a descriptor (its mesh's device layout, its own time arrays and,
 // optionally, a per-element factor on the squared edge lengths: a request's own speed field over
-// a resident mesh).  The blocks of all solves share one set of queue flags, solve i's blocks
-// being numbered bbase_i + b, and a queue entry carries the solve index, so the workgroups of the
-// launch pull blocks of any solve from one queue: small solves whose wavefront would leave most
-// of the GPU idle fill it together.  Tets and triangles keep separate queues and kernels.
+// a resident mesh).  The blocks of all solves of one element kind are numbered together, solve i's
+// blocks being kbase_i + b, and the workgroups of the launch find work among all of their words
+// (block_sched.h): small solves whose wavefront would leave most of the GPU idle fill it together.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -15,6 +14,7 @@
 #include <vector>
 
 #include "device.h"
+#include "visit_loop.h"
 
 namespace eik {
 
@@ -34,9 +34,11 @@ struct alignas(16) SolveDesc {
   float* T;
   float* seen;
   int64_t nv;
+  TriItems items;            // triangles
   int64_t nseen;
   int64_t out_off;           // first value of this solve in the gathered output
   int32_t bbase;             // first launch-wide block index
+  int32_t kbase;             // ... among the blocks of its element kind (launch_args)
   int32_t nblocks;
   int32_t dim;
   float large;
@@ -44,35 +46,29 @@ struct alignas(16) SolveDesc {
 
 struct MultiArgs {
   const SolveDesc* solves;
-  int32_t* queue;
-  uint32_t* qflag;
-  uint32_t* bstate;
-  QueueCtl* ctl;
-  uint32_t qmask;
-  int32_t bbits;
-  int32_t bmask;
+  LoopArgs loop;
+  int32_t* bsolve;           // per block of the kind: its solve
   unsigned long long* counters;
-  float eps;
-  int32_t max_inner;
   int32_t queue_cap;
   size_t rec_lds_bytes;
-  int64_t max_visits;
-  unsigned long long wait_limit;  // wall-clock ticks a queue wait may last (q_take)
 };
 
-// The solves of one element kind in a launch: their own queue and launch shape.  Shape 0
-// stages the element records in LDS (EIK_STAGE_LDS; lds[0] is 0 when the largest block's
-// records do not fit), shape 1 reads them from memory with smaller workgroups, the per-solve
-// factors applied at every use (batch.hip, k_visit_multi).
+// The solves of one element kind in a launch: their own words and launch shape.  Shape 0 stages the
+// element records in LDS (EIK_STAGE_LDS; lds[0] is 0 when the largest block's records do not fit),
+// shape 1 reads them from memory with smaller workgroups, the per-solve factors applied at every use
+// (batch.hip, k_visit_multi); shape 2 keeps them in registers (visit_loop.h; res_bt is 0 when the
+// largest block does not fit).
 struct Group {
   int dim = 3;
   bool present = false;
-  int32_t* queue = nullptr;
-  QueueCtl* qctl = nullptr;
-  uint32_t qcap = 0;
-  size_t lds[2] = {0, 0};
+  unsigned long long* words = nullptr;
+  unsigned char* sctl = nullptr;
+  int32_t* bsolve = nullptr;
+  size_t lds[3] = {0, 0, 0};
   size_t rec_lds_bytes = 0;  // shape 0
   int32_t queue_cap = 0;
+  int32_t max_local = 0, max_elem = 0, max_items = 0;
+  int res_bt = 0;            // shape 2: threads
   int shape = 0;             // chosen per launch (launch_args)
   int grid = 0;
   int wpe = 4;               // register budget of the visit kernel: waves per SIMD (group_grid)
@@ -90,12 +86,10 @@ struct Launch {
   int64_t cap_blocks = 0, cap_nv = 0, cap_seeds = 0;
   SolveDesc* dsolves = nullptr;
   SolveDesc* hsolves = nullptr;  // pinned
-  uint32_t* qflag = nullptr;
-  uint32_t* bstate = nullptr;
+  bool merged = false;  // both kinds in shape 2: one kernel visits them (launch_args)
   unsigned long long* counters = nullptr;
   float* out = nullptr;
-  int32_t *d_sseed = nullptr, *d_vseed = nullptr, *d_nseed = nullptr;
-  float* d_fseed = nullptr;
+  int32_t* d_seed = nullptr;  // as h_seed
   int32_t* h_seed = nullptr;  // pinned: [solve x cap][vertex x cap][value bits x cap][count]
   float* h_out = nullptr;     // pinned: gathered times
   unsigned long long* h_cnt = nullptr;
@@ -128,8 +122,8 @@ int launch_issue(Launch& L, int32_t nsolves, int64_t total_blocks, int64_t total
 // to the pinned buffer, on L.stream.
 int launch_output(Launch& L, int32_t nsolves, int64_t total_nv);
 void launch_stats(const Launch& L, float kernel_ms, eik_solve_stats_t* st);
-// After a finished launch: EIK_ERR_TIMEOUT if workgroups abandoned queue waits and a queue
-// never reached its end (check_queue_end), else EIK_OK.
+// After a finished launch: EIK_ERR_TIMEOUT if workgroups gave up waiting and a kind never reached
+// its end (check_end), else EIK_OK.
 int launch_check_end(const Launch& L);
 
 }  // namespace eik

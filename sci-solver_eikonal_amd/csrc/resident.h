@@ -22,11 +22,13 @@ namespace eik {
 
 // Items of the triangle blocks: block b's items are [start, start + count) of the arrays.
 // id: slots of the two other corners and the target, 10 bits each (a | b << 10 | target << 20);
-// len: {|a - target|^2, |b - target|^2, |a - b|^2, height of the target}.
+// len: {|a - target|^2, |b - target|^2, |a - b|^2, height of the target}; rec: the item's element
+// record within the block.
 struct TriItems {
   const int2* range;
   const uint32_t* id;
   const float4* len;
+  const uint16_t* rec;
 };
 constexpr int kItemSlotBits = 10;
 constexpr int kItemSlots = 1 << kItemSlotBits;  // local vertices of a block with items
@@ -51,8 +53,11 @@ __device__ __forceinline__ int this_thread() {
   return t;
 }
 
+// rmult: a factor per record of the block on its squared lengths, or null (a factor f scales the
+// heights by sqrt(f)).
 template <int N, int BT>
-__device__ __forceinline__ void tri_load(TriRegs<N>& r, const TriItems& t, int2 range) {
+__device__ __forceinline__ void tri_load(TriRegs<N>& r, const TriItems& t, int2 range,
+                                         const float* rmult) {
   const int tid = this_thread();
 #pragma unroll
   for (int u = 0; u < N; ++u) {
@@ -64,6 +69,17 @@ __device__ __forceinline__ void tri_load(TriRegs<N>& r, const TriItems& t, int2 
     r.lb[u] = l.y;
     r.lab[u] = l.z;
     r.h[u] = l.w;
+  }
+  if (rmult) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int i = u * BT + tid;
+      const float f = i < range.y ? rmult[t.rec[range.x + i]] : 1.f;
+      r.la[u] *= f;
+      r.lb[u] *= f;
+      r.lab[u] *= f;
+      r.h[u] *= __builtin_sqrtf(f);
+    }
   }
 }
 
@@ -120,10 +136,22 @@ __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large,
   return changed;
 }
 
+// Two non-negative values as fp16, rounded towards zero; and back.
+__device__ __forceinline__ uint32_t half_pair(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+}
+__device__ __forceinline__ float half_lo(uint32_t p) {
+  return (float)__builtin_bit_cast(_Float16, (uint16_t)p);
+}
+__device__ __forceinline__ float half_hi(uint32_t p) {
+  return (float)__builtin_bit_cast(_Float16, (uint16_t)(p >> 16));
+}
+
 template <int N>
 struct TetRegs {
   uint32_t v01[N], v23[N];     // corner slots, 16 bits each
-  float h0[N], h1[N], h2[N], h3[N];  // heights; +inf: the corner is not owned
+  // heights in fp16, rounded down (they stay lower bounds of every solve); +inf: not owned
+  uint32_t h01[N], h23[N];
   float p0[N], p1[N], p2[N], p3[N];  // corner times at the last selection
 };
 
@@ -135,9 +163,10 @@ __device__ __forceinline__ void copy_to_lds(const uint4* from, uint4* wave_base)
 }
 
 // Loads the thread's records: slots and heights to registers, slots and lengths to LDS.
+// rmult as in tri_load.
 template <int N, int BT>
 __device__ __forceinline__ void tet_load(TetRegs<N>& r, const void* recs, const BlockDesc& d,
-                                         uint4* sA, uint4* sB) {
+                                         uint4* sA, uint4* sB, const float* rmult) {
   const uint4* p = reinterpret_cast<const uint4*>(recs) + 3 * (int64_t)d.estart;
   const int tid = this_thread();
   const int wave = __builtin_amdgcn_readfirstlane(tid & ~63);
@@ -146,26 +175,33 @@ __device__ __forceinline__ void tet_load(TetRegs<N>& r, const void* recs, const 
     const int e = u * BT + tid;
     const bool in = e < d.nelem;
     const uint4* q = p + 3 * (in ? e : 0);
-    if (in) {
+    if (in && !rmult) {
       copy_to_lds(q, sA + u * BT + wave);
       copy_to_lds(q + 1, sB + u * BT + wave);
     }
     const uint2 v = *reinterpret_cast<const uint2*>(q);
-    const uint4 h = q[2];
+    const uint4 hq = q[2];
+    float h0 = __uint_as_float(hq.x), h1 = __uint_as_float(hq.y);
+    float h2 = __uint_as_float(hq.z), h3 = __uint_as_float(hq.w);
+    if (rmult && in) {
+      const float f = rmult[e], sf = __builtin_sqrtf(f);
+      const uint4 a = q[0], b = q[1];
+      sA[e] = make_uint4(a.x, a.y, __float_as_uint(__uint_as_float(a.z) * f),
+                         __float_as_uint(__uint_as_float(a.w) * f));
+      sB[e] = make_uint4(__float_as_uint(__uint_as_float(b.x) * f),
+                         __float_as_uint(__uint_as_float(b.y) * f),
+                         __float_as_uint(__uint_as_float(b.z) * f),
+                         __float_as_uint(__uint_as_float(b.w) * f));
+      h0 *= sf;
+      h1 *= sf;
+      h2 *= sf;
+      h3 *= sf;
+    }
+    const unsigned n = in ? (unsigned)d.nown : 0u;
     r.v01[u] = v.x;
     r.v23[u] = v.y;
-    r.h0[u] = __uint_as_float(h.x);
-    r.h1[u] = __uint_as_float(h.y);
-    r.h2[u] = __uint_as_float(h.z);
-    r.h3[u] = __uint_as_float(h.w);
-  }
-#pragma unroll
-  for (int u = 0; u < N; ++u) {
-    const unsigned n = u * BT + tid < d.nelem ? (unsigned)d.nown : 0u;
-    r.h0[u] = (r.v01[u] & 0xffffu) < n ? r.h0[u] : EIK_INF;
-    r.h1[u] = (r.v01[u] >> 16) < n ? r.h1[u] : EIK_INF;
-    r.h2[u] = (r.v23[u] & 0xffffu) < n ? r.h2[u] : EIK_INF;
-    r.h3[u] = (r.v23[u] >> 16) < n ? r.h3[u] : EIK_INF;
+    r.h01[u] = half_pair((v.x & 0xffffu) < n ? h0 : EIK_INF, (v.x >> 16) < n ? h1 : EIK_INF);
+    r.h23[u] = half_pair((v.y & 0xffffu) < n ? h2 : EIK_INF, (v.y >> 16) < n ? h3 : EIK_INF);
   }
 }
 
@@ -228,8 +264,10 @@ __device__ __forceinline__ void tet_select(TetRegs<N>& r, const float* sT, float
     const float m01 = __builtin_fminf(t0[u], t1[u]), m23 = __builtin_fminf(t2[u], t3[u]);
     const float mn0 = __builtin_fminf(t1[u], m23), mn1 = __builtin_fminf(t0[u], m23);
     const float mn2 = __builtin_fminf(m01, t3[u]), mn3 = __builtin_fminf(m01, t2[u]);
-    unsigned s = (t0[u] > mn0 + r.h0[u] ? 1u : 0u) | (t1[u] > mn1 + r.h1[u] ? 2u : 0u) |
-                 (t2[u] > mn2 + r.h2[u] ? 4u : 0u) | (t3[u] > mn3 + r.h3[u] ? 8u : 0u);
+    unsigned s = (t0[u] > mn0 + half_lo(r.h01[u]) ? 1u : 0u) |
+                 (t1[u] > mn1 + half_hi(r.h01[u]) ? 2u : 0u) |
+                 (t2[u] > mn2 + half_lo(r.h23[u]) ? 4u : 0u) |
+                 (t3[u] > mn3 + half_hi(r.h23[u]) ? 8u : 0u);
     // one corner alone changed: it has no new solve itself
     const unsigned f = (f0 ? 1u : 0u) | (f1 ? 2u : 0u) | (f2 ? 4u : 0u) | (f3 ? 8u : 0u);
     if ((f & (f - 1u)) == 0u) s &= ~f;

@@ -11,8 +11,7 @@
 #include <vector>
 
 #include "device.h"
-#include "resident.h"
-#include "block_sched.h"
+#include "visit_loop.h"
 
 namespace eik {
 
@@ -27,7 +26,7 @@ static int dev_free(DeviceState* d) {
                   d->dep_start, d->dep, d->owner, d->T,      d->out,      d->chg,
                   d->self,   d->list[0], d->list[1], d->count, d->counters, d->sync_acc, d->seeds,
                   d->seedvals, d->words, d->sctl,
-                  d->item_range, d->item_id, d->item_len};
+                  d->item_range, d->item_id, d->item_len, d->item_rec};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (d->h_seed) (void)hipHostFree(d->h_seed);
@@ -66,29 +65,6 @@ int ensure_stream(Mesh& m) {
 // ------------------------------------------------------------------------------------------
 // Kernels
 // ------------------------------------------------------------------------------------------
-__global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
-// The per-solve resets in one launch: segment k sets n[k] 32-bit words at p[k] to v[k]
-// (a launch per array cost about 5 us each, most of a small solve's set-up).
-struct FillSegs {
-  static constexpr int kMax = 10;
-  int32_t* p[kMax];
-  int64_t n[kMax];
-  int32_t v[kMax];
-  int count;
-  unsigned long long* words = nullptr;  // block words, set to clean (block_sched.h)
-  int64_t nwords = 0;
-  void add(void* ptr, int64_t words, int32_t value) {
-    p[count] = reinterpret_cast<int32_t*>(ptr);
-    n[count] = words;
-    v[count] = value;
-    ++count;
-  }
-};
-
 __global__ void k_fill_segs(FillSegs f) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -97,16 +73,15 @@ __global__ void k_fill_segs(FillSegs f) {
     const int32_t v = f.v[k];
     for (int64_t i = i0; i < f.n[k]; i += stride) p[i] = v;
   }
-  for (int64_t i = i0; i < f.nwords; i += stride) f.words[i] = kClean;
+  for (int k = 0; k < 2; ++k)
+    for (int64_t i = i0; i < f.nwords[k]; i += stride) f.words[k][i] = kClean;
 }
 
-static unsigned fill_grid(const FillSegs& f) {
-  int64_t most = 0;
+void launch_fill(const FillSegs& f, hipStream_t s) {
+  int64_t most = std::max<int64_t>(1, std::max(f.nwords[0], f.nwords[1]));
   for (int k = 0; k < f.count; ++k) most = std::max(most, f.n[k]);
-  return (unsigned)std::min<int64_t>(grid1d(most, 256), 2048);
-}
-static void launch_fill(const FillSegs& f, hipStream_t s) {
-  hipLaunchKernelGGL(k_fill_segs, dim3(fill_grid(f)), dim3(256), 0, s, f);
+  hipLaunchKernelGGL(k_fill_segs, dim3((unsigned)std::min<int64_t>(grid1d(most, 256), 2048)),
+                     dim3(256), 0, s, f);
 }
 
 // seeds: caller ids -> new ids; T = value; the owner block of each seed is marked changed
@@ -278,249 +253,24 @@ __device__ __forceinline__ void write_out(const SolveArgs& a, int block) {
     a.out[i] = load_T<true>(a.v.T + a.iperm[i]);
 }
 
-// Blocks seen waiting when a tet block is claimed from which on its visit runs up to max_inner sweeps:
-// while work waits, a block is loaded for more than one sweep (96^3 cube with 16 sources, 1 sweep
-// always / 1 / 8 / 16 waiting blocks: 1.66 / 1.52 / 1.52 / 1.57 ms); while workgroups wait for work,
-// one sweep, whose times reach the dependents sooner.
-constexpr int kCrowd = 8;
-
-// One whole wave: the next block, with the time spent looking in the workgroup's tally.
-__device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned long long* acc) {
-  const unsigned long long w0 = wall_clock64();
-  const int32_t b = sched_find(s, f);
-  if (__lane_id() == 0) {
-    acc[6] += wall_clock64() - w0;
-    if (b == kGaveUp) acc[kCntAbandoned] += 1;
+struct SingleBlocks {
+  const SolveArgs& a;
+  __device__ __forceinline__ BlockData operator()(int32_t b) const {
+    return {a.v.blocks, a.v.elems, a.v.halo, a.v.T,   a.v.seen, a.v.vmask,
+            a.dep_start, a.dep,    nullptr,  a.items, b,        0};
   }
-  return b;
-}
+};
 
-// The persistent kernel over blocks whose element data fits the workgroup's registers
-// (resident.h): N items or elements per thread.  Blocks are found and handed on as block_sched.h
-// says; a workgroup that visits a block again, at once or when it is dirty again and nothing smaller
-// waits, keeps its registers and LDS, and only times are read again.  A visit of a tet block is one
-// sweep while few blocks wait (kCrowd); a block that has not converged is visited again at once
-// unless a block of the same owner waits with a smaller time.
-// What bounds it: the chain of a visit (64^3 cube: 3.0 us a sweep, 0.4 us until its times have landed,
-// 0.8 us of marks and release, 2 us to load a block into the registers and LDS every third visit), and
-// on large tet meshes the loads too (96^3: 86,000 of 40 KB in 1.5 ms).  Held to 128 VGPRs, so that four
-// workgroups fit a CU: with 45 of them spilled the 96^3 solve took 2.1 ms, without 1.7.
-// Visit kernels, against the staged records of visit_block and one queue ring: 64^3 cube 1.045 ->
-// 0.664 ms, 96^3 with 16 sources 3.67 -> 1.53, 33^3 tensor 0.448 -> 0.295, 16^3 0.285 -> 0.172; level-8
-// icosphere 3.29 -> 1.70, level-7 anisotropic 1.02 -> 0.55, level 5 0.328 -> 0.169, 32^2 square 0.158 ->
-// 0.081.
 template <int DIM, int N, int BT>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_resident(SolveArgs a) {
   extern __shared__ uint4 lds4[];
-  __shared__ int sFlag[3];      // a sweep's "a time fell", in a ring over the sweeps
-  __shared__ int sQn[2];        // work-item counters of alternate sweeps (tets)
-  __shared__ unsigned sMark[2]; // dependents whose halo holds a vertex lowered in this visit
-  __shared__ int sBlock;
-  __shared__ unsigned sWaiting; // smallest key of the owner's waiting blocks when last looked
-  __shared__ unsigned sKey;     // smallest time the visit lowered
-  __shared__ int sCrowd;        // dirty blocks seen waiting when this one was claimed
-  __shared__ unsigned long long sAcc[kNumCounters];
-  const int tid = threadIdx.x;
-  uint4* sA = lds4;
-  uint4* sB = sA + (DIM == 3 ? a.max_elem : 0);
-  float* sT = reinterpret_cast<float*>(sB + (DIM == 3 ? a.max_elem : 0));
-  float* sP = sT + a.max_local;
-  int* sHidx = reinterpret_cast<int*>(sP + a.max_local);
-  uint16_t* sQ = reinterpret_cast<uint16_t*>(sHidx + a.max_local);
-  const float large = a.v.large, eps = a.v.eps;
-  if (tid < kNumCounters) sAcc[tid] = 0;
-  if (tid < 3) sFlag[tid] = 0;
-  if (tid < 2) sQn[tid] = 0;
-  if (tid < 2) sMark[tid] = 0;
-  if (tid == 0) sKey = kClean;
-  Finder f;
-  if (tid < 64) sched_enter(a.s, f);
-  int ring = 0;  // sweeps run so far, modulo 3
-  int qc = 0;
-  uint32_t solves = 0;
-  if (tid < 64) {
-    const int32_t nb = find_next(a.s, f, sAcc);
-    if (tid == 0) {
-      sBlock = nb;
-      sCrowd = f.others;
-    }
-  }
-  __syncthreads();
-  int b = __builtin_amdgcn_readfirstlane(sBlock);
-  while (b >= 0) {
-    unsigned long long t0 = wall_clock64();
-    const int cur = b;
-    // the resident block: one owned vertex per thread, its items or elements in registers
-    const BlockDesc d = a.v.blocks[b];
-    const uint32_t slot = sched_slot(a.s, b);
-    float* seen = a.v.seen + d.vstart + d.hstart;
-    const int32_t s0 = a.dep_start[b];
-    const int ndep = a.dep_start[b + 1] - s0;
-    float own = 0.f;  // the owned vertex's time as last published
-    uint64_t vm = 0;
-    uint32_t dep_slot = 0;
-    std::conditional_t<DIM == 2, TriRegs<N>, TetRegs<N>> r;
-    const int t = this_thread();
-    if (t < d.nown) {
-      own = load_T<true>(a.v.T + d.vstart + t);
-      sP[t] = seen[t];
-      vm = a.v.vmask[d.vstart + t];
-      sT[t] = own;
-    }
-    for (int i = t; i < d.nhalo; i += BT) {
-      const int32_t h = a.v.halo[d.hstart + i];
-      sHidx[i] = h;
-      sP[d.nown + i] = seen[d.nown + i];
-      sT[d.nown + i] = load_T<true>(a.v.T + h);
-    }
-    if (t < ndep) dep_slot = sched_slot(a.s, a.dep[s0 + t]);
-    if constexpr (DIM == 2)
-      tri_load<N, BT>(r, a.items, a.items.range[b]);
-    else
-      tet_load<N, BT>(r, a.v.elems, d, sA, sB);
-    wait_memory();  // the copies to LDS too
-    __syncthreads();
-    if constexpr (DIM == 2) tri_seen<N>(r, sP);
-    else tet_seen<N>(r, sP);
-    unsigned long long t1 = wall_clock64();
-    bool rerun = false;
-    unsigned waiting = kClean;  // smallest key of the owner's other blocks when last looked
-    // visits of this block: the next one at once, or when the block is dirty again and nothing
-    // smaller waits
-    for (;;) {
-      const int inner = DIM == 2 || sCrowd >= kCrowd ? a.v.max_inner : 1;
-      uint64_t marks = 0;  // dependents holding this thread's vertex, if it fell
-      uint32_t key = kClean;
-      float own_last = own;
-      int sweep = 0;
-      bool conv = false;
-      while (sweep < inner) {
-        bool ch = false;
-        int nq = 1;
-        if constexpr (DIM == 2) {
-          ch = tri_sweep<N>(r, sT, large, eps, solves);
-        } else {
-          tet_select<N, BT>(r, sT, eps, sQ, &sQn[qc]);
-          __syncthreads();
-          nq = sQn[qc];
-          if (tid == 0) sQn[qc ^ 1] = 0;
-          qc ^= 1;
-          if (nq) ch = tet_solve<N, BT>(r, sA, sB, sQ, nq, sT, large, eps, solves);
-        }
-        if (ch) sFlag[ring] = 1;
-        // (no pair selected: no time fell, and no thread waits for another's solve)
-        if (nq) __syncthreads();
-        const int any = nq ? sFlag[ring] : 0;
-        ring = ring == 2 ? 0 : ring + 1;
-        if (tid == 0) sFlag[ring == 2 ? 0 : ring + 1] = 0;
-        ++sweep;
-        // publish the owned times that fell
-        own_last = own;
-        if (tid < d.nown) {
-          const float v = sT[tid];
-          if (v < own) {
-            own = v;
-            (void)__hip_atomic_fetch_min(reinterpret_cast<unsigned*>(a.v.T + d.vstart + tid),
-                                         __float_as_uint(v), __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-            marks |= vm;
-            key = __float_as_uint(v);
-          }
-        }
-        if (!any) {
-          conv = true;
-          break;
-        }
-      }
-      const unsigned long long t2 = wall_clock64();
-      // visits beyond the bound mark nothing more (runaway guard)
-      const bool cap_ok = (int64_t)sAcc[0] < a.max_visits;
-      const bool more = !conv && cap_ok;
-      // marks made from here on are seen by the halo loads of the next visit or after it
-      if (more && tid == 0) sched_again(a.s, slot);
-      // reduced over the wave first: the compiler turns an LDS or with a uniform address into a
-      // scalar loop over the lanes (a third of a triangle sweep)
-      if (__ballot(key != kClean)) {
-        const uint32_t lo = wave_or((uint32_t)marks), hi = wave_or((uint32_t)(marks >> 32));
-        key = wave_umin(key);
-        if (__lane_id() == 63) {
-          atomicMin(&sKey, key);
-          if (lo) atomicOr(&sMark[0], lo);
-          if (hi) atomicOr(&sMark[1], hi);
-        }
-      }
-      // the published times have reached the device's coherence point before the dependents are
-      // marked
-      wait_memory();
-      __syncthreads();
-      const unsigned long long tq = wall_clock64();
-      const uint32_t vkey = sKey;
-      // visited again at once, unless another of the owner's blocks waits with a smaller time
-      const bool again = more && !(waiting < vkey);
-      if (tid < 64) {
-        const uint64_t mask = (uint64_t)sMark[0] | ((uint64_t)sMark[1] << 32);
-        if (cap_ok && tid < ndep && ((mask >> tid) & 1ull)) sched_mark(a.s, dep_slot, vkey);
-        if (tid < 2) sMark[tid] = 0;
-        if (tid == 0) {
-          VisitResult vr;
-          vr.sweeps = sweep;
-          vr.t_load = t1 - t0;
-          vr.t_sweep = t2 - t1;
-          vr.t_wb = tq - t2;
-          tally_visit(sAcc, d, vr, 0, a.elem_bytes, tq - t0, rerun, rerun);
-        }
-        if (again) {
-          const uint32_t w = sched_waiting(a.s);
-          if (tid == 0) sWaiting = w;
-          if (tid == 0) sAcc[10] += wall_clock64() - tq;
-        } else {
-          wait_memory();  // the marks have landed before this block can count as clean
-          if (tid == 0) sched_leave(a.s, slot, more ? vkey : kClean);
-          if (tid == 0) sAcc[10] += wall_clock64() - tq;
-          const int32_t nb = find_next(a.s, f, sAcc);
-          if (tid == 0) {
-            sBlock = nb;
-            sCrowd = f.others;
-            sWaiting = kClean;
-          }
-        }
-      } else if (again) {
-        // the halo times of the next visit (by the waves that mark nothing)
-        for (int i = tid - 64; i < d.nhalo; i += BT - 64)
-          sT[d.nown + i] = load_T<true>(a.v.T + sHidx[i]);
-      }
-      if (!again) {
-        // what this visit evaluated the block's elements with: every time, but for the owned
-        // vertices that fell in the last sweep of a visit cut off by the sweep cap.  A later
-        // visit that misses these (they are plain stores) evaluates more than it has to.
-        if (tid < d.nown) seen[tid] = conv ? own : own_last;
-        for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = sT[d.nown + i];
-      }
-      __syncthreads();
-      waiting = sWaiting;
-      if (tid == 0) sKey = kClean;
-      t0 = t1 = wall_clock64();
-      rerun = again;
-      if (again) continue;
-      b = __builtin_amdgcn_readfirstlane(sBlock);
-      if (b != cur) break;
-      // the same block, still resident: only times may have fallen (the owned ones if another
-      // workgroup visited the block meanwhile)
-      if (tid < d.nown) {
-        own = load_T<true>(a.v.T + d.vstart + tid);
-        sT[tid] = own;
-      }
-      for (int i = tid; i < d.nhalo; i += BT) sT[d.nown + i] = load_T<true>(a.v.T + sHidx[i]);
-      __syncthreads();
-      t1 = wall_clock64();
-    }
-  }
-  write_out(a, sBlock);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) solves += __shfl_down(solves, off, 64);
-  if (__lane_id() == 0 && solves) atomicAdd(&sAcc[3], (unsigned long long)solves);
-  __syncthreads();
-  if (tid < kNumCounters && sAcc[tid]) atomicAdd(&a.counters[tid], sAcc[tid]);
+  __shared__ LoopShared sh;
+  if (threadIdx.x < kNumCounters) sh.acc[threadIdx.x] = 0;
+  const LoopArgs la = {a.s, a.v.eps, a.v.max_inner, a.max_visits, a.max_local, a.max_elem};
+  const int end = resident_loop<DIM, N, BT>(la, SingleBlocks{a}, blockIdx.x, lds4, sh);
+  write_out(a, end);
+  if (threadIdx.x < kNumCounters && sh.acc[threadIdx.x])
+    atomicAdd(&a.counters[threadIdx.x], sh.acc[threadIdx.x]);
 }
 
 // Seeds of a solve of the scheduler above: the sources' times, and the owner block of each source
@@ -555,7 +305,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
   const int tid = threadIdx.x;
   if (tid < kNumCounters) sAcc[tid] = 0;
   Finder f;
-  if (tid < 64) sched_enter(a.s, f);
+  if (tid < 64) sched_enter(a.s, f, blockIdx.x);
   for (;;) {
     if (tid < 64) {
       const int32_t nb = find_next(a.s, f, sAcc);
@@ -640,7 +390,8 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
 // The items of every triangle block (TriItems) from its records: one workgroup per block, items in
 // record order.  mask: the record's updatable corners; corners not owned have no item.
 __global__ __launch_bounds__(256) void k_tri_items(const BlockDesc* blocks, const uint4* recs,
-                                                   const int2* range, uint32_t* id, float4* len) {
+                                                   const int2* range, uint32_t* id, float4* len,
+                                                   uint16_t* rec) {
   __shared__ int sWave[4];
   const BlockDesc d = blocks[blockIdx.x];
   int at = range[blockIdx.x].x;
@@ -662,14 +413,17 @@ __global__ __launch_bounds__(256) void k_tri_items(const BlockDesc* blocks, cons
     // the corner order and lengths of tri_rotation
     if (m & 1u) {
       id[q] = x.v1 | (x.v2 << kItemSlotBits) | ((uint32_t)x.v0 << (2 * kItemSlotBits));
+      rec[q] = (uint16_t)e;
       len[q++] = make_float4(x.L0, x.L2, x.L1, x.H0);
     }
     if (m & 2u) {
       id[q] = x.v0 | (x.v2 << kItemSlotBits) | ((uint32_t)x.v1 << (2 * kItemSlotBits));
+      rec[q] = (uint16_t)e;
       len[q++] = make_float4(x.L0, x.L1, x.L2, x.H1);
     }
     if (m & 4u) {
       id[q] = x.v0 | (x.v1 << kItemSlotBits) | ((uint32_t)x.v2 << (2 * kItemSlotBits));
+      rec[q] = (uint16_t)e;
       len[q++] = make_float4(x.L2, x.L1, x.L0, x.H2);
     }
     at += total;
@@ -818,9 +572,10 @@ int upload_layout(Mesh& m) {
 
 static const void* resident_kernel(int dim, int n, int bt) {
   if (dim == 3)
-    return bt == 256   ? (const void*)k_visit_resident<3, 4, 256>
-           : bt == 512 ? (const void*)k_visit_resident<3, 4, 512>
-                       : (const void*)k_visit_resident<3, 4, 1024>;
+    return n == 4 && bt == 256 ? (const void*)k_visit_resident<3, 4, 256>
+           : bt == 256         ? (const void*)k_visit_resident<3, kTetN<256>, 256>
+           : bt == 512         ? (const void*)k_visit_resident<3, kTetN<512>, 512>
+                               : (const void*)k_visit_resident<3, kTetN<1024>, 1024>;
   return n == 2      ? (const void*)k_visit_resident<2, 2, 256>
          : bt == 256 ? (const void*)k_visit_resident<2, 4, 256>
          : bt == 512 ? (const void*)k_visit_resident<2, 4, 512>
@@ -838,17 +593,15 @@ static int setup_resident(Mesh& m, size_t max_lds) {
   d->res_n = 0;
   if (L.vmask.empty()) return EIK_OK;
   const int32_t need = m.dim == 3 ? L.max_elem : L.max_items;
-  if (m.dim == 2 && need <= 2 * 256) d->res_n = 2, d->res_bt = 256;
-  else if (need <= 4 * 256) d->res_n = 4, d->res_bt = 256;
-  else if (need <= 4 * 512) d->res_n = 4, d->res_bt = 512;
-  else if (need <= 4 * 1024) d->res_n = 4, d->res_bt = 1024;
+  static const int shapes[2][4][2] = {{{2, 256}, {4, 256}, {4, 512}, {4, 1024}},
+                                      {{4, 256}, {kTetN<256>, 256}, {kTetN<512>, 512}, {kTetN<1024>, 1024}}};
+  for (const auto& sh : shapes[m.dim == 3 ? 1 : 0])
+    if (d->res_n == 0 && need <= sh[0] * sh[1]) d->res_n = sh[0], d->res_bt = sh[1];
   if (d->res_n == 0 || L.max_own > d->res_bt || (m.dim == 2 && L.max_local > kItemSlots)) {
     d->res_n = 0;
     return EIK_OK;
   }
-  d->res_lds = sizeof(float) * 3 * (size_t)L.max_local;
-  if (m.dim == 3)
-    d->res_lds += 2 * sizeof(uint4) * (size_t)L.max_elem + sizeof(uint16_t) * (size_t)L.max_items;
+  d->res_lds = loop_lds_bytes(m.dim, L.max_local, L.max_elem, L.max_items);
   if (d->res_lds > max_lds) {
     d->res_n = 0;
     return EIK_OK;
@@ -871,8 +624,10 @@ static int setup_resident(Mesh& m, size_t max_lds) {
   if (rc) return rc;
   HIP_TRY(hipMalloc((void**)&d->item_id, sizeof(uint32_t) * std::max<int64_t>(n, 1)));
   HIP_TRY(hipMalloc((void**)&d->item_len, sizeof(float4) * std::max<int64_t>(n, 1)));
+  HIP_TRY(hipMalloc((void**)&d->item_rec, sizeof(uint16_t) * std::max<int64_t>(n, 1)));
   hipLaunchKernelGGL(k_tri_items, dim3(L.nblocks), dim3(256), 0, d->stream, d->blocks,
-                     (const uint4*)d->elems, d->item_range, d->item_id, d->item_len);
+                     (const uint4*)d->elems, d->item_range, d->item_id, d->item_len,
+                     d->item_rec);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(d->stream));  // the host copy of the ranges has been read
   return EIK_OK;
@@ -1033,9 +788,7 @@ static int32_t async_inner_sweeps(int dim, int32_t requested) {
   return requested > 0 ? requested : (dim == 2 ? 3 : default_inner_sweeps(dim, 0));
 }
 
-// After a launch whose workgroups gave up waiting: EIK_OK if the solve still reached its end (the
-// result is complete), else EIK_ERR_TIMEOUT.  Synchronises stream s.
-static int check_end(const unsigned char* sctl, hipStream_t s, unsigned long long abandoned) {
+int check_end(const unsigned char* sctl, hipStream_t s, unsigned long long abandoned) {
   uint32_t done = 0;
   HIP_TRY(hipMemcpyAsync(&done, sctl + kSchedCtlBytes / 2, sizeof(done), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
@@ -1101,7 +854,7 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   a.s.done = reinterpret_cast<uint32_t*>(b.sctl + kSchedCtlBytes / 2);
   sched_shape(a.s, d->nblocks, grid);
   a.s.wait_limit = wait_limit_ticks(d->device, o.wait_limit_us);
-  a.items = {d->item_range, d->item_id, d->item_len};
+  a.items = {d->item_range, d->item_id, d->item_len, d->item_rec};
   a.dep_start = d->dep_start;
   a.dep = d->dep;
   a.iperm = d->iperm;
@@ -1118,12 +871,11 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   a.max_elem = d->max_elem;
   a.rec_lds_bytes = k.stage ? d->rec_lds_bytes : 0;
   FillSegs f;
-  f.count = 0;
   f.add(b.T, m.nv, (int32_t)__builtin_bit_cast(uint32_t, a.v.large));
   f.add(b.seen, d->nseen, (int32_t)__builtin_bit_cast(uint32_t, EIK_INF));
   f.add(b.counters, 2 * kNumCounters, 0);
-  f.words = b.words;
-  f.nwords = (int64_t)a.s.owners * a.s.stride;
+  f.words[0] = b.words;
+  f.nwords[0] = (int64_t)a.s.owners * a.s.stride;
   f.add(b.sctl, kSchedCtlBytes / 4, 0);
   launch_fill(f, s);
   hipLaunchKernelGGL(k_sched_seed, seed_grid(nseeds), dim3(64), 0, s, a.s, seeds, seedvals, nseeds,
@@ -1236,7 +988,6 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     if (rc) return rc;
   } else {
     FillSegs f;
-    f.count = 0;
     f.add(d->T, m->nv, (int32_t)__builtin_bit_cast(uint32_t, large));
     f.add(d->seen, d->nseen, (int32_t)__builtin_bit_cast(uint32_t, EIK_INF));
     f.add(d->chg, d->nblocks, -1);

@@ -1,0 +1,326 @@
+// visit_loop.h -- the loop of a persistent workgroup over register-resident blocks (device code),
+// shared by single solves (solver.hip) and multi-solve launches (batch.hip).
+#pragma once
+
+#include <type_traits>
+
+#include "block_sched.h"
+#include "device.h"
+#include "resident.h"
+
+namespace eik {
+
+// Elements per thread of the tet shapes: with 256 and 512 threads as many as 128 VGPRs hold beside the
+// solver, so that a block takes the smaller workgroup (the smallest blocks have a shape of 4).
+template <int BT>
+constexpr int kTetN = BT == 1024 ? 4 : 6;
+
+// What a visit reads of a block's mesh and solve.
+struct BlockData {
+  const BlockDesc* blocks;
+  const void* elems;
+  const int32_t* halo;
+  float* T;
+  float* seen;
+  const uint64_t* vmask;
+  const int32_t* dep_start;
+  const int32_t* dep;
+  const float* rmult;  // a factor per record on the squared lengths, or null
+  TriItems items;      // triangles
+  int32_t b;           // the block within its mesh
+  int32_t base;        // launch-wide index of its mesh's first block
+};
+
+struct LoopArgs {
+  Sched s;
+  float eps;
+  int32_t max_inner;
+  int64_t max_visits;  // runaway guard: visits of one workgroup after which it marks nothing
+  int32_t max_local;   // LDS strides: local vertices and elements of the largest block
+  int32_t max_elem;
+};
+
+// The workgroup's static LDS.
+struct LoopShared {
+  unsigned long long acc[kNumCounters];  // its tally
+  int flag[3];       // a sweep's "a time fell", in a ring over the sweeps
+  int qn[2];         // work-item counters of alternate sweeps (tets)
+  unsigned mark[2];  // dependents whose halo holds a vertex lowered in this visit
+  int block;
+  unsigned waiting;  // smallest key of the owner's waiting blocks when last looked
+  unsigned key;      // smallest time the visit lowered
+  int crowd;         // dirty blocks seen waiting when this one was claimed
+};
+
+// Dynamic LDS of the loop, bytes.
+inline size_t loop_lds_bytes(int dim, int32_t max_local, int32_t max_elem, int32_t max_items) {
+  size_t n = sizeof(float) * 3 * (size_t)max_local;
+  if (dim == 3) n += 2 * sizeof(uint4) * (size_t)max_elem + sizeof(uint16_t) * (size_t)max_items;
+  return n;
+}
+
+// Blocks seen waiting when a tet block is claimed from which on its visit runs up to max_inner sweeps:
+// while work waits, a block is loaded for more than one sweep (96^3 cube with 16 sources, 1 sweep
+// always / 1 / 8 / 16 waiting blocks: 1.66 / 1.52 / 1.52 / 1.57 ms); while workgroups wait for work,
+// one sweep, whose times reach the dependents sooner.
+constexpr int kCrowd = 8;
+
+// One whole wave: the next block (look: or kNothing), with the time spent in the workgroup's tally.
+__device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned long long* acc,
+                                             bool look = false) {
+  const unsigned long long w0 = wall_clock64();
+  const int32_t b = look ? sched_look(s, f) : sched_find(s, f);
+  if (__lane_id() == 0) {
+    acc[6] += wall_clock64() - w0;
+    if (b == kGaveUp) acc[kCntAbandoned] += 1;
+  }
+  return b;
+}
+
+// The loop of one workgroup over the blocks of a launch, until the solve has ended or it gives up:
+// blocks whose element data fits the workgroup's registers
+// (resident.h): N items or elements per thread.  Blocks are found and handed on as block_sched.h
+// says; a workgroup that visits a block again, at once or when it is dirty again and nothing smaller
+// waits, keeps its registers and LDS, and only times are read again.  A visit of a tet block is one
+// sweep while few blocks wait (kCrowd); a block that has not converged is visited again at once
+// unless a block of the same owner waits with a smaller time.
+// What bounds it: the chain of a visit (64^3 cube: 3.0 us a sweep, 0.4 us until its times have landed,
+// 0.8 us of marks and release, 2 us to load a block into the registers and LDS every third visit), and
+// on large tet meshes the loads too (96^3: 86,000 of 40 KB in 1.5 ms).  Held to 128 VGPRs, so that four
+// workgroups fit a CU: with 45 of them spilled the 96^3 solve took 2.1 ms, without 1.7.
+// Visit kernels, against the staged records of visit_block and one queue ring: 64^3 cube 1.045 ->
+// 0.664 ms, 96^3 with 16 sources 3.67 -> 1.53, 33^3 tensor 0.448 -> 0.295, 16^3 0.285 -> 0.172; level-8
+// icosphere 3.29 -> 1.70, level-7 anisotropic 1.02 -> 0.55, level 5 0.328 -> 0.169, 32^2 square 0.158 ->
+// 0.081.
+// blocks(g) gives the data of launch-wide block g; me is the workgroup's owner index.  Returns kNoWork or kGaveUp.  The workgroup's tally
+// is added to sh.acc, which the caller has cleared (behind a barrier) and flushes.
+template <int DIM, int N, int BT, class Blocks>
+__device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& blocks, uint32_t me,
+                                             uint4* lds4, LoopShared& sh) {
+  const int tid = threadIdx.x;
+  uint4* sA = lds4;
+  uint4* sB = sA + (DIM == 3 ? a.max_elem : 0);
+  float* sT = reinterpret_cast<float*>(sB + (DIM == 3 ? a.max_elem : 0));
+  float* sP = sT + a.max_local;
+  int* sHidx = reinterpret_cast<int*>(sP + a.max_local);
+  uint16_t* sQ = reinterpret_cast<uint16_t*>(sHidx + a.max_local);
+  const float eps = a.eps, large = DIM == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
+  // (the barrier before the first visit orders these)
+  if (tid < 3) sh.flag[tid] = 0;
+  if (tid < 2) sh.qn[tid] = 0;
+  if (tid < 2) sh.mark[tid] = 0;
+  if (tid == 0) sh.key = kClean;
+  // the second wave looks for work, while the first hands on what the last visit did
+  const bool finder = tid >= 64 && tid < 128;
+  Finder f;
+  if (finder) sched_enter(a.s, f, me);
+  int ring = 0;  // sweeps run so far, modulo 3
+  int qc = 0;
+  uint32_t solves = 0;
+  __syncthreads();
+  if (finder) {
+    const int32_t nb = find_next(a.s, f, sh.acc);
+    if (tid == 64) {
+      sh.block = nb;
+      sh.crowd = f.others;
+    }
+  }
+  __syncthreads();
+  int b = __builtin_amdgcn_readfirstlane(sh.block);
+  while (b >= 0) {
+    unsigned long long t0 = wall_clock64();
+    const int cur = b;
+    // the resident block: one owned vertex per thread, its items or elements in registers
+    const uint32_t slot = sched_slot(a.s, b);
+    const BlockData m = blocks(b);
+    const BlockDesc d = m.blocks[m.b];
+    float* T = m.T;
+    float* seen = m.seen + d.vstart + d.hstart;
+    const int32_t s0 = m.dep_start[m.b];
+    const int ndep = m.dep_start[m.b + 1] - s0;
+    const float* rmult = m.rmult ? m.rmult + d.estart : nullptr;
+    float own = 0.f;  // the owned vertex's time as last published
+    uint64_t vm = 0;
+    uint32_t dep_slot = 0;
+    std::conditional_t<DIM == 2, TriRegs<N>, TetRegs<N>> r;
+    const int t = this_thread();
+    if (t < d.nown) {
+      own = load_T<true>(T + d.vstart + t);
+      sP[t] = seen[t];
+      vm = m.vmask[d.vstart + t];
+      sT[t] = own;
+    }
+    for (int i = t; i < d.nhalo; i += BT) {
+      const int32_t h = m.halo[d.hstart + i];
+      sHidx[i] = h;
+      sP[d.nown + i] = seen[d.nown + i];
+      sT[d.nown + i] = load_T<true>(T + h);
+    }
+    if (t < ndep) dep_slot = sched_slot(a.s, m.base + m.dep[s0 + t]);
+    if constexpr (DIM == 2)
+      tri_load<N, BT>(r, m.items, m.items.range[m.b], rmult);
+    else
+      tet_load<N, BT>(r, m.elems, d, sA, sB, rmult);
+    wait_memory();  // the copies to LDS too
+    __syncthreads();
+    if constexpr (DIM == 2) tri_seen<N>(r, sP);
+    else tet_seen<N>(r, sP);
+    unsigned long long t1 = wall_clock64();
+    bool rerun = false;
+    unsigned waiting = kClean;  // smallest key of the owner's other blocks when last looked
+    // visits of this block: the next one at once, or when the block is dirty again and nothing
+    // smaller waits
+    for (;;) {
+      const int inner = DIM == 2 || sh.crowd >= kCrowd ? a.max_inner : 1;
+      uint64_t marks = 0;  // dependents holding this thread's vertex, if it fell
+      uint32_t key = kClean;
+      float own_last = own;
+      int sweep = 0;
+      bool conv = false;
+      while (sweep < inner) {
+        bool ch = false;
+        int nq = 1;
+        if constexpr (DIM == 2) {
+          ch = tri_sweep<N>(r, sT, large, eps, solves);
+        } else {
+          tet_select<N, BT>(r, sT, eps, sQ, &sh.qn[qc]);
+          __syncthreads();
+          nq = sh.qn[qc];
+          if (tid == 0) sh.qn[qc ^ 1] = 0;
+          qc ^= 1;
+          if (nq) ch = tet_solve<N, BT>(r, sA, sB, sQ, nq, sT, large, eps, solves);
+        }
+        if (ch) sh.flag[ring] = 1;
+        // (no pair selected: no time fell, and no thread waits for another's solve)
+        if (nq) __syncthreads();
+        const int any = nq ? sh.flag[ring] : 0;
+        ring = ring == 2 ? 0 : ring + 1;
+        if (tid == 0) sh.flag[ring == 2 ? 0 : ring + 1] = 0;
+        ++sweep;
+        // publish the owned times that fell
+        own_last = own;
+        if (tid < d.nown) {
+          const float v = sT[tid];
+          if (v < own) {
+            own = v;
+            (void)__hip_atomic_fetch_min(reinterpret_cast<unsigned*>(T + d.vstart + tid),
+                                         __float_as_uint(v), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+            marks |= vm;
+            key = __float_as_uint(v);
+          }
+        }
+        if (!any) {
+          conv = true;
+          break;
+        }
+      }
+      const unsigned long long t2 = wall_clock64();
+      // visits beyond the bound mark nothing more (runaway guard)
+      const bool cap_ok = (int64_t)sh.acc[0] < a.max_visits;
+      const bool more = !conv && cap_ok;
+      // marks made from here on are seen by the halo loads of the next visit or after it
+      if (more && tid == 0) sched_again(a.s, slot);
+      // reduced over the wave first: the compiler turns an LDS or with a uniform address into a
+      // scalar loop over the lanes (a third of a triangle sweep)
+      if (__ballot(key != kClean)) {
+        const uint32_t lo = wave_or((uint32_t)marks), hi = wave_or((uint32_t)(marks >> 32));
+        key = wave_umin(key);
+        if (__lane_id() == 63) {
+          atomicMin(&sh.key, key);
+          if (lo) atomicOr(&sh.mark[0], lo);
+          if (hi) atomicOr(&sh.mark[1], hi);
+        }
+      }
+      // the published times have reached the device's coherence point before the dependents are
+      // marked
+      wait_memory();
+      __syncthreads();
+      const unsigned long long tq = wall_clock64();
+      const uint32_t vkey = sh.key;
+      // visited again at once, unless another of the owner's blocks waits with a smaller time
+      const bool again = more && !(waiting < vkey);
+      if (tid < 64) {
+        const uint64_t mask = (uint64_t)sh.mark[0] | ((uint64_t)sh.mark[1] << 32);
+        if (cap_ok && tid < ndep && ((mask >> tid) & 1ull)) sched_mark(a.s, dep_slot, vkey);
+        if (tid < 2) sh.mark[tid] = 0;
+        if (tid == 0) {
+          VisitResult vr;
+          vr.sweeps = sweep;
+          vr.t_load = t1 - t0;
+          vr.t_sweep = t2 - t1;
+          vr.t_wb = tq - t2;
+          tally_visit(sh.acc, d, vr, 0, kAlgoElemBytes<DIM>, tq - t0, rerun, rerun);
+        }
+        if (again) {
+          const uint32_t w = sched_waiting(a.s, me);
+          if (tid == 0) sh.waiting = w;
+          if (tid == 0) sh.acc[10] += wall_clock64() - tq;
+        } else {
+          wait_memory();  // the marks have landed before this block can count as clean
+          if (tid == 0) {
+            sched_leave(a.s, slot, more ? vkey : kClean);
+            sh.waiting = kClean;
+            sh.acc[10] += wall_clock64() - tq;
+          }
+        }
+      } else if (!again) {
+        if (finder) {
+          const int32_t nb = a.s.per_owner > 1 ? find_next(a.s, f, sh.acc, true) : kNothing;
+          if (tid == 64) {
+            sh.block = nb;
+            sh.crowd = f.others;
+          }
+        }
+      } else {
+        // the halo times of the next visit (by the waves that mark nothing)
+        for (int i = tid - 64; i < d.nhalo; i += BT - 64)
+          sT[d.nown + i] = load_T<true>(T + sHidx[i]);
+      }
+      if (!again) {
+        // what this visit evaluated the block's elements with: every time, but for the owned
+        // vertices that fell in the last sweep of a visit cut off by the sweep cap.  A later
+        // visit that misses these (they are plain stores) evaluates more than it has to.
+        if (tid < d.nown) seen[tid] = conv ? own : own_last;
+        for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = sT[d.nown + i];
+      }
+      __syncthreads();
+      waiting = sh.waiting;
+      if (tid == 0) sh.key = kClean;
+      t0 = t1 = wall_clock64();
+      rerun = again;
+      if (again) continue;
+      b = __builtin_amdgcn_readfirstlane(sh.block);
+      if (b == kNothing) {
+        __syncthreads();
+        if (finder) {
+          const int32_t nb = find_next(a.s, f, sh.acc);
+          if (tid == 64) {
+            sh.block = nb;
+            sh.crowd = f.others;
+          }
+        }
+        __syncthreads();
+        b = __builtin_amdgcn_readfirstlane(sh.block);
+      }
+      if (b != cur) break;
+      // the same block, still resident: only times may have fallen (the owned ones if another
+      // workgroup visited the block meanwhile)
+      if (tid < d.nown) {
+        own = load_T<true>(T + d.vstart + tid);
+        sT[tid] = own;
+      }
+      for (int i = tid; i < d.nhalo; i += BT) sT[d.nown + i] = load_T<true>(T + sHidx[i]);
+      __syncthreads();
+      t1 = wall_clock64();
+    }
+  }
+  unsigned long long all = solves;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) all += __shfl_down(all, off, 64);
+  if (__lane_id() == 0 && all) atomicAdd(&sh.acc[3], all);
+  __syncthreads();
+  return b;
+}
+
+}  // namespace eik
