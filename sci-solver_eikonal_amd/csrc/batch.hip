@@ -205,7 +205,7 @@ struct MultiBlocks {
 // the workgroups begin with each kind and go on to the other when it has ended, so that a launch of
 // both takes about as long as the longer one instead of the sum, without two persistent kernels
 // waiting for each other's slots.
-template <int KINDS, int BT>
+template <int KINDS, int N3, int N2, int BT>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_multi_resident(
     MultiArgs a3, MultiArgs a2) {
   extern __shared__ uint4 lds4[];
@@ -217,10 +217,10 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const uint32_t me = KINDS != 3 ? blockIdx.x
                         : pass == 0 ? blockIdx.x >> 1 : gridDim.x == 1 ? 0u : 0xffffffffu;
     if constexpr ((KINDS & 1) != 0) {
-      if (tets) resident_loop<3, kTetN<BT>, BT>(a3.loop, MultiBlocks{a3.solves, a3.bsolve}, me, lds4, sh);
+      if (tets) resident_loop<3, N3, BT>(a3.loop, MultiBlocks{a3.solves, a3.bsolve}, me, lds4, sh);
     }
     if constexpr ((KINDS & 2) != 0) {
-      if (!tets) resident_loop<2, 4, BT>(a2.loop, MultiBlocks{a2.solves, a2.bsolve}, me, lds4, sh);
+      if (!tets) resident_loop<2, N2, BT>(a2.loop, MultiBlocks{a2.solves, a2.bsolve}, me, lds4, sh);
     }
   }
   unsigned long long* counters = KINDS == 2 ? a2.counters : a3.counters;
@@ -228,14 +228,20 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     atomicAdd(&counters[threadIdx.x], sh.acc[threadIdx.x]);
 }
 
-template <int KINDS>
-static const void* multi_resident(int bt) {
-  return bt == 256   ? (const void*)k_visit_multi_resident<KINDS, 256>
-         : bt == 512 ? (const void*)k_visit_multi_resident<KINDS, 512>
-                     : (const void*)k_visit_multi_resident<KINDS, 1024>;
-}
-static const void* multi_resident(int kinds, int bt) {
-  return kinds == 1 ? multi_resident<1>(bt) : kinds == 2 ? multi_resident<2>(bt) : multi_resident<3>(bt);
+// Elements and items per thread of a workgroup of bt threads: what the largest block of the launch
+// needs (n2: 1, 2 or 4 of the smallest that do).
+static const void* multi_resident(int kinds, int bt, int n3, int n2) {
+#define EIK_MULTI(n3_, n2_, bt_)                                                        \
+  return kinds == 1 ? (const void*)k_visit_multi_resident<1, n3_, 1, bt_>               \
+         : kinds == 2 ? (const void*)k_visit_multi_resident<2, 1, n2_, bt_>             \
+                      : (const void*)k_visit_multi_resident<3, n3_, n2_, bt_>
+  if (bt == 256 && n3 <= 4 && n2 <= 1) EIK_MULTI(4, 1, 256);
+  if (bt == 256 && n2 <= 1) EIK_MULTI(kTetN<256>, 1, 256);
+  if (bt == 512 && n2 <= 1) EIK_MULTI(kTetN<512>, 1, 512);
+  if (bt == 512 && n2 <= 2) EIK_MULTI(kTetN<512>, 2, 512);
+  if (bt == 512) EIK_MULTI(kTetN<512>, 4, 512);
+  EIK_MULTI(kTetN<1024>, 4, 1024);
+#undef EIK_MULTI
 }
 
 // ------------------------------------------------------------------------------------------
@@ -328,12 +334,29 @@ static void launch_visits(const Group& g, size_t lds, hipStream_t s, const Multi
 // Blocks per resident workgroup from which on a launch of tet blocks reads its records from memory.
 constexpr int kBusyBlocks = 24;
 
+// The register-resident kernel of a launch of these kinds (fn: null if their blocks do not fit): the
+// larger workgroup and LDS of the two.
+struct ResLaunch {
+  const void* fn;
+  int bt;
+  size_t lds;
+};
+static ResLaunch res_launch(const Launch& L, int kinds) {
+  const Group &g3 = L.grp[0], &g2 = L.grp[1];
+  if (((kinds & 1) && !g3.res_bt) || ((kinds & 2) && !g2.res_bt)) return {nullptr, 0, 0};
+  ResLaunch r = {nullptr, std::max(kinds & 1 ? g3.res_bt : 0, kinds & 2 ? g2.res_bt : 0),
+                 std::max(kinds & 1 ? g3.lds[2] : 0, kinds & 2 ? g2.lds[2] : 0)};
+  r.fn = multi_resident(kinds, r.bt, kinds & 1 ? (g3.max_elem + r.bt - 1) / r.bt : 0,
+                        kinds & 2 ? (g2.max_items + r.bt - 1) / r.bt : 0);
+  return r;
+}
+
 // Resident workgroups of a register-resident launch.
-static int resident_grid(const void* fn, int bt, size_t lds, int requested, int* out) {
+static int resident_grid(const ResLaunch& r, int requested, int* out) {
   int dev = 0, ncu = 0, per = 0;
   HIP_TRY(hipGetDevice(&dev));
   HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, bt, lds));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, r.fn, r.bt, r.lds));
   const int resident = std::min(std::max(1, ncu * std::max(per, 1)), 64 * ncu);
   *out = requested > 0 ? std::min(requested, resident) : resident;
   return EIK_OK;
@@ -389,10 +412,13 @@ int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
       g.max_elem = std::max(g.max_elem, Ly.max_elem);
       g.max_items = std::max(g.max_items, Ly.max_items);
       resident = resident && m->dev->res_n != 0;
-      g.res_bt = std::max(g.res_bt, (int)m->dev->res_bt);
     }
-    if (!resident) g.res_bt = 0;
     if (!g.present) continue;
+    const int need = g.dim == 3 ? g.max_elem : g.max_items;
+    static const int shapes[2][3][2] = {{{1, 256}, {4, 512}, {4, 1024}},
+                                        {{kTetN<256>, 256}, {kTetN<512>, 512}, {kTetN<1024>, 1024}}};
+    for (const auto& sh : shapes[g.dim == 3 ? 1 : 0])
+      if (resident && g.res_bt == 0 && need <= sh[0] * sh[1] && max_own <= sh[1]) g.res_bt = sh[1];
     Layout probe;
     probe.max_local = max_local;
     probe.max_own = max_own;
@@ -435,18 +461,9 @@ int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
   // the register-resident kernels that may run, for their LDS (a merged launch takes the larger
   // workgroup and LDS of the two kinds)
   for (int kinds = 1; kinds <= 3; ++kinds) {
-    int bt = 0;
-    size_t lds = 0;
-    bool all = true;
-    for (int gi = 0; gi < 2; ++gi) {
-      if (!((kinds >> gi) & 1)) continue;
-      all = all && L.grp[gi].res_bt > 0;
-      bt = std::max(bt, L.grp[gi].res_bt);
-      lds = std::max(lds, L.grp[gi].lds[2]);
-    }
-    if (all && lds > 65536)
-      HIP_TRY(hipFuncSetAttribute(multi_resident(kinds, bt),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const ResLaunch r = res_launch(L, kinds);
+    if (r.fn && r.lds > 65536)
+      HIP_TRY(hipFuncSetAttribute(r.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)r.lds));
   }
   L.cap_solves = cap_solves;
   L.cap_blocks = cap_blocks;
@@ -527,7 +544,7 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
     // direct, ms: 14 blocks per resident workgroup 2.41 / 3.83 (192 vertices per block), 21 3.34 / 3.44
     // (128) and 3.06 / 3.17 (64), 28 4.39 / 3.64 (192), 48 8.6 / 5.6 (192).  Triangle blocks are as
     // small resident: level-7 spheres 1.5 / 10.8.
-    int per = 0, rc = resident_grid(multi_resident(1 << gi, g.res_bt), g.res_bt, g.lds[2], 0, &per);
+    int per = 0, rc = resident_grid(res_launch(L, 1 << gi), 0, &per);
     if (rc) return rc;
     g.shape = gi == 0 && kblocks[0] > (int64_t)kBusyBlocks * per ? 1 : 2;
   }
@@ -537,10 +554,7 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
     if (!g.present) continue;
     int rc;
     if (g.shape == 2) {
-      const Group& h = L.merged ? L.grp[1 - gi] : g;
-      const int bt = std::max(g.res_bt, h.res_bt);
-      rc = resident_grid(multi_resident(L.merged ? 3 : 1 << gi, bt), bt, std::max(g.lds[2], h.lds[2]),
-                         o.workgroups, &g.grid);
+      rc = resident_grid(res_launch(L, L.merged ? 3 : 1 << gi), o.workgroups, &g.grid);
       // no more than one workgroup per block
       const int64_t most = L.merged ? 2 * std::max(kblocks[0], kblocks[1]) : kblocks[gi];
       g.grid = (int)std::min<int64_t>(g.grid, std::max<int64_t>(most, 1));
@@ -621,15 +635,11 @@ int launch_issue(Launch& L, int32_t nsolves, int64_t total_blocks, int64_t total
   if (g2.present && g2.shape == 0) launch_visits<2, kBlockThreads>(g2, g2.lds[0], s, a[1], sd);
   if (g2.present && g2.shape == 1) launch_visits<2, kDirectThreads>(g2, g2.lds[1], s, a[1], sd);
   void* args[] = {(void*)&a[0], (void*)&a[1]};
-  if (L.merged) {
-    const int bt = std::max(g3.res_bt, g2.res_bt);
-    HIP_TRY(hipLaunchKernel(multi_resident(3, bt), dim3(g3.grid), dim3(bt), args,
-                            std::max(g3.lds[2], g2.lds[2]), s));
-  } else {
-    for (int gi = 0; gi < 2; ++gi)
-      if (L.grp[gi].present && L.grp[gi].shape == 2)
-        HIP_TRY(hipLaunchKernel(multi_resident(1 << gi, L.grp[gi].res_bt), dim3(L.grp[gi].grid),
-                                dim3(L.grp[gi].res_bt), args, L.grp[gi].lds[2], s));
+  for (int gi = 0; gi < 2; ++gi) {
+    const Group& g = L.grp[gi];
+    if (!g.present || g.shape != 2 || (L.merged && gi == 1)) continue;
+    const ResLaunch r = res_launch(L, L.merged ? 3 : 1 << gi);
+    HIP_TRY(hipLaunchKernel(r.fn, dim3(g.grid), dim3(r.bt), args, r.lds, s));
   }
   HIP_TRY(hipMemcpyAsync(L.h_cnt, L.counters, sizeof(unsigned long long) * kNumCounters,
                          hipMemcpyDeviceToHost, s));

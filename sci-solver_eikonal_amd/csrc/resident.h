@@ -38,11 +38,20 @@ __device__ __forceinline__ bool fell(float last, float now, float eps) {
   return last - now > eps * now;
 }
 
+// What a sweep tests first it does for every item, changed or not, and with the instructions issued
+// on two thirds of all cycles (96^3 cube) their number counts: so an item holds the LDS offsets of its
+// corners' times instead of slots, and, for each corner, the time below which it counts as fallen,
+// last / (1 + eps), instead of the last time.
+__device__ __forceinline__ float fall_below(float last, float keep) { return last * keep; }
+__device__ __forceinline__ float time_at(const float* sT, uint32_t offset) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(sT) + offset);
+}
+
 template <int N>
 struct TriRegs {
-  uint32_t id[N];
+  uint32_t ab[N], t[N];  // LDS offsets of the two other corners, 16 bits each, and of the target
   float la[N], lb[N], lab[N], h[N];
-  float pa[N], pb[N];  // times of the two other corners at the last evaluation
+  float pa[N], pb[N];  // the two other corners: fallen below this since the last evaluation
 };
 
 // The thread index, opaque: what is computed from it is computed where it is used, not hoisted out of
@@ -63,7 +72,9 @@ __device__ __forceinline__ void tri_load(TriRegs<N>& r, const TriItems& t, int2 
   for (int u = 0; u < N; ++u) {
     const int i = u * BT + tid;
     const bool in = i < range.y;
-    r.id[u] = in ? t.id[range.x + i] : 0u;
+    const uint32_t id = in ? t.id[range.x + i] : 0u;
+    r.ab[u] = (id << 2 & 4 * (kItemSlots - 1)) | (id >> kItemSlotBits & (kItemSlots - 1)) << 18;
+    r.t[u] = id >> (2 * kItemSlotBits) << 2;
     const float4 l = in ? t.len[range.x + i] : make_float4(1.f, 1.f, 1.f, EIK_INF);
     r.la[u] = l.x;
     r.lb[u] = l.y;
@@ -83,23 +94,19 @@ __device__ __forceinline__ void tri_load(TriRegs<N>& r, const TriItems& t, int2 
   }
 }
 
-__device__ __forceinline__ int slot_a(uint32_t id) { return id & (kItemSlots - 1); }
-__device__ __forceinline__ int slot_b(uint32_t id) { return (id >> kItemSlotBits) & (kItemSlots - 1); }
-__device__ __forceinline__ int slot_t(uint32_t id) { return id >> (2 * kItemSlotBits); }
-
 template <int N>
-__device__ __forceinline__ void tri_seen(TriRegs<N>& r, const float* sP) {
+__device__ __forceinline__ void tri_seen(TriRegs<N>& r, const float* sP, float keep) {
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    r.pa[u] = sP[slot_a(r.id[u])];
-    r.pb[u] = sP[slot_b(r.id[u])];
+    r.pa[u] = fall_below(time_at(sP, r.ab[u] & 0xffffu), keep);
+    r.pb[u] = fall_below(time_at(sP, r.ab[u] >> 16), keep);
   }
 }
 
 // One sweep over the thread's items.  Returns whether it lowered a time.
 template <int N>
 __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large, float eps,
-                                          unsigned& solves) {
+                                          float keep, unsigned& solves) {
   float ta[N], tb[N], tk[N];
   // What a solve computes from the lengths alone stays in registers from sweep to sweep where there
   // is room (N = 2); for more items it would be spilled, so it is computed again.
@@ -109,16 +116,16 @@ __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large,
   }
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    ta[u] = sT[slot_a(r.id[u])];
-    tb[u] = sT[slot_b(r.id[u])];
-    tk[u] = sT[slot_t(r.id[u])];
+    ta[u] = time_at(sT, r.ab[u] & 0xffffu);
+    tb[u] = time_at(sT, r.ab[u] >> 16);
+    tk[u] = time_at(sT, r.t[u]);
   }
   bool changed = false;
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    if (!(fell(r.pa[u], ta[u], eps) || fell(r.pb[u], tb[u], eps))) continue;
-    r.pa[u] = ta[u];
-    r.pb[u] = tb[u];
+    if (!(ta[u] < r.pa[u] || tb[u] < r.pb[u])) continue;
+    r.pa[u] = fall_below(ta[u], keep);
+    r.pb[u] = fall_below(tb[u], keep);
     // nothing below the smaller time plus the height; unknown times are `large`, and no time
     // is above that
     if (!(tk[u] > __builtin_fminf(ta[u], tb[u]) + r.h[u])) continue;
@@ -129,30 +136,42 @@ __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large,
       cand = tri_corner_solve_wide(ta[u], tb[u], r.la[u], r.lb[u], r.lab[u], large);
     cand = __builtin_fmaxf(cand, 0.f);
     if (cand < tk[u]) {
-      atomicMin(reinterpret_cast<unsigned*>(&sT[slot_t(r.id[u])]), __float_as_uint(cand));
+      atomicMin(reinterpret_cast<unsigned*>(reinterpret_cast<char*>(sT) + r.t[u]), __float_as_uint(cand));
       changed |= fell(tk[u], cand, eps);
     }
   }
   return changed;
 }
 
-// Two non-negative values as fp16, rounded towards zero; and back.
+// Two non-negative values as fp16, rounded towards zero; and a sum with one of
+// them, in one instruction.
 __device__ __forceinline__ uint32_t half_pair(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
-__device__ __forceinline__ float half_lo(uint32_t p) {
-  return (float)__builtin_bit_cast(_Float16, (uint16_t)p);
+__device__ __forceinline__ float add_half_lo(float x, uint32_t p) {
+  float y;
+  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(x), "v"(p));
+  return y;
 }
-__device__ __forceinline__ float half_hi(uint32_t p) {
-  return (float)__builtin_bit_cast(_Float16, (uint16_t)(p >> 16));
+__device__ __forceinline__ float add_half_hi(float x, uint32_t p) {
+  float y;
+  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(x), "v"(p));
+  return y;
+}
+
+// The smallest of three times, which are not negative: as integers, which need no quieting of NaNs.
+__device__ __forceinline__ float time_min(float a, float b, float c) {
+  const uint32_t x = __float_as_uint(a), y = __float_as_uint(b), z = __float_as_uint(c);
+  const uint32_t m = x < y ? x : y;
+  return __uint_as_float(m < z ? m : z);
 }
 
 template <int N>
 struct TetRegs {
-  uint32_t v01[N], v23[N];     // corner slots, 16 bits each
+  uint32_t v01[N], v23[N];     // LDS offsets of the corners' times, 16 bits each
   // heights in fp16, rounded down (they stay lower bounds of every solve); +inf: not owned
   uint32_t h01[N], h23[N];
-  float p0[N], p1[N], p2[N], p3[N];  // corner times at the last selection
+  float p0[N], p1[N], p2[N], p3[N];  // the corners: fallen below this since the last selection
 };
 
 // Copies 16 bytes per lane from memory straight to LDS (lane i of the wave to base + 16 i), so that
@@ -198,21 +217,21 @@ __device__ __forceinline__ void tet_load(TetRegs<N>& r, const void* recs, const 
       h3 *= sf;
     }
     const unsigned n = in ? (unsigned)d.nown : 0u;
-    r.v01[u] = v.x;
-    r.v23[u] = v.y;
+    r.v01[u] = v.x << 2;  // (the LDS holds fewer than 2^14 times)
+    r.v23[u] = v.y << 2;
     r.h01[u] = half_pair((v.x & 0xffffu) < n ? h0 : EIK_INF, (v.x >> 16) < n ? h1 : EIK_INF);
     r.h23[u] = half_pair((v.y & 0xffffu) < n ? h2 : EIK_INF, (v.y >> 16) < n ? h3 : EIK_INF);
   }
 }
 
 template <int N>
-__device__ __forceinline__ void tet_seen(TetRegs<N>& r, const float* sP) {
+__device__ __forceinline__ void tet_seen(TetRegs<N>& r, const float* sP, float keep) {
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    r.p0[u] = sP[r.v01[u] & 0xffffu];
-    r.p1[u] = sP[r.v01[u] >> 16];
-    r.p2[u] = sP[r.v23[u] & 0xffffu];
-    r.p3[u] = sP[r.v23[u] >> 16];
+    r.p0[u] = fall_below(time_at(sP, r.v01[u] & 0xffffu), keep);
+    r.p1[u] = fall_below(time_at(sP, r.v01[u] >> 16), keep);
+    r.p2[u] = fall_below(time_at(sP, r.v23[u] & 0xffffu), keep);
+    r.p3[u] = fall_below(time_at(sP, r.v23[u] >> 16), keep);
   }
 }
 
@@ -239,50 +258,68 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
   return (uint32_t)x;
 }
 
+// A queued pair: thread and, in the low five bits, its element's place u and the corner, 4 u + k.
+template <int BT>
+__device__ __forceinline__ int item_elem(int item) { return (item >> 2 & 7) * BT + (item >> 5); }
+
+// Adds to an LDS counter, by one lane, without the scan over the lanes that the compiler makes of an
+// atomic with a result; returns the value before.
+__device__ __forceinline__ int lds_take(int* counter, int n) {
+  int old;
+  asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)"
+               : "=v"(old)
+               : "v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) int*)counter), "v"(n)
+               : "memory");
+  return old;
+}
+
 // Appends the (element, corner) pairs of the thread's elements that can improve to the queue.
+// About 190 vector instructions a wave for N = 4 (350 with slots, last times, quieted minima and
+// converted heights): the visits of the 64^3 cube 0.677 -> 0.650 ms, of the 96^3 cube 1.50 -> 1.44.
 template <int N, int BT>
-__device__ __forceinline__ void tet_select(TetRegs<N>& r, const float* sT, float eps, uint16_t* sQ,
-                                           int* qn) {
+__device__ __forceinline__ void tet_select(TetRegs<N>& r, int nelem, const float* sT, float keep,
+                                           uint16_t* sQ, int* qn) {
+  static_assert(N <= 8 && BT <= 2048, "queued pairs have 5 bits for the place, 11 for the thread");
+  // places of this wave that hold an element (64^3 cube 0.651 -> 0.633 ms with the others left out)
+  const int places = (nelem - __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63) + BT - 1) / BT;
   float t0[N], t1[N], t2[N], t3[N];
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    t0[u] = sT[r.v01[u] & 0xffffu];
-    t1[u] = sT[r.v01[u] >> 16];
-    t2[u] = sT[r.v23[u] & 0xffffu];
-    t3[u] = sT[r.v23[u] >> 16];
+    if (u >= 2 && u >= places) break;
+    t0[u] = time_at(sT, r.v01[u] & 0xffffu);
+    t1[u] = time_at(sT, r.v01[u] >> 16);
+    t2[u] = time_at(sT, r.v23[u] & 0xffffu);
+    t3[u] = time_at(sT, r.v23[u] >> 16);
   }
   unsigned sel = 0;
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    const bool f0 = fell(r.p0[u], t0[u], eps), f1 = fell(r.p1[u], t1[u], eps);
-    const bool f2 = fell(r.p2[u], t2[u], eps), f3 = fell(r.p3[u], t3[u], eps);
+    if (u >= 2 && u >= places) break;
+    const bool f0 = t0[u] < r.p0[u], f1 = t1[u] < r.p1[u];
+    const bool f2 = t2[u] < r.p2[u], f3 = t3[u] < r.p3[u];
     if (!(f0 || f1 || f2 || f3)) continue;
-    r.p0[u] = t0[u];
-    r.p1[u] = t1[u];
-    r.p2[u] = t2[u];
-    r.p3[u] = t3[u];
-    const float m01 = __builtin_fminf(t0[u], t1[u]), m23 = __builtin_fminf(t2[u], t3[u]);
-    const float mn0 = __builtin_fminf(t1[u], m23), mn1 = __builtin_fminf(t0[u], m23);
-    const float mn2 = __builtin_fminf(m01, t3[u]), mn3 = __builtin_fminf(m01, t2[u]);
-    unsigned s = (t0[u] > mn0 + half_lo(r.h01[u]) ? 1u : 0u) |
-                 (t1[u] > mn1 + half_hi(r.h01[u]) ? 2u : 0u) |
-                 (t2[u] > mn2 + half_lo(r.h23[u]) ? 4u : 0u) |
-                 (t3[u] > mn3 + half_hi(r.h23[u]) ? 8u : 0u);
-    // one corner alone changed: it has no new solve itself
-    const unsigned f = (f0 ? 1u : 0u) | (f1 ? 2u : 0u) | (f2 ? 4u : 0u) | (f3 ? 8u : 0u);
-    if ((f & (f - 1u)) == 0u) s &= ~f;
-    sel |= s << (4 * u);
+    r.p0[u] = fall_below(t0[u], keep);
+    r.p1[u] = fall_below(t1[u], keep);
+    r.p2[u] = fall_below(t2[u], keep);
+    r.p3[u] = fall_below(t3[u], keep);
+    // a corner is solved again if another one fell and it lies above the smallest of the others by
+    // more than its height
+    const bool c0 = t0[u] > add_half_lo(time_min(t1[u], t2[u], t3[u]), r.h01[u]);
+    const bool c1 = t1[u] > add_half_hi(time_min(t0[u], t2[u], t3[u]), r.h01[u]);
+    const bool c2 = t2[u] > add_half_lo(time_min(t0[u], t1[u], t3[u]), r.h23[u]);
+    const bool c3 = t3[u] > add_half_hi(time_min(t0[u], t1[u], t2[u]), r.h23[u]);
+    sel |= (c0 && (f1 || f2 || f3) ? 1u << 4 * u : 0u) | (c1 && (f0 || f2 || f3) ? 2u << 4 * u : 0u);
+    sel |= (c2 && (f0 || f1 || f3) ? 4u << 4 * u : 0u) | (c3 && (f0 || f1 || f2) ? 8u << 4 * u : 0u);
   }
   if (__ballot(sel != 0u) == 0ull) return;
   const int n = __popc(sel);
   const int end = wave_scan(n);
   int base = 0;
-  if (__lane_id() == 63) base = atomicAdd(qn, end);
+  if (__lane_id() == 63) base = lds_take(qn, end);
   base = __builtin_amdgcn_readlane(base, 63);
-  for (int q = base + end - n; sel; ++q, sel &= sel - 1u) {
-    const int k = __ffs(sel) - 1;
-    sQ[q] = (uint16_t)((((k >> 2) * BT + (int)threadIdx.x) << 2) | (k & 3));
-  }
+  const int me = (int)threadIdx.x << 5;
+  for (int q = base + end - n; sel; ++q, sel &= sel - 1u)
+    sQ[q] = (uint16_t)(me | (__ffs(sel) - 1));
 }
 
 struct TetItem {
@@ -291,12 +328,14 @@ struct TetItem {
   int k;
 };
 
+template <int BT>
 __device__ __forceinline__ TetItem tet_item(const uint4* sA, const uint4* sB, int item,
                                             const float* sT) {
   TetItem x;
+  const int e = item_elem<BT>(item);
   x.k = item & 3;
-  x.a = sA[item >> 2];
-  x.b = sB[item >> 2];
+  x.a = sA[e];
+  x.b = sB[e];
   x.t0 = sT[x.a.x & 0xffffu];
   x.t1 = sT[x.a.x >> 16];
   x.t2 = sT[x.a.y & 0xffffu];
@@ -326,7 +365,7 @@ __device__ __forceinline__ bool tet_solve_ill(TetRegs<N>& r, const uint4* sA, co
   asm volatile("" : : "v"(&keep) : "memory");  // in memory, not in registers
   bool changed = false;
   for (int q = threadIdx.x; q < nq; q += BT) {
-    const TetItem x = tet_item(sA, sB, sQ[q], sT);
+    const TetItem x = tet_item<BT>(sA, sB, sQ[q], sT);
     const float cand = tet_rotation_wide(
         x.k, x.t0, x.t1, x.t2, x.t3, __uint_as_float(x.a.z), __uint_as_float(x.a.w),
         __uint_as_float(x.b.x), __uint_as_float(x.b.y), __uint_as_float(x.b.z),
@@ -345,7 +384,7 @@ __device__ __forceinline__ bool tet_solve(TetRegs<N>& r, const uint4* sA, const 
                                           float eps, unsigned& solves) {
   bool changed = false, ill = false;
   for (int q = threadIdx.x; q < nq; q += BT) {
-    const TetItem x = tet_item(sA, sB, sQ[q], sT);
+    const TetItem x = tet_item<BT>(sA, sB, sQ[q], sT);
     ++solves;
     bool bad = false;
     const float cand = tet_rotation<kReport>(

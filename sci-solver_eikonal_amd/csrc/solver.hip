@@ -572,19 +572,26 @@ int upload_layout(Mesh& m) {
 
 static const void* resident_kernel(int dim, int n, int bt) {
   if (dim == 3)
-    return n == 4 && bt == 256 ? (const void*)k_visit_resident<3, 4, 256>
-           : bt == 256         ? (const void*)k_visit_resident<3, kTetN<256>, 256>
-           : bt == 512         ? (const void*)k_visit_resident<3, kTetN<512>, 512>
-                               : (const void*)k_visit_resident<3, kTetN<1024>, 1024>;
-  return n == 2      ? (const void*)k_visit_resident<2, 2, 256>
-         : bt == 256 ? (const void*)k_visit_resident<2, 4, 256>
-         : bt == 512 ? (const void*)k_visit_resident<2, 4, 512>
-                     : (const void*)k_visit_resident<2, 4, 1024>;
+    return n == 2                        ? (const void*)k_visit_resident<3, 2, 512>
+           : n == 4 && bt == 256         ? (const void*)k_visit_resident<3, 4, 256>
+           : bt == 256                   ? (const void*)k_visit_resident<3, kTetN<256>, 256>
+           : bt == 512                   ? (const void*)k_visit_resident<3, kTetN<512>, 512>
+                                         : (const void*)k_visit_resident<3, kTetN<1024>, 1024>;
+  return bt == 256    ? (const void*)k_visit_resident<2, 1, 256>
+         : bt == 1024 ? (const void*)k_visit_resident<2, 4, 1024>
+         : n == 1     ? (const void*)k_visit_resident<2, 1, 512>
+         : n == 2     ? (const void*)k_visit_resident<2, 2, 512>
+                      : (const void*)k_visit_resident<2, 4, 512>;
 }
 
 // The shape of the register-resident visits for this layout, and the triangle items.  A block
 // qualifies when one thread can hold each owned vertex and N x BT items (triangles) or elements
-// (tets) cover it; N and BT grow with the largest block.
+// (tets) cover it.  The shapes go from the smallest: few items per thread make the chain of a sweep
+// short (64-vertex triangle blocks, 1 per thread of 512 / 2 per thread of 256: level-7 anisotropic
+// icosphere 0.49 / 0.56 ms, level 8 1.56 / 1.67, 32^2 square 0.065 / 0.078; 301^2 square with
+// obtuse angles, up to 700 items, 2 of 512 / 4 of 256: 0.33 / 0.50).  A tet block keeps 40 KB and a CU
+// holds four of 256 threads or two of 512, so the wider workgroup is for meshes whose blocks it holds
+// all at once (16^3 cube 0.149 against 0.164 ms, 64^3 0.775 against 0.653).
 static int setup_resident(Mesh& m, size_t max_lds) {
   DeviceState* d = m.dev;
   const Layout& L = m.layout;
@@ -592,12 +599,19 @@ static int setup_resident(Mesh& m, size_t max_lds) {
   d->max_elem = L.max_elem;
   d->res_n = 0;
   if (L.vmask.empty()) return EIK_OK;
+  int dev = 0, ncu = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   const int32_t need = m.dim == 3 ? L.max_elem : L.max_items;
-  static const int shapes[2][4][2] = {{{2, 256}, {4, 256}, {4, 512}, {4, 1024}},
-                                      {{4, 256}, {kTetN<256>, 256}, {kTetN<512>, 512}, {kTetN<1024>, 1024}}};
-  for (const auto& sh : shapes[m.dim == 3 ? 1 : 0])
-    if (d->res_n == 0 && need <= sh[0] * sh[1]) d->res_n = sh[0], d->res_bt = sh[1];
-  if (d->res_n == 0 || L.max_own > d->res_bt || (m.dim == 2 && L.max_local > kItemSlots)) {
+  static const int shapes[2][5][2] = {
+      {{1, 256}, {1, 512}, {2, 512}, {4, 512}, {4, 1024}},
+      {{2, 512}, {4, 256}, {kTetN<256>, 256}, {kTetN<512>, 512}, {kTetN<1024>, 1024}}};
+  for (int i = m.dim == 3 && L.nblocks > 2 * ncu ? 1 : 0; i < 5 && d->res_n == 0; ++i) {
+    const int* sh = shapes[m.dim == 3 ? 1 : 0][i];
+    if (need <= sh[0] * sh[1] && L.max_own <= sh[1]) d->res_n = sh[0], d->res_bt = sh[1];
+  }
+  if (d->res_n == 0) return EIK_OK;
+  if (m.dim == 2 && L.max_local > kItemSlots) {
     d->res_n = 0;
     return EIK_OK;
   }
@@ -761,9 +775,8 @@ static VisitKernel visit_kernel(const DeviceState* d, int32_t stage_records) {
 
 // Workgroups of the single-solve persistent kernel: one per block while they all fit, so that every
 // block stays resident with its owner, else all that fit (64^3 cube, 4,292 blocks: 1.61 ms at 256,
-// 0.99 at 512, 0.72 at 1,024; 96^3, 14,261 blocks: 5.12, 2.90, 1.82).  Triangle meshes stop at three
-// per CU (level-7 anisotropic icosphere, 2,560 blocks: 0.76 ms at 256, 0.57 at 512, 0.55 at 768, 0.60
-// at 1,024; level 8, 10,240 blocks: 2.65, 1.88, 1.70, 1.69).
+// 0.99 at 512, 0.72 at 1,024; 96^3, 14,261 blocks: 5.12, 2.90, 1.82).  Triangle meshes
+// whose blocks take 256 threads stop at three per CU: beyond that, waiting workgroups only add traffic.
 static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t nblocks, int* out) {
   int dev = 0, ncu = 0, per_cu = 0;
   HIP_TRY(hipGetDevice(&dev));

@@ -52,9 +52,12 @@ struct LoopShared {
   int crowd;         // dirty blocks seen waiting when this one was claimed
 };
 
+// Words of an LDS array of local vertices; what follows three of them is 16-byte aligned.
+__host__ __device__ inline int32_t lds_stride(int32_t max_local) { return (max_local + 3) & ~3; }
+
 // Dynamic LDS of the loop, bytes.
 inline size_t loop_lds_bytes(int dim, int32_t max_local, int32_t max_elem, int32_t max_items) {
-  size_t n = sizeof(float) * 3 * (size_t)max_local;
+  size_t n = sizeof(float) * 3 * (size_t)lds_stride(max_local);
   if (dim == 3) n += 2 * sizeof(uint4) * (size_t)max_elem + sizeof(uint16_t) * (size_t)max_items;
   return n;
 }
@@ -98,13 +101,15 @@ template <int DIM, int N, int BT, class Blocks>
 __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& blocks, uint32_t me,
                                              uint4* lds4, LoopShared& sh) {
   const int tid = threadIdx.x;
-  uint4* sA = lds4;
+  // the times first: their offsets in the LDS are constants of the instructions that read them
+  const int ls = lds_stride(a.max_local);
+  float* sT = reinterpret_cast<float*>(lds4);
+  float* sP = sT + ls;
+  int* sHidx = reinterpret_cast<int*>(sP + ls);
+  uint4* sA = reinterpret_cast<uint4*>(sHidx + ls);
   uint4* sB = sA + (DIM == 3 ? a.max_elem : 0);
-  float* sT = reinterpret_cast<float*>(sB + (DIM == 3 ? a.max_elem : 0));
-  float* sP = sT + a.max_local;
-  int* sHidx = reinterpret_cast<int*>(sP + a.max_local);
-  uint16_t* sQ = reinterpret_cast<uint16_t*>(sHidx + a.max_local);
-  const float eps = a.eps, large = DIM == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
+  uint16_t* sQ = reinterpret_cast<uint16_t*>(sB + (DIM == 3 ? a.max_elem : 0));
+  const float eps = a.eps, keep = 1.f / (1.f + a.eps), large = DIM == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
   // (the barrier before the first visit orders these)
   if (tid < 3) sh.flag[tid] = 0;
   if (tid < 2) sh.qn[tid] = 0;
@@ -163,8 +168,8 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       tet_load<N, BT>(r, m.elems, d, sA, sB, rmult);
     wait_memory();  // the copies to LDS too
     __syncthreads();
-    if constexpr (DIM == 2) tri_seen<N>(r, sP);
-    else tet_seen<N>(r, sP);
+    if constexpr (DIM == 2) tri_seen<N>(r, sP, keep);
+    else tet_seen<N>(r, sP, keep);
     unsigned long long t1 = wall_clock64();
     bool rerun = false;
     unsigned waiting = kClean;  // smallest key of the owner's other blocks when last looked
@@ -181,9 +186,9 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
         bool ch = false;
         int nq = 1;
         if constexpr (DIM == 2) {
-          ch = tri_sweep<N>(r, sT, large, eps, solves);
+          ch = tri_sweep<N>(r, sT, large, eps, keep, solves);
         } else {
-          tet_select<N, BT>(r, sT, eps, sQ, &sh.qn[qc]);
+          tet_select<N, BT>(r, d.nelem, sT, keep, sQ, &sh.qn[qc]);
           __syncthreads();
           nq = sh.qn[qc];
           if (tid == 0) sh.qn[qc ^ 1] = 0;
