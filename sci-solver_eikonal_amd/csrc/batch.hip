@@ -205,7 +205,7 @@ struct MultiBlocks {
 // the workgroups begin with each kind and go on to the other when it has ended, so that a launch of
 // both takes about as long as the longer one instead of the sum, without two persistent kernels
 // waiting for each other's slots.
-template <int KINDS, int N3, int N2, int BT>
+template <int KINDS, int N3, int N2, int BT, bool CAP>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_multi_resident(
     MultiArgs a3, MultiArgs a2) {
   extern __shared__ uint4 lds4[];
@@ -217,10 +217,10 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const uint32_t me = KINDS != 3 ? blockIdx.x
                         : pass == 0 ? blockIdx.x >> 1 : gridDim.x == 1 ? 0u : 0xffffffffu;
     if constexpr ((KINDS & 1) != 0) {
-      if (tets) resident_loop<3, N3, BT>(a3.loop, MultiBlocks{a3.solves, a3.bsolve}, me, lds4, sh);
+      if (tets) resident_loop<3, N3, BT, CAP>(a3.loop, MultiBlocks{a3.solves, a3.bsolve}, me, lds4, sh);
     }
     if constexpr ((KINDS & 2) != 0) {
-      if (!tets) resident_loop<2, N2, BT>(a2.loop, MultiBlocks{a2.solves, a2.bsolve}, me, lds4, sh);
+      if (!tets) resident_loop<2, N2, BT, false>(a2.loop, MultiBlocks{a2.solves, a2.bsolve}, me, lds4, sh);
     }
   }
   unsigned long long* counters = KINDS == 2 ? a2.counters : a3.counters;
@@ -229,18 +229,21 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 }
 
 // Elements and items per thread of a workgroup of bt threads: what the largest block of the launch
-// needs (n2: 1, 2 or 4 of the smallest that do).
-static const void* multi_resident(int kinds, int bt, int n3, int n2) {
-#define EIK_MULTI(n3_, n2_, bt_)                                                        \
-  return kinds == 1 ? (const void*)k_visit_multi_resident<1, n3_, 1, bt_>               \
-         : kinds == 2 ? (const void*)k_visit_multi_resident<2, 1, n2_, bt_>             \
-                      : (const void*)k_visit_multi_resident<3, n3_, n2_, bt_>
-  if (bt == 256 && n3 <= 4 && n2 <= 1) EIK_MULTI(4, 1, 256);
-  if (bt == 256 && n2 <= 1) EIK_MULTI(kTetN<256>, 1, 256);
-  if (bt == 512 && n2 <= 1) EIK_MULTI(kTetN<512>, 1, 512);
-  if (bt == 512 && n2 <= 2) EIK_MULTI(kTetN<512>, 2, 512);
-  if (bt == 512) EIK_MULTI(kTetN<512>, 4, 512);
-  EIK_MULTI(kTetN<1024>, 4, 1024);
+// needs (n2: 1, 2 or 4 of the smallest that do); cap: the queue of the tets holds fewer than all pairs.
+static const void* multi_resident(int kinds, int bt, int n3, int n2, bool cap) {
+#define EIK_MULTI(n3_, n2_, bt_, cap_)                                                        \
+  return kinds == 1 ? (const void*)k_visit_multi_resident<1, n3_, 1, bt_, cap_>               \
+         : kinds == 2 ? (const void*)k_visit_multi_resident<2, 1, n2_, bt_, false>            \
+                      : (const void*)k_visit_multi_resident<3, n3_, n2_, bt_, cap_>
+  if (bt == 256 && n3 <= 4 && n2 <= 1) EIK_MULTI(4, 1, 256, false);
+  if (bt == 256 && n2 <= 1) EIK_MULTI(kTetN<256>, 1, 256, false);
+  if (bt == 512 && n2 <= 1 && cap) EIK_MULTI(kTetN<512>, 1, 512, true);
+  if (bt == 512 && n2 <= 1) EIK_MULTI(kTetN<512>, 1, 512, false);
+  if (bt == 512 && n2 <= 2 && cap) EIK_MULTI(kTetN<512>, 2, 512, true);
+  if (bt == 512 && n2 <= 2) EIK_MULTI(kTetN<512>, 2, 512, false);
+  if (bt == 512 && cap) EIK_MULTI(kTetN<512>, 4, 512, true);
+  if (bt == 512) EIK_MULTI(kTetN<512>, 4, 512, false);
+  EIK_MULTI(kTetN<1024>, 4, 1024, false);
 #undef EIK_MULTI
 }
 
@@ -331,7 +334,7 @@ static void launch_visits(const Group& g, size_t lds, hipStream_t s, const Multi
     hipLaunchKernelGGL((k_visit_multi<DIM, BT, 4>), dim3(g.grid), dim3(BT), lds, s, a, sd);
 }
 
-// Blocks per resident workgroup from which on a launch of tet blocks reads its records from memory.
+// Blocks per resident workgroup from which on a launch of tet blocks may read its records from memory.
 constexpr int kBusyBlocks = 24;
 
 // The register-resident kernel of a launch of these kinds (fn: null if their blocks do not fit): the
@@ -339,15 +342,23 @@ constexpr int kBusyBlocks = 24;
 struct ResLaunch {
   const void* fn;
   int bt;
+  int32_t queue;  // LoopArgs::max_queue of the tets
   size_t lds;
 };
 static ResLaunch res_launch(const Launch& L, int kinds) {
   const Group &g3 = L.grp[0], &g2 = L.grp[1];
-  if (((kinds & 1) && !g3.res_bt) || ((kinds & 2) && !g2.res_bt)) return {nullptr, 0, 0};
-  ResLaunch r = {nullptr, std::max(kinds & 1 ? g3.res_bt : 0, kinds & 2 ? g2.res_bt : 0),
-                 std::max(kinds & 1 ? g3.lds[2] : 0, kinds & 2 ? g2.lds[2] : 0)};
-  r.fn = multi_resident(kinds, r.bt, kinds & 1 ? (g3.max_elem + r.bt - 1) / r.bt : 0,
-                        kinds & 2 ? (g2.max_items + r.bt - 1) / r.bt : 0);
+  const bool tets = kinds & 1, tris = kinds & 2;
+  if ((tets && !g3.res_bt) || (tris && !g2.res_bt)) return {nullptr, 0, 0, 0};
+  ResLaunch r = {nullptr, std::max(tets ? g3.res_bt : 0, tris ? g2.res_bt : 0), 0, 0};
+  if (tets) {
+    r.queue = loop_queue(3, r.bt, g3.max_local, g3.max_elem, g3.max_items);
+    r.lds = loop_lds_bytes(3, g3.max_local, g3.max_elem, r.queue);
+  }
+  if (tris) r.lds = std::max(r.lds, loop_lds_bytes(2, g2.max_local, g2.max_elem, 0));
+  if (r.lds > (size_t)L.max_lds) return {nullptr, 0, 0, 0};
+  r.fn = multi_resident(kinds, r.bt, tets ? (g3.max_elem + r.bt - 1) / r.bt : 0,
+                        tris ? (g2.max_items + r.bt - 1) / r.bt : 0,
+                        tets && r.queue < g3.max_items);
   return r;
 }
 
@@ -386,6 +397,7 @@ int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
     L.device = dev;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0)
       max_lds = v - 1024;
+    L.max_lds = max_lds;
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   }
   // per element kind: LDS for its largest block, with the records read from memory (the
@@ -448,10 +460,6 @@ int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
     }
     g.rec_lds_bytes = rec_bytes;
     g.queue_cap = qcap_l;
-    if (g.res_bt) {
-      g.lds[2] = loop_lds_bytes(g.dim, g.max_local, g.max_elem, g.max_items);
-      if (g.lds[2] > (size_t)max_lds) g.res_bt = 0;
-    }
     // at most 64 workgroups per CU own words
     HIP_TRY(hipMalloc((void**)&g.words, sizeof(unsigned long long) *
                                             sched_max_words(cap_blocks, 64 * (size_t)std::max(ncu, 1))));
@@ -525,6 +533,8 @@ static void launch_bases(SolveDesc* sd, int32_t nsolves, int64_t n[2]) {
 int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solve_opts_t& o,
                 MultiArgs a[2]) {
   if (total_blocks >= (1ll << 30)) return fail(EIK_ERR_CAPACITY, "too many blocks in one launch");
+  int ncu = 0;
+  HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, L.device));
   // the blocks of each kind, numbered together
   int64_t kblocks[2];
   launch_bases(L.hsolves, nsolves, kblocks);
@@ -537,18 +547,24 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
                                     "staging; use fewer vertices per block or read the records "
                                     "from memory (EIK_STAGE_AUTO)");
     g.shape = o.stage_records == EIK_STAGE_LDS ? 0 : 1;
-    if (o.stage_records != EIK_STAGE_AUTO || g.res_bt == 0) continue;
-    // Register-resident visits, whose chain is short, unless there are so many tet blocks that every
-    // workgroup stays busy from its first visit to its last: then the records are read from memory at
-    // every use by smaller workgroups, of which more fit a CU.  Cubes of 16..48 vertices a side, resident /
-    // direct, ms: 14 blocks per resident workgroup 2.41 / 3.83 (192 vertices per block), 21 3.34 / 3.44
-    // (128) and 3.06 / 3.17 (64), 28 4.39 / 3.64 (192), 48 8.6 / 5.6 (192).  Triangle blocks are as
-    // small resident: level-7 spheres 1.5 / 10.8.
+    if (o.stage_records != EIK_STAGE_AUTO || !res_launch(L, 1 << gi).fn) continue;
+    // Register-resident visits, whose chain is short.  With so many tet blocks that every workgroup
+    // stays busy, though, what counts is how much of the meshes a CU holds at once: where that is
+    // less than 1,024 threads and 3,500 elements, the records are read from memory at every use by
+    // smaller workgroups, of which more fit.  64 cubes of 16..48 vertices a side, resident / from
+    // memory, ms: 48 vertices per block (2,800 elements a CU) 5.92 / 5.49, 64 (3,540) 5.12 / 5.26, 80
+    // 4.91 / 5.11, 96 (768 threads) 5.44 / 5.12, 128 (3,040) 6.40 / 5.05, 160 (3,560) 5.45 / 5.36, 192
+    // (4,270) 5.01 / 5.65, 208 (one workgroup) 7.90 / 5.72; with fewer blocks, 21 per workgroup of 128
+    // vertices 3.34 / 3.44, 14 of 192 2.41 / 3.83.  Triangle blocks are as small resident: level-7
+    // spheres 1.5 / 10.8.
     int per = 0, rc = resident_grid(res_launch(L, 1 << gi), 0, &per);
     if (rc) return rc;
-    g.shape = gi == 0 && kblocks[0] > (int64_t)kBusyBlocks * per ? 1 : 2;
+    const int cu = std::max(1, per / std::max(1, ncu));
+    const bool holds = cu * g.res_bt >= 1024 && cu * g.max_elem >= 3500;
+    g.shape = gi == 0 && !holds && kblocks[0] > (int64_t)kBusyBlocks * per ? 1 : 2;
   }
-  L.merged = L.grp[0].present && L.grp[1].present && L.grp[0].shape == 2 && L.grp[1].shape == 2;
+  L.merged = L.grp[0].present && L.grp[1].present && L.grp[0].shape == 2 && L.grp[1].shape == 2 &&
+             res_launch(L, 3).fn != nullptr;
   for (int gi = 0; gi < 2; ++gi) {
     Group& g = L.grp[gi];
     if (!g.present) continue;
@@ -580,6 +596,7 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
     x.loop.max_visits = (int64_t)(o.max_iterations > 0 ? o.max_iterations : 1000) * std::max<int64_t>(total_blocks, 1);
     x.loop.max_local = g.max_local;
     x.loop.max_elem = g.max_elem;
+    x.loop.max_queue = g.shape == 2 ? res_launch(L, L.merged ? 3 : 1 << gi).queue : 0;
     x.bsolve = g.bsolve;
     x.counters = L.counters;
     x.queue_cap = g.queue_cap;

@@ -86,6 +86,8 @@ struct DeviceState {
   // elements per thread (0: the blocks do not fit), threads, LDS strides and bytes, and for
   // triangles the items (resident.h, TriItems)
   int32_t res_n = 0, res_bt = 0;
+  int32_t max_queue = 0;
+  bool res_cap = false;  // the work-item queue holds fewer pairs than a block has
   int32_t max_local = 0, max_elem = 0;
   size_t res_lds = 0;
   int2* item_range = nullptr;

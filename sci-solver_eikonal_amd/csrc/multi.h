@@ -64,7 +64,7 @@ struct Group {
   unsigned long long* words = nullptr;
   unsigned char* sctl = nullptr;
   int32_t* bsolve = nullptr;
-  size_t lds[3] = {0, 0, 0};
+  size_t lds[2] = {0, 0};    // shapes 0 and 1
   size_t rec_lds_bytes = 0;  // shape 0
   int32_t queue_cap = 0;
   int32_t max_local = 0, max_elem = 0, max_items = 0;
@@ -79,6 +79,7 @@ struct Group {
 // seeds.  The descriptors are written per launch from the pinned hsolves.
 struct Launch {
   int device = -1;
+  int max_lds = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   Group grp[2];  // tets, triangles

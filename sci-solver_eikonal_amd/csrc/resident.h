@@ -273,12 +273,13 @@ __device__ __forceinline__ int lds_take(int* counter, int n) {
   return old;
 }
 
-// Appends the (element, corner) pairs of the thread's elements that can improve to the queue.
+// Appends the (element, corner) pairs of the thread's elements that can improve to the queue.  CAP:
+// it may hold fewer than a block has, max_queue; sets *again, and *full to the visit's number, if it did not hold them.
 // About 190 vector instructions a wave for N = 4 (350 with slots, last times, quieted minima and
 // converted heights): the visits of the 64^3 cube 0.677 -> 0.650 ms, of the 96^3 cube 1.50 -> 1.44.
-template <int N, int BT>
+template <int N, int BT, bool CAP>
 __device__ __forceinline__ void tet_select(TetRegs<N>& r, int nelem, const float* sT, float keep,
-                                           uint16_t* sQ, int* qn) {
+                                           uint16_t* sQ, int max_queue, int* qn, int* again, int* full, int visit) {
   static_assert(N <= 8 && BT <= 2048, "queued pairs have 5 bits for the place, 11 for the thread");
   // places of this wave that hold an element (64^3 cube 0.651 -> 0.633 ms with the others left out)
   const int places = (nelem - __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63) + BT - 1) / BT;
@@ -318,8 +319,18 @@ __device__ __forceinline__ void tet_select(TetRegs<N>& r, int nelem, const float
   if (__lane_id() == 63) base = lds_take(qn, end);
   base = __builtin_amdgcn_readlane(base, 63);
   const int me = (int)threadIdx.x << 5;
-  for (int q = base + end - n; sel; ++q, sel &= sel - 1u)
-    sQ[q] = (uint16_t)(me | (__ffs(sel) - 1));
+  int q = base + end - n;
+  if (!CAP || __builtin_expect(base + __builtin_amdgcn_readlane(end, 63) <= max_queue, 1)) {
+    for (; sel; ++q, sel &= sel - 1u) sQ[q] = (uint16_t)(me | (__ffs(sel) - 1));
+  } else {
+    for (; sel && q < max_queue; ++q, sel &= sel - 1u) sQ[q] = (uint16_t)(me | (__ffs(sel) - 1));
+    // what a full queue turns away counts as not evaluated, and another sweep follows
+    *again = 1;
+    *full = visit;
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (sel >> (4 * u) & 15u) r.p0[u] = r.p1[u] = r.p2[u] = r.p3[u] = EIK_INF;
+  }
 }
 
 struct TetItem {

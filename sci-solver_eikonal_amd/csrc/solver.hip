@@ -241,6 +241,7 @@ struct SolveArgs {
   int32_t elem_bytes;  // algorithmic bytes per element (visit_algo_bytes)
   int32_t max_local;   // LDS strides: local vertices and elements of the largest block
   int32_t max_elem;
+  int32_t max_queue;
   size_t rec_lds_bytes;  // k_visit_general: staged records
 };
 
@@ -261,13 +262,13 @@ struct SingleBlocks {
   }
 };
 
-template <int DIM, int N, int BT>
+template <int DIM, int N, int BT, bool CAP = false>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_resident(SolveArgs a) {
   extern __shared__ uint4 lds4[];
   __shared__ LoopShared sh;
   if (threadIdx.x < kNumCounters) sh.acc[threadIdx.x] = 0;
-  const LoopArgs la = {a.s, a.v.eps, a.v.max_inner, a.max_visits, a.max_local, a.max_elem};
-  const int end = resident_loop<DIM, N, BT>(la, SingleBlocks{a}, blockIdx.x, lds4, sh);
+  const LoopArgs la = {a.s, a.v.eps, a.v.max_inner, a.max_visits, a.max_local, a.max_elem, a.max_queue};
+  const int end = resident_loop<DIM, N, BT, CAP>(la, SingleBlocks{a}, blockIdx.x, lds4, sh);
   write_out(a, end);
   if (threadIdx.x < kNumCounters && sh.acc[threadIdx.x])
     atomicAdd(&a.counters[threadIdx.x], sh.acc[threadIdx.x]);
@@ -570,11 +571,12 @@ int upload_layout(Mesh& m) {
   return EIK_OK;
 }
 
-static const void* resident_kernel(int dim, int n, int bt) {
+static const void* resident_kernel(int dim, int n, int bt, bool cap) {
   if (dim == 3)
     return n == 2                        ? (const void*)k_visit_resident<3, 2, 512>
            : n == 4 && bt == 256         ? (const void*)k_visit_resident<3, 4, 256>
            : bt == 256                   ? (const void*)k_visit_resident<3, kTetN<256>, 256>
+           : bt == 512 && cap            ? (const void*)k_visit_resident<3, kTetN<512>, 512, true>
            : bt == 512                   ? (const void*)k_visit_resident<3, kTetN<512>, 512>
                                          : (const void*)k_visit_resident<3, kTetN<1024>, 1024>;
   return bt == 256    ? (const void*)k_visit_resident<2, 1, 256>
@@ -615,13 +617,15 @@ static int setup_resident(Mesh& m, size_t max_lds) {
     d->res_n = 0;
     return EIK_OK;
   }
-  d->res_lds = loop_lds_bytes(m.dim, L.max_local, L.max_elem, L.max_items);
+  d->max_queue = loop_queue(m.dim, d->res_bt, L.max_local, L.max_elem, L.max_items);
+  d->res_cap = m.dim == 3 && d->max_queue < L.max_items;
+  d->res_lds = loop_lds_bytes(m.dim, L.max_local, L.max_elem, d->max_queue);
   if (d->res_lds > max_lds) {
     d->res_n = 0;
     return EIK_OK;
   }
   if (d->res_lds > 65536)
-    HIP_TRY(hipFuncSetAttribute(resident_kernel(m.dim, d->res_n, d->res_bt),
+    HIP_TRY(hipFuncSetAttribute(resident_kernel(m.dim, d->res_n, d->res_bt, d->res_cap),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)d->res_lds));
   if (m.dim == 3) return EIK_OK;
   std::vector<int2> range(L.nblocks);
@@ -764,7 +768,7 @@ static VisitKernel visit_kernel(const DeviceState* d, int32_t stage_records) {
   if (d->res_n && stage_records != EIK_STAGE_MEMORY) {
     k.threads = d->res_bt;
     k.lds = d->res_lds;
-    k.fn = resident_kernel(d->dim, d->res_n, d->res_bt);
+    k.fn = resident_kernel(d->dim, d->res_n, d->res_bt, d->res_cap);
     return k;
   }
   k.threads = kBlockThreads;
@@ -881,6 +885,7 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   a.max_visits = (int64_t)(o.max_iterations > 0 ? o.max_iterations : 1000) * d->nblocks;
   a.elem_bytes = m.dim == 3 ? kAlgoElemBytes<3> : kAlgoElemBytes<2>;
   a.max_local = d->max_local;
+  a.max_queue = d->max_queue;
   a.max_elem = d->max_elem;
   a.rec_lds_bytes = k.stage ? d->rec_lds_bytes : 0;
   FillSegs f;

@@ -38,12 +38,14 @@ struct LoopArgs {
   int64_t max_visits;  // runaway guard: visits of one workgroup after which it marks nothing
   int32_t max_local;   // LDS strides: local vertices and elements of the largest block
   int32_t max_elem;
+  int32_t max_queue;   // pairs the work-item queue holds (tets)
 };
 
 // The workgroup's static LDS.
 struct LoopShared {
   unsigned long long acc[kNumCounters];  // its tally
   int flag[3];       // a sweep's "a time fell", in a ring over the sweeps
+  int full;          // the last visit with a sweep that selected more pairs than the queue holds
   int qn[2];         // work-item counters of alternate sweeps (tets)
   unsigned mark[2];  // dependents whose halo holds a vertex lowered in this visit
   int block;
@@ -55,11 +57,26 @@ struct LoopShared {
 // Words of an LDS array of local vertices; what follows three of them is 16-byte aligned.
 __host__ __device__ inline int32_t lds_stride(int32_t max_local) { return (max_local + 3) & ~3; }
 
-// Dynamic LDS of the loop, bytes.
-inline size_t loop_lds_bytes(int dim, int32_t max_local, int32_t max_elem, int32_t max_items) {
+// Dynamic LDS of the loop, bytes, with a work-item queue of max_queue pairs (tets).
+inline size_t loop_lds_bytes(int dim, int32_t max_local, int32_t max_elem, int32_t max_queue) {
   size_t n = sizeof(float) * 3 * (size_t)lds_stride(max_local);
-  if (dim == 3) n += 2 * sizeof(uint4) * (size_t)max_elem + sizeof(uint16_t) * (size_t)max_items;
+  if (dim == 3) n += 2 * sizeof(uint4) * (size_t)max_elem + sizeof(uint16_t) * (size_t)max_queue;
   return n;
+}
+
+// Pairs the work-item queue holds: all a block has, unless that costs the CU a workgroup and as many
+// as it has elements do not (a sweep selects about a tenth of the pairs; what a full queue turns
+// away is selected again by the next sweep).  For the workgroups of 512 threads: 64 cubes at 192 vertices
+// per block 8.1 -> 5.2 ms with two of them instead of one.
+inline int32_t loop_queue(int dim, int bt, int32_t max_local, int32_t max_elem, int32_t max_items) {
+  if (dim != 3) return 0;
+  if (bt != 512) return max_items;
+  // what each of the CU's workgroups has beside the static LDS
+  const size_t most = 163840 / (1024 / bt) - ((sizeof(LoopShared) + 15) & ~(size_t)15);
+  const size_t none = loop_lds_bytes(dim, max_local, max_elem, 0);
+  if (none + sizeof(uint16_t) * (size_t)max_items <= most) return max_items;
+  if (none + sizeof(uint16_t) * (size_t)max_elem > most) return max_items;
+  return (int32_t)((most - none) / sizeof(uint16_t));
 }
 
 // Blocks seen waiting when a tet block is claimed from which on its visit runs up to max_inner sweeps:
@@ -97,7 +114,7 @@ __device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned
 // 0.081.
 // blocks(g) gives the data of launch-wide block g; me is the workgroup's owner index.  Returns kNoWork or kGaveUp.  The workgroup's tally
 // is added to sh.acc, which the caller has cleared (behind a barrier) and flushes.
-template <int DIM, int N, int BT, class Blocks>
+template <int DIM, int N, int BT, bool CAP, class Blocks>
 __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& blocks, uint32_t me,
                                              uint4* lds4, LoopShared& sh) {
   const int tid = threadIdx.x;
@@ -115,6 +132,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
   if (tid < 2) sh.qn[tid] = 0;
   if (tid < 2) sh.mark[tid] = 0;
   if (tid == 0) sh.key = kClean;
+  if (tid == 0) sh.full = 0;
   // the second wave looks for work, while the first hands on what the last visit did
   const bool finder = tid >= 64 && tid < 128;
   Finder f;
@@ -122,6 +140,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
   int ring = 0;  // sweeps run so far, modulo 3
   int qc = 0;
   uint32_t solves = 0;
+  int visit = 1;
   __syncthreads();
   if (finder) {
     const int32_t nb = find_next(a.s, f, sh.acc);
@@ -188,9 +207,11 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
         if constexpr (DIM == 2) {
           ch = tri_sweep<N>(r, sT, large, eps, keep, solves);
         } else {
-          tet_select<N, BT>(r, d.nelem, sT, keep, sQ, &sh.qn[qc]);
+          tet_select<N, BT, CAP>(r, d.nelem, sT, keep, sQ, a.max_queue, &sh.qn[qc], &sh.flag[ring],
+                            &sh.full, visit);
           __syncthreads();
           nq = sh.qn[qc];
+          if (CAP) nq = min(nq, a.max_queue);
           if (tid == 0) sh.qn[qc ^ 1] = 0;
           qc ^= 1;
           if (nq) ch = tet_solve<N, BT>(r, sA, sB, sQ, nq, sT, large, eps, solves);
@@ -243,8 +264,11 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       __syncthreads();
       const unsigned long long tq = wall_clock64();
       const uint32_t vkey = sh.key;
+      const bool full = DIM == 3 && CAP && sh.full == visit;
+      ++visit;
+      const uint32_t lkey = full ? 0u : vkey;  // what the block waits with: its smallest new time
       // visited again at once, unless another of the owner's blocks waits with a smaller time
-      const bool again = more && !(waiting < vkey);
+      const bool again = more && !(waiting < lkey);
       if (tid < 64) {
         const uint64_t mask = (uint64_t)sh.mark[0] | ((uint64_t)sh.mark[1] << 32);
         if (cap_ok && tid < ndep && ((mask >> tid) & 1ull)) sched_mark(a.s, dep_slot, vkey);
@@ -264,7 +288,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
         } else {
           wait_memory();  // the marks have landed before this block can count as clean
           if (tid == 0) {
-            sched_leave(a.s, slot, more ? vkey : kClean);
+            sched_leave(a.s, slot, more ? lkey : kClean);
             sh.waiting = kClean;
             sh.acc[10] += wall_clock64() - tq;
           }
@@ -286,8 +310,9 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
         // what this visit evaluated the block's elements with: every time, but for the owned
         // vertices that fell in the last sweep of a visit cut off by the sweep cap.  A later
         // visit that misses these (they are plain stores) evaluates more than it has to.
-        if (tid < d.nown) seen[tid] = conv ? own : own_last;
-        for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = sT[d.nown + i];
+        // After a full queue, nothing counts as evaluated.
+        if (tid < d.nown) seen[tid] = full ? EIK_INF : conv ? own : own_last;
+        for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = full ? EIK_INF : sT[d.nown + i];
       }
       __syncthreads();
       waiting = sh.waiting;

@@ -80,3 +80,21 @@ def test_busy_launch(E):
         Ts, _ = b.solve(seeds)
         for i in (0, solves // 2, solves - 1):
             _same(Ts[i], m.solve(seeds[i])[0])
+
+
+@pytest.mark.parametrize("vpb", [188, 192])
+def test_full_queue(E, vpb):
+    """Blocks whose queue holds fewer pairs than they have, so that two fit a CU, with every vertex a
+    source: the first sweep selects most pairs of a block.  As many pairs as a queue turns away are
+    selected again.  Against the synchronous scheduler, whose queue holds them all."""
+    m = E.Mesh.kuhn_cube(24, 0.2, seed=vpb)
+    m.partition(vpb)
+    rng = np.random.default_rng(vpb)
+    seeds = np.arange(m.nv, dtype=np.int32)
+    values = rng.uniform(0.0, 4.0, m.nv).astype(np.float32)
+    ref, _ = m.solve(seeds, values, scheduler=E.SCHED_SYNC)
+    T, _ = m.solve(seeds, values)
+    _same(T, ref)
+    Ts, _ = E.Batch([m, m]).solve([seeds, seeds], [values, values])
+    _same(Ts[0], ref)
+    _same(Ts[1], ref)
