@@ -46,8 +46,6 @@ struct DeviceState {
   void* elems = nullptr;
   int32_t* halo = nullptr;
   int32_t* iperm = nullptr;
-  int32_t* sup_start = nullptr;
-  int32_t* sup = nullptr;
   int32_t* dep_start = nullptr;
   int32_t* dep = nullptr;
   int32_t* owner = nullptr;
@@ -61,10 +59,9 @@ struct DeviceState {
   int32_t* rec_elem = nullptr;
   int32_t rec_lds = 0;
   size_t rec_lds_bytes = 0;
-  int32_t* chg = nullptr;
-  int32_t* self = nullptr;
+  int32_t* stamp[2] = {nullptr, nullptr};  // synchronous scheduler (Active), by parity of the iteration
   int32_t* list[2] = {nullptr, nullptr};
-  int32_t* count = nullptr;  // active counts of even and odd iterations, last visited iteration
+  int32_t* count = nullptr;  // active counts of iterations modulo 3, last visited iteration
   unsigned long long* counters = nullptr;
   unsigned long long* sync_acc = nullptr;  // kSyncSlots * kSyncSlotWords
   int32_t* seeds = nullptr;
@@ -74,7 +71,9 @@ struct DeviceState {
   // (2 * seed_cap words) on the way in, the counters on the way out
   int32_t* h_seed = nullptr;
   unsigned long long* h_cnt = nullptr;
-  float* h_out = nullptr;  // behind h_cnt: a small mesh's times (kSmallOut)
+  // behind h_cnt: a word that the synchronous scheduler's iterations write, a small mesh's times
+  // (kSmallOut)
+  float* h_out = nullptr;
   // persistent scheduler (block_sched.h): block words and control words
   unsigned long long* words = nullptr;
   unsigned char* sctl = nullptr;

@@ -22,9 +22,9 @@ constexpr int64_t kSmallOut = 65536;
 static int dev_free(DeviceState* d) {
   if (!d) return EIK_OK;
   for (float* p : d->hist) (void)hipFree(p);
-  void* ptrs[] = {d->esel, d->elen, d->rec_elem, d->vmask, d->vh_start, d->vh_pos, d->seen, d->blocks, d->elems,  d->halo,  d->iperm,   d->sup_start, d->sup,
-                  d->dep_start, d->dep, d->owner, d->T,      d->out,      d->chg,
-                  d->self,   d->list[0], d->list[1], d->count, d->counters, d->sync_acc, d->seeds,
+  void* ptrs[] = {d->esel, d->elen, d->rec_elem, d->vmask, d->vh_start, d->vh_pos, d->seen, d->blocks, d->elems,  d->halo,  d->iperm,
+                  d->dep_start, d->dep, d->owner, d->T,      d->out,      d->stamp[0],
+                  d->stamp[1], d->list[0], d->list[1], d->count, d->counters, d->sync_acc, d->seeds,
                   d->seedvals, d->words, d->sctl,
                   d->item_range, d->item_id, d->item_len, d->item_rec};
   for (void* p : ptrs)
@@ -84,80 +84,57 @@ void launch_fill(const FillSegs& f, hipStream_t s) {
                      dim3(256), 0, s, f);
 }
 
-// seeds: caller ids -> new ids; T = value; the owner block of each seed is marked changed
-// (boundary and self) at stamp 0 so the first activation pass schedules it and its dependents.
-// A seed outside [0, nv) is skipped (the entry point that takes seeds in device memory cannot
-// check them on the host).  chg / self may be null (the persistent scheduler needs no stamps).
-__global__ void k_seed(const int32_t* seeds, const float* vals, int64_t n, const int32_t* iperm,
-                       const int32_t* owner, float* T, int32_t* chg, int32_t* self, int64_t nv) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || seeds[i] < 0 || seeds[i] >= nv) return;
-  int32_t v = iperm[seeds[i]];
-  atomicMin(reinterpret_cast<unsigned*>(&T[v]), __float_as_uint(vals ? vals[i] : 0.f));
-  int32_t b = owner[v];
-  if (chg) chg[b] = 0;
-  if (self) self[b] = 0;
+// The active blocks of an iteration of the synchronous scheduler: their number and list, and per
+// block the last iteration it was put on a list of this parity.
+struct Active {
+  int32_t* stamp;
+  int32_t* list;
+  int32_t* count;
+};
+
+// One whole wave: lane j of the first m puts block c on the list of iteration it, unless it is there.
+__device__ __forceinline__ void activate(const Active& next, int32_t it, bool mine, int32_t c) {
+  const bool add = mine && atomicExch(&next.stamp[c], it) != it;
+  const uint64_t bal = __ballot(add);
+  if (!bal) return;
+  int base = 0;
+  if (__lane_id() == 0) base = atomicAdd(next.count, __popcll(bal));
+  base = __builtin_amdgcn_readfirstlane(base);
+  if (add) next.list[base + __popcll(bal & lane_mask_lt())] = c;
 }
 
-// Next active list: block c is active at iteration it+1 if it did not converge in iteration it
-// or a block it depends on (a supplier of its halo) changed boundary values in iteration it.
-// Replaces the reference's host loop over blockCon and m_BlockNeighbor
-// (meshFIM3dEikonal.cu:445-488, 518-527; meshFIM2d_eikonal.cu:730-799).
-// The workgroups from act_wgs on copy T to snap instead (the per-iteration history, when snap
-// is set and the iteration just ended visited a block: *count_cur > 0), which saves a launch
-// per iteration.
-__global__ void k_activate(int32_t nb, const int32_t* __restrict__ sup_start,
-                           const int32_t* __restrict__ sup, const int32_t* __restrict__ chg,
-                           const int32_t* __restrict__ self, int32_t it, int32_t* __restrict__ list,
-                           int32_t* __restrict__ count, int32_t act_wgs, const float* __restrict__ T,
-                           int64_t nv, const int32_t* __restrict__ count_cur,
-                           float* __restrict__ snap) {
-  if ((int32_t)blockIdx.x >= act_wgs) {
-    if (!snap || *count_cur <= 0) return;
-    const int64_t stride = (int64_t)(gridDim.x - act_wgs) * blockDim.x;
-    for (int64_t i = (int64_t)(blockIdx.x - act_wgs) * blockDim.x + threadIdx.x; i < nv; i += stride)
-      snap[i] = T[i];
-    return;
-  }
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  bool act = false;
-  if (c < nb) {
-    // suppliers 16 at a time, all their loads in flight at once (a block of the 64^3 cube has
-    // 13 on average): two memory round trips per batch instead of two per supplier
-    constexpr int kB = 16;
-    const int s1 = sup_start[c + 1];
-    act = self[c] == it;
-    for (int s = sup_start[c]; !act && s < s1; s += kB) {
-      int32_t g[kB], v[kB];
-#pragma unroll
-      for (int j = 0; j < kB; ++j) g[j] = s + j < s1 ? sup[s + j] : -1;
-#pragma unroll
-      for (int j = 0; j < kB; ++j) v[j] = g[j] >= 0 ? chg[g[j]] : -2;  // stamps are >= -1
-#pragma unroll
-      for (int j = 0; j < kB; ++j) act |= v[j] == it;
+// seeds: caller ids -> new ids; T = value; the owner block of each seed and its dependents are active
+// in iteration 1 (one workgroup per seed).
+__global__ void k_sync_seed(const int32_t* seeds, const float* vals, int64_t n, const int32_t* iperm,
+                            const int32_t* owner, const int32_t* dep_start, const int32_t* dep,
+                            float* T, Active next) {
+  for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const int32_t v = iperm[seeds[i]];
+    if (threadIdx.x == 0)
+      atomicMin(reinterpret_cast<unsigned*>(&T[v]), __float_as_uint(vals ? vals[i] : 0.f));
+    const int32_t b = owner[v], s0 = dep_start[b], nd = dep_start[b + 1] - s0;
+    for (int j0 = 0; j0 <= nd; j0 += 64) {
+      const int j = j0 + (int)threadIdx.x;
+      activate(next, 1, j <= nd, j < nd ? dep[s0 + j] : b);
     }
   }
-  uint64_t bal = __ballot(act);
-  int n = __popcll(bal);
-  int base = 0;
-  if (__lane_id() == 0 && n) base = atomicAdd(count, n);
-  base = __shfl(base, 0, 64);
-  if (act) list[base + __popcll(bal & lane_mask_lt())] = c;
 }
 
 struct SyncArgs {
   VisitArgs v;
   size_t rec_lds_bytes;
-  const int32_t* list;
-  const int32_t* count;  // active blocks of this iteration (the grid may be larger)
-  int32_t* count_next;   // cleared here: the activation after this iteration fills it
-  int32_t* iters;        // outer iterations that visited at least one block
+  Active now, next;
+  int32_t* count_after;      // cleared here: the visits of the next iteration fill it
+  int32_t* last;             // the last iteration that visited a block
+  unsigned long long* told;  // pinned host memory: last << 32 | it, once iteration it has begun
+  const int32_t* dep;
+  int32_t nb;
   int32_t it;
-  int32_t* chg;
-  int32_t* self;
-  unsigned long long* acc;  // kSyncSlots slot lines of counters
-  int32_t elem_bytes;  // algorithmic bytes per element (visit_algo_bytes)
+  float* snap;               // the times after this iteration (the per-iteration history), or null
+  unsigned long long* acc;   // kSyncSlots slot lines of counters
+  int32_t elem_bytes;        // algorithmic bytes per element (visit_algo_bytes)
 };
+constexpr int kSnapBlocks = 16;  // blocks whose times a workgroup copies to the history
 
 // Adds one visit's counters to the workgroup's slot line (kSyncSlots lines, summed by
 // k_sum_slots after the solve).
@@ -193,22 +170,41 @@ __global__ void k_sum_slots(const unsigned long long* acc, unsigned long long* c
   counters[k] += s;
 }
 
-// One outer iteration: workgroup i visits the i-th active block.  The host enqueues several
-// iterations without waiting, so the grid covers every block and the workgroups beyond this
-// iteration's active count leave at once (an iteration after convergence is empty).
+// One outer iteration: workgroup i visits the i-th active block and puts the blocks whose halo holds a
+// vertex it lowered, and itself if it did not converge, on the list of the next iteration.  Replaces
+// the reference's host loop over blockCon and m_BlockNeighbor (meshFIM3dEikonal.cu:445-488, 518-527;
+// meshFIM2d_eikonal.cu:730-799).  The host enqueues several iterations without waiting, so the grid
+// covers every block and the workgroups beyond this iteration's active count leave at once (an
+// iteration after convergence is empty).  For the history, a visit writes its block's times, and
+// the workgroups from nb on copy those of the blocks that are not active, which no one changes now:
+// one launch per iteration (48^3 cube with history, 43 iterations, in all: 1.35 -> 1.06 ms; a launch
+// that looked through every block's suppliers took 5 us of each, the host's waits 0.2 ms).
 template <int DIM>
 __global__ __launch_bounds__(kBlockThreads) void k_visit_sync(SyncArgs a) {
   extern __shared__ uint4 lds4[];
   __shared__ int sFlag[4];
   __shared__ int sQn[2];  // work-item counters of alternate chunks
   __shared__ unsigned long long sRed;
-  const int n = *a.count;
+  const int n = *a.now.count;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *a.count_next = 0;
-    if (n > 0) *a.iters = a.it;
+    *a.count_after = 0;
+    const int32_t last = n > 0 ? a.it : *a.last;
+    *a.last = last;
+    __hip_atomic_store(a.told, (unsigned long long)last << 32 | (unsigned)a.it, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if ((int)blockIdx.x >= a.nb) {
+    if (n <= 0) return;
+    const int c0 = ((int)blockIdx.x - a.nb) * kSnapBlocks;
+    for (int c = c0 + (int)(threadIdx.x >> 6); c < min(c0 + kSnapBlocks, a.nb); c += kBlockThreads / 64) {
+      if (a.now.stamp[c] == a.it) continue;
+      const BlockDesc d = a.v.blocks[c];
+      for (int i = (int)__lane_id(); i < d.nown; i += 64) a.snap[d.vstart + i] = a.v.T[d.vstart + i];
+    }
+    return;
   }
   if ((int)blockIdx.x >= n) return;
-  const int b = a.list[blockIdx.x];
+  const int b = a.now.list[blockIdx.x];
   const BlockDesc d = a.v.blocks[b];
   VisitLds l = carve_lds<DIM>(lds4, a.rec_lds_bytes, a.v.queue_cap, d);
   if (threadIdx.x == 0) sRed = 0;
@@ -216,10 +212,17 @@ __global__ __launch_bounds__(kBlockThreads) void k_visit_sync(SyncArgs a) {
   const unsigned long long t0 = wall_clock64();
   VisitResult r = visit_block<DIM, false>(a.v, b, l.rec, l.T, l.old, l.chg, l.hidx, l.vm, l.q, l.mark,
                                           sFlag, sQn, &solves);
-  if (threadIdx.x == 0) {
-    if (r.bnd_changed) a.chg[b] = a.it;
-    if (!r.converged) a.self[b] = a.it;
+  if (threadIdx.x < 64) {
+    const int32_t s0 = a.v.dep_start[b];
+    const int nd = r.bnd_changed ? a.v.dep_start[b + 1] - s0 : 0;
+    const int m = nd + (r.converged ? 0 : 1);
+    for (int j0 = 0; j0 < m; j0 += 64) {
+      const int j = j0 + (int)threadIdx.x;
+      activate(a.next, a.it + 1, j < m, j < nd ? a.dep[s0 + j] : b);
+    }
   }
+  if (a.snap)
+    for (int i = (int)threadIdx.x; i < d.nown; i += kBlockThreads) a.snap[d.vstart + i] = l.T[i];
   block_counters(a.acc, d, r.sweeps, solves, a.elem_bytes, wall_clock64() - t0, r, &sRed);
 }
 
@@ -543,8 +546,6 @@ int upload_layout(Mesh& m) {
   }
   if ((rc = upload(&d->halo, L.halo, s))) return rc;
   if ((rc = upload(&d->iperm, L.iperm, s))) return rc;
-  if ((rc = upload(&d->sup_start, L.sup_start, s))) return rc;
-  if ((rc = upload(&d->sup, L.sup, s))) return rc;
   if ((rc = upload(&d->dep_start, L.dep_start, s))) return rc;
   if ((rc = upload(&d->dep, L.dep, s))) return rc;
   if ((rc = upload(&d->owner, L.owner, s))) return rc;
@@ -557,8 +558,8 @@ int upload_layout(Mesh& m) {
   HIP_TRY(hipMalloc((void**)&d->out, sizeof(float) * m.nv));
   d->nseen = m.nv + (int64_t)L.halo.size();
   HIP_TRY(hipMalloc((void**)&d->seen, sizeof(float) * d->nseen));
-  HIP_TRY(hipMalloc((void**)&d->chg, sizeof(int32_t) * L.nblocks));
-  HIP_TRY(hipMalloc((void**)&d->self, sizeof(int32_t) * L.nblocks));
+  HIP_TRY(hipMalloc((void**)&d->stamp[0], sizeof(int32_t) * L.nblocks));
+  HIP_TRY(hipMalloc((void**)&d->stamp[1], sizeof(int32_t) * L.nblocks));
   HIP_TRY(hipMalloc((void**)&d->list[0], sizeof(int32_t) * L.nblocks));
   HIP_TRY(hipMalloc((void**)&d->list[1], sizeof(int32_t) * L.nblocks));
   HIP_TRY(hipMalloc((void**)&d->count, sizeof(int32_t) * 4));
@@ -651,27 +652,42 @@ static int setup_resident(Mesh& m, size_t max_lds) {
   return EIK_OK;
 }
 
-// Outer iterations are enqueued kSyncChunk at a time and the host reads the next iteration's
-// active count once per chunk (the reference copies block flags back and forth and synchronises
-// several times per iteration, meshFIM3dEikonal.cu:431-531).  Iterations enqueued after
-// convergence find no active block and cost one near-empty launch each.
-constexpr int kSyncChunk = 8;
+// Iterations enqueued beyond the one that has begun last.  The device tells the host which that is
+// (SyncArgs::told), so that the stream does not run empty while the host waits to learn whether there is
+// another (the reference copies block flags back and forth and synchronises several times per
+// iteration, meshFIM3dEikonal.cu:431-531; a wait for every eight iterations left the device idle for 35
+// us each).  Iterations enqueued after convergence find no active block and cost one near-empty launch each.
+constexpr int kSyncAhead = 5;
 
-static int solve_sync(Mesh& m, const eik_solve_opts_t& o, eik_solve_stats_t& st) {
+// Waits until an iteration has begun.  (The stream is asked only after a while: the question puts a
+// marker into it, which costs the device 6 us.)
+static int sync_wait(const unsigned long long* told, int64_t it, hipStream_t s) {
+  auto begun = [&] { return (int64_t)(uint32_t)__atomic_load_n(told, __ATOMIC_ACQUIRE) >= it; };
+  for (;;) {
+    const auto t0 = std::chrono::steady_clock::now();
+    do {
+      for (int spin = 0; spin < 256; ++spin)
+        if (begun()) return EIK_OK;
+    } while (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(20));
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    HIP_TRY(e);
+    return begun() ? EIK_OK : fail(EIK_ERR_HIP, "an iteration ended without a sign");
+  }
+}
+
+static int solve_sync(Mesh& m, const eik_solve_opts_t& o) {
   DeviceState* d = m.dev;
   hipStream_t s = d->stream;
   const int32_t nb = d->nblocks;
   const float large = m.dim == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
-  // d->count (cleared with the solve's other arrays): [0], [1] the active counts of even and odd
-  // iterations, [2] the last iteration that visited a block
+  // d->count (cleared with the solve's other arrays): the active counts of iterations modulo 3, the
+  // last iteration that visited a block
   int32_t* cnt = d->count;
-  // activation for iteration 1 from the seed stamps (stamp 0)
-  const int32_t act_wgs = (int32_t)grid1d(nb, 256);
-  hipLaunchKernelGGL(k_activate, dim3(act_wgs), dim3(256), 0, s, nb, d->sup_start, d->sup,
-                     d->chg, d->self, 0, d->list[1], cnt + 1, act_wgs, nullptr, (int64_t)0,
-                     nullptr, nullptr);
-  HIP_TRY(hipGetLastError());
+  unsigned long long* told = d->h_cnt + kNumCounters;
+  __atomic_store_n(told, 0ull, __ATOMIC_RELEASE);
   SyncArgs a;
+  a.snap = nullptr;
   a.v.blocks = d->blocks;
   a.v.elems = d->elems;
   a.v.halo = d->halo;
@@ -695,60 +711,49 @@ static int solve_sync(Mesh& m, const eik_solve_opts_t& o, eik_solve_stats_t& st)
   a.v.lens = nullptr;
   a.v.dep_start = d->dep_start;
   a.rec_lds_bytes = stage ? d->rec_lds_bytes : 0;
-  a.chg = d->chg;
-  a.self = d->self;
   a.acc = d->sync_acc;
   a.elem_bytes = m.dim == 3 ? kAlgoElemBytes<3> : kAlgoElemBytes<2>;
-  a.iters = cnt + 2;
+  a.last = cnt + 3;
+  a.told = told;
+  a.dep = d->dep;
+  a.nb = nb;
   // values only decrease, so the loop ends; the cap bounds it on pathological inputs
   const int64_t cap = o.max_iterations > 0 ? o.max_iterations : 1000000;
-  int32_t* h = reinterpret_cast<int32_t*>(d->h_cnt);  // pinned, free until the counters return
   int64_t it = 0;
   HIP_TRY(hipEventRecord(d->evA, s));
   while (it < cap) {
-    const int64_t n = std::min<int64_t>(kSyncChunk, cap - it);
-    for (int64_t k = 0; k < n; ++k) {
-      ++it;
-      const int p = (int)(it & 1);
-      a.list = d->list[p];
-      a.count = cnt + p;
-      a.count_next = cnt + (p ^ 1);
-      a.it = (int32_t)it;
-      if (m.dim == 3)
-        hipLaunchKernelGGL(k_visit_sync<3>, dim3(nb), dim3(kBlockThreads), lds, s, a);
-      else
-        hipLaunchKernelGGL(k_visit_sync<2>, dim3(nb), dim3(kBlockThreads), lds, s, a);
-      HIP_TRY(hipGetLastError());
-      float* snap = nullptr;
-      unsigned snap_wgs = 0;
-      if (o.record_history) {
-        const size_t slot = (size_t)(it - 1);
-        while (d->hist.size() <= slot / kHistChunk) {
-          float* c = nullptr;
-          HIP_TRY(hipMalloc((void**)&c, sizeof(float) * kHistChunk * (size_t)m.nv));
-          d->hist.push_back(c);
-        }
-        snap = d->hist[slot / kHistChunk] + (slot % kHistChunk) * (size_t)m.nv;
-        snap_wgs = (unsigned)std::min<int64_t>(grid1d(m.nv, 256), 1024);
-      }
-      hipLaunchKernelGGL(k_activate, dim3((unsigned)act_wgs + snap_wgs), dim3(256), 0, s, nb,
-                         d->sup_start, d->sup, d->chg, d->self, (int32_t)it, d->list[p ^ 1],
-                         cnt + (p ^ 1), act_wgs, d->T, m.nv, cnt + p, snap);
-      HIP_TRY(hipGetLastError());
+    if (it >= kSyncAhead) {
+      int rc = sync_wait(told, it + 1 - kSyncAhead, s);
+      if (rc) return rc;
     }
-    HIP_TRY(hipEventRecord(d->evB, s));
-    HIP_TRY(hipMemcpyAsync(h, cnt, sizeof(int32_t) * 3, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (h[(it + 1) & 1] == 0) break;  // the next iteration has no active block
+    const unsigned long long t = __atomic_load_n(told, __ATOMIC_ACQUIRE);
+    if ((t >> 32) < (uint32_t)t) break;  // an iteration without an active block has begun
+    ++it;
+    a.now = {d->stamp[it & 1], d->list[it & 1], cnt + it % 3};
+    a.next = {d->stamp[~it & 1], d->list[~it & 1], cnt + (it + 1) % 3};
+    a.count_after = cnt + (it + 2) % 3;
+    a.it = (int32_t)it;
+    unsigned snap_wgs = 0;
+    if (o.record_history) {
+      const size_t slot = (size_t)(it - 1);
+      while (d->hist.size() <= slot / kHistChunk) {
+        float* c = nullptr;
+        HIP_TRY(hipMalloc((void**)&c, sizeof(float) * kHistChunk * (size_t)m.nv));
+        d->hist.push_back(c);
+      }
+      a.snap = d->hist[slot / kHistChunk] + (slot % kHistChunk) * (size_t)m.nv;
+      snap_wgs = (unsigned)grid1d(nb, kSnapBlocks);
+    }
+    const dim3 grid((unsigned)nb + snap_wgs);
+    if (m.dim == 3)
+      hipLaunchKernelGGL(k_visit_sync<3>, grid, dim3(kBlockThreads), lds, s, a);
+    else
+      hipLaunchKernelGGL(k_visit_sync<2>, grid, dim3(kBlockThreads), lds, s, a);
+    HIP_TRY(hipGetLastError());
   }
+  HIP_TRY(hipEventRecord(d->evB, s));
   hipLaunchKernelGGL(k_sum_slots, dim3(1), dim3(64), 0, s, d->sync_acc, d->counters);
   HIP_TRY(hipGetLastError());
-  float vms = 0.f;
-  HIP_TRY(hipEventElapsedTime(&vms, d->evA, d->evB));
-  st.visit_ms = vms;
-  st.outer_iterations = h[2];
-  st.visit_launches = h[2];
-  if (o.record_history) d->hist_len = h[2];
   return EIK_OK;
 }
 
@@ -983,9 +988,9 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     d->seed_cap = nseeds;
   }
   if (!d->h_cnt) {
-    HIP_TRY(hipHostMalloc((void**)&d->h_cnt, sizeof(unsigned long long) * kNumCounters +
+    HIP_TRY(hipHostMalloc((void**)&d->h_cnt, sizeof(unsigned long long) * (kNumCounters + 1) +
                                                  sizeof(float) * std::min(m->nv, kSmallOut)));
-    d->h_out = reinterpret_cast<float*>(d->h_cnt + kNumCounters);
+    d->h_out = reinterpret_cast<float*>(d->h_cnt + kNumCounters + 1);
   }
   d->hist_len = 0;
   int32_t* h_vals = d->h_seed + d->seed_cap;
@@ -1008,17 +1013,17 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     FillSegs f;
     f.add(d->T, m->nv, (int32_t)__builtin_bit_cast(uint32_t, large));
     f.add(d->seen, d->nseen, (int32_t)__builtin_bit_cast(uint32_t, EIK_INF));
-    f.add(d->chg, d->nblocks, -1);
-    f.add(d->self, d->nblocks, -1);
+    f.add(d->stamp[0], d->nblocks, -1);
+    f.add(d->stamp[1], d->nblocks, -1);
     f.add(d->counters, 2 * kNumCounters, 0);
     f.add(d->count, 4, 0);
     f.add(d->sync_acc, 2 * kSyncSlots * kSyncSlotWords, 0);
     launch_fill(f, s);
-    hipLaunchKernelGGL(k_seed, dim3(grid1d(nseeds, 256)), dim3(256), 0, s, d->seeds,
-                       seed_vals ? d->seedvals : nullptr, nseeds, d->iperm, d->owner, d->T, d->chg,
-                       d->self, m->nv);
+    hipLaunchKernelGGL(k_sync_seed, seed_grid(nseeds), dim3(64), 0, s, d->seeds,
+                       seed_vals ? d->seedvals : nullptr, nseeds, d->iperm, d->owner, d->dep_start,
+                       d->dep, d->T, Active{d->stamp[1], d->list[1], d->count + 1});
     HIP_TRY(hipGetLastError());
-    if ((rc = solve_sync(*m, o, st))) return rc;
+    if ((rc = solve_sync(*m, o))) return rc;
     if (T_out)
       hipLaunchKernelGGL(k_gather, dim3(grid1d(m->nv, 256)), dim3(256), 0, s, d->T, d->iperm, m->nv,
                          d->out);
@@ -1032,13 +1037,12 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     HIP_TRY(hipMemcpyAsync(d->h_out, d->out, sizeof(float) * m->nv, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
   const unsigned long long* cnt = d->h_cnt;
-  if (async) {
-    float vms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&vms, d->evA, d->evB));
-    st.visit_ms = vms;
-    st.visit_launches = 1;
-    st.outer_iterations = 1;
-  }
+  float vms = 0.f;
+  HIP_TRY(hipEventElapsedTime(&vms, d->evA, d->evB));
+  st.visit_ms = vms;
+  st.outer_iterations = async ? 1 : (int64_t)(d->h_cnt[kNumCounters] >> 32);
+  st.visit_launches = st.outer_iterations;
+  if (!async && o.record_history) d->hist_len = (decltype(d->hist_len))st.outer_iterations;
   auto t1 = std::chrono::steady_clock::now();
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, d->ev0, d->ev1));
