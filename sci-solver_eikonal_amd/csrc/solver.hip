@@ -133,6 +133,8 @@ struct SyncArgs {
   float* snap;               // the times after this iteration (the per-iteration history), or null
   unsigned long long* acc;   // kSyncSlots slot lines of counters
   int32_t elem_bytes;        // algorithmic bytes per element (visit_algo_bytes)
+  TriItems items;            // register-resident visits: triangles, and the LDS (LoopArgs)
+  int32_t max_local, max_elem, max_queue;
 };
 constexpr int kSnapBlocks = 16;  // blocks whose times a workgroup copies to the history
 
@@ -179,12 +181,9 @@ __global__ void k_sum_slots(const unsigned long long* acc, unsigned long long* c
 // the workgroups from nb on copy those of the blocks that are not active, which no one changes now:
 // one launch per iteration (48^3 cube with history, 43 iterations, in all: 1.35 -> 1.06 ms; a launch
 // that looked through every block's suppliers took 5 us of each, the host's waits 0.2 ms).
-template <int DIM>
-__global__ __launch_bounds__(kBlockThreads) void k_visit_sync(SyncArgs a) {
-  extern __shared__ uint4 lds4[];
-  __shared__ int sFlag[4];
-  __shared__ int sQn[2];  // work-item counters of alternate chunks
-  __shared__ unsigned long long sRed;
+//
+// The block this workgroup visits, or -1 (the history copy done).
+__device__ __forceinline__ int sync_begin(const SyncArgs& a) {
   const int n = *a.now.count;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     *a.count_after = 0;
@@ -193,18 +192,41 @@ __global__ __launch_bounds__(kBlockThreads) void k_visit_sync(SyncArgs a) {
     __hip_atomic_store(a.told, (unsigned long long)last << 32 | (unsigned)a.it, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
   }
-  if ((int)blockIdx.x >= a.nb) {
-    if (n <= 0) return;
-    const int c0 = ((int)blockIdx.x - a.nb) * kSnapBlocks;
-    for (int c = c0 + (int)(threadIdx.x >> 6); c < min(c0 + kSnapBlocks, a.nb); c += kBlockThreads / 64) {
-      if (a.now.stamp[c] == a.it) continue;
-      const BlockDesc d = a.v.blocks[c];
-      for (int i = (int)__lane_id(); i < d.nown; i += 64) a.snap[d.vstart + i] = a.v.T[d.vstart + i];
-    }
-    return;
+  if ((int)blockIdx.x < a.nb) return (int)blockIdx.x < n ? a.now.list[blockIdx.x] : -1;
+  if (n <= 0) return -1;
+  const int c0 = ((int)blockIdx.x - a.nb) * kSnapBlocks;
+  for (int c = c0 + (int)(threadIdx.x >> 6); c < min(c0 + kSnapBlocks, a.nb); c += (int)(blockDim.x >> 6)) {
+    if (a.now.stamp[c] == a.it) continue;
+    const BlockDesc d = a.v.blocks[c];
+    for (int i = (int)__lane_id(); i < d.nown; i += 64) a.snap[d.vstart + i] = a.v.T[d.vstart + i];
   }
-  if ((int)blockIdx.x >= n) return;
-  const int b = a.now.list[blockIdx.x];
+  return -1;
+}
+
+// After a visit: the next iteration's blocks (first wave), the history.
+__device__ __forceinline__ void sync_end(const SyncArgs& a, int b, const BlockDesc& d, bool bnd_changed,
+                                         bool converged, const float* sT) {
+  if (threadIdx.x < 64) {
+    const int32_t s0 = a.v.dep_start[b];
+    const int nd = bnd_changed ? a.v.dep_start[b + 1] - s0 : 0;
+    const int m = nd + (converged ? 0 : 1);
+    for (int j0 = 0; j0 < m; j0 += 64) {
+      const int j = j0 + (int)threadIdx.x;
+      activate(a.next, a.it + 1, j < m, j < nd ? a.dep[s0 + j] : b);
+    }
+  }
+  if (a.snap)
+    for (int i = (int)threadIdx.x; i < d.nown; i += (int)blockDim.x) a.snap[d.vstart + i] = sT[i];
+}
+
+template <int DIM>
+__global__ __launch_bounds__(kBlockThreads) void k_visit_sync(SyncArgs a) {
+  extern __shared__ uint4 lds4[];
+  __shared__ int sFlag[4];
+  __shared__ int sQn[2];  // work-item counters of alternate chunks
+  __shared__ unsigned long long sRed;
+  const int b = sync_begin(a);
+  if (b < 0) return;
   const BlockDesc d = a.v.blocks[b];
   VisitLds l = carve_lds<DIM>(lds4, a.rec_lds_bytes, a.v.queue_cap, d);
   if (threadIdx.x == 0) sRed = 0;
@@ -212,18 +234,107 @@ __global__ __launch_bounds__(kBlockThreads) void k_visit_sync(SyncArgs a) {
   const unsigned long long t0 = wall_clock64();
   VisitResult r = visit_block<DIM, false>(a.v, b, l.rec, l.T, l.old, l.chg, l.hidx, l.vm, l.q, l.mark,
                                           sFlag, sQn, &solves);
-  if (threadIdx.x < 64) {
-    const int32_t s0 = a.v.dep_start[b];
-    const int nd = r.bnd_changed ? a.v.dep_start[b + 1] - s0 : 0;
-    const int m = nd + (r.converged ? 0 : 1);
-    for (int j0 = 0; j0 < m; j0 += 64) {
-      const int j = j0 + (int)threadIdx.x;
-      activate(a.next, a.it + 1, j < m, j < nd ? a.dep[s0 + j] : b);
+  sync_end(a, b, d, r.bnd_changed, r.converged, l.T);
+  block_counters(a.acc, d, r.sweeps, solves, a.elem_bytes, wall_clock64() - t0, r, &sRed);
+}
+
+// The same visit with the block's element data in registers (resident.h), where the blocks fit: its
+// sweeps are the ones of the persistent kernel (visit_loop.h).  Kernel ms against k_visit_sync: 48^3
+// cube with history 0.91 -> 0.82, 64^3 1.60 -> 1.51, 96^3 with 16 sources 3.87 -> 3.65, level-7
+// anisotropic icosphere 1.42 -> 1.22, level 5 0.45 -> 0.30, 32^2 square 0.21 -> 0.14.
+template <int DIM, int N, int BT, bool CAP = false>
+__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_visit_sync_resident(SyncArgs a) {
+  extern __shared__ uint4 lds4[];
+  __shared__ int sFlag[3], sQn[2], sBnd, sFull;
+  __shared__ unsigned long long sRed;
+  const int b = sync_begin(a);
+  if (b < 0) return;
+  const BlockDesc d = a.v.blocks[b];
+  const int tid = threadIdx.x;
+  const int ls = lds_stride(a.max_local);
+  float* sT = reinterpret_cast<float*>(lds4);
+  float* sP = sT + ls;
+  uint4* sA = reinterpret_cast<uint4*>(sP + 2 * ls);
+  uint4* sB = sA + (DIM == 3 ? a.max_elem : 0);
+  uint16_t* sQ = reinterpret_cast<uint16_t*>(sB + (DIM == 3 ? a.max_elem : 0));
+  const float eps = a.v.eps, keep = 1.f / (1.f + eps), large = a.v.large;
+  float* T = a.v.T;
+  float* seen = a.v.seen + d.vstart + d.hstart;
+  if (tid < 3) sFlag[tid] = 0;
+  if (tid < 2) sQn[tid] = 0;
+  if (tid == 0) {
+    sRed = 0;
+    sBnd = sFull = 0;
+  }
+  const unsigned long long t0 = wall_clock64();
+  float own = 0.f;
+  if (tid < d.nown) {
+    own = T[d.vstart + tid];
+    sP[tid] = seen[tid];
+    sT[tid] = own;
+  }
+  for (int i = tid; i < d.nhalo; i += BT) {
+    sP[d.nown + i] = seen[d.nown + i];
+    sT[d.nown + i] = T[a.v.halo[d.hstart + i]];
+  }
+  std::conditional_t<DIM == 2, TriRegs<N>, TetRegs<N>> r;
+  if constexpr (DIM == 2) tri_load<N, BT>(r, a.items, a.items.range[b], nullptr);
+  else tet_load<N, BT>(r, a.v.elems, d, sA, sB, nullptr);
+  wait_memory();  // the copies to LDS too
+  __syncthreads();
+  if constexpr (DIM == 2) tri_seen<N>(r, sP, keep);
+  else tet_seen<N>(r, sP, keep);
+  const unsigned long long t1 = wall_clock64();
+  uint32_t solves = 0;
+  float last = own;  // the owned time before the last sweep
+  bool conv = false;
+  int sweep = 0;
+  while (sweep < a.v.max_inner && !conv) {
+    const int f = sweep % 3;
+    bool ch = false;
+    int nq = 1;
+    if constexpr (DIM == 2) {
+      ch = tri_sweep<N>(r, sT, large, eps, keep, solves);
+    } else {
+      tet_select<N, BT, CAP>(r, d.nelem, sT, keep, sQ, a.max_queue, &sQn[sweep & 1], &sFlag[f], &sFull,
+                             sweep + 1);
+      __syncthreads();
+      nq = sQn[sweep & 1];
+      if (CAP) nq = min(nq, a.max_queue);
+      if (tid == 0) sQn[(sweep & 1) ^ 1] = 0;
+      if (nq) ch = tet_solve<N, BT>(r, sA, sB, sQ, nq, sT, large, eps, solves);
+    }
+    if (ch) sFlag[f] = 1;
+    wait_memory();
+    __syncthreads();
+    conv = !sFlag[f];
+    if (tid == 0) sFlag[(f + 2) % 3] = 0;
+    ++sweep;
+    if (!conv && sweep < a.v.max_inner) {
+      if (tid < d.nown) last = sT[tid];
+      if constexpr (DIM == 2) __syncthreads();  // (read before the next sweep lowers it)
     }
   }
-  if (a.snap)
-    for (int i = (int)threadIdx.x; i < d.nown; i += kBlockThreads) a.snap[d.vstart + i] = l.T[i];
-  block_counters(a.acc, d, r.sweeps, solves, a.elem_bytes, wall_clock64() - t0, r, &sRed);
+  const unsigned long long t2 = wall_clock64();
+  // What this visit evaluated the block's elements with: every time, but for the owned vertices that
+  // fell in the last sweep of a visit cut off by the sweep cap; after a full queue, nothing.
+  const bool full = DIM == 3 && CAP && !conv && sFull == sweep;
+  if (tid < d.nown) {
+    const float v = sT[tid];
+    seen[tid] = full ? EIK_INF : conv ? v : last;
+    if (v < own) {
+      T[d.vstart + tid] = v;
+      if (tid >= d.nbnd0) sBnd = 1;
+    }
+  }
+  for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = full ? EIK_INF : sT[d.nown + i];
+  __syncthreads();
+  sync_end(a, b, d, sBnd != 0, conv, sT);
+  VisitResult vr;
+  vr.t_load = t1 - t0;
+  vr.t_sweep = t2 - t1;
+  vr.t_wb = wall_clock64() - t2;
+  block_counters(a.acc, d, sweep, solves, a.elem_bytes, wall_clock64() - t0, vr, &sRed);
 }
 
 static dim3 seed_grid(int64_t nseeds) {
@@ -572,19 +683,28 @@ int upload_layout(Mesh& m) {
   return EIK_OK;
 }
 
-static const void* resident_kernel(int dim, int n, int bt, bool cap) {
-  if (dim == 3)
-    return n == 2                        ? (const void*)k_visit_resident<3, 2, 512>
-           : n == 4 && bt == 256         ? (const void*)k_visit_resident<3, 4, 256>
-           : bt == 256                   ? (const void*)k_visit_resident<3, kTetN<256>, 256>
-           : bt == 512 && cap            ? (const void*)k_visit_resident<3, kTetN<512>, 512, true>
-           : bt == 512                   ? (const void*)k_visit_resident<3, kTetN<512>, 512>
-                                         : (const void*)k_visit_resident<3, kTetN<1024>, 1024>;
-  return bt == 256    ? (const void*)k_visit_resident<2, 1, 256>
-         : bt == 1024 ? (const void*)k_visit_resident<2, 4, 1024>
-         : n == 1     ? (const void*)k_visit_resident<2, 1, 512>
-         : n == 2     ? (const void*)k_visit_resident<2, 2, 512>
-                      : (const void*)k_visit_resident<2, 4, 512>;
+struct ResidentKernels {
+  const void* loop;  // k_visit_resident
+  const void* sync;  // k_visit_sync_resident
+};
+template <int DIM, int N, int BT, bool CAP = false>
+static ResidentKernels resident_pair() {
+  return {(const void*)k_visit_resident<DIM, N, BT, CAP>, (const void*)k_visit_sync_resident<DIM, N, BT, CAP>};
+}
+static ResidentKernels resident_kernels(const DeviceState* d) {
+  const int n = d->res_n, bt = d->res_bt;
+  if (d->dim == 3)
+    return n == 2                   ? resident_pair<3, 2, 512>()
+           : n == 4 && bt == 256    ? resident_pair<3, 4, 256>()
+           : bt == 256              ? resident_pair<3, kTetN<256>, 256>()
+           : bt == 512 && d->res_cap ? resident_pair<3, kTetN<512>, 512, true>()
+           : bt == 512              ? resident_pair<3, kTetN<512>, 512>()
+                                    : resident_pair<3, kTetN<1024>, 1024>();
+  return bt == 256    ? resident_pair<2, 1, 256>()
+         : bt == 1024 ? resident_pair<2, 4, 1024>()
+         : n == 1     ? resident_pair<2, 1, 512>()
+         : n == 2     ? resident_pair<2, 2, 512>()
+                      : resident_pair<2, 4, 512>();
 }
 
 // The shape of the register-resident visits for this layout, and the triangle items.  A block
@@ -626,8 +746,8 @@ static int setup_resident(Mesh& m, size_t max_lds) {
     return EIK_OK;
   }
   if (d->res_lds > 65536)
-    HIP_TRY(hipFuncSetAttribute(resident_kernel(m.dim, d->res_n, d->res_bt, d->res_cap),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)d->res_lds));
+    for (const void* k : {resident_kernels(d).loop, resident_kernels(d).sync})
+      HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)d->res_lds));
   if (m.dim == 3) return EIK_OK;
   std::vector<int2> range(L.nblocks);
   int64_t n = 0;
@@ -716,10 +836,16 @@ static int solve_sync(Mesh& m, const eik_solve_opts_t& o) {
   a.last = cnt + 3;
   a.told = told;
   a.dep = d->dep;
+  a.items = {d->item_range, d->item_id, d->item_len, d->item_rec};
+  a.max_local = d->max_local;
+  a.max_elem = d->max_elem;
+  a.max_queue = d->max_queue;
   a.nb = nb;
   // values only decrease, so the loop ends; the cap bounds it on pathological inputs
   const int64_t cap = o.max_iterations > 0 ? o.max_iterations : 1000000;
   int64_t it = 0;
+  const bool resident = d->res_n != 0 && o.stage_records == EIK_STAGE_AUTO;
+  void* args[] = {(void*)&a};
   HIP_TRY(hipEventRecord(d->evA, s));
   while (it < cap) {
     if (it >= kSyncAhead) {
@@ -745,7 +871,9 @@ static int solve_sync(Mesh& m, const eik_solve_opts_t& o) {
       snap_wgs = (unsigned)grid1d(nb, kSnapBlocks);
     }
     const dim3 grid((unsigned)nb + snap_wgs);
-    if (m.dim == 3)
+    if (resident)
+      HIP_TRY(hipLaunchKernel(resident_kernels(d).sync, grid, dim3(d->res_bt), args, d->res_lds, s));
+    else if (m.dim == 3)
       hipLaunchKernelGGL(k_visit_sync<3>, grid, dim3(kBlockThreads), lds, s, a);
     else
       hipLaunchKernelGGL(k_visit_sync<2>, grid, dim3(kBlockThreads), lds, s, a);
@@ -773,7 +901,7 @@ static VisitKernel visit_kernel(const DeviceState* d, int32_t stage_records) {
   if (d->res_n && stage_records != EIK_STAGE_MEMORY) {
     k.threads = d->res_bt;
     k.lds = d->res_lds;
-    k.fn = resident_kernel(d->dim, d->res_n, d->res_bt, d->res_cap);
+    k.fn = resident_kernels(d).loop;
     return k;
   }
   k.threads = kBlockThreads;
