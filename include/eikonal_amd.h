@@ -208,7 +208,8 @@ typedef struct {
 void eik_solve_opts_default(eik_solve_opts_t* opts);
 
 typedef struct {
-  double kernel_ms;        /* device time of the solve (HIP events on the handle's stream) */
+  double kernel_ms;        /* device time of the solve, from its first kernel's start (async: by the
+                              device's clock; sync, batch: HIP events on the handle's stream) */
   double wall_ms;          /* host time of the solve call (excludes mesh upload) */
   int64_t outer_iterations;/* sync: outer iterations; async: 1 */
   int64_t block_visits;    /* block visits (the reference's "total iteration number",
@@ -220,8 +221,7 @@ typedef struct {
                               tet (20 per triangle) + 4 B per owned and halo time read + 4 B per
                               owned time written + 4 */
   int64_t history_len;     /* iterations stored (record_history) */
-  double visit_ms;         /* device time of the block-visit kernel launches (HIP events on the
-                              handle's stream around each launch) */
+  double visit_ms;         /* device time of the block-visit kernel launches (measured likewise) */
   int64_t visit_launches;  /* block-visit kernel launches */
   double busy_ms;          /* time inside block visits, summed over workgroups */
   double wait_ms;          /* async: time workgroups waited for work, summed */

@@ -127,6 +127,7 @@ struct FillSegs {
   int count = 0;
   unsigned long long* words[2] = {nullptr, nullptr};  // block words (block_sched.h)
   int64_t nwords[2] = {0, 0};
+  unsigned long long* begin = nullptr;  // gets the device clock
   void add(void* ptr, int64_t words32, int32_t value) {
     p[count] = reinterpret_cast<int32_t*>(ptr);
     n[count] = words32;

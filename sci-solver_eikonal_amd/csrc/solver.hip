@@ -18,6 +18,8 @@ namespace eik {
 // Results of up to this many vertices are copied out through pinned memory in the solve's one wait;
 // larger ones straight to the caller's memory after it.
 constexpr int64_t kSmallOut = 65536;
+// Up to this many seeds are read from pinned host memory by the kernel that needs them, without a copy.
+constexpr int64_t kDirectSeeds = 1024;
 
 static int dev_free(DeviceState* d) {
   if (!d) return EIK_OK;
@@ -66,6 +68,7 @@ int ensure_stream(Mesh& m) {
 // Kernels
 // ------------------------------------------------------------------------------------------
 __global__ void k_fill_segs(FillSegs f) {
+  if (f.begin && blockIdx.x == 0 && threadIdx.x == 0) *f.begin = wall_clock64();
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   for (int k = 0; k < f.count; ++k) {
@@ -349,6 +352,7 @@ struct SolveArgs {
   const int32_t* dep;
   const int32_t* iperm;
   float* out;          // the times in caller order, written when the solve has ended (or null)
+  unsigned long long* told;  // pinned host memory: the last one copies the counters here (or null)
   int64_t nv;
   unsigned long long* counters;
   int64_t max_visits;  // runaway guard: visits of one workgroup after which it marks nothing
@@ -368,6 +372,28 @@ __device__ __forceinline__ void write_out(const SolveArgs& a, int block) {
     a.out[i] = load_T<true>(a.v.T + a.iperm[i]);
 }
 
+// The end of a workgroup: its tally, and, if it is the last one, the sums to the host, with the ticks at
+// which the solve and its visits began and this one.
+__device__ __forceinline__ void finish(const SolveArgs& a, const unsigned long long* acc) {
+  if (threadIdx.x < kNumCounters && acc[threadIdx.x])
+    atomicAdd(&a.counters[threadIdx.x], acc[threadIdx.x]);
+  if (!a.told || threadIdx.x >= 64) return;
+  wait_memory();
+  unsigned before = 0;
+  // (workgroups that have finished: a control word of its own line)
+  if (threadIdx.x == 0) before = atomicAdd(reinterpret_cast<unsigned*>(a.s.ctl) + kSchedCtlBytes / 16, 1u);
+  if (__builtin_amdgcn_readfirstlane(before) + 1u != gridDim.x) return;
+  if (threadIdx.x <= kNumCounters)
+    __hip_atomic_store(&a.told[threadIdx.x], load_word(&a.counters[threadIdx.x]), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  if (threadIdx.x == 0) a.told[kNumCounters + 2] = wall_clock64();
+}
+
+// The start of the visit launch (the fill before it left its own behind the counters).
+__device__ __forceinline__ void begin(const SolveArgs& a) {
+  if (a.told && blockIdx.x == 0 && threadIdx.x == 0) a.told[kNumCounters + 1] = wall_clock64();
+}
+
 struct SingleBlocks {
   const SolveArgs& a;
   __device__ __forceinline__ BlockData operator()(int32_t b) const {
@@ -381,11 +407,11 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   extern __shared__ uint4 lds4[];
   __shared__ LoopShared sh;
   if (threadIdx.x < kNumCounters) sh.acc[threadIdx.x] = 0;
+  begin(a);
   const LoopArgs la = {a.s, a.v.eps, a.v.max_inner, a.max_visits, a.max_local, a.max_elem, a.max_queue};
   const int end = resident_loop<DIM, N, BT, CAP>(la, SingleBlocks{a}, blockIdx.x, lds4, sh);
   write_out(a, end);
-  if (threadIdx.x < kNumCounters && sh.acc[threadIdx.x])
-    atomicAdd(&a.counters[threadIdx.x], sh.acc[threadIdx.x]);
+  finish(a, sh.acc);
 }
 
 // Seeds of a solve of the scheduler above: the sources' times, and the owner block of each source
@@ -418,6 +444,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
   __shared__ unsigned long long sRed;
   __shared__ unsigned long long sAcc[kNumCounters];
   const int tid = threadIdx.x;
+  begin(a);
   if (tid < kNumCounters) sAcc[tid] = 0;
   Finder f;
   if (tid < 64) sched_enter(a.s, f, blockIdx.x);
@@ -499,7 +526,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
     }
   }
   write_out(a, sBlock);
-  if (tid < kNumCounters && sAcc[tid]) atomicAdd(&a.counters[tid], sAcc[tid]);
+  finish(a, sAcc);
 }
 
 // The items of every triangle block (TriItems) from its records: one workgroup per block, items in
@@ -674,7 +701,7 @@ int upload_layout(Mesh& m) {
   HIP_TRY(hipMalloc((void**)&d->list[0], sizeof(int32_t) * L.nblocks));
   HIP_TRY(hipMalloc((void**)&d->list[1], sizeof(int32_t) * L.nblocks));
   HIP_TRY(hipMalloc((void**)&d->count, sizeof(int32_t) * 4));
-  HIP_TRY(hipMalloc((void**)&d->counters, sizeof(unsigned long long) * kNumCounters));
+  HIP_TRY(hipMalloc((void**)&d->counters, sizeof(unsigned long long) * (kNumCounters + 1)));
   HIP_TRY(hipMalloc((void**)&d->sync_acc, sizeof(unsigned long long) * kSyncSlots * kSyncSlotWords));
   HIP_TRY(hipStreamSynchronize(s));
   rc = setup_resident(m, (size_t)max_lds);
@@ -976,7 +1003,7 @@ struct AsyncBufs {
 // rather than memsets, so that a caller may capture this into a graph.
 static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBufs& b,
                          const int32_t* seeds, const float* seedvals, int64_t nseeds, float* out,
-                         hipStream_t s, hipEvent_t before, hipEvent_t after) {
+                         unsigned long long* told, hipStream_t s) {
   const DeviceState* d = m.dev;
   const VisitKernel k = visit_kernel(d, o.stage_records);
   int grid = 0;
@@ -1011,6 +1038,7 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   a.out = out;
   a.nv = m.nv;
   a.counters = b.counters;
+  a.told = told;
   // runaway guard: a workgroup that has made this many visits marks no more blocks (its visits
   // still finish), so a solve ends even if it never converged; the bound is max_iterations
   // outer iterations' worth of visits of every block (1000 without a cap), far above what a
@@ -1025,6 +1053,7 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   f.add(b.T, m.nv, (int32_t)__builtin_bit_cast(uint32_t, a.v.large));
   f.add(b.seen, d->nseen, (int32_t)__builtin_bit_cast(uint32_t, EIK_INF));
   f.add(b.counters, 2 * kNumCounters, 0);
+  if (told) f.begin = b.counters + kNumCounters;
   f.words[0] = b.words;
   f.nwords[0] = (int64_t)a.s.owners * a.s.stride;
   f.add(b.sctl, kSchedCtlBytes / 4, 0);
@@ -1032,10 +1061,8 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   hipLaunchKernelGGL(k_sched_seed, seed_grid(nseeds), dim3(64), 0, s, a.s, seeds, seedvals, nseeds,
                      d->iperm, d->owner, d->dep_start, d->dep, b.T, m.nv);
   HIP_TRY(hipGetLastError());
-  if (before) HIP_TRY(hipEventRecord(before, s));
   void* args[] = {(void*)&a};
   HIP_TRY(hipLaunchKernel(k.fn, dim3(grid), dim3(k.threads), args, k.lds, s));
-  if (after) HIP_TRY(hipEventRecord(after, s));
   return EIK_OK;
 }
 
@@ -1116,26 +1143,36 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     d->seed_cap = nseeds;
   }
   if (!d->h_cnt) {
-    HIP_TRY(hipHostMalloc((void**)&d->h_cnt, sizeof(unsigned long long) * (kNumCounters + 1) +
+    HIP_TRY(hipHostMalloc((void**)&d->h_cnt, sizeof(unsigned long long) * (kNumCounters + 3) +
                                                  sizeof(float) * std::min(m->nv, kSmallOut)));
-    d->h_out = reinterpret_cast<float*>(d->h_cnt + kNumCounters + 1);
+    d->h_out = reinterpret_cast<float*>(d->h_cnt + kNumCounters + 3);
   }
   d->hist_len = 0;
   int32_t* h_vals = d->h_seed + d->seed_cap;
   std::memcpy(d->h_seed, seeds, sizeof(int32_t) * nseeds);
   if (seed_vals) std::memcpy(h_vals, seed_vals, sizeof(float) * nseeds);
-  HIP_TRY(hipEventRecord(d->ev0, s));
-  HIP_TRY(hipMemcpyAsync(d->seeds, d->h_seed, sizeof(int32_t) * nseeds, hipMemcpyHostToDevice, s));
-  if (seed_vals)
-    HIP_TRY(hipMemcpyAsync(d->seedvals, h_vals, sizeof(float) * nseeds, hipMemcpyHostToDevice, s));
+  const bool async = o.scheduler == EIK_SCHED_ASYNC;
+  // (the persistent kernel tells its times itself: an event is a packet of its own, 2 us)
+  if (!async) HIP_TRY(hipEventRecord(d->ev0, s));
+  // a few seeds are read where they are, in pinned memory
+  const bool direct_seeds = nseeds <= kDirectSeeds;
+  if (!direct_seeds) {
+    HIP_TRY(hipMemcpyAsync(d->seeds, d->h_seed, sizeof(int32_t) * nseeds, hipMemcpyHostToDevice, s));
+    if (seed_vals)
+      HIP_TRY(hipMemcpyAsync(d->seedvals, h_vals, sizeof(float) * nseeds, hipMemcpyHostToDevice, s));
+  }
+  const int32_t* dev_seeds = direct_seeds ? d->h_seed : d->seeds;
+  const float* dev_vals = !seed_vals ? nullptr
+                          : direct_seeds ? reinterpret_cast<const float*>(h_vals) : d->seedvals;
+  // a small result comes back in the solve's one wait, through pinned memory
+  const bool small = T_out && m->nv <= kSmallOut;
   eik_solve_stats_t st;
   std::memset(&st, 0, sizeof(st));
-  const bool async = o.scheduler == EIK_SCHED_ASYNC;
   if (async) {
     if ((rc = ensure_words(d))) return rc;
     const AsyncBufs bufs = {d->T, d->seen, d->words, d->sctl, d->counters};
-    rc = enqueue_async(*m, o, bufs, d->seeds, seed_vals ? d->seedvals : nullptr, nseeds,
-                       T_out ? d->out : nullptr, s, d->evA, d->evB);
+    rc = enqueue_async(*m, o, bufs, dev_seeds, dev_vals, nseeds,
+                       small ? d->h_out : T_out ? d->out : nullptr, d->h_cnt, s);
     if (rc) return rc;
   } else {
     FillSegs f;
@@ -1147,8 +1184,7 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     f.add(d->count, 4, 0);
     f.add(d->sync_acc, 2 * kSyncSlots * kSyncSlotWords, 0);
     launch_fill(f, s);
-    hipLaunchKernelGGL(k_sync_seed, seed_grid(nseeds), dim3(64), 0, s, d->seeds,
-                       seed_vals ? d->seedvals : nullptr, nseeds, d->iperm, d->owner, d->dep_start,
+    hipLaunchKernelGGL(k_sync_seed, seed_grid(nseeds), dim3(64), 0, s, dev_seeds, dev_vals, nseeds, d->iperm, d->owner, d->dep_start,
                        d->dep, d->T, Active{d->stamp[1], d->list[1], d->count + 1});
     HIP_TRY(hipGetLastError());
     if ((rc = solve_sync(*m, o))) return rc;
@@ -1156,25 +1192,26 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
       hipLaunchKernelGGL(k_gather, dim3(grid1d(m->nv, 256)), dim3(256), 0, s, d->T, d->iperm, m->nv,
                          d->out);
   }
-  HIP_TRY(hipEventRecord(d->ev1, s));
-  HIP_TRY(hipMemcpyAsync(d->h_cnt, d->counters, sizeof(unsigned long long) * kNumCounters,
-                         hipMemcpyDeviceToHost, s));
-  // a small result comes back in the same wait, through pinned memory
-  const bool small = T_out && m->nv <= kSmallOut;
-  if (small)
-    HIP_TRY(hipMemcpyAsync(d->h_out, d->out, sizeof(float) * m->nv, hipMemcpyDeviceToHost, s));
+  if (!async) {
+    HIP_TRY(hipEventRecord(d->ev1, s));
+    HIP_TRY(hipMemcpyAsync(d->h_cnt, d->counters, sizeof(unsigned long long) * kNumCounters,
+                           hipMemcpyDeviceToHost, s));
+    if (small)
+      HIP_TRY(hipMemcpyAsync(d->h_out, d->out, sizeof(float) * m->nv, hipMemcpyDeviceToHost, s));
+  }
   HIP_TRY(hipStreamSynchronize(s));
   const unsigned long long* cnt = d->h_cnt;
-  float vms = 0.f;
-  HIP_TRY(hipEventElapsedTime(&vms, d->evA, d->evB));
-  st.visit_ms = vms;
+  if (!async) {
+    float ms = 0.f, vms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&ms, d->ev0, d->ev1));
+    HIP_TRY(hipEventElapsedTime(&vms, d->evA, d->evB));
+    st.kernel_ms = ms;
+    st.visit_ms = vms;
+  }
   st.outer_iterations = async ? 1 : (int64_t)(d->h_cnt[kNumCounters] >> 32);
   st.visit_launches = st.outer_iterations;
   if (!async && o.record_history) d->hist_len = (decltype(d->hist_len))st.outer_iterations;
   auto t1 = std::chrono::steady_clock::now();
-  float ms = 0.f;
-  HIP_TRY(hipEventElapsedTime(&ms, d->ev0, d->ev1));
-  st.kernel_ms = ms;
   st.wall_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
   st.block_visits = (int64_t)cnt[0];
   st.vertex_updates = (int64_t)cnt[1];
@@ -1186,6 +1223,10 @@ int eik_solve(eik_mesh_t h, const int32_t* seeds, int64_t nseeds, const float* s
     int khz = 0;
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, d->device) == hipSuccess &&
         khz > 0) {
+      if (async) {
+        st.kernel_ms = (double)(cnt[kNumCounters + 2] - cnt[kNumCounters]) / khz;
+        st.visit_ms = (double)(cnt[kNumCounters + 2] - cnt[kNumCounters + 1]) / khz;
+      }
       st.busy_ms = (double)cnt[5] / khz;
       st.wait_ms = (double)cnt[6] / khz;
       st.load_ms = (double)cnt[7] / khz;
@@ -1336,7 +1377,7 @@ int eik_solve_noalloc(eik_mesh_t h, const int32_t* seeds_dev, int64_t nseeds, fl
   eik_solve_opts_t o;
   eik_solve_opts_default(&o);
   return enqueue_async(*m, o, b, seeds_dev, nullptr, nseeds, T_out_dev,
-                       stream ? reinterpret_cast<hipStream_t>(stream) : d->stream, nullptr, nullptr);
+                       nullptr, stream ? reinterpret_cast<hipStream_t>(stream) : d->stream);
 }
 
 }  // extern "C"
