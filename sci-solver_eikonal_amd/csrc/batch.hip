@@ -192,6 +192,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
 }
 
 struct MultiBlocks {
+  static constexpr bool kSingle = false;
   const SolveDesc* solves;
   const int32_t* bsolve;
   __device__ __forceinline__ BlockData operator()(int32_t g) const {

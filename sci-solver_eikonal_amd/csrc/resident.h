@@ -273,6 +273,19 @@ __device__ __forceinline__ int lds_take(int* counter, int n) {
   return old;
 }
 
+// LDS atomics without a result, of one lane, as they are (see lds_take).  The caller waits for them
+// (wait_memory) before its barrier.
+__device__ __forceinline__ void lds_min(unsigned* p, unsigned v) {
+  asm volatile("ds_min_u32 %0, %1"
+               :: "v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned*)p), "v"(v)
+               : "memory");
+}
+__device__ __forceinline__ void lds_or(unsigned* p, unsigned v) {
+  asm volatile("ds_or_b32 %0, %1"
+               :: "v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned*)p), "v"(v)
+               : "memory");
+}
+
 // Appends the (element, corner) pairs of the thread's elements that can improve to the queue.  CAP:
 // it may hold fewer than a block has, max_queue; sets *again, and *full to the visit's number, if it did not hold them.
 // About 190 vector instructions a wave for N = 4 (350 with slots, last times, quieted minima and

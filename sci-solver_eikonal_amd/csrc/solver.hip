@@ -395,6 +395,7 @@ __device__ __forceinline__ void begin(const SolveArgs& a) {
 }
 
 struct SingleBlocks {
+  static constexpr bool kSingle = true;
   const SolveArgs& a;
   __device__ __forceinline__ BlockData operator()(int32_t b) const {
     return {a.v.blocks, a.v.elems, a.v.halo, a.v.T,   a.v.seen, a.v.vmask,

@@ -44,6 +44,7 @@ struct LoopArgs {
 // The workgroup's static LDS.
 struct LoopShared {
   unsigned long long acc[kNumCounters];  // its tally
+  int64_t max_visits;  // LoopArgs (read here with what it is compared with)
   int flag[3];       // a sweep's "a time fell", in a ring over the sweeps
   int full;          // the last visit with a sweep that selected more pairs than the queue holds
   int qn[2];         // work-item counters of alternate sweeps (tets)
@@ -131,7 +132,10 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
   if (tid < 3) sh.flag[tid] = 0;
   if (tid < 2) sh.qn[tid] = 0;
   if (tid < 2) sh.mark[tid] = 0;
-  if (tid == 0) sh.key = kClean;
+  if (tid == 0) {
+    sh.key = kClean;
+    sh.max_visits = a.max_visits;
+  }
   if (tid == 0) sh.full = 0;
   // the second wave looks for work, while the first hands on what the last visit did
   const bool finder = tid >= 64 && tid < 128;
@@ -243,21 +247,29 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       }
       const unsigned long long t2 = wall_clock64();
       // visits beyond the bound mark nothing more (runaway guard)
-      const bool cap_ok = (int64_t)sh.acc[0] < a.max_visits;
+      const bool cap_ok = (int64_t)sh.acc[0] < sh.max_visits;
       const bool more = !conv && cap_ok;
       // marks made from here on are seen by the halo loads of the next visit or after it
       if (more && tid == 0) sched_again(a.s, slot);
-      // reduced over the wave first: the compiler turns an LDS or with a uniform address into a
-      // scalar loop over the lanes (a third of a triangle sweep)
+      // reduced over the wave first, and by one lane: the compiler turns an LDS atomic with a uniform
+      // address into a scalar loop over the lanes (a third of a triangle sweep)
       if (__ballot(key != kClean)) {
         const uint32_t lo = wave_or((uint32_t)marks), hi = wave_or((uint32_t)(marks >> 32));
         key = wave_umin(key);
         if (__lane_id() == 63) {
-          atomicMin(&sh.key, key);
-          if (lo) atomicOr(&sh.mark[0], lo);
-          if (hi) atomicOr(&sh.mark[1], hi);
+          lds_min(&sh.key, key);
+          lds_or(&sh.mark[0], lo);
+          lds_or(&sh.mark[1], hi);
         }
       }
+      // What the owner's other blocks wait with, for the next visit's decision.  In single solves of
+      // triangles, most of whose visits are followed by another, it is loaded in the same wait as the
+      // publishing: 301^2 square with 16 sources 0.334 -> 0.322 ms, level-8 icosphere 1.56 -> 1.51 (in
+      // launches of several solves, with more visits that converge, 1.88 -> 1.93).
+      constexpr bool kEarlyLook = DIM == 2 && Blocks::kSingle;
+      unsigned long long word = ~0ull;
+      if (kEarlyLook && tid < 64 && (uint32_t)tid < a.s.per_owner && a.s.per_owner > 1)
+        word = load_word(&a.s.word[me * a.s.stride + tid]);
       // the published times have reached the device's coherence point before the dependents are
       // marked
       wait_memory();
@@ -282,7 +294,10 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
           tally_visit(sh.acc, d, vr, 0, kAlgoElemBytes<DIM>, tq - t0, rerun, rerun);
         }
         if (again) {
-          const uint32_t w = sched_waiting(a.s, me);
+          // (with one block per owner there is no other, and no wait for its word: 33^3 cube 0.281 ->
+          // 0.267 ms, level-5 icosphere 0.130 -> 0.118)
+          const uint32_t w = kEarlyLook ? wave_umin((word >> 32) == 0ull ? (uint32_t)word : kClean)
+                             : a.s.per_owner > 1 ? sched_waiting(a.s, me) : kClean;
           if (tid == 0) sh.waiting = w;
           if (tid == 0) sh.acc[10] += wall_clock64() - tq;
         } else {
