@@ -167,14 +167,15 @@ int eik_partition_labels(eik_mesh_t mesh, int32_t* labels_out);
 /* meshFIM3dEikonal.cu:285-566; meshFIM2dEikonal::GenerateData, meshFIM2d_eikonal.cu:349-864) */
 /* ---------------------------------------------------------------------------------------- */
 
-#define EIK_SCHED_SYNC 0   /* one launch per outer iteration, host reads the active count */
-#define EIK_SCHED_ASYNC 1  /* one persistent launch with a device work queue */
+#define EIK_SCHED_SYNC 0   /* one launch per outer iteration */
+#define EIK_SCHED_ASYNC 1  /* one persistent launch with a device scheduler */
 
 /* Element records of a block visit: copied to LDS once per visit, or read from memory (L1/L2)
- * at every use with smaller workgroups, more of them per CU.  AUTO stages the persistent single
- * solve (one solve's wavefront is latency-bound: fewer, faster visits win) and reads from
- * memory in the one-launch-per-iteration solve and in multi-solve launches (batches, serving:
- * throughput-bound, more resident workgroups win). */
+ * at every use with smaller workgroups, more of them per CU.  AUTO keeps a block's element data in
+ * registers and LDS where the blocks fit (up to about 4,000 tets or 4,000 triangle corners a block);
+ * else it stages the persistent single solve's and reads from memory in the
+ * one-launch-per-iteration solve and in multi-solve launches, there also where a launch has so
+ * many blocks that smaller workgroups are faster. */
 #define EIK_STAGE_AUTO 0
 #define EIK_STAGE_LDS 1
 #define EIK_STAGE_MEMORY 2
@@ -187,21 +188,20 @@ typedef struct {
                               <= 0 (the default) chooses per element kind: 2 for tets, 4 for
                               triangles, 3 for triangles in the async single solve (the
                               reference runs 2 in 3D, 7 in 2D).  The async scheduler runs one
-                              sweep per tet visit while few blocks are pending and then re-runs
+                              sweep per tet visit while few blocks wait and then re-runs
                               an unconverged block at once in the same workgroup (stats.reruns) */
   float eps;               /* relative: a decrease by more than eps * T marks a vertex changed
                               (its elements are re-solved) and keeps its block unconverged;
                               default 0, the exact fixed point (the reference stops at an
                               absolute 1e-5, CUDADefines.h:20) */
   int32_t record_history;  /* sync only: keep T after every outer iteration */
-  int32_t workgroups;      /* async: persistent workgroups (0 = auto, sized to the fronts:
-                              about 5 x (blocks^2 x seeds)^(1/3) for tets, 3 x sqrt(blocks x
-                              seeds) for triangles, at least one per CU, at most all that fit) */
+  int32_t workgroups;      /* async: persistent workgroups (0 = auto: one per block, at most all
+                              that fit) */
   int32_t stage_records;   /* EIK_STAGE_*: where a block visit reads its element records */
   int32_t wait_limit_us;   /* async / batch / served: longest wait of a persistent workgroup
-                              for queued work, in microseconds (0 = 10 s, the default; < 0 is
-                              invalid).  A workgroup that waits longer exits; if the queue then
-                              never reaches its end the solve fails with EIK_ERR_TIMEOUT, so a
+                              for work, in microseconds (0 = 10 s, the default; < 0 is
+                              invalid).  A workgroup that waits longer exits; if the solve then
+                              never reaches its end it fails with EIK_ERR_TIMEOUT, so a
                               solve cannot hang the caller.  Normal waits last microseconds. */
 } eik_solve_opts_t;
 
@@ -228,10 +228,10 @@ typedef struct {
   double load_ms;          /* parts of busy_ms: staging loads, sweeps, write-back */
   double sweep_ms;
   double writeback_ms;
-  double queue_ms;         /* async: queueing dependents and releasing blocks, summed */
+  double queue_ms;         /* async: marking dependents and releasing blocks, summed */
   int64_t reruns;          /* async: visits that directly followed the same workgroup's visit of
-                              the same block (no queue round trip; records still staged) */
-  int64_t abandoned_waits; /* async / batch: queue waits that outlasted wait_limit_us (0 in a
+                              the same block (element data still on the CU) */
+  int64_t abandoned_waits; /* async / batch: waits for work that outlasted wait_limit_us (0 in a
                               healthy solve) */
   int64_t algo_bytes_loaded; /* algo_bytes without the element term of the re-runs whose element
                                 records were still staged in LDS from the visit before (they
@@ -254,7 +254,7 @@ int eik_solve(eik_mesh_t mesh, const int32_t* seeds, int64_t nseeds, const float
  * cannot allocate device memory: code under HIP graph capture, serving loops, harnesses that
  * forbid hipMalloc.  No counterpart in the reference (its solve allocates on every call,
  * meshFIM3dEikonal.cu:368-389).  Allocates nothing and does not synchronise: the solve's state
- * (times, the seen values, the work queue, its flags and counters) lives in a device array of the
+ * (times, the seen values, the scheduler's words and counters) lives in a device array of the
  * library of 64 MiB per device, held until the process ends; a mesh whose state needs more fails
  * with EIK_ERR_CAPACITY (tet meshes up to about 3 M vertices fit at 64 vertices per block;
  * larger ones use eik_solve).

@@ -939,8 +939,9 @@ static VisitKernel visit_kernel(const DeviceState* d, int32_t stage_records) {
 }
 
 // Workgroups of the single-solve persistent kernel: one per block while they all fit, so that every
-// block stays resident with its owner, else all that fit (64^3 cube, 4,292 blocks: 1.61 ms at 256,
-// 0.99 at 512, 0.72 at 1,024; 96^3, 14,261 blocks: 5.12, 2.90, 1.82).  Triangle meshes
+// block stays resident with its owner, else all that fit (64^3 cube, 4,292 blocks: 1.29 ms at 256,
+// 0.81 at 512, 0.66 at 768, 0.63 at 1,024; level-8 icosphere, 10,240 blocks of 512 threads: 2.10 at 256,
+// 1.73 at 384, 1.57 at 512).  Triangle meshes
 // whose blocks take 256 threads stop at three per CU: beyond that, waiting workgroups only add traffic.
 static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t nblocks, int* out) {
   int dev = 0, ncu = 0, per_cu = 0;
@@ -1356,12 +1357,17 @@ int eik_solve_noalloc(eik_mesh_t h, const int32_t* seeds_dev, int64_t nseeds, fl
   HIP_TRY(hipGetDevice(&dev));
   if (dev != d->device)
     return fail(EIK_ERR_STATE, "the current device is not the one the mesh was uploaded to");
-  int ncu = 0;
-  HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  eik_solve_opts_t o;
+  eik_solve_opts_default(&o);
+  int grid = 0;
+  int rc = persistent_grid(m->dim, visit_kernel(d, o.stage_records), o.workgroups, d->nblocks, &grid);
+  if (rc) return rc;
+  Sched words;
+  sched_shape(words, d->nblocks, grid);
   // [control words][counters][block words][T][seen], 256-byte aligned
   const size_t o_cnt = align256(kSchedCtlBytes);
   const size_t o_word = o_cnt + align256(sizeof(unsigned long long) * kNumCounters);
-  const size_t o_T = o_word + align256(sizeof(unsigned long long) * sched_max_words((size_t)d->nblocks, 64 * (size_t)std::max(ncu, 1)));
+  const size_t o_T = o_word + align256(sizeof(unsigned long long) * (size_t)words.owners * words.stride);
   const size_t o_seen = o_T + align256(sizeof(float) * (size_t)m->nv);
   const size_t need = o_seen + align256(sizeof(float) * (size_t)d->nseen);
   if (need > kScratchBytes)
@@ -1369,14 +1375,12 @@ int eik_solve_noalloc(eik_mesh_t h, const int32_t* seeds_dev, int64_t nseeds, fl
                                       " bytes of solve state; the allocation-free solve has " +
                                       std::to_string(kScratchBytes) + " (use eik_solve)");
   unsigned char* base = nullptr;
-  int rc = scratch_address(dev, &base);
+  rc = scratch_address(dev, &base);
   if (rc) return rc;
   // the array keeps the previous call's contents: everything the solve reads first is reset
   const AsyncBufs b = {reinterpret_cast<float*>(base + o_T), reinterpret_cast<float*>(base + o_seen),
                        reinterpret_cast<unsigned long long*>(base + o_word), base,
                        reinterpret_cast<unsigned long long*>(base + o_cnt)};
-  eik_solve_opts_t o;
-  eik_solve_opts_default(&o);
   return enqueue_async(*m, o, b, seeds_dev, nullptr, nseeds, T_out_dev,
                        nullptr, stream ? reinterpret_cast<hipStream_t>(stream) : d->stream);
 }

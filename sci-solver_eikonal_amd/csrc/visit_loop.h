@@ -105,16 +105,18 @@ __device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned
 // waits, keeps its registers and LDS, and only times are read again.  A visit of a tet block is one
 // sweep while few blocks wait (kCrowd); a block that has not converged is visited again at once
 // unless a block of the same owner waits with a smaller time.
-// What bounds it: the chain of a visit (64^3 cube: 3.0 us a sweep, 0.4 us until its times have landed,
-// 0.8 us of marks and release, 2 us to load a block into the registers and LDS every third visit), and
-// on large tet meshes the loads too (96^3: 86,000 of 40 KB in 1.5 ms).  Held to 128 VGPRs, so that four
+// What bounds it: the chain of a visit (64^3 cube: 2.7 us a sweep, of which 2.3 us without other
+// workgroups on the CU, 0.4 us until its times have landed, 1.0 us of marks and halo loads, 3.1 us to load a
+// block into the registers and LDS every third visit), and on large tet meshes the instructions too:
+// the 96^3 solve keeps the vector units issuing for half of its time.  Held to 128 VGPRs, so that four
 // workgroups fit a CU: with 45 of them spilled the 96^3 solve took 2.1 ms, without 1.7.
 // Visit kernels, against the staged records of visit_block and one queue ring: 64^3 cube 1.045 ->
-// 0.664 ms, 96^3 with 16 sources 3.67 -> 1.53, 33^3 tensor 0.448 -> 0.295, 16^3 0.285 -> 0.172; level-8
-// icosphere 3.29 -> 1.70, level-7 anisotropic 1.02 -> 0.55, level 5 0.328 -> 0.169, 32^2 square 0.158 ->
-// 0.081.
-// blocks(g) gives the data of launch-wide block g; me is the workgroup's owner index.  Returns kNoWork or kGaveUp.  The workgroup's tally
-// is added to sh.acc, which the caller has cleared (behind a barrier) and flushes.
+// 0.63 ms, 96^3 with 16 sources 3.67 -> 1.41, 33^3 tensor 0.448 -> 0.267, 16^3 0.285 -> 0.135; level-8
+// icosphere 3.29 -> 1.51, level-7 anisotropic 1.02 -> 0.48, level 5 0.328 -> 0.118, 32^2 square 0.158 ->
+// 0.057.
+// blocks(g) gives the data of launch-wide block g; me is the workgroup's owner index.  Returns kNoWork
+// or kGaveUp.  The workgroup's tally is added to sh.acc, which the caller has cleared (behind a
+// barrier) and flushes.
 template <int DIM, int N, int BT, bool CAP, class Blocks>
 __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& blocks, uint32_t me,
                                              uint4* lds4, LoopShared& sh) {
