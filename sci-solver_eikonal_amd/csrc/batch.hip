@@ -335,7 +335,8 @@ static void launch_visits(const Group& g, size_t lds, hipStream_t s, const Multi
     hipLaunchKernelGGL((k_visit_multi<DIM, BT, 4>), dim3(g.grid), dim3(BT), lds, s, a, sd);
 }
 
-// Blocks per resident workgroup from which on a launch of tet blocks may read its records from memory.
+// Blocks per resident workgroup from which on a launch of tet blocks reads its records from memory (twice
+// as many where the CUs hold enough of them resident).
 constexpr int kBusyBlocks = 24;
 
 // The register-resident kernel of a launch of these kinds (fn: null if their blocks do not fit): the
@@ -556,13 +557,16 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
     // memory, ms: 48 vertices per block (2,800 elements a CU) 5.92 / 5.49, 64 (3,540) 5.12 / 5.26, 80
     // 4.91 / 5.11, 96 (768 threads) 5.44 / 5.12, 128 (3,040) 6.40 / 5.05, 160 (3,560) 5.45 / 5.36, 192
     // (4,270) 5.01 / 5.65, 208 (one workgroup) 7.90 / 5.72; with fewer blocks, 21 per workgroup of 128
-    // vertices 3.34 / 3.44, 14 of 192 2.41 / 3.83.  Triangle blocks are as small resident: level-7
+    // vertices 3.34 / 3.44, 14 of 192 2.41 / 3.83.  With twice as many blocks per workgroup the launch's ramp
+    // and end, where the long visits from memory wait, no longer count: 64 / 192 vertices per block, 90 / 60
+    // per workgroup 11.7 / 10.2 and 11.5 / 10.1, 180 / 120 23.8 / 19.0 and 23.3 / 18.1; 43 / 29 5.18 / 5.29
+    // and 5.22 / 5.64.  Triangle blocks are as small resident: level-7
     // spheres 1.5 / 10.8.
     int per = 0, rc = resident_grid(res_launch(L, 1 << gi), 0, &per);
     if (rc) return rc;
     const int cu = std::max(1, per / std::max(1, ncu));
     const bool holds = cu * g.res_bt >= 1024 && cu * g.max_elem >= 3500;
-    g.shape = gi == 0 && !holds && kblocks[0] > (int64_t)kBusyBlocks * per ? 1 : 2;
+    g.shape = gi == 0 && kblocks[0] > (int64_t)(holds ? 2 : 1) * kBusyBlocks * per ? 1 : 2;
   }
   L.merged = L.grp[0].present && L.grp[1].present && L.grp[0].shape == 2 && L.grp[1].shape == 2 &&
              res_launch(L, 3).fn != nullptr;

@@ -68,7 +68,7 @@ def test_shapes_with_factors(E, vpb, workgroups, kinds):
 
 
 def test_busy_launch(E):
-    """More than 24 one-vertex tet blocks for each of the at most 1,024 workgroups of 256 threads that
+    """More than 24 one-vertex (too small to fill a CU) tet blocks for each of the at most 1,024 workgroups of 256 threads that
     are resident: records read from memory; one solve fewer than that: register-resident."""
     m = E.Mesh.kuhn_cube(11, 0.2, seed=3)
     m.partition(1)
