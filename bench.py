@@ -33,9 +33,9 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 # kernel sources it was measured on.  A summary whose hash differs from the current sources is
 # stale and gives no figure (traffic null).
 PROFILES = {
-    "fim3d_kuhn64_lognormal": "k_visit_async_fim3d_kuhn64_lognormal.md",
+    "fim3d_kuhn64_lognormal": "k_visit_resident_fim3d_kuhn64_lognormal.md",
     "batch256_kuhn16to48_twolayer": "k_visit_multi_batch256_kuhn16to48.md",
-    "ico7_aniso_4src": "k_visit_async_ico7_aniso.md",
+    "ico7_aniso_4src": "k_visit_resident_ico7_aniso.md",
 }
 
 
