@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fim_kernels.h"
+#include "lane_ops.h"
 
 namespace eik {
 
@@ -78,14 +79,6 @@ __device__ __forceinline__ uint32_t* lock_of(const Sched& s, uint32_t slot) {
 // Marks a block dirty with a key; no result is waited for.
 __device__ __forceinline__ void sched_mark(const Sched& s, uint32_t slot, uint32_t key) {
   (void)__hip_atomic_fetch_min(key_of(s, slot), key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Waits until this wave's memory operations have completed at the device's coherence point
-// (vmcnt covers loads, stores and atomics, with or without a result).
-__device__ __forceinline__ void wait_memory() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0);
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
 // What one wave of a workgroup keeps between its searches.

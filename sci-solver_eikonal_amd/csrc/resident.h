@@ -17,6 +17,7 @@
 #pragma once
 
 #include "fim_kernels.h"
+#include "lane_ops.h"
 
 namespace eik {
 
@@ -143,22 +144,6 @@ __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large,
   return changed;
 }
 
-// Two non-negative values as fp16, rounded towards zero; and a sum with one of
-// them, in one instruction.
-__device__ __forceinline__ uint32_t half_pair(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-}
-__device__ __forceinline__ float add_half_lo(float x, uint32_t p) {
-  float y;
-  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(x), "v"(p));
-  return y;
-}
-__device__ __forceinline__ float add_half_hi(float x, uint32_t p) {
-  float y;
-  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(x), "v"(p));
-  return y;
-}
-
 // The smallest of three times, which are not negative: as integers, which need no quieting of NaNs.
 __device__ __forceinline__ float time_min(float a, float b, float c) {
   const uint32_t x = __float_as_uint(a), y = __float_as_uint(b), z = __float_as_uint(c);
@@ -173,13 +158,6 @@ struct TetRegs {
   uint32_t h01[N], h23[N];
   float p0[N], p1[N], p2[N], p3[N];  // the corners: fallen below this since the last selection
 };
-
-// Copies 16 bytes per lane from memory straight to LDS (lane i of the wave to base + 16 i), so that
-// no register holds them on the way.
-__device__ __forceinline__ void copy_to_lds(const uint4* from, uint4* wave_base) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
-                                   (__attribute__((address_space(3))) void*)wave_base, 16, 0, 0);
-}
 
 // Loads the thread's records: slots and heights to registers, slots and lengths to LDS.
 // rmult as in tri_load.
@@ -261,30 +239,6 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
 // A queued pair: thread and, in the low five bits, its element's place u and the corner, 4 u + k.
 template <int BT>
 __device__ __forceinline__ int item_elem(int item) { return (item >> 2 & 7) * BT + (item >> 5); }
-
-// Adds to an LDS counter, by one lane, without the scan over the lanes that the compiler makes of an
-// atomic with a result; returns the value before.
-__device__ __forceinline__ int lds_take(int* counter, int n) {
-  int old;
-  asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)"
-               : "=v"(old)
-               : "v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) int*)counter), "v"(n)
-               : "memory");
-  return old;
-}
-
-// LDS atomics without a result, of one lane, as they are (see lds_take).  The caller waits for them
-// (wait_memory) before its barrier.
-__device__ __forceinline__ void lds_min(unsigned* p, unsigned v) {
-  asm volatile("ds_min_u32 %0, %1"
-               :: "v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned*)p), "v"(v)
-               : "memory");
-}
-__device__ __forceinline__ void lds_or(unsigned* p, unsigned v) {
-  asm volatile("ds_or_b32 %0, %1"
-               :: "v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned*)p), "v"(v)
-               : "memory");
-}
 
 // Appends the (element, corner) pairs of the thread's elements that can improve to the queue.  CAP:
 // it may hold fewer than a block has, max_queue; sets *again, and *full to the visit's number, if it did not hold them.
