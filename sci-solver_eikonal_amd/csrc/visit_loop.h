@@ -204,7 +204,12 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       const int inner = DIM == 2 || sh.crowd >= kCrowd ? a.max_inner : 1;
       uint64_t marks = 0;  // dependents holding this thread's vertex, if it fell
       uint32_t key = kClean;
-      float own_last = own;
+      // The owned time that a visit cut off by the sweep cap leaves in `seen`: at least every value that the
+      // block's elements were last evaluated with.  For tets the time before the last sweep.  For triangles
+      // the one published before that: no barrier parts the publishing from the next sweep, which lowers
+      // times in place, so the time published after the last sweep but one may be one of the last sweep's
+      // already, which items evaluated before it fell have not seen.
+      float own_last = own, own_seen = own;
       int sweep = 0;
       bool conv = false;
       while (sweep < inner) {
@@ -230,6 +235,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
         if (tid == 0) sh.flag[ring == 2 ? 0 : ring + 1] = 0;
         ++sweep;
         // publish the owned times that fell
+        own_seen = DIM == 2 ? own_last : own;
         own_last = own;
         if (tid < d.nown) {
           const float v = sT[tid];
@@ -286,6 +292,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       if (tid < 64) {
         const uint64_t mask = (uint64_t)sh.mark[0] | ((uint64_t)sh.mark[1] << 32);
         if (cap_ok && tid < ndep && ((mask >> tid) & 1ull)) sched_mark(a.s, dep_slot, vkey);
+        __builtin_amdgcn_wave_barrier();  // (the mask has been read by every lane)
         if (tid < 2) sh.mark[tid] = 0;
         if (tid == 0) {
           VisitResult vr;
@@ -328,7 +335,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
         // vertices that fell in the last sweep of a visit cut off by the sweep cap.  A later
         // visit that misses these (they are plain stores) evaluates more than it has to.
         // After a full queue, nothing counts as evaluated.
-        if (tid < d.nown) seen[tid] = full ? EIK_INF : conv ? own : own_last;
+        if (tid < d.nown) seen[tid] = full ? EIK_INF : conv ? own : own_seen;
         for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = full ? EIK_INF : sT[d.nown + i];
       }
       __syncthreads();

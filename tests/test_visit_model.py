@@ -1,0 +1,52 @@
+"""CPU checks of the persistent workgroups' loop (no device): csrc/visit_loop.h, block_sched.h and
+resident.h as they are, built for the host with a model of waves, barriers and late atomics
+(tests/cpp/simt), run whole solves on real layouts with the waves interleaved at random
+(tests/cpp/visit_model.cpp).  Every solve must end by itself with no block waiting, and no corner solve
+of any element may then lower a time."""
+import glob
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+CLANG = "/opt/rocm/llvm/bin/clang++"
+CSRC = os.path.join(ROOT, "sci-solver_eikonal_amd", "csrc")
+CPP = os.path.join(ROOT, "tests", "cpp")
+
+
+@pytest.fixture(scope="module")
+def visit_model(tmp_path_factory):
+    if not os.path.exists(CLANG):
+        pytest.skip("clang++ is not installed")
+    d = tmp_path_factory.mktemp("visit_model")
+    # the headers, with the host's definitions of the few operations written as instructions
+    for h in glob.glob(os.path.join(CSRC, "*.h")):
+        shutil.copy(h, d)
+    shutil.copy(os.path.join(CPP, "simt", "lane_ops.h"), d)
+    exe = d / "visit_model"
+    subprocess.run([CLANG, "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(CPP, "simt"),
+                    "-I", str(d), "-I", os.path.join(ROOT, "include"), "-I", "/opt/rocm/include",
+                    os.path.join(CPP, "visit_model.cpp")] +
+                   [os.path.join(CSRC, f) for f in ("mesh.cpp", "partition.cpp", "layout.cpp")] +
+                   ["-o", str(exe), "-lpthread"], check=True, capture_output=True)
+    return str(exe)
+
+
+def _run(exe, *args):
+    r = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+    return r.stdout
+
+
+# kind and items or elements per thread, mesh size, vertices per block, workgroups, inner sweeps, runs
+@pytest.mark.parametrize("kind,size,vpb,groups,inner,runs", [
+    ("tri1", 3, 32, 1, 3, 12), ("tri1", 3, 32, 3, 2, 12), ("tri2", 3, 90, 1, 3, 20),
+    ("tri2", 4, 90, 2, 3, 6), ("tri1", 3, 16, 2, 1, 8), ("tri1", 2, 32, 6, 3, 10),
+    ("tet4", 5, 20, 2, 2, 15), ("tet4", 5, 20, 9, 2, 15), ("tet2", 4, 60, 2, 3, 10)])
+def test_solves_end_at_a_fixed_point(visit_model, kind, size, vpb, groups, inner, runs):
+    """Blocks cut off by the sweep cap and left for another, more blocks than workgroups, one per workgroup."""
+    out = _run(visit_model, kind, size, vpb, groups, inner, runs, 7, 0)
+    assert "unfinished 0, failures 0" in out, out
