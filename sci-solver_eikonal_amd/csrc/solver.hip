@@ -351,7 +351,7 @@ struct SolveArgs {
   const int32_t* dep_start;
   const int32_t* dep;
   const int32_t* iperm;
-  float* out;          // the times in caller order, written when the solve has ended (or null)
+  float* out;          // the times in caller order, written at the end of the launch (or null)
   unsigned long long* told;  // pinned host memory: the last one copies the counters here (or null)
   int64_t nv;
   unsigned long long* counters;
@@ -362,15 +362,6 @@ struct SolveArgs {
   int32_t max_queue;
   size_t rec_lds_bytes;  // k_visit_general: staged records
 };
-
-// After the end of the solve (block == kNoWork: every visit has ended and every published time has
-// landed), the launch's workgroups write the times in caller order.
-__device__ __forceinline__ void write_out(const SolveArgs& a, int block) {
-  if (!a.out || block != kNoWork) return;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.nv; i += stride)
-    a.out[i] = load_T<true>(a.v.T + a.iperm[i]);
-}
 
 // The end of a workgroup: its tally, and, if it is the last one, the sums to the host, with the ticks at
 // which the solve and its visits began and this one.
@@ -411,7 +402,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   begin(a);
   const LoopArgs la = {a.s, a.v.eps, a.v.max_inner, a.max_visits, a.max_local, a.max_elem, a.max_queue};
   const int end = resident_loop<DIM, N, BT, CAP>(la, SingleBlocks{a}, blockIdx.x, lds4, sh);
-  write_out(a, end);
+  write_times(a.s, end, a.v.T, a.iperm, a.nv, a.out, &sh.block);
   finish(a, sh.acc);
 }
 
@@ -526,7 +517,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
       rerun = true;
     }
   }
-  write_out(a, sBlock);
+  write_times(a.s, __builtin_amdgcn_readfirstlane(sBlock), a.v.T, a.iperm, a.nv, a.out, &sBlock);
   finish(a, sAcc);
 }
 
@@ -1030,7 +1021,7 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   a.v.dep_start = d->dep_start;
   a.s.word = b.words;
   a.s.ctl = reinterpret_cast<unsigned long long*>(b.sctl);
-  a.s.done = reinterpret_cast<uint32_t*>(b.sctl + kSchedCtlBytes / 2);
+  a.s.done = reinterpret_cast<unsigned long long*>(b.sctl + kSchedCtlBytes / 2);
   sched_shape(a.s, d->nblocks, grid);
   a.s.wait_limit = wait_limit_ticks(d->device, o.wait_limit_us);
   a.items = {d->item_range, d->item_id, d->item_len, d->item_rec};

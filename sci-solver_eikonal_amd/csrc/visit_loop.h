@@ -93,9 +93,37 @@ __device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned
   const int32_t b = look ? sched_look(s, f) : sched_find(s, f);
   if (__lane_id() == 0) {
     acc[6] += wall_clock64() - w0;
-    if (b == kGaveUp) acc[kCntAbandoned] += 1;
+    if (b == kGaveUp || b == kGaveUpLast) acc[kCntAbandoned] += 1;
   }
   return b;
+}
+
+// Writes a solve's times in caller order, when a workgroup of the launch found no further block (end).  At
+// the end of the solve (every visit has ended and every published time has landed) each workgroup writes a
+// stripe of them.  Where workgroups gave up before, their stripes would be missing: the ones that found the
+// end, or the last to give up (whose times are not final), write stretches that they take from a counter
+// until none is left.
+constexpr int64_t kOutStretch = 8192;
+__device__ __forceinline__ void write_times(const Sched& s, int end, const float* T, const int32_t* iperm,
+                                            int64_t nv, float* out, int* next) {
+  if (!out || end == kGaveUp) return;
+  if (end == kNoWork) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += stride)
+      out[i] = load_T<true>(T + iperm[i]);
+    return;
+  }
+  uint32_t* taken = reinterpret_cast<uint32_t*>(s.done + 1);
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0)
+      *next = (int)(uint32_t)__hip_atomic_fetch_add(taken, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int64_t from = (int64_t)(uint32_t)*next * kOutStretch;
+    if (from >= nv) return;
+    const int64_t to = from + kOutStretch < nv ? from + kOutStretch : nv;
+    for (int64_t i = from + threadIdx.x; i < to; i += blockDim.x) out[i] = load_T<true>(T + iperm[i]);
+  }
 }
 
 // The loop of one workgroup over the blocks of a launch, until the solve has ended or it gives up:
@@ -114,8 +142,8 @@ __device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned
 // 0.63 ms, 96^3 with 16 sources 3.67 -> 1.41, 33^3 tensor 0.448 -> 0.267, 16^3 0.285 -> 0.135; level-8
 // icosphere 3.29 -> 1.51, level-7 anisotropic 1.02 -> 0.48, level 5 0.328 -> 0.118, 32^2 square 0.158 ->
 // 0.057.
-// blocks(g) gives the data of launch-wide block g; me is the workgroup's owner index.  Returns kNoWork
-// or kGaveUp.  The workgroup's tally is added to sh.acc, which the caller has cleared (behind a
+// blocks(g) gives the data of launch-wide block g; me is the workgroup's owner index.  Returns why there
+// is no further block (block_sched.h).  The workgroup's tally is added to sh.acc, which the caller has cleared (behind a
 // barrier) and flushes.
 template <int DIM, int N, int BT, bool CAP, class Blocks>
 __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& blocks, uint32_t me,

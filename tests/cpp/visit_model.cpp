@@ -4,7 +4,8 @@
 //
 // Every solve must end by itself with all block words clean, and its times must be a fixed point: no
 // corner solve of any element gives less than its target's time (the solver and its arithmetic are
-// those of the visits).
+// those of the visits).  The output must be the times in caller order, complete, whether or not
+// workgroups gave up waiting before the end.
 //
 // usage: visit_model <tri N|tet N> <mesh size> <vertices per block> <workgroups> <inner sweeps> <runs>
 //                    <seed> <wait limit, steps; 0: none>
@@ -59,7 +60,7 @@ Items tri_items(const Layout& L) {
 struct Solve {
   const Mesh& m;
   Items items;
-  std::vector<float> T, seen;
+  std::vector<float> T, seen, out;
   std::vector<unsigned long long> words;
   alignas(256) unsigned char ctl[kSchedCtlBytes] = {};
   LoopArgs a = {};
@@ -141,11 +142,12 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
   std::mt19937_64 rng(seed);
   Solve s(m);
   const float large = DIM == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
-  int failures = 0, gave_up = 0, unfinished = 0;
+  int failures = 0, gave_up = 0, unfinished = 0, shortened = 0;
   long long visits = 0;
   for (int run = 0; run < runs; ++run) {
     s.T.assign((size_t)m.nv, large);
     s.seen.assign((size_t)m.nv + L.halo.size(), EIK_INF);
+    s.out.assign((size_t)m.nv, -1.f);
     std::memset(s.ctl, 0, sizeof s.ctl);
     Sched& sc = s.a.s;
     sched_shape(sc, L.nblocks, groups);
@@ -178,6 +180,7 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
     const char* err = simt::run((unsigned)groups, BT, seed * 1000003u + (uint64_t)run, [&] {
       Group& g = gs[blockIdx.x];
       const int end = resident_loop<DIM, N, BT, false>(s.a, blocks, blockIdx.x, g.lds.data(), g.sh);
+      write_times(s.a.s, end, s.T.data(), L.iperm.data(), m.nv, s.out.data(), &g.sh.block);
       g.end = end;
     });
     if (err) {
@@ -185,15 +188,24 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
       return 1;
     }
     bool ended = false;
+    const int before = gave_up;
     for (Group& g : gs) {
-      ended = ended || g.end == kNoWork;
-      gave_up += g.end == kGaveUp;
+      ended = ended || g.end == kNoWork || g.end == kNoWorkFew;
+      gave_up += g.end == kGaveUp || g.end == kGaveUpLast;
       visits += (long long)g.sh.acc[0];
+    }
+    const int given = gave_up - before;
+    int unwritten = 0;
+    for (int64_t v = 0; v < m.nv; ++v) unwritten += s.out[(size_t)v] != s.T[(size_t)L.iperm[(size_t)v]];
+    if (unwritten) {
+      ++failures;
+      std::printf("run %d: %d of %lld times not written\n", run, unwritten, (long long)m.nv);
     }
     if (!ended) {
       ++unfinished;
       continue;
     }
+    shortened += given > 0;
     int dirty = 0;
     for (unsigned long long w : s.words) dirty += w != (unsigned long long)kClean;
     const int bad = improvable(s);
@@ -202,8 +214,8 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
       std::printf("run %d: ended with %d words not clean, %d solves that lower a time\n", run, dirty, bad);
     }
   }
-  std::printf("%d runs of %d blocks, %lld visits, gave up %d, unfinished %d, failures %d\n", runs, L.nblocks,
-              visits, gave_up, unfinished, failures);
+  std::printf("%d runs of %d blocks, %lld visits, gave up %d, ended short %d, unfinished %d, failures %d\n",
+              runs, L.nblocks, visits, gave_up, shortened, unfinished, failures);
   return failures ? 1 : 0;
 }
 

@@ -50,3 +50,11 @@ def test_solves_end_at_a_fixed_point(visit_model, kind, size, vpb, groups, inner
     """Blocks cut off by the sweep cap and left for another, more blocks than workgroups, one per workgroup."""
     out = _run(visit_model, kind, size, vpb, groups, inner, runs, 7, 0)
     assert "unfinished 0, failures 0" in out, out
+
+
+# the wait limit in scheduling steps
+@pytest.mark.parametrize("kind,size,vpb,groups,limit", [
+    ("tri1", 2, 32, 6, 300), ("tri1", 2, 32, 6, 1500), ("tri1", 2, 32, 6, 6000), ("tet4", 4, 20, 3, 300)])
+def test_every_time_is_written_when_workgroups_give_up(visit_model, kind, size, vpb, groups, limit):
+    out = _run(visit_model, kind, size, vpb, groups, 3, 20, 1, limit)
+    assert "gave up 0," not in out and "failures 0" in out, out
