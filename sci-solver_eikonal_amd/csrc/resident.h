@@ -34,16 +34,18 @@ struct TriItems {
 constexpr int kItemSlotBits = 10;
 constexpr int kItemSlots = 1 << kItemSlotBits;  // local vertices of a block with items
 
-// A time that has fallen since `last`, by more than eps relative (eps = 0: at all).
+// Whether a fall counts as a change, after which a visit sweeps again: by more than eps relative (eps = 0:
+// at all).
 __device__ __forceinline__ bool fell(float last, float now, float eps) {
   return last - now > eps * now;
 }
 
 // What a sweep tests first it does for every item, changed or not, and with the instructions issued
 // on two thirds of all cycles (96^3 cube) their number counts: so an item holds the LDS offsets of its
-// corners' times instead of slots, and, for each corner, the time below which it counts as fallen,
-// last / (1 + eps), instead of the last time.
-__device__ __forceinline__ float fall_below(float last, float keep) { return last * keep; }
+// corners' times instead of slots.  A corner counts as fallen if it lies below its last time at all,
+// whatever eps: falls within eps are many, and where each had to exceed it alone, with a block's record of
+// evaluated times starting anew at every visit, their sum was lost (persistent solves at eps = 0.01,
+// largest relative error: 32^3 cube 3e-2, now 1e-5; level-7 icosphere 7e-2, now 9e-3).
 __device__ __forceinline__ float time_at(const float* sT, uint32_t offset) {
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(sT) + offset);
 }
@@ -52,7 +54,7 @@ template <int N>
 struct TriRegs {
   uint32_t ab[N], t[N];  // LDS offsets of the two other corners, 16 bits each, and of the target
   float la[N], lb[N], lab[N], h[N];
-  float pa[N], pb[N];  // the two other corners: fallen below this since the last evaluation
+  float pa[N], pb[N];  // the two other corners' times at the last evaluation
 };
 
 // The thread index, opaque: what is computed from it is computed where it is used, not hoisted out of
@@ -96,18 +98,18 @@ __device__ __forceinline__ void tri_load(TriRegs<N>& r, const TriItems& t, int2 
 }
 
 template <int N>
-__device__ __forceinline__ void tri_seen(TriRegs<N>& r, const float* sP, float keep) {
+__device__ __forceinline__ void tri_seen(TriRegs<N>& r, const float* sP) {
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    r.pa[u] = fall_below(time_at(sP, r.ab[u] & 0xffffu), keep);
-    r.pb[u] = fall_below(time_at(sP, r.ab[u] >> 16), keep);
+    r.pa[u] = time_at(sP, r.ab[u] & 0xffffu);
+    r.pb[u] = time_at(sP, r.ab[u] >> 16);
   }
 }
 
 // One sweep over the thread's items.  Returns whether it lowered a time.
 template <int N>
 __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large, float eps,
-                                          float keep, unsigned& solves) {
+                                          unsigned& solves) {
   float ta[N], tb[N], tk[N];
   // What a solve computes from the lengths alone stays in registers from sweep to sweep where there
   // is room (N = 2); for more items it would be spilled, so it is computed again.
@@ -125,8 +127,8 @@ __device__ __forceinline__ bool tri_sweep(TriRegs<N>& r, float* sT, float large,
 #pragma unroll
   for (int u = 0; u < N; ++u) {
     if (!(ta[u] < r.pa[u] || tb[u] < r.pb[u])) continue;
-    r.pa[u] = fall_below(ta[u], keep);
-    r.pb[u] = fall_below(tb[u], keep);
+    r.pa[u] = ta[u];
+    r.pb[u] = tb[u];
     // nothing below the smaller time plus the height; unknown times are `large`, and no time
     // is above that
     if (!(tk[u] > __builtin_fminf(ta[u], tb[u]) + r.h[u])) continue;
@@ -156,7 +158,7 @@ struct TetRegs {
   uint32_t v01[N], v23[N];     // LDS offsets of the corners' times, 16 bits each
   // heights in fp16, rounded down (they stay lower bounds of every solve); +inf: not owned
   uint32_t h01[N], h23[N];
-  float p0[N], p1[N], p2[N], p3[N];  // the corners: fallen below this since the last selection
+  float p0[N], p1[N], p2[N], p3[N];  // the corners' times at the last selection
 };
 
 // Loads the thread's records: slots and heights to registers, slots and lengths to LDS.
@@ -203,13 +205,13 @@ __device__ __forceinline__ void tet_load(TetRegs<N>& r, const void* recs, const 
 }
 
 template <int N>
-__device__ __forceinline__ void tet_seen(TetRegs<N>& r, const float* sP, float keep) {
+__device__ __forceinline__ void tet_seen(TetRegs<N>& r, const float* sP) {
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    r.p0[u] = fall_below(time_at(sP, r.v01[u] & 0xffffu), keep);
-    r.p1[u] = fall_below(time_at(sP, r.v01[u] >> 16), keep);
-    r.p2[u] = fall_below(time_at(sP, r.v23[u] & 0xffffu), keep);
-    r.p3[u] = fall_below(time_at(sP, r.v23[u] >> 16), keep);
+    r.p0[u] = time_at(sP, r.v01[u] & 0xffffu);
+    r.p1[u] = time_at(sP, r.v01[u] >> 16);
+    r.p2[u] = time_at(sP, r.v23[u] & 0xffffu);
+    r.p3[u] = time_at(sP, r.v23[u] >> 16);
   }
 }
 
@@ -245,7 +247,7 @@ __device__ __forceinline__ int item_elem(int item) { return (item >> 2 & 7) * BT
 // About 190 vector instructions a wave for N = 4 (350 with slots, last times, quieted minima and
 // converted heights): the visits of the 64^3 cube 0.677 -> 0.650 ms, of the 96^3 cube 1.50 -> 1.44.
 template <int N, int BT, bool CAP>
-__device__ __forceinline__ void tet_select(TetRegs<N>& r, int nelem, const float* sT, float keep,
+__device__ __forceinline__ void tet_select(TetRegs<N>& r, int nelem, const float* sT,
                                            uint16_t* sQ, int max_queue, int* qn, int* again, int* full, int visit) {
   static_assert(N <= 8 && BT <= 2048, "queued pairs have 5 bits for the place, 11 for the thread");
   // places of this wave that hold an element (64^3 cube 0.651 -> 0.633 ms with the others left out)
@@ -266,10 +268,10 @@ __device__ __forceinline__ void tet_select(TetRegs<N>& r, int nelem, const float
     const bool f0 = t0[u] < r.p0[u], f1 = t1[u] < r.p1[u];
     const bool f2 = t2[u] < r.p2[u], f3 = t3[u] < r.p3[u];
     if (!(f0 || f1 || f2 || f3)) continue;
-    r.p0[u] = fall_below(t0[u], keep);
-    r.p1[u] = fall_below(t1[u], keep);
-    r.p2[u] = fall_below(t2[u], keep);
-    r.p3[u] = fall_below(t3[u], keep);
+    r.p0[u] = t0[u];
+    r.p1[u] = t1[u];
+    r.p2[u] = t2[u];
+    r.p3[u] = t3[u];
     // a corner is solved again if another one fell and it lies above the smallest of the others by
     // more than its height
     const bool c0 = t0[u] > add_half_lo(time_min(t1[u], t2[u], t3[u]), r.h01[u]);

@@ -260,7 +260,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   uint4* sA = reinterpret_cast<uint4*>(sP + 2 * ls);
   uint4* sB = sA + (DIM == 3 ? a.max_elem : 0);
   uint16_t* sQ = reinterpret_cast<uint16_t*>(sB + (DIM == 3 ? a.max_elem : 0));
-  const float eps = a.v.eps, keep = 1.f / (1.f + eps), large = a.v.large;
+  const float eps = a.v.eps, large = a.v.large;
   float* T = a.v.T;
   float* seen = a.v.seen + d.vstart + d.hstart;
   if (tid < 3) sFlag[tid] = 0;
@@ -285,8 +285,8 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   else tet_load<N, BT>(r, a.v.elems, d, sA, sB, nullptr);
   wait_memory();  // the copies to LDS too
   __syncthreads();
-  if constexpr (DIM == 2) tri_seen<N>(r, sP, keep);
-  else tet_seen<N>(r, sP, keep);
+  if constexpr (DIM == 2) tri_seen<N>(r, sP);
+  else tet_seen<N>(r, sP);
   const unsigned long long t1 = wall_clock64();
   uint32_t solves = 0;
   float last = own;  // the owned time before the last sweep
@@ -297,9 +297,9 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     bool ch = false;
     int nq = 1;
     if constexpr (DIM == 2) {
-      ch = tri_sweep<N>(r, sT, large, eps, keep, solves);
+      ch = tri_sweep<N>(r, sT, large, eps, solves);
     } else {
-      tet_select<N, BT, CAP>(r, d.nelem, sT, keep, sQ, a.max_queue, &sQn[sweep & 1], &sFlag[f], &sFull,
+      tet_select<N, BT, CAP>(r, d.nelem, sT, sQ, a.max_queue, &sQn[sweep & 1], &sFlag[f], &sFull,
                              sweep + 1);
       __syncthreads();
       nq = sQn[sweep & 1];

@@ -157,7 +157,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
   uint4* sA = reinterpret_cast<uint4*>(sHidx + ls);
   uint4* sB = sA + (DIM == 3 ? a.max_elem : 0);
   uint16_t* sQ = reinterpret_cast<uint16_t*>(sB + (DIM == 3 ? a.max_elem : 0));
-  const float eps = a.eps, keep = 1.f / (1.f + a.eps), large = DIM == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
+  const float eps = a.eps, large = DIM == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
   // (the barrier before the first visit orders these)
   if (tid < 3) sh.flag[tid] = 0;
   if (tid < 2) sh.qn[tid] = 0;
@@ -221,8 +221,8 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       tet_load<N, BT>(r, m.elems, d, sA, sB, rmult);
     wait_memory();  // the copies to LDS too
     __syncthreads();
-    if constexpr (DIM == 2) tri_seen<N>(r, sP, keep);
-    else tet_seen<N>(r, sP, keep);
+    if constexpr (DIM == 2) tri_seen<N>(r, sP);
+    else tet_seen<N>(r, sP);
     unsigned long long t1 = wall_clock64();
     bool rerun = false;
     unsigned waiting = kClean;  // smallest key of the owner's other blocks when last looked
@@ -232,7 +232,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       const int inner = DIM == 2 || sh.crowd >= kCrowd ? a.max_inner : 1;
       uint64_t marks = 0;  // dependents holding this thread's vertex, if it fell
       uint32_t key = kClean;
-      // The owned time that a visit cut off by the sweep cap leaves in `seen`: at least every value that the
+      // The owned time left in `seen` by a visit whose last sweep lowered times: at least every value that the
       // block's elements were last evaluated with.  For tets the time before the last sweep.  For triangles
       // the one published before that: no barrier parts the publishing from the next sweep, which lowers
       // times in place, so the time published after the last sweep but one may be one of the last sweep's
@@ -244,9 +244,9 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
         bool ch = false;
         int nq = 1;
         if constexpr (DIM == 2) {
-          ch = tri_sweep<N>(r, sT, large, eps, keep, solves);
+          ch = tri_sweep<N>(r, sT, large, eps, solves);
         } else {
-          tet_select<N, BT, CAP>(r, d.nelem, sT, keep, sQ, a.max_queue, &sh.qn[qc], &sh.flag[ring],
+          tet_select<N, BT, CAP>(r, d.nelem, sT, sQ, a.max_queue, &sh.qn[qc], &sh.flag[ring],
                             &sh.full, visit);
           __syncthreads();
           nq = sh.qn[qc];
@@ -360,10 +360,10 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       }
       if (!again) {
         // what this visit evaluated the block's elements with: every time, but for the owned
-        // vertices that fell in the last sweep of a visit cut off by the sweep cap.  A later
-        // visit that misses these (they are plain stores) evaluates more than it has to.
-        // After a full queue, nothing counts as evaluated.
-        if (tid < d.nown) seen[tid] = full ? EIK_INF : conv ? own : own_seen;
+        // vertices that fell in the last sweep of a visit cut off by the sweep cap (or one that ended
+        // with falls within eps).  A later visit that misses these (they are plain stores) evaluates
+        // more than it has to.  After a full queue, nothing counts as evaluated.
+        if (tid < d.nown) seen[tid] = full ? EIK_INF : conv && eps == 0.f ? own : own_seen;
         for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = full ? EIK_INF : sT[d.nown + i];
       }
       __syncthreads();

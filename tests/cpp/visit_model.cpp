@@ -8,7 +8,10 @@
 // workgroups gave up waiting before the end.
 //
 // usage: visit_model <tri N|tet N> <mesh size> <vertices per block> <workgroups> <inner sweeps> <runs>
-//                    <seed> <wait limit, steps; 0: none>
+//                    <seed> <wait limit, steps; 0: none> [eps]
+// With eps > 0 a visit ends when a sweep lowers nothing by more than that, and what its last sweep
+// lowered counts as evaluated; a fall of a halo vertex is evaluated, however small: only the corner
+// solves from halo vertices alone are looked at then.
 #include <hip/hip_runtime.h>
 
 #include "visit_loop.h"
@@ -92,7 +95,7 @@ struct ModelBlocks {
 };
 
 // Corner solves that give less than their target's time (owned corners of every record).
-int improvable(const Solve& s) {
+int improvable(const Solve& s, bool halo_only) {
   const Mesh& m = s.m;
   const Layout& L = m.layout;
   int bad = 0;
@@ -105,6 +108,9 @@ int improvable(const Solve& s) {
         t[k] = s.T[(size_t)(v[k] < d.nown ? d.vstart + v[k] : L.halo[(size_t)(d.hstart + v[k] - d.nown)])];
       for (int k = 0; k < K; ++k) {
         if (v[k] >= d.nown) continue;
+        bool owned = false;
+        for (int j = 0; j < K; ++j) owned = owned || (j != k && v[j] < d.nown);
+        if (halo_only && owned) continue;
         float least = EIK_INF, cand, h;
         for (int j = 0; j < K; ++j)
           if (j != k) least = std::min(least, t[j]);
@@ -132,7 +138,7 @@ struct Group {
 };
 
 template <int DIM, int N, int BT>
-int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned long long limit) {
+int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned long long limit, float eps) {
   const Layout& L = m.layout;
   const int need = DIM == 3 ? L.max_elem : L.max_items;
   if (need > N * BT || L.max_own > BT || L.max_local > kItemSlots || L.vmask.empty()) {
@@ -156,7 +162,7 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
     sc.ctl = reinterpret_cast<unsigned long long*>(s.ctl);
     sc.done = reinterpret_cast<decltype(sc.done)>(s.ctl + kSchedCtlBytes / 2);
     sc.wait_limit = limit ? limit : ~0ull;
-    s.a.eps = 0.f;
+    s.a.eps = eps;
     s.a.max_inner = inner;
     s.a.max_visits = 1 << 30;
     s.a.max_local = L.max_local;
@@ -208,7 +214,7 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
     shortened += given > 0;
     int dirty = 0;
     for (unsigned long long w : s.words) dirty += w != (unsigned long long)kClean;
-    const int bad = improvable(s);
+    const int bad = improvable(s, eps > 0.f);
     if (dirty || bad) {
       ++failures;
       std::printf("run %d: ended with %d words not clean, %d solves that lower a time\n", run, dirty, bad);
@@ -222,12 +228,13 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
 }  // namespace
 
 int main(int argc, char** argv) {
-  if (argc != 9) return 2;
+  if (argc != 9 && argc != 10) return 2;
   const std::string kind = argv[1];
   const int size = std::atoi(argv[2]), vpb = std::atoi(argv[3]), groups = std::atoi(argv[4]);
   const int inner = std::atoi(argv[5]), runs = std::atoi(argv[6]);
   const uint64_t seed = std::strtoull(argv[7], nullptr, 10);
   const unsigned long long limit = std::strtoull(argv[8], nullptr, 10);
+  const float eps = argc == 10 ? (float)std::atof(argv[9]) : 0.f;
   Mesh m;
   if (kind[3] == ' ' || kind.size() < 4) return 2;
   const bool tets = kind.substr(0, 3) == "tet";
@@ -240,9 +247,9 @@ int main(int argc, char** argv) {
   if (!tets) tri_virtual_faces(m);
   if (partition_by_size(m, vpb) || build_layout(m)) return 2;
   const int n = std::atoi(kind.c_str() + 3);
-  if (tets) return n == 2 ? run_solves<3, 2, 512>(m, groups, inner, runs, seed, limit)
-                          : run_solves<3, 4, 256>(m, groups, inner, runs, seed, limit);
-  return n == 1   ? run_solves<2, 1, 256>(m, groups, inner, runs, seed, limit)
-         : n == 2 ? run_solves<2, 2, 512>(m, groups, inner, runs, seed, limit)
-                  : run_solves<2, 4, 512>(m, groups, inner, runs, seed, limit);
+  if (tets) return n == 2 ? run_solves<3, 2, 512>(m, groups, inner, runs, seed, limit, eps)
+                          : run_solves<3, 4, 256>(m, groups, inner, runs, seed, limit, eps);
+  return n == 1   ? run_solves<2, 1, 256>(m, groups, inner, runs, seed, limit, eps)
+         : n == 2 ? run_solves<2, 2, 512>(m, groups, inner, runs, seed, limit, eps)
+                  : run_solves<2, 4, 512>(m, groups, inner, runs, seed, limit, eps);
 }

@@ -58,3 +58,10 @@ def test_solves_end_at_a_fixed_point(visit_model, kind, size, vpb, groups, inner
 def test_every_time_is_written_when_workgroups_give_up(visit_model, kind, size, vpb, groups, limit):
     out = _run(visit_model, kind, size, vpb, groups, 3, 20, 1, limit)
     assert "gave up 0," not in out and "failures 0" in out, out
+
+
+@pytest.mark.parametrize("kind,size,vpb,groups,eps", [
+    ("tet4", 5, 8, 2, 0.05), ("tet4", 5, 8, 9, 0.01), ("tri1", 3, 4, 3, 0.05), ("tri1", 3, 8, 7, 0.01)])
+def test_small_falls_of_halo_vertices_are_evaluated(visit_model, kind, size, vpb, groups, eps):
+    out = _run(visit_model, kind, size, vpb, groups, 2, 10, 3, 0, eps)
+    assert "unfinished 0, failures 0" in out, out
