@@ -932,9 +932,16 @@ static VisitKernel visit_kernel(const DeviceState* d, int32_t stage_records) {
 // Workgroups of the single-solve persistent kernel: one per block while they all fit, so that every
 // block stays resident with its owner, else all that fit (64^3 cube, 4,292 blocks: 1.29 ms at 256,
 // 0.81 at 512, 0.66 at 768, 0.63 at 1,024; level-8 icosphere, 10,240 blocks of 512 threads: 2.10 at 256,
-// 1.73 at 384, 1.57 at 512).  Triangle meshes
-// whose blocks take 256 threads stop at three per CU: beyond that, waiting workgroups only add traffic.
-static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t nblocks, int* out) {
+// 1.73 at 384, 1.57 at 512).  Where a triangle mesh has more blocks than fit and they take 256 threads, of
+// which a CU holds more than are of use, the grid is sized to the fronts, which are curves: six workgroups
+// per block of a front of sqrt(blocks x sources) blocks, one to three per CU.  Beyond that, workgroups visit
+// blocks whose suppliers are still changing, and poll (in registers, 768 workgroups / this rule: level-5
+// icosphere at 8 vertices per block 0.56 / 0.27 ms, level 6 at 32 0.60 / 0.34, level 7 at 32 0.79 / 0.73,
+// level 8 at 32 1.69 / 1.69; general kernel, records from memory, level 7 with 4 sources at 128 1.93 / 1.65,
+// level 7 at 200 1.50 / 1.18).  The other triangle shapes, two to a CU, take all that fit (level 7 with one
+// source at 303 / 512: 0.72 / 0.68).
+static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t nblocks, int64_t nseeds,
+                           int* out) {
   int dev = 0, ncu = 0, per_cu = 0;
   HIP_TRY(hipGetDevice(&dev));
   HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -945,7 +952,11 @@ static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t
     *out = std::min(requested, resident);
     return EIK_OK;
   }
-  const int most = dim == 2 ? std::min(resident, 3 * ncu) : resident;
+  int most = dim == 2 ? std::min(resident, 3 * ncu) : resident;
+  if (dim == 2 && k.threads == kBlockThreads && nblocks > most) {
+    const double front = 6.0 * std::sqrt((double)nblocks * (double)std::max<int64_t>(nseeds, 1));
+    most = (int)std::min<double>(most, std::max<double>(ncu, front));
+  }
   *out = (int)std::min<int64_t>(most, std::max<int64_t>(nblocks, 1));
   return EIK_OK;
 }
@@ -1000,7 +1011,7 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   const DeviceState* d = m.dev;
   const VisitKernel k = visit_kernel(d, o.stage_records);
   int grid = 0;
-  int rc = persistent_grid(m.dim, k, o.workgroups, d->nblocks, &grid);
+  int rc = persistent_grid(m.dim, k, o.workgroups, d->nblocks, nseeds, &grid);
   if (rc) return rc;
   SolveArgs a;
   a.v.blocks = d->blocks;
@@ -1351,7 +1362,7 @@ int eik_solve_noalloc(eik_mesh_t h, const int32_t* seeds_dev, int64_t nseeds, fl
   eik_solve_opts_t o;
   eik_solve_opts_default(&o);
   int grid = 0;
-  int rc = persistent_grid(m->dim, visit_kernel(d, o.stage_records), o.workgroups, d->nblocks, &grid);
+  int rc = persistent_grid(m->dim, visit_kernel(d, o.stage_records), o.workgroups, d->nblocks, nseeds, &grid);
   if (rc) return rc;
   Sched words;
   sched_shape(words, d->nblocks, grid);
