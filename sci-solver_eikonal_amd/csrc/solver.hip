@@ -912,12 +912,12 @@ struct VisitKernel {
   bool stage;  // k_visit_general: records staged in LDS
 };
 
-// Register-resident visits where the blocks fit them, unless the records are to be read from
-// memory; else the general kernel, its records staged in LDS where they fit.
+// Register-resident visits where the blocks fit them, unless the caller asks for staged records or for
+// records read from memory; else the general kernel, its records staged in LDS where they fit.
 static VisitKernel visit_kernel(const DeviceState* d, int32_t stage_records) {
   VisitKernel k;
   k.stage = d->rec_lds && stage_records != EIK_STAGE_MEMORY;
-  if (d->res_n && stage_records != EIK_STAGE_MEMORY) {
+  if (d->res_n && stage_records == EIK_STAGE_AUTO) {
     k.threads = d->res_bt;
     k.lds = d->res_lds;
     k.fn = resident_kernels(d).loop;
