@@ -591,7 +591,7 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
     x.solves = L.dsolves;
     x.loop.s.word = g.words;
     x.loop.s.ctl = reinterpret_cast<unsigned long long*>(g.sctl);
-    x.loop.s.done = reinterpret_cast<unsigned long long*>(g.sctl + kSchedCtlBytes / 2);
+    x.loop.s.done = reinterpret_cast<uint32_t*>(g.sctl + kSchedCtlBytes / 2);
     // a merged launch's even workgroups own the tet blocks, its odd ones the triangle blocks
     sched_shape(x.loop.s, std::max<int64_t>(kblocks[gi], 1),
                 L.merged ? std::max(1, (g.grid + 1 - gi) / 2) : g.grid);

@@ -32,7 +32,8 @@ constexpr size_t kSchedCtlBytes = 512;  // ctl, and done in a line of its own
 struct Sched {
   unsigned long long* word;  // per slot
   unsigned long long* ctl;   // (times busy) << 32 | busy workgroups
-  unsigned long long* done;  // 1 in the low half: the solve has ended; high half: workgroups that gave up
+  uint32_t* done;            // 1: the solve has ended; then, in one word of 64 bits with it, the workgroups
+                             // that gave up, and in the next word the stretches taken (write_times)
   uint32_t owners;           // G: workgroups of the launch
   uint32_t per_owner;        // words per owner
   uint32_t stride;           // slots from one owner's words to the next's
@@ -91,9 +92,7 @@ struct Finder {
   uint64_t waits = 0; // those of the last look that were dirty (one block per owner)
 };
 
-// No block: the solve has ended; nothing now; this workgroup gave up its wait; the solve has ended, and
-// workgroups had given up before; all workgroups gave up, this one last.
-constexpr int32_t kNoWork = -1, kNothing = -2, kGaveUp = -3, kNoWorkFew = -4, kGaveUpLast = -5;
+constexpr int32_t kNoWork = -1, kNothing = -2, kGaveUp = -3;
 
 // Smallest value over the lanes of a wave (uniform).
 __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
@@ -147,13 +146,13 @@ __device__ __forceinline__ bool sched_claim(const Sched& s, Finder& f, uint32_t 
   return __builtin_amdgcn_readfirstlane(got) != 0u;
 }
 
-// One look: a block for this workgroup, claimed; kNoWork or kNoWorkFew at the end of the solve; kNothing
-// if there is none now.  Called by one whole wave.
+// One look: a block for this workgroup, claimed; kNoWork at the end of the solve; kNothing if there is
+// none now.  Called by one whole wave.
 __device__ __forceinline__ int32_t sched_look(const Sched& s, Finder& f) {
   const uint32_t lane = __lane_id();
   const uint32_t own = f.me * s.stride;
   const uint32_t total = s.owners * s.stride;
-  const unsigned long long dn = load_word(s.done);
+  const uint32_t dn = __hip_atomic_load(s.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   uint32_t key = kClean, at = 0;
   for (uint32_t base = lane; base < s.per_owner && f.me < s.owners; base += 64) {
     const unsigned long long v = load_word(&s.word[own + base]);
@@ -183,28 +182,15 @@ __device__ __forceinline__ int32_t sched_look(const Sched& s, Finder& f) {
   }
   const uint32_t best = wave_umin(key);
   // (done is not set while a workgroup is busy; one that is never leaves without lowering ctl)
-  if (best == kClean) {
-    if (f.busy || __builtin_amdgcn_readfirstlane((uint32_t)dn) == 0u) return kNothing;
-    return __builtin_amdgcn_readfirstlane((uint32_t)(dn >> 32)) ? kNoWorkFew : kNoWork;
-  }
+  if (best == kClean) return !f.busy && __builtin_amdgcn_readfirstlane(dn) ? kNoWork : kNothing;
   const int l = __ffsll((unsigned long long)__ballot(key == best)) - 1;
   f.others = __popcll(__ballot(key != kClean)) - 1;
   const uint32_t slot = (uint32_t)__builtin_amdgcn_readlane((int)at, l);
   return sched_claim(s, f, slot, best) ? sched_block(s, slot) : kNothing;
 }
 
-// A workgroup whose wait has outlasted the limit leaves, counted, unless the solve has ended meanwhile.
-// Whoever finds the end after that finds the count with it: it was added before done was set.
-__device__ __forceinline__ int32_t sched_give_up(const Sched& s) {
-  unsigned long long old = 0;
-  if (__lane_id() == 0)
-    old = __hip_atomic_fetch_add(s.done, 1ull << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (__builtin_amdgcn_readfirstlane((uint32_t)old)) return kNoWorkFew;
-  return __builtin_amdgcn_readfirstlane((uint32_t)(old >> 32)) + 1u == s.owners ? kGaveUpLast : kGaveUp;
-}
-
-// The next block for this workgroup, claimed; kNoWork or kNoWorkFew at the end of the solve; kGaveUp or
-// kGaveUpLast when the wait outlasted s.wait_limit.  Called by one whole wave, when every mark and release of the
+// The next block for this workgroup, claimed; kNoWork at the end of the solve; kGaveUp when the
+// wait outlasted s.wait_limit.  Called by one whole wave, when every mark and release of the
 // workgroup's visits has landed.
 __device__ __forceinline__ int32_t sched_find(const Sched& s, Finder& f) {
   unsigned long long since = 0;
@@ -219,13 +205,12 @@ __device__ __forceinline__ int32_t sched_find(const Sched& s, Finder& f) {
       const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)old);
       if (lo == 1u && sched_all_clean(s) && __lane_id() == 0 &&
           __hip_atomic_load(s.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == old - 1ull)
-        __hip_atomic_store(reinterpret_cast<uint32_t*>(s.done), 1u, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(s.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       since = wall_clock64();
       continue;
     }
     if (since == 0) since = wall_clock64();
-    else if (wall_clock64() - since > s.wait_limit) return sched_give_up(s);
+    else if (wall_clock64() - since > s.wait_limit) return kGaveUp;
     __builtin_amdgcn_s_sleep(1);
   }
 }

@@ -1032,7 +1032,7 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   a.v.dep_start = d->dep_start;
   a.s.word = b.words;
   a.s.ctl = reinterpret_cast<unsigned long long*>(b.sctl);
-  a.s.done = reinterpret_cast<unsigned long long*>(b.sctl + kSchedCtlBytes / 2);
+  a.s.done = reinterpret_cast<uint32_t*>(b.sctl + kSchedCtlBytes / 2);
   sched_shape(a.s, d->nblocks, grid);
   a.s.wait_limit = wait_limit_ticks(d->device, o.wait_limit_us);
   a.items = {d->item_range, d->item_id, d->item_len, d->item_rec};

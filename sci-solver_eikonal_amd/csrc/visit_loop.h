@@ -93,34 +93,48 @@ __device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned
   const int32_t b = look ? sched_look(s, f) : sched_find(s, f);
   if (__lane_id() == 0) {
     acc[6] += wall_clock64() - w0;
-    if (b == kGaveUp || b == kGaveUpLast) acc[kCntAbandoned] += 1;
+    if (b == kGaveUp) acc[kCntAbandoned] += 1;
   }
   return b;
 }
 
-// Writes a solve's times in caller order, when a workgroup of the launch found no further block (end).  At
-// the end of the solve (every visit has ended and every published time has landed) each workgroup writes a
-// stripe of them.  Where workgroups gave up before, their stripes would be missing: the ones that found the
-// end, or the last to give up (whose times are not final), write stretches that they take from a counter
-// until none is left.
+// Writes a solve's times in caller order, when a workgroup has found no further block (end).  At the end of
+// the solve (every visit has ended and every published time has landed) each workgroup writes a stripe of
+// them.  Where workgroups have given up, their stripes would be missing: the ones that find the end, or
+// the last to give up (then the times are not final), write stretches that they take from a counter until
+// none is left.  A workgroup that gives up counts itself in the word that says that the solve has ended:
+// either it finds the end there, or whoever finds the end later finds the count.  (Counted and looked at
+// here, not where blocks are found: there it cost every look registers, level-8 icosphere 1.64 -> 1.71 ms.)
 constexpr int64_t kOutStretch = 8192;
 __device__ __forceinline__ void write_times(const Sched& s, int end, const float* T, const int32_t* iperm,
-                                            int64_t nv, float* out, int* next) {
-  if (!out || end == kGaveUp) return;
-  if (end == kNoWork) {
+                                            int64_t nv, float* out, int* shared) {
+  if (!out) return;
+  enum { kStripe, kStretches, kNothingToWrite };
+  __syncthreads();  // (the shared word has been read)
+  if (threadIdx.x == 0) {
+    unsigned long long* word = reinterpret_cast<unsigned long long*>(s.done);
+    if (end == kNoWork) {
+      *shared = load_word(word) >> 32 ? kStretches : kStripe;
+    } else {
+      const unsigned long long old =
+          __hip_atomic_fetch_add(word, 1ull << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *shared = (uint32_t)old || (uint32_t)(old >> 32) + 1u == s.owners ? kStretches : kNothingToWrite;
+    }
+  }
+  __syncthreads();
+  const int what = __builtin_amdgcn_readfirstlane(*shared);
+  if (what == kStripe) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += stride)
       out[i] = load_T<true>(T + iperm[i]);
-    return;
   }
-  uint32_t* taken = reinterpret_cast<uint32_t*>(s.done + 1);
-  for (;;) {
+  while (what == kStretches) {
     __syncthreads();
     if (threadIdx.x == 0)
-      *next = (int)(uint32_t)__hip_atomic_fetch_add(taken, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *shared = (int)(uint32_t)__hip_atomic_fetch_add(s.done + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    const int64_t from = (int64_t)(uint32_t)*next * kOutStretch;
-    if (from >= nv) return;
+    const int64_t from = (int64_t)*shared * kOutStretch;
+    if (from >= nv) break;
     const int64_t to = from + kOutStretch < nv ? from + kOutStretch : nv;
     for (int64_t i = from + threadIdx.x; i < to; i += blockDim.x) out[i] = load_T<true>(T + iperm[i]);
   }
@@ -142,8 +156,8 @@ __device__ __forceinline__ void write_times(const Sched& s, int end, const float
 // 0.63 ms, 96^3 with 16 sources 3.67 -> 1.41, 33^3 tensor 0.448 -> 0.267, 16^3 0.285 -> 0.135; level-8
 // icosphere 3.29 -> 1.51, level-7 anisotropic 1.02 -> 0.48, level 5 0.328 -> 0.118, 32^2 square 0.158 ->
 // 0.057.
-// blocks(g) gives the data of launch-wide block g; me is the workgroup's owner index.  Returns why there
-// is no further block (block_sched.h).  The workgroup's tally is added to sh.acc, which the caller has cleared (behind a
+// blocks(g) gives the data of launch-wide block g; me is the workgroup's owner index.  Returns kNoWork
+// or kGaveUp.  The workgroup's tally is added to sh.acc, which the caller has cleared (behind a
 // barrier) and flushes.
 template <int DIM, int N, int BT, bool CAP, class Blocks>
 __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& blocks, uint32_t me,
@@ -360,10 +374,10 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       }
       if (!again) {
         // what this visit evaluated the block's elements with: every time, but for the owned
-        // vertices that fell in the last sweep of a visit cut off by the sweep cap (or one that ended
-        // with falls within eps).  A later visit that misses these (they are plain stores) evaluates
-        // more than it has to.  After a full queue, nothing counts as evaluated.
-        if (tid < d.nown) seen[tid] = full ? EIK_INF : conv && eps == 0.f ? own : own_seen;
+        // vertices that fell in the last sweep of a visit cut off by the sweep cap (triangles: or of one
+        // that ended with falls within eps).  A later visit that misses these (they are plain stores)
+        // evaluates more than it has to.  After a full queue, nothing counts as evaluated.
+        if (tid < d.nown) seen[tid] = full ? EIK_INF : conv && (DIM == 3 || eps == 0.f) ? own : own_seen;
         for (int i = tid; i < d.nhalo; i += BT) seen[d.nown + i] = full ? EIK_INF : sT[d.nown + i];
       }
       __syncthreads();

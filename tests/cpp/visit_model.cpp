@@ -196,8 +196,8 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
     bool ended = false;
     const int before = gave_up;
     for (Group& g : gs) {
-      ended = ended || g.end == kNoWork || g.end == kNoWorkFew;
-      gave_up += g.end == kGaveUp || g.end == kGaveUpLast;
+      ended = ended || g.end == kNoWork;
+      gave_up += g.end == kGaveUp;
       visits += (long long)g.sh.acc[0];
     }
     const int given = gave_up - before;
