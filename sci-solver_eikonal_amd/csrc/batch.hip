@@ -198,7 +198,7 @@ struct MultiBlocks {
   __device__ __forceinline__ BlockData operator()(int32_t g) const {
     const SolveDesc& s = solves[bsolve[g]];
     return {s.blocks, s.elems, s.halo,  s.T,     s.seen,      s.vmask,
-            s.dep_start, s.dep, s.rmult, s.items, g - s.kbase, s.kbase};
+            s.dep_start, s.dep, s.rmult, s.height_unit, s.items, g - s.kbase, s.kbase};
   }
 };
 
@@ -516,6 +516,7 @@ void solve_desc(SolveDesc& s, Mesh* m, float* T, float* seen, const float* rmult
   s.seen = seen;
   s.nv = m->nv;
   s.items = {d->item_range, d->item_id, d->item_len, d->item_rec};
+  s.height_unit = d->height_unit;
   s.nseen = d->nseen;
   s.nblocks = d->nblocks;
   s.dim = m->dim;

@@ -88,6 +88,7 @@ struct DeviceState {
   int32_t max_queue = 0;
   bool res_cap = false;  // the work-item queue holds fewer pairs than a block has
   int32_t max_local = 0, max_elem = 0;
+  float height_unit = 1.f;
   size_t res_lds = 0;
   int2* item_range = nullptr;
   uint32_t* item_id = nullptr;

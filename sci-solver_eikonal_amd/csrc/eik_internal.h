@@ -76,6 +76,7 @@ struct Layout {
   // virtual face only the obtuse one)
   std::vector<int32_t> items;
   int32_t max_items = 0;
+  float height_unit = 1.f;  // of the tets' largest height (height_unit)
   int64_t total_elems = 0;
   bool valid = false;
 };
@@ -110,6 +111,12 @@ struct Mesh {
 // 2.11 ms vs 2.55 ms at 2; the front needs more sweeps to cross an 8 x 8 block).
 inline int32_t default_inner_sweeps(int dim, int32_t requested) {
   return requested > 0 ? requested : (dim == 3 ? 2 : 4);
+}
+
+// The power of two 2^(x - 15): the unit in which a height m 2^x, 1/2 <= m < 1, is 2^14 to 2^15.  (Its
+// reciprocal is finite: x is kept in range.)
+inline constexpr float height_unit(int x) {
+  return __builtin_bit_cast(float, (uint32_t)(127 - 15 + (x < -110 ? -110 : x)) << 23);
 }
 
 // errors ----------------------------------------------------------------------------------

@@ -19,20 +19,9 @@ __device__ __forceinline__ void wait_memory() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// Two non-negative values as fp16, rounded towards zero; and a sum with one of
-// them, in one instruction.
+// Two non-negative values as fp16, rounded towards zero.
 __device__ __forceinline__ uint32_t half_pair(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-}
-__device__ __forceinline__ float add_half_lo(float x, uint32_t p) {
-  float y;
-  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(x), "v"(p));
-  return y;
-}
-__device__ __forceinline__ float add_half_hi(float x, uint32_t p) {
-  float y;
-  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(x), "v"(p));
-  return y;
 }
 
 // Copies 16 bytes per lane from memory straight to LDS (lane i of the wave to base + 16 i), so that

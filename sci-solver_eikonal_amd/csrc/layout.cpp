@@ -208,6 +208,13 @@ int build_layout(Mesh& m) {
       tri_heights(Le, He);
     }
   });
+  if (m.dim == 3) {
+    float most = 0.f;
+    for (float h : eH) most = std::isfinite(h) ? std::max(most, h) : most;
+    int x = 0;
+    (void)std::frexp(most, &x);
+    L.height_unit = height_unit(x);
+  }
   L.blocks.resize(nb);
   if (m.dim == 3) L.tets.resize(total); else L.tris.resize(total);
   L.items.assign(nb, 0);

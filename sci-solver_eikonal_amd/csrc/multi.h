@@ -35,6 +35,7 @@ struct alignas(16) SolveDesc {
   float* seen;
   int64_t nv;
   TriItems items;            // triangles
+  float height_unit;         // tets (BlockData)
   int64_t nseen;
   int64_t out_off;           // first value of this solve in the gathered output
   int32_t bbase;             // first launch-wide block index

@@ -138,6 +138,7 @@ struct SyncArgs {
   int32_t elem_bytes;        // algorithmic bytes per element (visit_algo_bytes)
   TriItems items;            // register-resident visits: triangles, and the LDS (LoopArgs)
   int32_t max_local, max_elem, max_queue;
+  float height_unit;
 };
 constexpr int kSnapBlocks = 16;  // blocks whose times a workgroup copies to the history
 
@@ -282,7 +283,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   }
   std::conditional_t<DIM == 2, TriRegs<N>, TetRegs<N>> r;
   if constexpr (DIM == 2) tri_load<N, BT>(r, a.items, a.items.range[b], nullptr);
-  else tet_load<N, BT>(r, a.v.elems, d, sA, sB, nullptr);
+  else tet_load<N, BT>(r, a.v.elems, d, sA, sB, a.height_unit, nullptr);
   wait_memory();  // the copies to LDS too
   __syncthreads();
   if constexpr (DIM == 2) tri_seen<N>(r, sP);
@@ -360,6 +361,7 @@ struct SolveArgs {
   int32_t max_local;   // LDS strides: local vertices and elements of the largest block
   int32_t max_elem;
   int32_t max_queue;
+  float height_unit;     // tets (BlockData)
   size_t rec_lds_bytes;  // k_visit_general: staged records
 };
 
@@ -390,7 +392,7 @@ struct SingleBlocks {
   const SolveArgs& a;
   __device__ __forceinline__ BlockData operator()(int32_t b) const {
     return {a.v.blocks, a.v.elems, a.v.halo, a.v.T,   a.v.seen, a.v.vmask,
-            a.dep_start, a.dep,    nullptr,  a.items, b,        0};
+            a.dep_start, a.dep,    nullptr,  a.height_unit, a.items, b, 0};
   }
 };
 
@@ -739,6 +741,7 @@ static int setup_resident(Mesh& m, size_t max_lds) {
   const Layout& L = m.layout;
   d->max_local = L.max_local;
   d->max_elem = L.max_elem;
+  d->height_unit = L.height_unit;
   d->res_n = 0;
   if (L.vmask.empty()) return EIK_OK;
   int dev = 0, ncu = 0;
@@ -859,6 +862,7 @@ static int solve_sync(Mesh& m, const eik_solve_opts_t& o) {
   a.max_local = d->max_local;
   a.max_elem = d->max_elem;
   a.max_queue = d->max_queue;
+  a.height_unit = d->height_unit;
   a.nb = nb;
   // values only decrease, so the loop ends; the cap bounds it on pathological inputs
   const int64_t cap = o.max_iterations > 0 ? o.max_iterations : 1000000;
@@ -1052,6 +1056,7 @@ static int enqueue_async(const Mesh& m, const eik_solve_opts_t& o, const AsyncBu
   a.max_local = d->max_local;
   a.max_queue = d->max_queue;
   a.max_elem = d->max_elem;
+  a.height_unit = d->height_unit;
   a.rec_lds_bytes = k.stage ? d->rec_lds_bytes : 0;
   FillSegs f;
   f.add(b.T, m.nv, (int32_t)__builtin_bit_cast(uint32_t, a.v.large));

@@ -26,6 +26,7 @@ struct BlockData {
   const int32_t* dep_start;
   const int32_t* dep;
   const float* rmult;  // a factor per record on the squared lengths, or null
+  float unit;          // tets: of the heights (Layout::height_unit)
   TriItems items;      // triangles
   int32_t b;           // the block within its mesh
   int32_t base;        // launch-wide index of its mesh's first block
@@ -232,7 +233,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
     if constexpr (DIM == 2)
       tri_load<N, BT>(r, m.items, m.items.range[m.b], rmult);
     else
-      tet_load<N, BT>(r, m.elems, d, sA, sB, rmult);
+      tet_load<N, BT>(r, m.elems, d, sA, sB, m.unit, rmult);
     wait_memory();  // the copies to LDS too
     __syncthreads();
     if constexpr (DIM == 2) tri_seen<N>(r, sP);

@@ -64,6 +64,12 @@ inline int __ffs(unsigned v) { return __builtin_ffs((int)v); }
 inline int __ffsll(unsigned long long v) { return __builtin_ffsll((long long)v); }
 #define __builtin_amdgcn_sqrtf(x) std::sqrt((float)(x))
 #define __builtin_amdgcn_rcpf(x) (1.f / (float)(x))
+inline int simt_frexp_exp(float x) {
+  int e = 0;
+  if (x != 0.f && std::isfinite(x)) (void)std::frexp(x, &e);
+  return e;
+}
+#define __builtin_amdgcn_frexp_expf(x) simt_frexp_exp(x)
 
 // ------------------------------------------------------------------------------------------
 // fibers, waves, workgroups

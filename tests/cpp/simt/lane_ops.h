@@ -20,16 +20,7 @@ inline uint32_t half_down(float x) {
   __builtin_memcpy(&u, &h, 2);
   return u;
 }
-inline float half_up(uint32_t u) {
-  const uint16_t v = (uint16_t)u;
-  _Float16 h;
-  __builtin_memcpy(&h, &v, 2);
-  return (float)h;
-}
 inline uint32_t half_pair(float a, float b) { return half_down(a) | half_down(b) << 16; }
-inline float add_half_lo(float x, uint32_t p) { return x + half_up(p & 0xffffu); }
-inline float add_half_hi(float x, uint32_t p) { return x + half_up(p >> 16); }
-
 inline void copy_to_lds(const uint4* from, uint4* wave_base) { wave_base[simt::me().lane] = *from; }
 inline int lds_take(int* counter, int n) { return atomicAdd(counter, n); }
 inline void lds_min(unsigned* p, unsigned v) { atomicMin(p, v); }

@@ -87,6 +87,7 @@ struct ModelBlocks {
     d.dep_start = L.dep_start.data();
     d.dep = L.dep.data();
     d.rmult = nullptr;
+    d.unit = L.height_unit;
     d.items = {s.items.range.data(), s.items.id.data(), s.items.len.data(), s.items.rec.data()};
     d.b = b;
     d.base = 0;
