@@ -16,6 +16,7 @@
 #pragma once
 
 #include <hip/hip_runtime_api.h>
+#include <setjmp.h>
 #include <ucontext.h>
 
 #include <algorithm>
@@ -82,7 +83,9 @@ enum State { kReady, kWaveOp, kWait, kBarrier, kEnded };
 
 struct Wave;
 struct Thread {
-  ucontext_t ctx;
+  ucontext_t ctx;  // its first entry; later switches are jumps
+  jmp_buf at;
+  bool entered = false;
   std::unique_ptr<char[]> stack;
   State state = kReady;
   Dim tid, bid;
@@ -108,7 +111,7 @@ struct Group {
 };
 
 inline Thread* g_me = nullptr;
-inline ucontext_t g_main;
+inline jmp_buf g_main;
 inline unsigned long long g_clock = 0;
 inline std::mt19937_64 g_rng;
 inline Dim g_grid, g_block;
@@ -118,9 +121,14 @@ inline const char* g_error = nullptr;
 
 inline Thread& me() { return *g_me; }
 inline void to_scheduler() {
-  Thread* t = g_me;
-  swapcontext(&t->ctx, &g_main);
+  if (_setjmp(g_me->at) == 0) _longjmp(g_main, 1);
+}
+__attribute__((noinline)) inline void resume(Thread* t) {
   g_me = t;
+  if (_setjmp(g_main) != 0) return;
+  if (t->entered) _longjmp(t->at, 1);
+  t->entered = true;
+  setcontext(&t->ctx);
 }
 inline void yield() { to_scheduler(); }
 inline void entry() {
@@ -268,10 +276,7 @@ inline const char* run(unsigned groups, unsigned threads, uint64_t seed,
     if (stuck) return g_error ? g_error : "every thread waits";
     if (!w->pending.empty() && uniform() < 0.2) land(*w, g_rng() % w->pending.size());
     for (Thread* t : w->lanes)
-      if (t->state == kReady) {
-        g_me = t;
-        swapcontext(&g_main, &t->ctx);
-      }
+      if (t->state == kReady) resume(t);
     // the wave's operation, when all of its lanes have come to one
     size_t at_op = 0, at_barrier = 0, at_wait = 0, ended = 0, ready = 0;
     for (Thread* t : w->lanes) {

@@ -7,8 +7,9 @@
 // those of the visits).  The output must be the times in caller order, complete, whether or not
 // workgroups gave up waiting before the end.
 //
-// usage: visit_model <tri N|tet N> <mesh size> <vertices per block> <workgroups> <inner sweeps> <runs>
+// usage: visit_model <triN|tetN|cap4> <mesh size> <vertices per block> <workgroups> <inner sweeps> <runs>
 //                    <seed> <wait limit, steps; 0: none> [eps]
+// cap4: tets, 4 elements per thread, a work-item queue that holds a twentieth of a block's pairs.
 // With eps > 0 a visit ends when a sweep lowers nothing by more than that, and what its last sweep
 // lowered counts as evaluated; a fall of a halo vertex is evaluated, however small: only the corner
 // solves from halo vertices alone are looked at then.
@@ -138,7 +139,7 @@ struct Group {
   int end = 0;
 };
 
-template <int DIM, int N, int BT>
+template <int DIM, int N, int BT, bool CAP = false>
 int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned long long limit, float eps) {
   const Layout& L = m.layout;
   const int need = DIM == 3 ? L.max_elem : L.max_items;
@@ -168,7 +169,7 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
     s.a.max_visits = 1 << 30;
     s.a.max_local = L.max_local;
     s.a.max_elem = L.max_elem;
-    s.a.max_queue = DIM == 3 ? L.max_items : 0;
+    s.a.max_queue = DIM != 3 ? 0 : CAP ? L.max_items / 20 : L.max_items;
     const int nsrc = 1 + (int)(rng() % 3);
     for (int k = 0; k < nsrc; ++k) {
       const int32_t v = L.iperm[rng() % (uint64_t)m.nv], b = L.owner[(size_t)v];
@@ -186,7 +187,7 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
     const ModelBlocks blocks{s};
     const char* err = simt::run((unsigned)groups, BT, seed * 1000003u + (uint64_t)run, [&] {
       Group& g = gs[blockIdx.x];
-      const int end = resident_loop<DIM, N, BT, false>(s.a, blocks, blockIdx.x, g.lds.data(), g.sh);
+      const int end = resident_loop<DIM, N, BT, CAP>(s.a, blocks, blockIdx.x, g.lds.data(), g.sh);
       write_times(s.a.s, end, s.T.data(), L.iperm.data(), m.nv, s.out.data(), &g.sh.block);
       g.end = end;
     });
@@ -237,8 +238,8 @@ int main(int argc, char** argv) {
   const unsigned long long limit = std::strtoull(argv[8], nullptr, 10);
   const float eps = argc == 10 ? (float)std::atof(argv[9]) : 0.f;
   Mesh m;
-  if (kind[3] == ' ' || kind.size() < 4) return 2;
-  const bool tets = kind.substr(0, 3) == "tet";
+  if (kind.size() != 4) return 2;
+  const bool cap = kind == "cap4", tets = cap || kind.substr(0, 3) == "tet";
   if (tets ? gen_kuhn_cube(size, 0.2f, seed, m) : gen_icosphere(size, m)) return 2;
   // uneven speeds, so that times arrive out of order
   std::mt19937_64 rng(seed);
@@ -248,6 +249,7 @@ int main(int argc, char** argv) {
   if (!tets) tri_virtual_faces(m);
   if (partition_by_size(m, vpb) || build_layout(m)) return 2;
   const int n = std::atoi(kind.c_str() + 3);
+  if (cap) return run_solves<3, 4, 256, true>(m, groups, inner, runs, seed, limit, eps);
   if (tets) return n == 2 ? run_solves<3, 2, 512>(m, groups, inner, runs, seed, limit, eps)
                           : run_solves<3, 4, 256>(m, groups, inner, runs, seed, limit, eps);
   return n == 1   ? run_solves<2, 1, 256>(m, groups, inner, runs, seed, limit, eps)

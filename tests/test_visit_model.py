@@ -65,3 +65,10 @@ def test_every_time_is_written_when_workgroups_give_up(visit_model, kind, size, 
 def test_small_falls_of_halo_vertices_are_evaluated(visit_model, kind, size, vpb, groups, eps):
     out = _run(visit_model, kind, size, vpb, groups, 2, 10, 3, 0, eps)
     assert "unfinished 0, failures 0" in out, out
+
+
+@pytest.mark.parametrize("size,vpb,groups,inner", [(5, 20, 2, 2), (5, 40, 1, 3), (5, 20, 11, 1)])
+def test_a_full_queue_loses_nothing(visit_model, size, vpb, groups, inner):
+    """What a sweep cannot queue is selected again, in the next sweep or by the block's next visit."""
+    out = _run(visit_model, "cap4", size, vpb, groups, inner, 12, 9, 0)
+    assert "unfinished 0, failures 0" in out, out
