@@ -217,8 +217,9 @@ inline Result<T, F> atomic(T* p, F f) {
   return Result<T, F>(p, f);
 }
 
-// Runs `groups` workgroups of `threads` (a multiple of 64).  Returns null, or what went wrong.
-inline const char* run(unsigned groups, unsigned threads, uint64_t seed,
+// Runs `groups` workgroups of `threads` (a multiple of 64), at most `resident` at a time: a further one
+// starts when one has ended.  Returns null, or what went wrong.
+inline const char* run(unsigned groups, unsigned threads, uint64_t seed, unsigned resident,
                        const std::function<void()>& body, unsigned long long max_steps = 1ull << 33) {
   g_rng.seed(seed);
   g_clock = 1;
@@ -253,8 +254,13 @@ inline const char* run(unsigned groups, unsigned threads, uint64_t seed,
     }
   auto uniform = [] { return (double)(g_rng() >> 11) * 0x1p-53; };
   size_t left = ws.size();
-  std::vector<Wave*> order;
-  for (auto& w : ws) order.push_back(w.get());
+  std::vector<Wave*> order;  // the waves that run
+  unsigned started = 0;
+  auto start = [&] {
+    for (Wave* w : gs[started].waves) order.push_back(w);
+    ++started;
+  };
+  while (started < std::min(groups, resident)) start();
   while (left > 0) {
     if (++g_clock > max_steps) return "too many steps";
     if (g_clock % 256 == 2)
@@ -309,6 +315,10 @@ inline const char* run(unsigned groups, unsigned threads, uint64_t seed,
           order.erase(order.begin() + (long)i);
           break;
         }
+      bool gone = true;
+      for (Wave* v : gs[(size_t)w->group].waves)
+        for (Thread* t : v->lanes) gone = gone && t->state == kEnded;
+      if (gone && started < groups) start();
     }
     // the workgroup's barrier
     bool all = true, any_ended = false;

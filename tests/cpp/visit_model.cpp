@@ -8,7 +8,7 @@
 // workgroups gave up waiting before the end.
 //
 // usage: visit_model <triN|tetN|cap4> <mesh size> <vertices per block> <workgroups> <inner sweeps> <runs>
-//                    <seed> <wait limit, steps; 0: none> [eps]
+//                    <seed> <wait limit, steps; 0: none> [eps [workgroups that run at a time]]
 // cap4: tets, 4 elements per thread, a work-item queue that holds a twentieth of a block's pairs.
 // With eps > 0 a visit ends when a sweep lowers nothing by more than that, and what its last sweep
 // lowered counts as evaluated; a fall of a halo vertex is evaluated, however small: only the corner
@@ -140,7 +140,8 @@ struct Group {
 };
 
 template <int DIM, int N, int BT, bool CAP = false>
-int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned long long limit, float eps) {
+int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned long long limit, float eps,
+               int resident) {
   const Layout& L = m.layout;
   const int need = DIM == 3 ? L.max_elem : L.max_items;
   if (need > N * BT || L.max_own > BT || L.max_local > kItemSlots || L.vmask.empty()) {
@@ -185,7 +186,7 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
       std::memset(&g.sh, 0, sizeof g.sh);
     }
     const ModelBlocks blocks{s};
-    const char* err = simt::run((unsigned)groups, BT, seed * 1000003u + (uint64_t)run, [&] {
+    const char* err = simt::run((unsigned)groups, BT, seed * 1000003u + (uint64_t)run, (unsigned)resident, [&] {
       Group& g = gs[blockIdx.x];
       const int end = resident_loop<DIM, N, BT, CAP>(s.a, blocks, blockIdx.x, g.lds.data(), g.sh);
       write_times(s.a.s, end, s.T.data(), L.iperm.data(), m.nv, s.out.data(), &g.sh.block);
@@ -230,13 +231,14 @@ int run_solves(Mesh& m, int groups, int inner, int runs, uint64_t seed, unsigned
 }  // namespace
 
 int main(int argc, char** argv) {
-  if (argc != 9 && argc != 10) return 2;
+  if (argc < 9 || argc > 11) return 2;
   const std::string kind = argv[1];
   const int size = std::atoi(argv[2]), vpb = std::atoi(argv[3]), groups = std::atoi(argv[4]);
   const int inner = std::atoi(argv[5]), runs = std::atoi(argv[6]);
   const uint64_t seed = std::strtoull(argv[7], nullptr, 10);
   const unsigned long long limit = std::strtoull(argv[8], nullptr, 10);
-  const float eps = argc == 10 ? (float)std::atof(argv[9]) : 0.f;
+  const float eps = argc > 9 ? (float)std::atof(argv[9]) : 0.f;
+  const int resident = argc > 10 ? std::atoi(argv[10]) : groups;
   Mesh m;
   if (kind.size() != 4) return 2;
   const bool cap = kind == "cap4", tets = cap || kind.substr(0, 3) == "tet";
@@ -249,10 +251,10 @@ int main(int argc, char** argv) {
   if (!tets) tri_virtual_faces(m);
   if (partition_by_size(m, vpb) || build_layout(m)) return 2;
   const int n = std::atoi(kind.c_str() + 3);
-  if (cap) return run_solves<3, 4, 256, true>(m, groups, inner, runs, seed, limit, eps);
-  if (tets) return n == 2 ? run_solves<3, 2, 512>(m, groups, inner, runs, seed, limit, eps)
-                          : run_solves<3, 4, 256>(m, groups, inner, runs, seed, limit, eps);
-  return n == 1   ? run_solves<2, 1, 256>(m, groups, inner, runs, seed, limit, eps)
-         : n == 2 ? run_solves<2, 2, 512>(m, groups, inner, runs, seed, limit, eps)
-                  : run_solves<2, 4, 512>(m, groups, inner, runs, seed, limit, eps);
+  if (cap) return run_solves<3, 4, 256, true>(m, groups, inner, runs, seed, limit, eps, resident);
+  if (tets) return n == 2 ? run_solves<3, 2, 512>(m, groups, inner, runs, seed, limit, eps, resident)
+                          : run_solves<3, 4, 256>(m, groups, inner, runs, seed, limit, eps, resident);
+  return n == 1   ? run_solves<2, 1, 256>(m, groups, inner, runs, seed, limit, eps, resident)
+         : n == 2 ? run_solves<2, 2, 512>(m, groups, inner, runs, seed, limit, eps, resident)
+                  : run_solves<2, 4, 512>(m, groups, inner, runs, seed, limit, eps, resident);
 }

@@ -2,7 +2,8 @@
 resident.h as they are, built for the host with a model of waves, barriers and late atomics
 (tests/cpp/simt), run whole solves on real layouts with the waves interleaved at random
 (tests/cpp/visit_model.cpp).  Every solve must end by itself with no block waiting, and no corner solve
-of any element may then lower a time."""
+of any element may then lower a time.  The scheduler alone (block_sched.h) runs many launches of idle
+workgroups with visits of a few relaxations (tests/cpp/sched_model.cpp)."""
 import glob
 import os
 import shutil
@@ -17,22 +18,29 @@ CSRC = os.path.join(ROOT, "sci-solver_eikonal_amd", "csrc")
 CPP = os.path.join(ROOT, "tests", "cpp")
 
 
-@pytest.fixture(scope="module")
-def visit_model(tmp_path_factory):
+def _build(d, source, *more):
     if not os.path.exists(CLANG):
         pytest.skip("clang++ is not installed")
-    d = tmp_path_factory.mktemp("visit_model")
     # the headers, with the host's definitions of the few operations written as instructions
     for h in glob.glob(os.path.join(CSRC, "*.h")):
         shutil.copy(h, d)
     shutil.copy(os.path.join(CPP, "simt", "lane_ops.h"), d)
-    exe = d / "visit_model"
+    exe = d / "model"
     subprocess.run([CLANG, "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(CPP, "simt"),
                     "-I", str(d), "-I", os.path.join(ROOT, "include"), "-I", "/opt/rocm/include",
-                    os.path.join(CPP, "visit_model.cpp")] +
-                   [os.path.join(CSRC, f) for f in ("mesh.cpp", "partition.cpp", "layout.cpp")] +
+                    os.path.join(CPP, source)] + [os.path.join(CSRC, f) for f in more] +
                    ["-o", str(exe), "-lpthread"], check=True, capture_output=True)
     return str(exe)
+
+
+@pytest.fixture(scope="module")
+def visit_model(tmp_path_factory):
+    return _build(tmp_path_factory.mktemp("visit_model"), "visit_model.cpp", "mesh.cpp", "partition.cpp", "layout.cpp")
+
+
+@pytest.fixture(scope="module")
+def sched_model(tmp_path_factory):
+    return _build(tmp_path_factory.mktemp("sched_model"), "sched_model.cpp")
 
 
 def _run(exe, *args):
@@ -72,3 +80,17 @@ def test_a_full_queue_loses_nothing(visit_model, size, vpb, groups, inner):
     """What a sweep cannot queue is selected again, in the next sweep or by the block's next visit."""
     out = _run(visit_model, "cap4", size, vpb, groups, inner, 12, 9, 0)
     assert "unfinished 0, failures 0" in out, out
+
+
+@pytest.mark.parametrize("kind,size,vpb,groups,resident", [
+    ("tet4", 5, 20, 11, 3), ("tri1", 2, 32, 5, 1), ("tri1", 3, 32, 8, 3), ("tet4", 4, 20, 4, 2)])
+def test_blocks_of_workgroups_that_do_not_run_are_visited(visit_model, kind, size, vpb, groups, resident):
+    """A launch beside others: only some of its workgroups run until the solve has ended."""
+    out = _run(visit_model, kind, size, vpb, groups, 2, 8, 11, 0, 0, resident)
+    assert "unfinished 0, failures 0" in out, out
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_scheduler_ends_every_launch_and_no_earlier(sched_model, seed):
+    out = _run(sched_model, 350, seed)
+    assert "350 launches, failures 0" in out, out
