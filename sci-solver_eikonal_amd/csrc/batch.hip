@@ -629,7 +629,7 @@ int launch_output(Launch& L, int32_t nsolves, int64_t total_nv) {
   return EIK_OK;
 }
 
-int launch_issue(Launch& L, int32_t nsolves, int64_t total_blocks, int64_t total_nv,
+int launch_issue(Launch& L, int32_t nsolves, int64_t /*total_blocks*/, int64_t total_nv,
                  const MultiArgs a[2], bool upload_desc, bool output) {
   hipStream_t s = L.stream;
   const int64_t cap = L.cap_seeds;
@@ -759,16 +759,14 @@ static int batch_alloc(Batch* b, int64_t seed_cap) {
                         seed_cap);
   if (rc) return rc;
   b->seed_cap = b->L.cap_seeds;
-  int64_t so = 0, off = 0, bbase = 0;
+  int64_t so = 0, off = 0;
   for (size_t i = 0; i < b->meshes.size(); ++i) {
     Mesh* m = b->meshes[i];
     SolveDesc& s = b->L.hsolves[i];
     solve_desc(s, m, b->T + off, b->seen + so, b->rmult[i]);
     s.out_off = off;
-    s.bbase = (int32_t)bbase;
     so += s.nseen;
     off += m->nv;
-    bbase += s.nblocks;
   }
   int64_t n[2];
   launch_bases(b->L.hsolves, (int32_t)b->meshes.size(), n);

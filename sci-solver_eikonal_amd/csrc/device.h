@@ -1,5 +1,5 @@
 // device.h -- device state and the device-side pieces shared by the solve translation units:
-// the per-mesh device state, the persistent work queue, LDS carving and visit tallies.
+// the per-mesh device state, the per-solve resets, LDS carving and visit tallies.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -38,8 +38,7 @@ struct alignas(16) SolveDesc {
   float height_unit;         // tets (BlockData)
   int64_t nseen;
   int64_t out_off;           // first value of this solve in the gathered output
-  int32_t bbase;             // first launch-wide block index
-  int32_t kbase;             // ... among the blocks of its element kind (launch_args)
+  int32_t kbase;             // its first block among those of its element kind (launch_args)
   int32_t nblocks;
   int32_t dim;
   float large;
@@ -107,7 +106,7 @@ int partition_parallel(const std::vector<Mesh*>& ms, int32_t vpb);
 int launch_alloc(Launch& L, const std::vector<Mesh*>& kinds, int32_t cap_solves,
                  int64_t cap_blocks, int64_t cap_nv, int64_t cap_seeds);
 void launch_free(Launch& L);
-// Fills the descriptor of a solve of mesh m with the given arrays (out_off, bbase by caller).
+// Fills the descriptor of a solve of mesh m with the given arrays (out_off by caller).
 void solve_desc(SolveDesc& s, Mesh* m, float* T, float* seen, const float* rmult);
 // Per-record factors of mesh m (rmult, layout.total_elems values) from per-element factors
 // (mult, device), on stream s.

@@ -95,7 +95,7 @@ static void server_free(Server* s) {
 static int start_launch(Server* s, int k, std::vector<Request*>& rs) {
   Launch& L = s->L[k];
   Slots& z = s->slots[k];
-  int64_t off = 0, bbase = 0, nseeds = 0;
+  int64_t off = 0, nblocks = 0, nseeds = 0;
   const int64_t cap = L.cap_seeds;
   for (size_t j = 0; j < rs.size(); ++j) {
     Request* r = rs[j];
@@ -110,9 +110,8 @@ static int start_launch(Server* s, int k, std::vector<Request*>& rs) {
     SolveDesc& d = L.hsolves[j];
     solve_desc(d, m, z.T + (int64_t)j * s->max_nv, z.seen + (int64_t)j * s->max_nseen, rmult);
     d.out_off = off;
-    d.bbase = (int32_t)bbase;
     off += m->nv;
-    bbase += d.nblocks;
+    nblocks += d.nblocks;
     for (int32_t v : r->seeds) {
       L.h_seed[nseeds] = (int32_t)j;
       L.h_seed[cap + nseeds] = v;
@@ -126,10 +125,10 @@ static int start_launch(Server* s, int k, std::vector<Request*>& rs) {
   eik_solve_opts_default(&o);
   o.max_inner = s->opts.max_inner;
   MultiArgs a[2];
-  int rc = launch_args(L, (int32_t)rs.size(), bbase, o, a);
+  int rc = launch_args(L, (int32_t)rs.size(), nblocks, o, a);
   if (rc) return rc;
   HIP_TRY(hipEventRecord(L.ev0, L.stream));
-  rc = launch_issue(L, (int32_t)rs.size(), bbase, off, a, true);
+  rc = launch_issue(L, (int32_t)rs.size(), nblocks, off, a, true);
   if (rc) return rc;
   HIP_TRY(hipEventRecord(L.ev1, L.stream));
   return EIK_OK;
