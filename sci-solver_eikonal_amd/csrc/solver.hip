@@ -460,8 +460,9 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
     const int ndep = a.dep_start[b + 1] - s0;
     bool rerun = false;  // the previous visit of this workgroup was of block b, and this one's
                          // times are in LDS already (rerun_load)
-    // few blocks wait: one sweep of a tet block per visit (see kCrowd; larger here, where a load costs
-    // less beside the sweeps)
+    // few blocks wait: one sweep of a tet block per visit (see kCrowd; 1 / 3 / 8 times as many here, records
+    // from memory: 64^3 cube 1.04 / 1.04 / 1.05 ms, at 192 vertices per block 1.32 / 1.29 / 1.32, 96^3 with 16
+    // sources 2.95 / 3.01 / 3.30)
     const int inner = DIM == 3 && sCrowd < 3 * kCrowd ? 1 : 0;
     for (;;) {
       if (tid == 0) {
@@ -965,10 +966,10 @@ static int persistent_grid(int dim, const VisitKernel& k, int requested, int64_t
   return EIK_OK;
 }
 
-// Inner sweeps per visit of the single-solve persistent kernel when the caller leaves the
-// choice: triangle blocks, visited by the smaller grid above, measured best at 3 (icosphere
-// with 4 sources at 256 workgroups: 1.24 vs 1.30 ms at 4); other schedulers and launches keep
-// default_inner_sweeps.
+// Inner sweeps per visit of the single-solve persistent kernel when the caller leaves the choice: 3 for
+// triangles (visits at 2 / 3 / 4 / 5 sweeps, in registers: level-5 icosphere 176 / 167 / 170 / 172 us, level 7
+// with 4 sources 476 / 467 / 483 / 503, level 8 1,719 / 1,719 / 1,742 / 1,782; general kernel, level 7 1,063 /
+// 1,034 / 1,036 / 1,106); other schedulers and launches keep default_inner_sweeps.
 static int32_t async_inner_sweeps(int dim, int32_t requested) {
   return requested > 0 ? requested : (dim == 2 ? 3 : default_inner_sweeps(dim, 0));
 }
