@@ -111,7 +111,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     if (sBlock == kNothing) {
       __syncthreads();
       if (finder) {
-        const int32_t nb = find_next(s, f, sAcc);
+        const int32_t nb = find_next<true>(s, f, sAcc);
         if (tid == 64) sBlock = nb;
       }
       __syncthreads();
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         sAcc[10] += wall_clock64() - tq;
       }
     } else if (finder) {
-      const int32_t nb = find_next(s, f, sAcc, true);
+      const int32_t nb = find_next<true>(s, f, sAcc, true);
       if (tid == 64) sBlock = nb;
     }
     // The wait is written out: hipcc 7.2 leaves it away before a barrier that heads this loop, and a

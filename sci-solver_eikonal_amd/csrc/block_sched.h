@@ -88,7 +88,7 @@ struct Finder {
   uint32_t me;        // the workgroup's owner index; s.owners or more: it owns no blocks
   uint32_t probe;     // next slot to look at among all
   int others = 0;     // dirty blocks seen beside the one claimed
-  uint32_t idle = 0;  // looks so far (one block per owner)
+  uint32_t idle = 0;  // looks so far that may have gone without a window of all words
   uint64_t waits = 0; // those of the last look that were dirty (one block per owner)
 };
 
@@ -148,6 +148,14 @@ __device__ __forceinline__ bool sched_claim(const Sched& s, Finder& f, uint32_t 
 
 // One look: a block for this workgroup, claimed; kNoWork at the end of the solve; kNothing if there is
 // none now.  Called by one whole wave.
+// THIN: an idle workgroup looks at others' words at every 32nd look only, and sleeps between looks.  For the
+// general kernels of multi-solve launches, of whose small workgroups up to 16 fit a CU: with a few blocks
+// per owner, hundreds of idle ones read all words all the time, and every visit waited for that traffic
+// (24 level-6 icospheres at 500 vertices per block, 1,944 blocks, records from memory: 5.36 ms looking at a
+// window every time, 2.89 every 8th, 2.38 every 32nd with the sleep; 4 at 64, 2,560 blocks: 3.85 / 2.00 / 1.25).
+// The register-resident kernels, with fewer and larger workgroups, look every time (12 level-6 icospheres at
+// 64 vertices per block 0.81 ms, every 32nd 0.89).
+template <bool THIN = false>
 __device__ __forceinline__ int32_t sched_look(const Sched& s, Finder& f) {
   const uint32_t lane = __lane_id();
   const uint32_t own = f.me * s.stride;
@@ -162,7 +170,7 @@ __device__ __forceinline__ int32_t sched_look(const Sched& s, Finder& f) {
   // is near the smallest of the launch, and an idle workgroup finds what a busy owner leaves.
   // With one block per owner its owner visits it, resident; now and then a window is looked at
   // for blocks that stay dirty because their owner is not running (yet).
-  if (s.per_owner > 1 || (++f.idle & 63u) == 0u) {
+  if (s.per_owner > 1 ? !THIN || f.busy || (++f.idle & 31u) == 0u : (++f.idle & 63u) == 0u) {
     const uint32_t i = f.probe + lane;
     const unsigned long long v = i < total ? load_word(&s.word[i]) : (unsigned long long)kClean;
     bool take = (v >> 32) == 0ull;
@@ -192,10 +200,11 @@ __device__ __forceinline__ int32_t sched_look(const Sched& s, Finder& f) {
 // The next block for this workgroup, claimed; kNoWork at the end of the solve; kGaveUp when the
 // wait outlasted s.wait_limit.  Called by one whole wave, when every mark and release of the
 // workgroup's visits has landed.
+template <bool THIN = false>
 __device__ __forceinline__ int32_t sched_find(const Sched& s, Finder& f) {
   unsigned long long since = 0;
   for (;;) {
-    const int32_t b = sched_look(s, f);
+    const int32_t b = sched_look<THIN>(s, f);
     if (b != kNothing) return b;
     if (f.busy) {
       unsigned long long old = 0;
@@ -211,7 +220,7 @@ __device__ __forceinline__ int32_t sched_find(const Sched& s, Finder& f) {
     }
     if (since == 0) since = wall_clock64();
     else if (wall_clock64() - since > s.wait_limit) return kGaveUp;
-    __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_s_sleep(THIN ? 8 : 1);
   }
 }
 

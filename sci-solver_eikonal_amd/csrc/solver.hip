@@ -444,7 +444,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
   if (tid < 64) sched_enter(a.s, f, blockIdx.x);
   for (;;) {
     if (tid < 64) {
-      const int32_t nb = find_next(a.s, f, sAcc);
+      const int32_t nb = find_next<false>(a.s, f, sAcc);
       if (tid == 0) {
         sBlock = nb;
         sCrowd = f.others;

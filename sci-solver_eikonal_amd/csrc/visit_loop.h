@@ -87,11 +87,13 @@ inline int32_t loop_queue(int dim, int bt, int32_t max_local, int32_t max_elem, 
 // one sweep, whose times reach the dependents sooner.
 constexpr int kCrowd = 8;
 
-// One whole wave: the next block (look: or kNothing), with the time spent in the workgroup's tally.
+// One whole wave: the next block (look: or kNothing), with the time spent in the workgroup's tally.  THIN: see
+// sched_look.
+template <bool THIN>
 __device__ __forceinline__ int32_t find_next(const Sched& s, Finder& f, unsigned long long* acc,
                                              bool look = false) {
   const unsigned long long w0 = wall_clock64();
-  const int32_t b = look ? sched_look(s, f) : sched_find(s, f);
+  const int32_t b = look ? sched_look<THIN>(s, f) : sched_find<THIN>(s, f);
   if (__lane_id() == 0) {
     acc[6] += wall_clock64() - w0;
     if (b == kGaveUp) acc[kCntAbandoned] += 1;
@@ -192,7 +194,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
   int visit = 1;
   __syncthreads();
   if (finder) {
-    const int32_t nb = find_next(a.s, f, sh.acc);
+    const int32_t nb = find_next<false>(a.s, f, sh.acc);
     if (tid == 64) {
       sh.block = nb;
       sh.crowd = f.others;
@@ -364,7 +366,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
         }
       } else if (!again) {
         if (finder) {
-          const int32_t nb = a.s.per_owner > 1 ? find_next(a.s, f, sh.acc, true) : kNothing;
+          const int32_t nb = a.s.per_owner > 1 ? find_next<false>(a.s, f, sh.acc, true) : kNothing;
           if (tid == 64) {
             sh.block = nb;
             sh.crowd = f.others;
@@ -393,7 +395,7 @@ __device__ __forceinline__ int resident_loop(const LoopArgs& a, const Blocks& bl
       if (b == kNothing) {
         __syncthreads();
         if (finder) {
-          const int32_t nb = find_next(a.s, f, sh.acc);
+          const int32_t nb = find_next<false>(a.s, f, sh.acc);
           if (tid == 64) {
             sh.block = nb;
             sh.crowd = f.others;

@@ -69,6 +69,7 @@ struct Launch {
 };
 
 // One workgroup (one wave).
+template <bool THIN>
 int work(Launch& l) {
   const Sched& s = l.s;
   Finder f;
@@ -76,7 +77,7 @@ int work(Launch& l) {
   std::mt19937 own(blockIdx.x * 977u + 13u);  // the same in every lane
   int32_t b = kNothing;
   for (;;) {
-    if (b == kNothing) b = sched_find(s, f);
+    if (b == kNothing) b = sched_find<THIN>(s, f);
     if (b < 0) return b;
     const uint32_t slot = sched_slot(s, b);
     const auto& sup = l.g.sup[(size_t)b];
@@ -110,7 +111,7 @@ int work(Launch& l) {
       __builtin_amdgcn_wave_barrier();
       break;
     }
-    b = own() % 2 && s.per_owner > 1 ? sched_look(s, f) : kNothing;
+    b = own() % 2 && s.per_owner > 1 ? sched_look<THIN>(s, f) : kNothing;
   }
 }
 
@@ -142,7 +143,7 @@ int main(int argc, char** argv) {
       l.value[(size_t)s] = 0;
       l.words[sched_slot(l.s, s)] = 0ull;
     }
-    const char* err = simt::run((unsigned)groups, 64, rng(), 1 + (unsigned)rnd(groups), [&] { (void)work(l); });
+    const char* err = simt::run((unsigned)groups, 64, rng(), 1 + (unsigned)rnd(groups), [&] { (void)(i % 2 ? work<true>(l) : work<false>(l)); });
     int dirty = 0, wrong = 0;
     for (unsigned long long w : l.words) dirty += w != (unsigned long long)kClean;
     const std::vector<uint32_t> ref = shortest(l.g, seeds);
