@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <thread>
 
@@ -530,13 +531,16 @@ void solve_desc(SolveDesc& s, Mesh* m, float* T, float* seen, const float* rmult
   s.large = m->dim == 3 ? EIK_LARGENUM_3D : EIK_LARGENUM_2D;
 }
 
-// Numbers the blocks of each element kind over the launch's solves; n[0], n[1]: their numbers.
-static void launch_bases(SolveDesc* sd, int32_t nsolves, int64_t n[2]) {
+// Numbers the blocks of each element kind over the launch's solves; n[0], n[1]: their numbers, and of the
+// solves.
+static void launch_bases(SolveDesc* sd, int32_t nsolves, int64_t n[2], int32_t solves[2]) {
   n[0] = n[1] = 0;
+  solves[0] = solves[1] = 0;
   for (int32_t i = 0; i < nsolves; ++i) {
-    int64_t& k = n[sd[i].dim == 3 ? 0 : 1];
-    sd[i].kbase = (int32_t)k;
-    k += sd[i].nblocks;
+    const int kind = sd[i].dim == 3 ? 0 : 1;
+    sd[i].kbase = (int32_t)n[kind];
+    n[kind] += sd[i].nblocks;
+    ++solves[kind];
   }
 }
 
@@ -547,7 +551,8 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
   HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, L.device));
   // the blocks of each kind, numbered together
   int64_t kblocks[2];
-  launch_bases(L.hsolves, nsolves, kblocks);
+  int32_t ksolves[2];
+  launch_bases(L.hsolves, nsolves, kblocks, ksolves);
   for (int gi = 0; gi < 2; ++gi) {
     Group& g = L.grp[gi];
     std::memset(&a[gi], 0, sizeof(MultiArgs));
@@ -583,7 +588,15 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
     if (!g.present) continue;
     int rc;
     if (g.shape == 2) {
-      rc = resident_grid(res_launch(L, L.merged ? 3 : 1 << gi), o.workgroups, &g.grid);
+      const ResLaunch r = res_launch(L, L.merged ? 3 : 1 << gi);
+      rc = resident_grid(r, o.workgroups, &g.grid);
+      // More triangle blocks than workgroups of 256 threads: sized to the fronts, as in single solves
+      // (level-5 icosphere at 8 vertices per block 0.93 -> 0.36 ms, 4 of them 0.71 -> 0.59, 12 0.69; level 6
+      // at 32 0.96 -> 0.44, 2 0.90 -> 0.50; level 7 at 32 1.27 -> 0.95, 2 1.19 -> 1.15).
+      if (gi == 1 && !L.merged && r.bt == 256 && o.workgroups <= 0 && kblocks[1] > g.grid) {
+        const double front = 6.0 * std::sqrt((double)kblocks[1] * (double)ksolves[1]);
+        g.grid = (int)std::min<double>(g.grid, std::max<double>(ncu, front));
+      }
       // no more than one workgroup per block
       const int64_t most = L.merged ? 2 * std::max(kblocks[0], kblocks[1]) : kblocks[gi];
       g.grid = (int)std::min<int64_t>(g.grid, std::max<int64_t>(most, 1));
@@ -595,6 +608,8 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
                    : group_grid<2, kDirectThreads>(g.lds[1], o.workgroups, &g.grid, &g.wpe);
     }
     if (rc) return rc;
+    // (workgroups without a block of their own only poll: level-3 icosphere, 80 blocks, 0.31 -> 0.18 ms)
+    if (g.shape != 2) g.grid = (int)std::min<int64_t>(g.grid, std::max<int64_t>(kblocks[gi], 1));
     MultiArgs& x = a[gi];
     x.solves = L.dsolves;
     x.loop.s.word = g.words;
@@ -615,8 +630,6 @@ int launch_args(Launch& L, int32_t nsolves, int64_t total_blocks, const eik_solv
     x.queue_cap = g.queue_cap;
     x.rec_lds_bytes = g.shape == 0 ? g.rec_lds_bytes : 0;
   }
-    // (workgroups without a block of their own only poll: level-3 icosphere, 80 blocks, 0.31 -> 0.18 ms)
-    if (g.shape != 2) g.grid = (int)std::min<int64_t>(g.grid, std::max<int64_t>(kblocks[gi], 1));
   return EIK_OK;
 }
 
@@ -778,7 +791,8 @@ static int batch_alloc(Batch* b, int64_t seed_cap) {
     off += m->nv;
   }
   int64_t n[2];
-  launch_bases(b->L.hsolves, (int32_t)b->meshes.size(), n);
+  int32_t solves[2];
+  launch_bases(b->L.hsolves, (int32_t)b->meshes.size(), n, solves);
   HIP_TRY(hipMemcpy(b->L.dsolves, b->L.hsolves, sizeof(SolveDesc) * b->meshes.size(),
                     hipMemcpyHostToDevice));
   return EIK_OK;
