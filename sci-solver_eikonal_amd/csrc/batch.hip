@@ -861,7 +861,7 @@ static int batch_solve(Batch* b, const int64_t* seed_off, const int32_t* seeds,
     for (int64_t k = seed_off[i]; k < seed_off[i + 1]; ++k) {
       L.h_seed[k] = (int32_t)i;
       L.h_seed[cap + k] = seeds[k];
-      float v = seed_vals ? seed_vals[k] : 0.f;
+      float v = seed_vals ? seed_vals[k] + 0.f : 0.f;  // -0 counts as 0: the words order times
       std::memcpy(&L.h_seed[2 * cap + k], &v, 4);
     }
   L.h_seed[3 * cap] = (int32_t)nseeds;

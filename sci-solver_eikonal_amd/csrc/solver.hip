@@ -106,6 +106,11 @@ __device__ __forceinline__ void activate(const Active& next, int32_t it, bool mi
   if (add) next.list[base + __popcll(bal & lane_mask_lt())] = c;
 }
 
+// A source's time as the words order times: -0 counts as 0 (its own bits are the largest word).
+static __device__ __forceinline__ unsigned seed_key(const float* vals, int64_t i) {
+  return __float_as_uint(vals ? vals[i] + 0.f : 0.f);
+}
+
 // seeds: caller ids -> new ids; T = value; the owner block of each seed and its dependents are active
 // in iteration 1 (one workgroup per seed).
 __global__ void k_sync_seed(const int32_t* seeds, const float* vals, int64_t n, const int32_t* iperm,
@@ -114,7 +119,7 @@ __global__ void k_sync_seed(const int32_t* seeds, const float* vals, int64_t n, 
   for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
     const int32_t v = iperm[seeds[i]];
     if (threadIdx.x == 0)
-      atomicMin(reinterpret_cast<unsigned*>(&T[v]), __float_as_uint(vals ? vals[i] : 0.f));
+      atomicMin(reinterpret_cast<unsigned*>(&T[v]), seed_key(vals, i));
     const int32_t b = owner[v], s0 = dep_start[b], nd = dep_start[b + 1] - s0;
     for (int j0 = 0; j0 <= nd; j0 += 64) {
       const int j = j0 + (int)threadIdx.x;
@@ -418,10 +423,10 @@ __global__ void k_sched_seed(Sched s, const int32_t* seeds, const float* vals, i
     const int32_t v = iperm[seeds[i]];
     const int32_t b = owner[v];
     if (threadIdx.x == 0)
-      atomicMin(reinterpret_cast<unsigned*>(&T[v]), __float_as_uint(vals ? vals[i] : 0.f));
+      atomicMin(reinterpret_cast<unsigned*>(&T[v]), seed_key(vals, i));
     const int32_t s0 = dep_start[b], nd = dep_start[b + 1] - s0;
     for (int j = threadIdx.x; j <= nd; j += blockDim.x)
-      sched_mark(s, sched_slot(s, j == 0 ? b : dep[s0 + j - 1]), __float_as_uint(vals ? vals[i] : 0.f));
+      sched_mark(s, sched_slot(s, j == 0 ? b : dep[s0 + j - 1]), seed_key(vals, i));
   }
 }
 
