@@ -194,7 +194,10 @@ int build_layout(Mesh& m) {
   //    indices and the records; the halo lists are concatenated in block order
   const int nl = m.dim == 3 ? 6 : 3;
   std::vector<float> eL((size_t)ntot * nl), eH((size_t)ntot * k);
-  parallel_for(ntot, 4096, [&](int64_t e, int) {
+  struct alignas(64) Top { float h = 0.f; };  // a worker's largest finite height
+  const unsigned nworkers = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+  std::vector<Top> top(nworkers);
+  parallel_for(ntot, 4096, [&](int64_t e, int w) {
     const int32_t* c = elem_corners(e);
     float* Le = &eL[(size_t)e * nl];
     float* He = &eH[(size_t)e * k];
@@ -202,6 +205,8 @@ int build_layout(Mesh& m) {
       static const int pairs[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
       for (int p = 0; p < 6; ++p) Le[p] = (float)edge_len2(m, e, pairs[p][0], pairs[p][1]);
       tet_heights(Le, He);
+      for (int j = 0; j < 4; ++j)
+        if (He[j] > top[w].h && std::isfinite(He[j])) top[w].h = He[j];
     } else {
       const int64_t src = e < m.ne ? e : m.vorigin[e - m.ne];
       for (int p = 0; p < 3; ++p) Le[p] = (float)tri_edge_len2(m, src, c, p, (p + 1) % 3);
@@ -210,7 +215,7 @@ int build_layout(Mesh& m) {
   });
   if (m.dim == 3) {
     float most = 0.f;
-    for (float h : eH) most = std::isfinite(h) ? std::max(most, h) : most;
+    for (const Top& t : top) most = std::max(most, t.h);
     int x = 0;
     (void)std::frexp(most, &x);
     L.height_unit = height_unit(x);
@@ -221,7 +226,6 @@ int build_layout(Mesh& m) {
   L.rec_elem.resize(total);
   for (int64_t q = 0; q < total; ++q)
     L.rec_elem[q] = (int32_t)(elist[q] < m.ne ? elist[q] : m.vorigin[elist[q] - m.ne]);
-  const unsigned nworkers = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
   std::vector<std::vector<int32_t>> local(nworkers);  // new id -> local index in the block
   std::vector<std::vector<int32_t>> bhalo(nb);
   std::vector<int32_t> bad(nb, 0);  // 1: too many local vertices, 2: too many elements
@@ -238,7 +242,7 @@ int build_layout(Mesh& m) {
     d.pad = 0;
     std::vector<int32_t>& halo = bhalo[b];
     for (int32_t i = 0; i < d.nown; ++i) loc[d.vstart + i] = i;
-    int32_t nloc = d.nown;
+    int32_t nloc = d.nown, items = 0;
     for (int64_t q = eoff[b]; q < eoff[b + 1]; ++q) {
       const int64_t e = elist[q];
       const int32_t* c = elem_corners(e);
@@ -255,7 +259,7 @@ int build_layout(Mesh& m) {
         bad[b] = 1;
         break;
       }
-      for (int j = 0; j < (e < m.ne ? k : 1); ++j) L.items[b] += lv[j] < d.nown;
+      for (int j = 0; j < (e < m.ne ? k : 1); ++j) items += lv[j] < d.nown;
       const float* Le = &eL[(size_t)e * nl];
       const float* He = &eH[(size_t)e * k];
       if (m.dim == 3) {
@@ -272,6 +276,7 @@ int build_layout(Mesh& m) {
       }
     }
     d.nhalo = nloc - d.nown;
+    L.items[b] = items;
     if (!bad[b] && d.nelem > 16383) bad[b] = 2;
     // reset the map for the worker's next block
     for (int32_t i = 0; i < d.nown; ++i) loc[d.vstart + i] = -1;
