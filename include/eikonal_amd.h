@@ -36,7 +36,7 @@ extern "C" {
 #define EIK_ERR_CAPACITY 5 /* a block exceeds the kernel's local capacity */
 #define EIK_ERR_NOMEM 6    /* host or device allocation failed */
 #define EIK_ERR_TIMEOUT 7  /* async / batch / served solve: a workgroup waited longer than
-                              wait_limit_us for queued work and the queue never reached its end
+                              wait_limit_us for work and the solve never reached its end
                               (the result is incomplete; the device is left in a usable state) */
 
 #define EIK_LARGENUM_3D 1.0e9f
@@ -170,8 +170,8 @@ int eik_partition_labels(eik_mesh_t mesh, int32_t* labels_out);
 #define EIK_SCHED_SYNC 0   /* one launch per outer iteration */
 #define EIK_SCHED_ASYNC 1  /* one persistent launch with a device scheduler */
 
-/* Element records of a block visit: copied to LDS once per visit, or read from memory (L1/L2)
- * at every use with smaller workgroups, more of them per CU.  AUTO keeps a block's element data in
+/* Element records of a block visit: copied to LDS once per visit (LDS), or read from memory (L1/L2)
+ * at every use, with more workgroups per CU (MEMORY).  AUTO keeps a block's element data in
  * registers and LDS where the blocks fit (up to about 4,000 tets or 4,000 triangle corners a block);
  * else it stages the persistent single solve's and reads from memory in the
  * one-launch-per-iteration solve and in multi-solve launches, there also where a launch has so
@@ -196,7 +196,8 @@ typedef struct {
                               absolute 1e-5, CUDADefines.h:20) */
   int32_t record_history;  /* sync only: keep T after every outer iteration */
   int32_t workgroups;      /* async: persistent workgroups (0 = auto: one per block, at most all
-                              that fit) */
+                              that fit, or, of triangle blocks that take 256 threads, as many as the
+                              solve's fronts keep busy) */
   int32_t stage_records;   /* EIK_STAGE_*: where a block visit reads its element records */
   int32_t wait_limit_us;   /* async / batch / served: longest wait of a persistent workgroup
                               for work, in microseconds (0 = 10 s, the default; < 0 is
@@ -234,7 +235,7 @@ typedef struct {
   int64_t abandoned_waits; /* async / batch: waits for work that outlasted wait_limit_us (0 in a
                               healthy solve) */
   int64_t algo_bytes_loaded; /* algo_bytes without the element term of the re-runs whose element
-                                records were still staged in LDS from the visit before (they
+                                data was still in registers or LDS from the visit before (they
                                 read none from memory); equal to algo_bytes when records are
                                 read from memory at every use */
 } eik_solve_stats_t;
@@ -264,8 +265,8 @@ int eik_solve(eik_mesh_t mesh, const int32_t* seeds, int64_t nseeds, const float
  * the stream reaches the end of the work enqueued here.  stream: a hipStream_t, or NULL for the
  * mesh's stream.  Every call on a device shares that device's array: calls that overlap on one
  * device (different streams, or host threads) race and must be serialised by the caller.  The
- * call returns before the solve ends, so it reports no statistics and cannot report a queue
- * wait that outlasted the default wait limit (10 s; the result is then incomplete). */
+ * call returns before the solve ends, so it reports no statistics and cannot report a
+ * solve that did not reach its end within the default wait limit (10 s; the result is then incomplete). */
 int eik_solve_noalloc(eik_mesh_t mesh, const int32_t* seeds_dev, int64_t nseeds, float* T_out_dev,
                       void* stream);
 
@@ -335,8 +336,8 @@ typedef struct eik_batch* eik_batch_t;
  * threads; each mesh's device layout is uploaded (and stays usable by eik_solve).  The meshes
  * stay owned by the caller and must outlive the batch; re-partitioning a mesh invalidates the
  * batch.  A mesh may appear several times: every solve has its own time arrays and, with
- * eik_batch_set_factors, its own speed field.  EIK_ERR_CAPACITY if a block's times and work
- * queue do not fit the LDS; blocks whose element records do not fit it as well are solved with
+ * eik_batch_set_factors, its own speed field.  EIK_ERR_CAPACITY if a block's times and list
+ * of work do not fit the LDS; blocks whose element records do not fit it as well are solved with
  * the records read from memory (stage_records EIK_STAGE_LDS then fails with EIK_ERR_CAPACITY). */
 int eik_batch_create(const eik_mesh_t* meshes, int32_t n, eik_batch_t* out);
 int eik_batch_destroy(eik_batch_t batch);
